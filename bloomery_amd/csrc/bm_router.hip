@@ -43,6 +43,8 @@ __device__ unsigned long long g_router_timeline[kRouterTimelineRows * 8];
 #endif
 
 
+typedef float v4f __attribute__((ext_vector_type(4)));
+
 constexpr u32 kSiteRouter = 5; // crates/device/src/fault.rs:84-86
 
 // Sum / maximum over the wave, every lane ending with it: pairs, quads, eights and sixteens by data-parallel-primitive moves
@@ -414,7 +416,7 @@ __device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *ro
                 const float4 v = make_float4(__fmul_rn(__fmul_rn(scale, gv[j].x), xv[j].x), __fmul_rn(__fmul_rn(scale, gv[j].y), xv[j].y),
                                              __fmul_rn(__fmul_rn(scale, gv[j].z), xv[j].z), __fmul_rn(__fmul_rn(scale, gv[j].w), xv[j].w));
                 put4(xs, i, v);
-                if (normed_out && e0 == 0) reinterpret_cast<float4 *>(normed_out + (size_t)t * hidden)[i] = v;
+                if (normed_out && e0 <= 0) reinterpret_cast<float4 *>(normed_out + (size_t)t * hidden)[i] = v;
             }
         }
     } else {
@@ -439,7 +441,7 @@ __device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *ro
                 float *at = xs + (i & 7) * line + (i >> 3);
                 const float v = __fmul_rn(__fmul_rn(scale, gain[i]), *at); // written before the barrier above
                 *at = v;
-                if (normed_out && e0 == 0) normed_out[(size_t)t * hidden + i] = v;
+                if (normed_out && e0 <= 0) normed_out[(size_t)t * hidden + i] = v;
             }
         }
     }
@@ -454,7 +456,7 @@ __device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *ro
     // the dots)
     [[maybe_unused]] u32 *hand = nullptr;
     if constexpr (COH) hand = bm_global(bm_kernarg_at<u32 *>(offsetof(NormRouteArgs, late) + offsetof(NormRouteLate, hand)));
-    if (!gain && normed_out && e0 == 0) // the rows as they are (read after the barrier: other threads staged them)
+    if (!gain && normed_out && e0 <= 0) // the rows as they are (read after the barrier: other threads staged them)
         for (int i = tid; i < hidden; i += 256) normed_out[(size_t)t * hidden + i] = xs[(i & 7) * line + (i >> 3)];
     // every thread that stores a logit below is of the first wave: k_norm_route's hand-over (a device-scope count updated by
     // thread 0 behind the workgroup's barrier) publishes that wave's stores and relies on it
@@ -529,6 +531,27 @@ __global__ __launch_bounds__(256) void k_router_logits(const float *router, cons
     const int blocks_per_token = (n_exp + R - 1) / R;
     router_logits_body<R>(lds, router, x, gain, eps, n_exp, hidden, normed_out, logits, blockIdx.x / blocks_per_token,
                           (blockIdx.x % blocks_per_token) * R);
+}
+
+// A normed row as router_logits_body leaves it in LDS (value k at line k % 8, place k / 8) into column t of act_x.
+__device__ __forceinline__ void quant_normed_row(const float *xs, int hidden, int t, uint8_t *act_x, int q8k, u32 *fault, u32 layer) {
+    const int line = router_line(hidden), nb = hidden / 256, tid = threadIdx.x;
+    if (q8k) {
+        uint8_t *col = act_x + (size_t)t * nb * BM_Q8K_STRIDE;
+        for (int b = tid >> 6; b < nb; b += 4) { // a wave a 256-value block, four consecutive values a lane
+            const int k = 256 * b + 4 * (tid & 63);
+            const float *at = xs + (k & 7) * line + (k >> 3);
+            q8k_wave_block(make_float4(at[0], at[line], at[2 * line], at[3 * line]), col + (size_t)b * BM_Q8K_STRIDE, tid & 63, fault, layer);
+        }
+    } else {
+        uint8_t *col = act_x + (size_t)t * nb * BM_Q82_SB_EXT;
+        for (int k = 8 * tid; k < hidden; k += 2048) { // a quad of lanes a 32-value block, eight consecutive values a lane
+            float v8[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) v8[j] = xs[j * line + (k >> 3)];
+            q82_quad8(v8, col, nb, k >> 5, tid & 3, fault, layer);
+        }
+    }
 }
 
 // Norm, logits and routing in one launch (crates/gpu/src/route_softmax.rs:1667-1674 enqueue_norm_fused; the quantizer of
@@ -624,28 +647,179 @@ __global__ __launch_bounds__(256) void k_norm_route(const float *router, const f
         u32 *const fault = bm_global(late.fault);
         const u32 layer = late.layer;
         const int q8k = late.q8k;
-        const int line = router_line(hidden), nb = hidden / 256, tid = threadIdx.x;
-        const float *xs = reinterpret_cast<const float *>(lds); // value k at line k % 8, place k / 8
-        if (q8k) {
-            uint8_t *col = act_x + (size_t)tq * nb * BM_Q8K_STRIDE;
-            for (int b = tid >> 6; b < nb; b += 4) { // a wave a 256-value block, four consecutive values a lane
-                const int k = 256 * b + 4 * (tid & 63);
-                const float *at = xs + (k & 7) * line + (k >> 3);
-                q8k_wave_block(make_float4(at[0], at[line], at[2 * line], at[3 * line]), col + (size_t)b * BM_Q8K_STRIDE, tid & 63, fault, layer);
-            }
-        } else {
-            uint8_t *col = act_x + (size_t)tq * nb * BM_Q82_SB_EXT;
-            for (int k = 8 * tid; k < hidden; k += 2048) { // a quad of lanes a 32-value block, eight consecutive values a lane
-                float v8[8];
-#pragma unroll
-                for (int j = 0; j < 8; j++) v8[j] = xs[j * line + (k >> 3)];
-                q82_quad8(v8, col, nb, k >> 5, tid & 3, fault, layer);
-            }
-        }
+        quant_normed_row(reinterpret_cast<const float *>(lds), hidden, tq, act_x, q8k, fault, layer);
         return;
     }
     const u32 t = blockIdx.x / blocks_per_token;
     router_logits_body<R, true>(lds, router, x, gain, eps, n_exp, hidden, normed_out, logits, (int)t, (int)(blockIdx.x % blocks_per_token) * R);
+}
+
+// ---- many tokens
+
+// The norm of many tokens' rows, a workgroup a token: router_logits_body's row into normed_out and, with act_x, into the token's
+// quantized column.
+__global__ __launch_bounds__(256) void k_norm_rows(const float *x, const float *gain, float eps, int hidden, float *normed_out, uint8_t *act_x,
+                                                   int q8k, u32 *fault, u32 layer) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int t = (int)blockIdx.x;
+    router_logits_body<1>(lds, nullptr, x, gain, eps, 0, hidden, normed_out, nullptr, t, -1);
+    if (act_x) quant_normed_row(reinterpret_cast<const float *>(lds), hidden, t, act_x, q8k, fault, layer);
+}
+
+// The logits of many tokens' normed rows: tiles of tokens x experts on the matrix cores. v_mfma_f32_16x16x4_f32 runs four steps of
+// a 16 x 16 tile's multiply-add chains in increasing k, each with one rounding - fmaf's bits, subnormal values and signed zeros
+// included (checked over millions of values) - so accumulator l of a row dot is a chain of these instructions over its places,
+// and the logits are k_router_logits's bit for bit. Lane (row = lane % 16, s = lane / 16) of the instruction for accumulator l
+// holds value 8 (4 i + s) + l of its row, so over the eight accumulators a lane's operands are eight consecutive values. The chain
+// starts at -0 (a first product then keeps its own sign of zero, as the product that starts the CPU path's chain does), and
+// the places past a row's end hold -0 x 0.
+// A workgroup is four waves:
+//   SPLIT = 1: 16 tokens x 64 experts, a tile and its eight accumulators a wave;
+//   SPLIT = 4: the waves share one 16 x 16 tile, two accumulators each, which meet in LDS: a chain is then a quarter of the matrix
+//     instructions, the form for batches whose tiles would leave most of the card idle (it brings twice the bytes a value to LDS).
+// Both sides go through LDS in chunks of KC values a row, pieces of 16 bytes swizzled by the row's number so that sixteen rows at
+// one place fall on sixteen different bank groups. Three chunks: while chunk i is multiplied, chunk i + 1 is there already (so
+// operands are read a step ahead of their use, over the chunks' ends too), and chunk i + 2 goes in over chunk i - 1. The loads
+// (five chunks ahead), LDS stores and LDS reads stand one by one between the matrix instructions, in whose shadow they issue.
+// Without RAGGED the loop has no branch: a branch round an LDS store (for the padding of a last chunk) cost 55 ns a store, as
+// much as four matrix instructions, so rows that are whole groups of four chunks have a form of their own.
+// Bound: LDS traffic (16-byte reads and stores run at 64 to 80 bytes a cycle; a step of 32 values moves 26 KB a workgroup, 370 cycles,
+// against 256 of matrix instructions). Two tiles of experts a wave, which halve the reads of a matrix instruction, were no faster
+// (39.1 against 39.8 us at 4096 tokens: half the workgroups). Measured, with the norm's launch: 4096 tokens x 128 experts x 2048 values
+// 827 -> 40 us, 2048 tokens 416 -> 25, 333 tokens 71 -> 13.7, 64 tokens 16.7 -> 11.1; 1024 tokens x 256 experts x 7168 values
+// 2867 -> 64 us. The one-token workgroups of k_router_logits read and lay out the router's rows once a token.
+template <int SPLIT, int KC, bool RAGGED>
+__global__ __launch_bounds__(256) void k_router_tiles(const float *router, const float *x, int m, int n_exp, int hidden, float *logits) {
+    constexpr int kTok = 16, kExp = SPLIT == 1 ? 64 : 16, kAcc = 8 / SPLIT, kRows = kTok + kExp;
+    constexpr int kLine = KC / 4;                 // 16-byte pieces of a row's chunk
+    constexpr int kLoads = kRows * kLine / 256;   // pieces a thread brings in a chunk, of rows 256 / kLine apart,
+    constexpr int kTokLoads = kTok * kLine / 256; // the first of them pieces of tokens' rows
+    constexpr int kSteps = KC / 32, kSlots = kSteps * kAcc, kRing = 4;
+    static_assert(SPLIT == 1 || SPLIT == 4, "four waves: a tile each, or two accumulators of one tile each");
+    static_assert(kTok * kLine % 256 == 0 && kExp * kLine % 256 == 0 && KC % 64 == 0 && 256 % kLine == 0, "whole pieces a thread");
+    static_assert(2 * kLoads <= kSlots, "a slot of the chain for every load and every LDS store");
+    static_assert(kSteps % 2 == 0, "the two sets of operands alternate over whole chunks");
+    constexpr int kChunk = kRows * kLine;
+    extern __shared__ __align__(16) uint8_t lds[];
+    float4 *const s_buf = reinterpret_cast<float4 *>(lds); // three chunks: [kRows][kLine]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int exp_groups = (n_exp + kExp - 1) / kExp;
+    const int t0 = (int)(blockIdx.x / exp_groups) * kTok, e0 = (int)(blockIdx.x % exp_groups) * kExp;
+    const int chunks = (hidden + KC - 1) / KC, n4 = hidden / 4;
+    // what this thread brings of every chunk: piece `col` of rows row0, row0 + 256 / kLine, ..., tokens first
+    const int col = tid % kLine, row0 = tid / kLine;
+    const uint8_t *const x0 = reinterpret_cast<const uint8_t *>(x + (size_t)t0 * hidden);
+    const uint8_t *const w0 = reinterpret_cast<const uint8_t *>(router + (size_t)e0 * hidden);
+    u32 src[kLoads];
+    int dst[kLoads];
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) {
+        const int r = row0 + 256 / kLine * j;
+        const int in_tile = j < kTokLoads ? (t0 + r < m ? r : m - 1 - t0) : (e0 + r - kTok < n_exp ? r - kTok : n_exp - 1 - e0);
+        src[j] = (u32)in_tile * (u32)hidden * 4u + 16u * (u32)col;
+        dst[j] = r * kLine + (col ^ (r & 15));
+    }
+    // (places past a row's end, in the last chunk and behind it: the row's last piece, which park replaces)
+    const int past = col - (n4 - 1 - (chunks - 1) * kLine);
+    const u32 tail = past > 0 ? 16u * (u32)past : 0u;
+    float4 ring[kRing][kLoads];
+    auto fetch = [&](int i, int j, float4(&v)[kLoads]) {
+        const int c = i < chunks ? i : chunks - 1;
+        const u32 back = RAGGED && i >= chunks - 1 ? tail : 0u;
+        v[j] = *reinterpret_cast<const float4 *>((j < kTokLoads ? x0 : w0) + (size_t)c * (KC * 4) + (src[j] - back));
+    };
+    auto park = [&](int i, int j, int buf, const float4(&v)[kLoads]) { // a piece into LDS
+        float4 w = v[j];
+        if (RAGGED && (i >= chunks || (i == chunks - 1 && past > 0))) {
+            const float pad = j < kTokLoads ? -0.0f : 0.0f;
+            w = make_float4(pad, pad, pad, pad);
+        }
+        s_buf[buf + dst[j]] = w;
+    };
+#pragma unroll
+    for (int u = 0; u < kRing; u++)
+#pragma unroll
+        for (int j = 0; j < kLoads; j++) fetch(u, j, ring[u]);
+    const int l16 = lane & 15, ks = lane >> 4;
+    const int wexp = SPLIT == 1 ? 16 * wave : 0; // this wave's experts of the workgroup's
+    const int l0 = SPLIT == 1 ? 0 : kAcc * wave; // this wave's first accumulator
+    v4f acc[kAcc];
+#pragma unroll
+    for (int l = 0; l < kAcc; l++) acc[l] = v4f{-0.0f, -0.0f, -0.0f, -0.0f};
+    struct Step { // a lane's operands of 32 values: kAcc consecutive ones of its token's row and of its expert's row
+        float a[kAcc], b[kAcc];
+    };
+    // piece `part` of a step's operands, of kParts: values 8 (4 s + ks) + l0 .. of the lane's token row (first) and of its expert's
+    constexpr int kRowParts = kAcc == 2 ? 1 : 2, kParts = 2 * kRowParts;
+    static_assert(kParts <= kAcc, "a slot of the chain for every LDS read");
+    auto rd = [&](int buf, int s, int part, Step &st) {
+        const bool exp = part >= kRowParts;
+        const int j = part % kRowParts, r = exp ? kTok + wexp + l16 : l16;
+        float(&v)[kAcc] = exp ? st.b : st.a;
+        const float4 *row = s_buf + buf + r * kLine;
+        const int p = 8 * s + 2 * ks;
+        if constexpr (kAcc == 2) {
+            const float2 q = *reinterpret_cast<const float2 *>(reinterpret_cast<const float *>(row + ((p + (wave >> 1)) ^ (r & 15))) + 2 * (wave & 1));
+            v[0] = q.x, v[1] = q.y;
+        } else {
+            const float4 q = row[(p + j) ^ (r & 15)];
+            v[4 * j] = q.x, v[4 * j + 1] = q.y, v[4 * j + 2] = q.z, v[4 * j + 3] = q.w;
+        }
+    };
+    int now = 0, next = kChunk, over = 2 * kChunk; // the buffers of chunks i, i + 1, i + 2
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) park(0, j, now, ring[0]);
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) fetch(kRing, j, ring[0]);
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) park(1, j, next, ring[1]);
+    lds_barrier();
+    Step st[2];
+#pragma unroll
+    for (int r = 0; r < kParts; r++) rd(now, 0, r, st[0]);
+    for (int i = 0; i < chunks; i += kRing) {
+#pragma unroll
+        for (int u = 0; u < kRing; u++) {
+#pragma unroll
+            for (int s = 0; s < kSteps; s++) {
+#pragma unroll
+                for (int l = 0; l < kAcc; l++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    acc[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(st[s & 1].a[l], st[s & 1].b[l], acc[l], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (l < kParts) rd(s + 1 < kSteps ? now : next, (s + 1) % kSteps, l, st[(s + 1) & 1]);
+                    const int slot = s * kAcc + l;
+                    if (slot < kLoads) fetch(i + u + 1 + kRing, slot, ring[(u + 1) % kRing]);
+                    if (slot >= kSlots - kLoads) park(i + u + 2, slot - (kSlots - kLoads), over, ring[(u + 2) % kRing]);
+                }
+            }
+            lds_barrier();
+            const int done = now;
+            now = next, next = over, over = done;
+        }
+    }
+    // s_l = acc_l + acc_{l+4}, then (s_0 + s_2) + (s_1 + s_3); result v of a tile is token 4 ks + v against expert l16
+    if constexpr (SPLIT == 1) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const float s0 = __fadd_rn(acc[0][v], acc[4][v]), s1 = __fadd_rn(acc[1][v], acc[5][v]);
+            const float s2 = __fadd_rn(acc[2][v], acc[6][v]), s3 = __fadd_rn(acc[3][v], acc[7][v]);
+            const int t = t0 + 4 * ks + v, ex = e0 + wexp + l16;
+            if (t < m && ex < n_exp) logits[(size_t)t * n_exp + ex] = __fadd_rn(__fadd_rn(s0, s2), __fadd_rn(s1, s3));
+        }
+    } else {
+        __shared__ float s_acc[8][16][17];
+#pragma unroll
+        for (int l = 0; l < kAcc; l++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) s_acc[l0 + l][4 * ks + v][l16] = acc[l][v];
+        __syncthreads();
+        const int r = tid >> 4, c = tid & 15;
+        float s[4];
+#pragma unroll
+        for (int l = 0; l < 4; l++) s[l] = __fadd_rn(s_acc[l][r][c], s_acc[l + 4][r][c]);
+        if (t0 + r < m && e0 + c < n_exp) logits[(size_t)(t0 + r) * n_exp + e0 + c] = __fadd_rn(__fadd_rn(s[0], s[2]), __fadd_rn(s[1], s[3]));
+    }
 }
 
 // LDS of a workgroup of R rows: the token's row and the router rows, each as eight lines.
@@ -669,8 +843,40 @@ static int router_rows(int hidden, int m = 1 << 20, int n_exp = 1 << 20) {
 
 bool router_logits_fits(int hidden) { return router_rows(hidden) > 0; }
 
+// Whether the norm and the logits go as two launches, rows and then tiles: from ten million products on. Below that the one launch is
+// as short as the tiles' two (logits, one launch / two: 32 tokens x 128 experts x 2048 values 11.0 / 10.8 us, 16 tokens 6.3 / 10.7; 4 tokens x
+// 256 x 7168 13.8 / 25.1 us, 16 tokens 49.1 / 25.6). The tiles read normed rows from memory: a caller that wants none of them stays
+// with the one-token workgroups.
+static bool router_tiled(int m, int n_exp, int hidden, const float *gain, const float *normed_out) {
+    return (double)m * n_exp * hidden >= (double)(10 << 20) && (!gain || normed_out);
+}
+
+static hipError_t router_tiles(const Launch &L, const float *router, const float *x, const float *gain, float eps, int m, int n_exp,
+                               int hidden, float *normed_out, float *logits, uint8_t *act_x = nullptr, bool q8k = false) {
+    if (normed_out || act_x) {
+        const size_t lds = router_lds_bytes(0, hidden);
+        hipError_t e = allow_lds(k_norm_rows, lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_norm_rows, dim3((unsigned)m), dim3(256), lds, L.stream, x, gain, eps, hidden, normed_out, act_x, q8k ? 1 : 0, L.fault,
+                           L.layer);
+    }
+    auto launch = [&](auto kern, unsigned grid, unsigned rows, unsigned kc) {
+        const size_t lds = 3 * (size_t)rows * kc * sizeof(float);
+        hipError_t e = allow_lds(kern, lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, router, normed_out ? normed_out : x, m, n_exp, hidden, logits);
+        return hipGetLastError();
+    };
+    const unsigned t16 = (unsigned)((m + 15) / 16), e16 = (unsigned)((n_exp + 15) / 16), e64 = (e16 + 3) / 4;
+    // up to two split workgroups a compute unit (777 tokens x 128 experts: split 19.9, a tile a wave 24.0 us; 2048 tokens: 33.9 and 24.9)
+    if ((long)t16 * e16 <= 512)
+        return hidden % 512 ? launch(k_router_tiles<4, 128, true>, t16 * e16, 32, 128) : launch(k_router_tiles<4, 128, false>, t16 * e16, 32, 128);
+    return hidden % 256 ? launch(k_router_tiles<1, 64, true>, t16 * e64, 80, 64) : launch(k_router_tiles<1, 64, false>, t16 * e64, 80, 64);
+}
+
 hipError_t router_logits(const Launch &L, const float *router, const float *x, const float *gain, float eps, int m, int n_exp,
                          int hidden, float *normed_out, float *logits) {
+    if (router_tiled(m, n_exp, hidden, gain, normed_out)) return router_tiles(L, router, x, gain, eps, m, n_exp, hidden, normed_out, logits);
     const int rows = router_rows(hidden, m, n_exp);
     if (rows == 0) return hipErrorInvalidValue;
     const size_t lds = router_lds_bytes(rows, hidden);
@@ -696,6 +902,10 @@ hipError_t norm_route(const Launch &L, const float *router, const float *x, cons
     const int rows = router_rows(hidden, m, n_exp);
     if (rows == 0) return hipErrorInvalidValue;
     if (act_x && hidden % 256 != 0) return hipErrorInvalidValue;
+    if (router_tiled(m, n_exp, hidden, gain, normed_out)) {
+        const hipError_t e = router_tiles(L, router, x, gain, eps, m, n_exp, hidden, normed_out, logits, act_x, q8k);
+        return e != hipSuccess ? e : route_softmax(L, logits, m, n_exp, used, renorm, probs, ids, weights);
+    }
     const size_t lds = router_lds_bytes(rows, hidden);
     const unsigned grid = (unsigned)m * (unsigned)((n_exp + rows - 1) / rows) + (act_x ? (unsigned)m : 0u) + (unsigned)m;
 #define BM_NR(R, PER)                                                                                                  \

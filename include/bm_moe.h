@@ -437,7 +437,9 @@ int bm_router_logits(bm_ctx *ctx, const float *router_dev, const float *x_dev, c
  * hold an armed pattern between launches; its wait is bounded: BM_SITE_ROUTER and NaN weights if a logit never came) and
  * routes the token (after a wait that ran out: bm_fault_clear, which arms the words again, before the next call).
  * logits_dev is required; 1 .. 4096 tokens a launch. Launches of this entry that share a context must not
- * overlap (they share those words). */
+ * overlap (they share those words). From ten million products (tokens x experts x hidden) on, where normed_dev is given or
+ * gain_dev NULL, the call is three launches instead - the rows, the logits as tiles on the matrix cores, the routing - with the
+ * same bits in every output. */
 int bm_norm_route(bm_ctx *ctx, const float *router_dev, const float *x_dev, const float *gain_dev, float eps, int n_tokens,
                   int n_experts, int hidden, int top_k, int renorm, float *normed_dev, float *logits_dev, float *probs_dev,
                   uint32_t *ids_dev, float *weights_dev, bm_act *act_x);

@@ -290,6 +290,42 @@ def test_norm_route_is_the_two_launches_in_one(gpu, n_experts, hidden, m, top_k,
             b.free()
 
 
+@pytest.mark.parametrize("n_experts,hidden,m,with_gain", ((129, 2048, 49, True), (16, 2048, 330, False), (17, 2056, 400, True), (1000, 512, 33, True),
+                                                           (33, 520, 650, False), (130, 2048, 1100, True), (70, 2072, 2100, True), (65, 264, 4096, True)))
+def test_many_tokens_take_the_tiles_with_the_same_bits(gpu, n_experts, hidden, m, with_gain):
+    """Batches whose norm and logits go as rows and tiles (bm_router.hip, router_tiled): rows that are whole groups of chunks and
+    rows that are not, tiles cut off on both sides, the split and the whole form, rows of zeros and of one value among them;
+    normed rows and logits bit for bit against the oracle, routing and quantized columns as a launch of their own leaves them."""
+    rng = np.random.default_rng(1000 * n_experts + m)
+    router = normal_f32(rng, (n_experts, hidden), 0.05)
+    x = normal_f32(rng, (m, hidden)) * (10.0 ** rng.uniform(-2, 2, (m, 1))).astype(np.float32)
+    x[1] = 0.0
+    x[2, 1:] = 0.0
+    router[3, 8:] = -0.0
+    gain = (1.0 + normal_f32(rng, hidden, 0.2)).astype(np.float32) if with_gain else None
+    rd, xd = gpu.upload(router, np.float32), gpu.upload(x, np.float32)
+    gd = gpu.upload(gain, np.float32) if with_gain else None
+    top_k = min(8, n_experts)
+    normed, logits = gpu.buffer(np.float32, m * hidden).fill_bytes(0xFF), gpu.buffer(np.float32, m * n_experts).fill_bytes(0xFF)
+    ids, wts, ids2, wts2 = (gpu.buffer(t, m * top_k) for t in (np.uint32, np.float32, np.uint32, np.float32))
+    act = gpu.act(bm.Q4_K, hidden, m) if hidden % 256 == 0 else None
+    gpu.enqueue_norm_route(rd, xd, gd, 1e-6, m, n_experts, hidden, top_k, True, normed, logits, None, ids, wts, act_x=act)
+    want_n, want_l = ora.router_logits(router, x, gain, 1e-6)
+    assert_f32(normed.download(), want_n.reshape(-1), "normed rows")
+    assert np.array_equal(logits.download().view(np.uint32), want_l.reshape(-1).view(np.uint32)), "logits"
+    gpu.enqueue_route_softmax(logits, m, n_experts, top_k, True, None, ids2, wts2)
+    assert np.array_equal(ids.download(), ids2.download()) and np.array_equal(wts.download(), wts2.download())
+    if act is not None:
+        for t in (0, 1, m - 1):
+            assert np.array_equal(act.download(t), ora.quantize_col(bm.Q4_K, want_n.reshape(m, hidden)[t])), f"act_x column {t}"
+        act.free()
+    gpu.enqueue_router_logits(rd, xd, gd, 1e-6, m, n_experts, hidden, normed, logits.fill_bytes(0xFF))
+    assert np.array_equal(logits.download().view(np.uint32), want_l.reshape(-1).view(np.uint32)), "bm_router_logits"
+    for b in (rd, xd, gd, normed, logits, ids, wts, ids2, wts2):
+        if b is not None:
+            b.free()
+
+
 @pytest.mark.parametrize("n_experts,top_k", ((128, 8), (200, 6), (40, 4), (300, 8)))
 def test_norm_route_picks_among_equal_probabilities(gpu, n_experts, top_k):
     """Router rows that repeat give logits that are equal bit for bit: the fused launch's picks (by counting, for up to 256
