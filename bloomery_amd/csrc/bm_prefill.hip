@@ -1,4 +1,4 @@
-// Prefill: the grouped expert GEMM over a route table, on the int8 matrix cores, and the SwiGLU quantizer between
+// Prefill: the grouped expert GEMM over a route table, on the matrix cores, and the SwiGLU quantizer between
 // a gate/up pair and its down (crates/gpu/src/gemm/mod.rs:1-50).
 //
 // The route table is the reference's (crates/gpu/src/gemm/route.rs:1-60,109-125): `cols` lists the slots grouped by
@@ -7,13 +7,9 @@
 // refused count}.
 //
 // The GEMM's numbers are the decode path's, bit for bit: every (row, slot) value is the one-column row dot of
-// bm_device.hpp. The integer sums of each 16-value group come out of v_mfma_i32_16x16x32_i8 (16 rows x 16 slots,
-// exact; the other half of the 32 values zeroed on the weight side), and each enters the f32 accumulator of the CPU path's lane that
-// owns it, in the CPU path's order (crates/qdot/src/lib.rs:4363-4447 Q4_K, :4776-4874 Q6_K): eight accumulators a
+// bm_device.hpp. The integer sums of each 16-value group come out of the matrix cores exactly, and each enters the f32 accumulator
+// of the CPU path's lane that owns it, in the CPU path's order (crates/qdot/src/lib.rs:4363-4447 Q4_K, :4776-4874 Q6_K): eight accumulators a
 // value, the min term first, then the groups in increasing k, and the closing sum (t0 + t2) + (t1 + t3).
-// Activation scales come per 32 values in this form, so every group's sum is scaled on the vector ALU before it is
-// added: three operations a (row, slot, group) against one matrix instruction per 1024 of them. The kernel is bound
-// by that arithmetic, not by the matrix cores.
 #include <type_traits>
 
 #include "bm_gemm.hpp"
@@ -197,11 +193,6 @@ hipError_t swiglu_quant(const Launch &L, const float *g, const float *u, int m, 
 
 // ------------------------------------------------------------------------------------------------- GEMM
 
-// LDS of one workgroup: a super-block of the tile's 64 activation columns and of the slab's 64 weight rows, and the
-// rows' scale products. Strides are padded off the 128-byte bank period.
-constexpr int kActSb = BM_Q82_SB_REF + 64;   // a column's super-block: its two groups and its (d8, d8 * isum) pairs
-constexpr int kActStride = kActSb + 8;       // 360
-
 // (q6 - 32) of four codes a word, as signed bytes: q6 in 0..63.
 __device__ __forceinline__ u32 q6_minus_32(u32 q) {
     const u32 t = q ^ 0x20202020u;        // q >= 32: q - 32; q < 32: q + 32
@@ -209,318 +200,349 @@ __device__ __forceinline__ u32 q6_minus_32(u32 q) {
     return t | (m << 1) | (m << 2);
 }
 
-// LDS of the exact kernel, two buffers of: the part's activation columns (a super-block each), the slab's 64 weight
-// rows unpacked to a signed byte a code (Q4_K 0..15, Q6_K q6 - 32), so the arithmetic reads matrix operands as they
-// are, and the rows' 16 x 64 scale products. A page of zeros stands in for the half of an operand that must not count.
-// Strides: an operand read is 8 bytes a lane, served sixteen lanes at a time, the sixteen a wave's rows (or slots) at
-// one piece of a block: a stride of 8 x an odd number puts them on sixteen different bank pairs (rows 8 x 33, columns
-// 8 x 45). Strides of 16-byte multiples, which would let the staging store 16 bytes a lane, measured slower: the reads
-// then collide in pairs.
-constexpr int kRowStride = 256 + 8;
-constexpr int kColStride = kActStride; // 360
-constexpr int kRsStride = 68; // floats a row of the 16 x 64 scale products
-constexpr int kZeroPage = 256;
-__host__ __device__ constexpr size_t gemm_exact_buf_bytes(int slots) {
-    return (size_t)slots * kColStride + (size_t)kGemmBM * kRowStride + 16 * kRsStride * sizeof(float);
+// The exact form's LDS, half a super-block (128 values) at a time, twice: the slab's 64 weight rows and the tile's 64 columns as
+// f16 codes, 264 bytes a row (8 x an odd number: sixteen lanes of a wave read sixteen rows at one place, eight bytes each, from
+// sixteen different bank pairs), and the f32 factors, a line of 64 rows (or slots) each.
+constexpr int kXStride = 2 * 128 + 8;
+constexpr int kXCodes = 64 * kXStride; // rows of half 0, rows of half 1, columns of half 0, columns of half 1, the factors
+constexpr int kXLine = 80 * 4;         // bytes: the staging's sixteen rows of four lines land on different banks
+template <int WT>
+struct XLds {
+    static constexpr bool kMins = WT != BM_Q6K;
+    static constexpr int kScales = kMins ? 4 : 8;           // lines of scale products a half
+    static constexpr int kHalf = (kScales + 4) * kXLine;    // a half's factors: the scale products, and four lines of d8
+    static constexpr int kMinsAt = 2 * kHalf;               // and a super-block's: eight lines of mins, eight of d8 isum
+    static constexpr int kFactors = kMinsAt + (kMins ? 16 * kXLine : 0);
+    static constexpr size_t kBytes = 4 * (size_t)kXCodes + kFactors + sizeof(GemmLds);
+};
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef u32 v2u __attribute__((ext_vector_type(2)));
+typedef u32 v4u __attribute__((ext_vector_type(4)));
+
+// Two small integers given as f16 bit patterns 1024 + n, less `bias`: exact.
+__device__ __forceinline__ u32 h2_less(u32 x, float bias) {
+    const _Float16 b = (_Float16)bias;
+    return __builtin_bit_cast(u32, __builtin_bit_cast(v2h, x) - (v2h){b, b});
 }
-__host__ __device__ constexpr size_t gemm_exact_lds_bytes(int slots) {
-    return sizeof(GemmLds) + kZeroPage + 2 * gemm_exact_buf_bytes(slots);
+// The same of 1024 + 16 n: n - off.
+__device__ __forceinline__ u32 h2_16th(u32 x, float off) {
+    const _Float16 s = (_Float16)0.0625f, b = (_Float16)(-64.0f - off);
+    return __builtin_bit_cast(u32, __builtin_elementwise_fma(__builtin_bit_cast(v2h, x), (v2h){s, s}, (v2h){b, b}));
 }
 
-// Byte j (0..11) of the twelve scale bytes a Q4_K block holds after d and dmin, the bytes given as three words.
-__device__ __forceinline__ u32 q4k_scale_byte(u32 y, u32 z, u32 w, int j) {
-    const unsigned long long yz = ((unsigned long long)z << 32) | y;
-    const u32 a = (u32)(yz >> ((8 * j) & 63)), b = w >> ((8 * j) & 31);
-    return (j < 8 ? a : b) & 0xffu;
+// (x & mask) | bits in one instruction; from the plain expression the compiler makes two or three.
+__device__ __forceinline__ u32 and_or(u32 x, u32 mask, u32 bits) {
+    u32 r;
+    __asm__("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(bits));
+    return r;
 }
 
-// A workgroup of 4 CH waves takes 16 T CH slots of a tile (all 64, or a part of it: a tile's parts are workgroups of
-// their own) and a slab of 64 rows. Wave w works on rows 16 * (w & 3) .. and slots 16 T * (w >> 2) ..: T 16 x 16
-// products a 16-value group. v_mfma_i32_16x16x32_i8 sums over 32 values, lane / 16 = k / 8; a 16-value half comes out
-// of it when the lanes of the other half hand in zeros: those lanes read their weight operand from the zero page (an
-// address picked once, no instruction a product). 4 T results a lane, 32 T accumulators.
-// The next super-block is loaded to registers before the arithmetic on the present one and stored to the other
-// buffer after it: one barrier a super-block. Parts of 32 slots put two workgroups on a CU, and one's loads, LDS
-// stores and barrier then run under the other's arithmetic.
-template <int WT, int T, int CH>
-__global__ __launch_bounds__(256 * CH) void k_gemm(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
+// A workgroup of four waves takes a slab of 64 rows and a tile's 64 slots, a wave 32 x 32 of them.
+// Per (row, slot, 16-value group) the contract is acc[l] = fma(fl(scale d8), sum, acc[l]) over eight accumulators, one fused
+// multiply-add that only the vector ALU can do. The rest is on the matrix cores: the group's integer sum comes out of
+// v_mfma_f32_32x32x16_f16 as a float (codes of at most eight bits, sums below 2^24: exact, where an int8 product needs a
+// conversion a sum), fl(scale d8) over the tile is the outer product v_mfma_f32_32x32x1_2b_f32 (two blocks, or Q6_K's two
+// groups, an instruction; a product plus zero is the product's rounding), and a min term fma(d8 isum, min, acc) is the same
+// instruction with the accumulators as its addend.
+// Bound by the vector ALU (the f32 matrix instructions run on it too, 64 cycles each; the f16 ones beside it): 32 multiply-adds a
+// wave and 32 x 32 x 32 values, 16 multiply-adds' worth of outer products and about 30 instructions of staging, 300 of the 490
+// cycles measured. The staging of a half (bytes to f16, the factors) is cut in eight pieces between the groups of the half before
+// it, each behind the group's matrix instruction, and its bytes are asked for a whole half ahead: one barrier a half, no wait in
+// front of it. 78 KB: two workgroups a CU. 16384 slots of 128 experts, 768 rows of 2048 values Q4_K: 315 -> 225 us; 2048 rows of
+// 768 Q6_K: 378 -> 300 us, against int8 products with the scaling, the conversion and the mins on the vector ALU.
+template <int WT>
+__global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
                                                  const u32 *tiles, const u32 *n_tiles, u32 n_units, u32 slot_div,
-                                                 u32 n_slots, float *y) {
-    constexpr int kSlots = 16 * T * CH, kParts = kGemmBN / kSlots, kThreads = 256 * CH;
-    static_assert(kThreads == 8 * kGemmBM, "a thread a (row, eighth of the row's codes)");
-    constexpr size_t kBuf = gemm_exact_buf_bytes(kSlots);
-    constexpr int kWtsAt = kSlots * kColStride, kRsAt = kWtsAt + kGemmBM * kRowStride;
+                                                 u32 n_slots, float *y, u32 slabs) {
+    using X = XLds<WT>;
     extern __shared__ __align__(16) uint8_t lds[];
-    GemmLds *tab = reinterpret_cast<GemmLds *>(lds);
-    uint8_t *zeros = lds + sizeof(GemmLds);
-    uint8_t *buf0 = zeros + kZeroPage;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const u32 g = tile_of_block(blockIdx.x, n_units); // a unit: a row slab and a part of the tile
-    const u32 unit = slab_of_block(blockIdx.x, n_units);
-    const int row0 = (int)(unit / kParts) * kGemmBM, part0 = (int)(unit % kParts) * kSlots;
+    GemmLds *tab = reinterpret_cast<GemmLds *>(lds + 4 * kXCodes + X::kFactors);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const u32 g = tile_of_block(blockIdx.x, n_units);
+    int row0 = (int)(slab_of_block(blockIdx.x, n_units) * slabs) * kGemmBM; // of the slabs a workgroup takes one after the other
     const u32 count = n_tiles[0];
     if (g > count) return;
     if (g == count) { // the refused slots' rows: NaN (crates/gpu/src/gemm/grouped.rs:2283-2287)
-        const u32 refused = part0 == 0 ? n_tiles[1] : 0u;
-        for (u32 i = tid; i < refused * kGemmBM; i += blockDim.x) {
-            const u32 s = cols[n_slots - n_tiles[2] - refused + i / kGemmBM];
-            const int r = row0 + (int)(i % kGemmBM);
+        const u32 refused = n_tiles[1];
+        const u32 rows = slabs * kGemmBM;
+        for (u32 i = tid; i < refused * rows; i += 256) {
+            const u32 s = cols[n_slots - n_tiles[2] - refused + i / rows];
+            const int r = row0 + (int)(i % rows);
             if (r < rpe) y[(size_t)s * rpe + r] = bm_bits_f32(0x7fc00000u);
         }
         return;
     }
     const u32 e = tiles[2 * g], word = tiles[2 * g + 1];
-    const int start = (int)(word & 0xffffu) + part0, len = (int)(word >> 16) - part0;
-    if (len <= 0) return; // the tile ends before this part
-    if (tid < kSlots) {
+    const int start = (int)(word & 0xffffu), len = (int)(word >> 16);
+    if (tid < kGemmBN) {
         const u32 s = cols[start + (tid < len ? tid : 0)];
         tab->slot[tid] = s;
         tab->col[tid] = s / slot_div;
     }
-    if (tid < kZeroPage / 4) reinterpret_cast<u32 *>(zeros)[tid] = 0u;
     __syncthreads();
     constexpr int kBlock = bm_block_bytes<WT>();
-    constexpr bool kQ45 = WT == BM_Q4K || WT == BM_Q5K; // one walk: Q5_K is Q4_K with a fifth bit a code
-    constexpr int kCodesAt = WT == BM_Q5K ? 48 : 16;    // where a Q4_K / Q5_K block's nibbles start
+    constexpr bool kQ45 = X::kMins;                  // one walk: Q5_K is Q4_K with a fifth bit a code
+    constexpr int kCodesAt = WT == BM_Q5K ? 48 : 16; // where a Q4_K / Q5_K block's nibbles start
     const u32 row_bytes = (u32)nb * kBlock, col_bytes = (u32)nb * BM_Q82_SB_EXT;
 
-    // What a thread stages of every super-block: kActLoads 16-byte chunks of the activations (a column's super-block
-    // is 18 chunks of codes and 4 of (d8, d8 * isum) pairs), 16 code bytes of row tid / 8 (Q6_K: with the 16 bytes of
-    // high bits that go with them), and two of that row's sixteen scale products. The sources are fixed but for the
-    // super-block's offset: 32-bit offsets from the activations and from the expert's rows.
-    constexpr int kAc = kActSb / 16; // 22
-    constexpr int kActLoads = (kSlots * kAc + kThreads - 1) / kThreads;
-    u32 src_a[kActLoads], step_a[kActLoads]; // a chunk's offset in super-block 0 and its step a super-block
-    int dst_a[kActLoads];
-#pragma unroll
-    for (int t = 0; t < kActLoads; t++) {
-        int c = t * kThreads + tid;
-        c = c < kSlots * kAc ? c : kSlots * kAc - 1;
-        const int n = c / kAc, k = c % kAc;
-        const u32 colp = tab->col[n] * col_bytes;
-        // chunk k < 18: the codes, a step of 288 a super-block; else the pairs behind all the codes, a step of 64
-        src_a[t] = k < 18 ? colp + 16 * k : colp + (u32)nb * BM_Q82_SB_REF + 16 * (k - 18);
-        step_a[t] = k < 18 ? BM_Q82_SB_REF : 64;
-        dst_a[t] = n * kColStride + 16 * k;
-    }
+    // What a thread stages of every half: of row tid / 4 the sixteen code bytes 16 p .. of the half's 64 (p = tid % 4: low
+    // nibbles one 16-value group, high nibbles another), of column tid / 4 the codes 16 p .. and 64 + 16 p .., and of both
+    // the factors of the half's block p.
+    const int wr = tid >> 2, p = tid & 3;
     const uint8_t *we = w + (size_t)e * rpe * row_bytes;
-    const int wr = tid >> 3, pc = tid & 7; // the row and the eighth of its codes
-    const u32 src_w = (u32)(row0 + wr < rpe ? row0 + wr : rpe - 1) * row_bytes;
-    uint4 ra[kActLoads], rw, rqh, rhd = make_uint4(0, 0, 0, 0);
-    auto fetch = [&](int i) {
-#pragma unroll
-        for (int t = 0; t < kActLoads; t++) ra[t] = *reinterpret_cast<const uint4 *>(act + (src_a[t] + (u32)i * step_a[t]));
-        const uint8_t *blk = we + (src_w + (u32)i * kBlock);
+    auto row_at = [&](int first_row) { return (u32)(first_row + wr < rpe ? first_row + wr : rpe - 1) * row_bytes; };
+    const u32 acol = tab->col[wr] * col_bytes + 16 + 16 * p, apair = acol + (u32)nb * BM_Q82_SB_REF - 16 - 8 * p;
+    v4u rw, rq = {0, 0, 0, 0}, rh = {0, 0, 0, 0}, ra[2] = {};
+    float d8, y0 = 0.0f, y4 = 0.0f;
+    auto ld16 = [](const uint8_t *at) {
+        v4u v;
+        __builtin_memcpy(&v, at, 16);
+        return v;
+    };
+    struct At { // a super-block: of which row, and which
+        u32 row; // the row's offset in the expert's rows
+        int i;
+    };
+    auto fetch_row = [&](At at, auto half) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
+        const uint8_t *blk = we + (at.row + (u32)at.i * kBlock);
         if constexpr (kQ45) {
-            rw = *reinterpret_cast<const uint4 *>(blk + kCodesAt + 16 * pc);
-            if (pc == 0) rhd = *reinterpret_cast<const uint4 *>(blk); // d, dmin, the twelve scale bytes
-            // Q5_K: value n's fifth bit is bit n / 32 of high byte n % 32 (crates/gguf/src/quant.rs:769-816); these
-            // code bytes hold values 64 (pc / 2) + 16 (pc % 2) .. and the values 32 on
-            if constexpr (WT == BM_Q5K) rqh = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * (pc & 1));
-        } else { // half pc / 4: its ql bytes 16 (pc % 4) .. and the qh bytes that go with them
-            rw = bm_ld16u(blk + 64 * (pc >> 2) + 16 * (pc & 3));
-            rqh = bm_ld16u(blk + 128 + 32 * (pc >> 2) + 16 * (pc & 1));
-            rhd.x = bm_ld2u(blk + 208);          // d
-            rhd.y = bm_ld2u(blk + 192 + 2 * pc); // scales 2 pc, 2 pc + 1
+            rw = ld16(blk + kCodesAt + 64 * j + 16 * p);
+            // Q5_K: value n's fifth bit is bit n / 32 of high byte n % 32 (crates/gguf/src/quant.rs:769-816)
+            if constexpr (WT == BM_Q5K) rq = ld16(blk + 16 + 16 * (p & 1));
+        } else { // Q6_K: ql bytes 64 j + 16 p .. and the qh bytes that go with them
+            rw = ld16(blk + 64 * j + 16 * p);
+            rq = ld16(blk + 128 + 32 * j + 16 * (p & 1));
         }
     };
-    auto put16 = [](uint8_t *dst, u32 a, u32 b, u32 c, u32 d) {
-        *reinterpret_cast<uint2 *>(dst) = make_uint2(a, b);
-        *reinterpret_cast<uint2 *>(dst + 8) = make_uint2(c, d);
+    auto fetch_col = [&](int i, auto half, int q) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
+        ra[q] = ld16(act + (acol + (u32)(2 * i + j) * BM_Q82X4_STRIDE) + 64 * q);
     };
-    auto stash = [&](uint8_t *buf) {
+    const u32 k1024 = 0x64006400u, m4l = 0x000f000fu, m4h = 0x00f000f0u, m8 = 0x00ff00ffu, mx = WT == BM_Q5K ? 0x00100010u : 0x00300030u,
+              my = WT == BM_Q5K ? 0x01000100u : 0x03000300u;
+    // (explicit LDS addresses: a base a lane and constants; the reads volatile, so that eight-byte reads stay eight bytes: merged
+    // into sixteen they run at half the rate)
+    typedef __attribute__((address_space(3))) uint8_t *LdsB;
+    typedef __attribute__((address_space(3))) float *LdsF;
+    typedef const volatile __attribute__((address_space(3))) v2u *LdsV2;
+    typedef const volatile __attribute__((address_space(3))) float *LdsVF;
+    const LdsB my_put = (LdsB)lds + wr * kXStride + 32 * p, my_factor = (LdsB)lds + 4 * kXCodes + 4 * wr + kXLine * p;
+    auto put = [&](int at, u32 a, u32 b) { *(__attribute__((address_space(3))) v2u *)(my_put + at) = (v2u){a, b}; };
+    auto factor = [&](int at, float v) { *(LdsF)(my_factor + at) = v; };
+    // Word k of the sixteen code bytes of the row. Four codes a word become f16 in the order 0, 2, 1, 3 (rows and columns alike: a
+    // sum's terms may come in any order). Low nibbles: group p of the buffer's first four; high nibbles: of its second four (Q6_K:
+    // the values' own order).
+    auto stash_row = [&](auto half, int k) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
+        const u32 x = rw[k], x8 = x >> 8;
+        u32 l0 = and_or(x, m4l, k1024), l1 = and_or(x8, m4l, k1024), h0 = and_or(x, m4h, k1024), h1 = and_or(x8, m4h, k1024);
+        if constexpr (WT == BM_Q5K) { // the fifth bits of blocks 4 j + 2 (p / 2) and the one after
+            const u32 t = rq[k] >> (4 * j + 2 * (p >> 1));
+            l0 = and_or(t << 4, mx, l0);
+            l1 = and_or(t >> 4, mx, l1);
+            h0 = and_or(t << 7, my, h0);
+            h1 = and_or(t >> 1, my, h1);
+        }
+        if constexpr (WT == BM_Q6K) { // the two high bits of quarters p / 2 and p / 2 + 2
+            const u32 t = rq[k] >> (2 * (p >> 1)), t4 = t << 4, t8 = t >> 4;
+            l0 = and_or(t4, mx, l0);
+            l1 = and_or(t8, mx, l1);
+            h0 = and_or(t4, my, h0);
+            h1 = and_or(t8, my, h1);
+        }
+        constexpr float kOff = kQ45 ? 0.0f : 32.0f;
+        put(j * kXCodes + 8 * k, h2_less(l0, 1024.0f + kOff), h2_less(l1, 1024.0f + kOff));
+        put(j * kXCodes + 128 + 8 * k, h2_16th(h0, kOff), h2_16th(h1, kOff));
+    };
+    // Words 2 h and 2 h + 1 of the column's sixteen codes q.
+    auto stash_col = [&](auto half, int q, int h) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
 #pragma unroll
-        for (int t = 0; t < kActLoads; t++)
-            if (t * kThreads + tid < kSlots * kAc) put16(buf + dst_a[t], ra[t].x, ra[t].y, ra[t].z, ra[t].w);
-        const u32 ml = 0x0f0f0f0fu;
-        uint8_t *codes = buf + kWtsAt + wr * kRowStride;
-        float *rs = reinterpret_cast<float *>(buf + kRsAt); // [16][kRsStride]
+        for (int k = 2 * h; k < 2 * h + 2; k++) {
+            const u32 u = ra[q][k] ^ 0x80808080u;
+            put((2 + j) * kXCodes + 128 * q + 8 * k, h2_less(and_or(u, m8, k1024), 1152.0f), h2_less(and_or(u >> 8, m8, k1024), 1152.0f));
+        }
+    };
+    float r4 = 0.0f; // Q4_K, Q5_K: the scale product of block 4 + p, kept for the second half
+    auto stash_factors = [&](auto half) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
+        if constexpr (kQ45 && j == 0) { // crates/gguf/src/quant.rs:620-628 get_scale_min_k4
+            const float d = bm_half_to_f32((unsigned short)(rh.x & 0xffffu)), dmin = bm_half_to_f32((unsigned short)(rh.x >> 16));
+            const u32 b0 = (rh.y >> (8 * p)) & 0xffu, b4 = (rh.z >> (8 * p)) & 0xffu, b8 = (rh.w >> (8 * p)) & 0xffu;
+            factor(0, d * (float)(b0 & 63u));
+            r4 = d * (float)((b8 & 15u) | ((b0 >> 6) << 4));
+            factor(X::kMinsAt, -(dmin * (float)(b4 & 63u)));
+            factor(X::kMinsAt + 4 * kXLine, -(dmin * (float)((b8 >> 4) | ((b4 >> 6) << 4))));
+            factor(X::kMinsAt + 8 * kXLine, y0);
+            factor(X::kMinsAt + 12 * kXLine, y4);
+        } else if constexpr (kQ45) {
+            factor(X::kHalf, r4);
+        } else { // groups p and 4 + p of the half
+            const float d = bm_half_to_f32((unsigned short)rh.x);
+            factor(j * X::kHalf, d * (float)(int)(signed char)(rh.y & 0xffu));
+            factor(j * X::kHalf + 4 * kXLine, d * (float)(int)(signed char)(rh.z & 0xffu));
+        }
+        factor(j * X::kHalf + X::kScales * kXLine, d8);
+    };
+    auto fetch_factors = [&](At at, auto half) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
+        const uint8_t *blk = we + (at.row + (u32)at.i * kBlock);
         if constexpr (kQ45) {
-            // code bytes 16 pc ..: values 64 (pc / 2) + 16 (pc % 2) .. (low nibbles) and 32 on (high nibbles)
-            uint8_t *dst = codes + 64 * (pc >> 1) + 16 * (pc & 1);
-            if constexpr (WT == BM_Q5K) {
-                const u32 one = 0x01010101u;
-                const int s0 = 2 * (pc >> 1), s1 = s0 + 1; // the sub-blocks of the low and of the high nibbles
-                put16(dst, (rw.x & ml) | (((rqh.x >> s0) & one) << 4), (rw.y & ml) | (((rqh.y >> s0) & one) << 4),
-                      (rw.z & ml) | (((rqh.z >> s0) & one) << 4), (rw.w & ml) | (((rqh.w >> s0) & one) << 4));
-                put16(dst + 32, ((rw.x >> 4) & ml) | (((rqh.x >> s1) & one) << 4), ((rw.y >> 4) & ml) | (((rqh.y >> s1) & one) << 4),
-                      ((rw.z >> 4) & ml) | (((rqh.z >> s1) & one) << 4), ((rw.w >> 4) & ml) | (((rqh.w >> s1) & one) << 4));
-            } else {
-                put16(dst, rw.x & ml, rw.y & ml, rw.z & ml, rw.w & ml);
-                put16(dst + 32, (rw.x >> 4) & ml, (rw.y >> 4) & ml, (rw.z >> 4) & ml, (rw.w >> 4) & ml);
-            }
-            // the row's header from the lane that read it; scale and min of sub-block pc
-            // (crates/gguf/src/quant.rs:620-628 get_scale_min_k4)
-            const int from = 4 * (lane & ~7);
-            const u32 h0 = (u32)__builtin_amdgcn_ds_bpermute(from, (int)rhd.x), h1 = (u32)__builtin_amdgcn_ds_bpermute(from, (int)rhd.y),
-                      h2 = (u32)__builtin_amdgcn_ds_bpermute(from, (int)rhd.z), h3 = (u32)__builtin_amdgcn_ds_bpermute(from, (int)rhd.w);
-            const float d = bm_half_to_f32((unsigned short)(h0 & 0xffffu));
-            const float dmin = bm_half_to_f32((unsigned short)(h0 >> 16));
-            const u32 lo = q4k_scale_byte(h1, h2, h3, pc < 4 ? pc : pc + 4);     // pc < 4: sc[pc]; else sc[pc + 4]
-            const u32 b4 = q4k_scale_byte(h1, h2, h3, pc < 4 ? pc + 4 : pc - 4); // pc < 4: sc[pc + 4]; else sc[pc - 4]
-            const u32 b0 = q4k_scale_byte(h1, h2, h3, pc);                       // sc[pc]
-            const u32 scv = pc < 4 ? (lo & 63u) : ((lo & 15u) | ((b4 >> 6) << 4));
-            const u32 mv = pc < 4 ? (b4 & 63u) : ((lo >> 4) | ((b0 >> 6) << 4));
-            rs[pc * kRsStride + wr] = d * (float)scv;
-            rs[(8 + pc) * kRsStride + wr] = -(dmin * (float)mv);
+            if constexpr (j == 0) rh = ld16(blk); // d, dmin, the twelve scale bytes
         } else {
-            // low nibbles are quarter (pc % 4) / 2 of the half, high nibbles that quarter + 2; values 16 (pc % 2) ..
-#pragma unroll
-            for (int hn = 0; hn < 2; hn++) {
-                const int a4 = ((pc & 3) >> 1) + 2 * hn, ns = 4 * hn, hs = 2 * a4;
-                uint8_t *dst = codes + 128 * (pc >> 2) + 32 * a4 + 16 * (pc & 1);
-                const u32 mh = 0x03030303u;
-                put16(dst, q6_minus_32(((rw.x >> ns) & ml) | (((rqh.x >> hs) & mh) << 4)),
-                      q6_minus_32(((rw.y >> ns) & ml) | (((rqh.y >> hs) & mh) << 4)),
-                      q6_minus_32(((rw.z >> ns) & ml) | (((rqh.z >> hs) & mh) << 4)),
-                      q6_minus_32(((rw.w >> ns) & ml) | (((rqh.w >> hs) & mh) << 4)));
-            }
-            const float d = bm_half_to_f32((unsigned short)rhd.x);
-            rs[(2 * pc) * kRsStride + wr] = d * (float)(int)(signed char)(rhd.y & 0xffu);
-            rs[(2 * pc + 1) * kRsStride + wr] = d * (float)(int)(signed char)(rhd.y >> 8);
+            rh.x = bm_ld2u(blk + 208);         // d
+            rh.y = blk[192 + 8 * j + p];       // the scales of groups p
+            rh.z = blk[192 + 8 * j + 4 + p];   // and 4 + p
+        }
+        d8 = *reinterpret_cast<const float *>(act + (apair + 64 * (u32)at.i) + 32 * j); // of block 4 j + p
+        if constexpr (kQ45 && j == 0) { // d8 isum of blocks p and 4 + p
+            y0 = *reinterpret_cast<const float *>(act + (apair + 64 * (u32)at.i) + 4);
+            y4 = *reinterpret_cast<const float *>(act + (apair + 64 * (u32)at.i) + 36);
         }
     };
-    // this lane in its wave's 16 x 16 products: operand row / slot lane % 16, values 8 * (lane / 16) .. + 8 of a
-    // 32-value block; its four results of each product are rows 4 * (lane / 16) + v of slot lane % 16
-    const int rg = wv & 3, ch = wv >> 2, l16 = lane & 15, kg = lane >> 4;
-    int my_act[T];
-#pragma unroll
-    for (int t = 0; t < T; t++) my_act[t] = (16 * T * ch + 16 * t + l16) * kColStride;
-    // the weight operand of half h of a block: this lane's eight codes when they are of that half, else zeros
-    // (offsets from the buffer; the zero page lies below both buffers)
-    const int my_row = kWtsAt + (16 * rg + l16) * kRowStride + 8 * kg;
-    const int rbase = 16 * rg + 4 * kg; // result v sits in row rbase + v of the slab
-    const bool live = 16 * T * ch < len; // else none of this wave's slots is real
-    float acc[T][4][8];
-#pragma unroll
-    for (int t = 0; t < T; t++)
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-#pragma unroll
-            for (int l = 0; l < 8; l++) acc[t][v][l] = 0.0f;
-
-    auto arithmetic = [&](const uint8_t *buf) __attribute__((always_inline)) {
-        const float *rs = reinterpret_cast<const float *>(buf + kRsAt);
-        const uint8_t *my_a[2] = {kg < 2 ? buf + my_row : zeros, kg < 2 ? zeros : buf + my_row};
-        const float2 *pair[T]; // (d8, d8 * isum) a 32-block
-#pragma unroll
-        for (int t = 0; t < T; t++) pair[t] = reinterpret_cast<const float2 *>(buf + my_act[t] + BM_Q82_SB_REF);
-        if constexpr (kQ45) {
-            // the min terms first: accumulator l takes sub-block l's (crates/qdot/src/lib.rs:4389-4394)
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const float4 mn = *reinterpret_cast<const float4 *>(&rs[(8 + s) * kRsStride + rbase]);
-#pragma unroll
-                for (int t = 0; t < T; t++) {
-                    const float my = pair[t][s].y;
-                    acc[t][0][s] = fmaf(my, mn.x, acc[t][0][s]);
-                    acc[t][1][s] = fmaf(my, mn.y, acc[t][1][s]);
-                    acc[t][2][s] = fmaf(my, mn.z, acc[t][2][s]);
-                    acc[t][3][s] = fmaf(my, mn.w, acc[t][3][s]);
-                }
-            }
+    // Step st of eight of a half's staging. The codes of the half after it (super-block `next`) are asked for where a register's last
+    // word is done with, seven steps before its first use; the half's own factors at step 1, for step 7.
+    auto stash = [&](auto half, int st, At now, At next) __attribute__((always_inline)) {
+        constexpr std::integral_constant<int, 1 - decltype(half)::value> after{};
+        if (st == 0) fetch_factors(now, half);
+        if (st < 4) {
+            stash_row(half, st);
+            if (st == 3) fetch_row(next, after);
+        } else {
+            stash_col(half, (st - 4) >> 1, st & 1);
+            if (st & 1) fetch_col(next.i, after, (st - 4) >> 1);
         }
-        if constexpr (T == 1) {
-            // one product a 16-value group, sixteen a super-block: a group's matrix instruction is issued one group ahead
-            // of the vector work on its sums, and a block's LDS operands are read two blocks ahead
-            long a[2][2], b[2];
-            float d8[2];
-            float4 sv[2][2];
-            v4i sum[2];
-            auto rd = [&](int bk) {
+        if (st == 7) stash_factors(half);
+    };
+
+    // this lane in its wave's 32 x 32 products: operand slot and row lane % 32, eight of a group's sixteen values by lane / 32;
+    // result v is slot 8 (v / 4) + 4 (lane / 32) + v % 4 of row lane % 32
+    const int l32 = lane & 31, kh = lane >> 5;
+    const int wrow0 = 32 * (wv & 1), wslot0 = 32 * (wv >> 1);
+    const bool live = wslot0 < len;
+    v32f acc[4]; // accumulator l: [l / 2], results 16 (l % 2) ..
+
+    constexpr std::integral_constant<int, 0> kFirst{};
+    constexpr std::integral_constant<int, 1> kSecond{};
+    const LdsB my_row = (LdsB)lds + (wrow0 + l32) * kXStride + 16 * kh, my_col = (LdsB)lds + 2 * kXCodes + (wslot0 + l32) * kXStride + 16 * kh;
+    // the factors of an outer product's two blocks, or of a block's two groups (Q6_K: one d8 for both): a half of the lanes each
+    const LdsB my_sr = (LdsB)lds + 4 * kXCodes + 4 * (wrow0 + l32) + kh * kXLine;
+    const LdsB my_sc = (LdsB)lds + 4 * kXCodes + 4 * (wslot0 + l32) + (kQ45 ? kh : 0) * kXLine + X::kScales * kXLine;
+    const LdsB my_mr = my_sr + X::kMinsAt, my_mc = my_sc + X::kMinsAt + (8 - X::kScales) * kXLine;
+    // A half's arithmetic, a step a 16-value group, and in the shade of each step's outer product a piece of the staging of the half
+    // after it (super-block i1).
+    auto arithmetic = [&](auto half, At now, At next) __attribute__((always_inline)) {
+        constexpr int j = decltype(half)::value;
+        const v16f z16 = {};
+        const v32f z32 = {};
+        v4u a, b;
+        v16f sum;
+        v32f pd;
+        auto rd = [&](int gr) { // group gr of the half's eight
+            const int at = j * kXCodes + 32 * (kQ45 ? 4 * ((gr >> 1) & 1) + 2 * (gr >> 2) + (gr & 1) : gr), ct = j * kXCodes + 32 * gr;
+            const v2u a0 = *(LdsV2)(my_row + at), a1 = *(LdsV2)(my_row + at + 8), b0 = *(LdsV2)(my_col + ct), b1 = *(LdsV2)(my_col + ct + 8);
+            a = (v4u){a0.x, a0.y, a1.x, a1.y};
+            b = (v4u){b0.x, b0.y, b1.x, b1.y};
+        };
+        auto product = [&]() {
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, b), __builtin_bit_cast(v8h, a), z16, 0, 0, 0);
+        };
+        // Q4_K, Q5_K: one scale a block; Q6_K: one a group (crates/qdot/src/lib.rs:4403-4440, :4794-4809)
+        auto scale = [&](int gr) {
+            const float fc = *(LdsVF)(my_sc + j * X::kHalf + (gr >> 1) * kXLine), fr = *(LdsVF)(my_sr + j * X::kHalf + (kQ45 ? gr >> 1 : gr) * kXLine);
+            pd = __builtin_amdgcn_mfma_f32_32x32x1f32(fc, fr, z32, 0, 0, 0);
+        };
+        // the min terms come before a super-block's products: accumulator l takes sub-block l's (crates/qdot/src/lib.rs:4389-4394)
+        auto min_term = [&](int s) {
+            acc[s] = __builtin_amdgcn_mfma_f32_32x32x1f32(*(LdsVF)(my_mc + 2 * s * kXLine), *(LdsVF)(my_mr + 2 * s * kXLine), acc[s], 0, 0, 0);
+        };
+        rd(0);
+        if constexpr (kQ45 && j == 0) {
+            min_term(0);
+            min_term(2);
+        }
 #pragma unroll
-                for (int h = 0; h < 2; h++) a[bk & 1][h] = *reinterpret_cast<const long *>(my_a[h] + 32 * bk);
-                b[bk & 1] = *reinterpret_cast<const long *>(buf + my_act[0] + (bk >> 2) * BM_Q82X4_STRIDE + 16 + 32 * (bk & 3) + 8 * kg);
-                d8[bk & 1] = pair[0][bk].x;
-                sv[bk & 1][0] = *reinterpret_cast<const float4 *>(&rs[(kQ45 ? bk : 2 * bk) * kRsStride + rbase]);
-                if constexpr (!kQ45) sv[bk & 1][1] = *reinterpret_cast<const float4 *>(&rs[(2 * bk + 1) * kRsStride + rbase]);
-            };
-            auto product = [&](int g) {
-                const v4i z = {0, 0, 0, 0};
-                sum[g & 1] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[(g >> 1) & 1][g & 1], b[(g >> 1) & 1], z, 0, 0, 0);
-            };
-            rd(0);
-            rd(1);
-            product(0);
+        for (int gr = 0; gr < 8; gr++) {
+            const int bk = gr >> 1, h = gr & 1, l = 4 * h + bk, al = 16 * (l & 1), pb = 16 * (kQ45 ? bk & 1 : h);
+            product();
+            if ((gr & (kQ45 ? 3 : 1)) == 0) scale(gr);
+            if constexpr (kQ45 && j == 0) {
+                if (gr == 1) min_term(1);
+                if (gr == 3) min_term(3);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (gr + 1 < 8) rd(gr + 1);
+            stash(std::integral_constant<int, 1 - j>{}, gr, now, next);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int g = 0; g < 16; g++) {
-                const int bk = g >> 1, h = g & 1, l = 4 * h + (bk & 3);
-                if (g + 1 < 16) product(g + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                // Q4_K, Q5_K: one scale a block; Q6_K: one a group (crates/qdot/src/lib.rs:4403-4440, :4794-4809)
-                const float4 r = sv[bk & 1][kQ45 ? 0 : h];
-                const float dc = d8[bk & 1];
-                acc[0][0][l] = fmaf(r.x * dc, (float)sum[g & 1][0], acc[0][0][l]);
-                acc[0][1][l] = fmaf(r.y * dc, (float)sum[g & 1][1], acc[0][1][l]);
-                acc[0][2][l] = fmaf(r.z * dc, (float)sum[g & 1][2], acc[0][2][l]);
-                acc[0][3][l] = fmaf(r.w * dc, (float)sum[g & 1][3], acc[0][3][l]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (h == 1 && bk + 2 < 8) rd(bk + 2);
-            }
-            return;
-        }
-#pragma unroll
-        for (int bk = 0; bk < 8; bk++) { // 32-value block bk of the super-block: groups 2 bk (half 0) and 2 bk + 1
-            long a[2], b[T];
-#pragma unroll
-            for (int h = 0; h < 2; h++) a[h] = *reinterpret_cast<const long *>(my_a[h] + 32 * bk);
-            float d8[T];
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                b[t] = *reinterpret_cast<const long *>(buf + my_act[t] + (bk >> 2) * BM_Q82X4_STRIDE + 16 + 32 * (bk & 3) + 8 * kg);
-                d8[t] = pair[t][bk].x;
-            }
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                // Q4_K, Q5_K: one scale a block; Q6_K: one a group (crates/qdot/src/lib.rs:4403-4440, :4794-4809)
-                const float4 sv = *reinterpret_cast<const float4 *>(&rs[(kQ45 ? bk : 2 * bk + h) * kRsStride + rbase]);
-                const int l = 4 * h + (bk & 3);
-#pragma unroll
-                for (int t = 0; t < T; t++) {
-                    const v4i z = {0, 0, 0, 0};
-                    const v4i sum = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[h], b[t], z, 0, 0, 0);
-                    acc[t][0][l] = fmaf(sv.x * d8[t], (float)sum[0], acc[t][0][l]);
-                    acc[t][1][l] = fmaf(sv.y * d8[t], (float)sum[1], acc[t][1][l]);
-                    acc[t][2][l] = fmaf(sv.z * d8[t], (float)sum[2], acc[t][2][l]);
-                    acc[t][3][l] = fmaf(sv.w * d8[t], (float)sum[3], acc[t][3][l]);
-                }
-            }
+            for (int v = 0; v < 16; v++) acc[l >> 1][al + v] = fmaf(pd[pb + v], sum[v], acc[l >> 1][al + v]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
-    fetch(0);
-    stash(buf0);
+    auto stash_all = [&](auto half, At now, At next) __attribute__((always_inline)) {
+#pragma unroll
+        for (int st = 0; st < 8; st++) stash(half, st, now, next);
+    };
+    int left = (rpe - row0 + kGemmBM - 1) / kGemmBM; // slabs to do
+    left = left < (int)slabs ? left : (int)slabs;
+    At now = {row_at(row0), 0};
+    fetch_row(now, kFirst);
+    fetch_col(0, kFirst, 0);
+    fetch_col(0, kFirst, 1);
+    stash_all(kFirst, now, now);
     __syncthreads();
-    for (int i = 0; i < nb; i++) {
-        const bool more = i + 1 < nb;
-        if (more) fetch(i + 1);
-        if (live) arithmetic(buf0 + (size_t)(i & 1) * kBuf);
-        // the other buffer's last readers passed the barrier that ended the super-block before this one
-        if (more) stash(buf0 + (size_t)((i + 1) & 1) * kBuf);
-        __syncthreads();
-    }
-    // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order) and the store
-#pragma unroll
-    for (int t = 0; t < T; t++) {
-        const int n = 16 * T * ch + 16 * t + l16;
-        if (n < len) {
-            const size_t out = (size_t)tab->slot[n] * rpe + row0;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = rbase + v;
-                const float t0 = acc[t][v][0] + acc[t][v][4], t1 = acc[t][v][1] + acc[t][v][5];
-                const float t2 = acc[t][v][2] + acc[t][v][6], t3 = acc[t][v][3] + acc[t][v][7];
-                if (row0 + r < rpe) y[out + r] = (t0 + t2) + (t1 + t3);
+    // the super-block after `at`, in the next slab behind a slab's last (the very last: itself, staged for no reader)
+    auto following = [&](At at) {
+        if (at.i + 1 < nb) return At{at.row, at.i + 1};
+        return left > 1 ? At{row_at(row0 + kGemmBM), 0} : at;
+    };
+    // (a half's last readers passed the barrier that ended the half before)
+    if (!live) { // none of this wave's slots is real: it stages only
+        for (; left > 0; left--, row0 += kGemmBM)
+            for (int i = 0; i < nb; i++) {
+                const At next = following(now);
+                stash_all(kSecond, now, next);
+                __syncthreads();
+                stash_all(kFirst, next, next);
+                __syncthreads();
+                now = next;
             }
+        return;
+    }
+#pragma unroll
+    for (int l = 0; l < 4; l++)
+#pragma unroll
+        for (int v = 0; v < 32; v++) acc[l][v] = 0.0f;
+    for (; left > 0; left--, row0 += kGemmBM) {
+        for (int i = 0; i < nb; i++) {
+            const At next = following(now);
+            arithmetic(kFirst, now, next);
+            __syncthreads();
+            arithmetic(kSecond, next, next);
+            __syncthreads();
+            now = next;
+        }
+        // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order) and the store
+        const int row = row0 + wrow0 + l32;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int n = wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
+            const float t0 = acc[0][v] + acc[2][v], t1 = acc[0][16 + v] + acc[2][16 + v];
+            const float t2 = acc[1][v] + acc[3][v], t3 = acc[1][16 + v] + acc[3][16 + v];
+            if (row < rpe && n < len) y[(size_t)tab->slot[n] * rpe + row] = (t0 + t2) + (t1 + t3);
+#pragma unroll
+            for (int l = 0; l < 4; l++) acc[l][v] = acc[l][16 + v] = 0.0f;
         }
     }
 }
 
-// ------------------------------------------------------ one accumulator a value: whole-block matrix instructions
-
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 // The tolerance mode (BM_GEMM_FAST). The integer sums are the exact ones, formed by matrix instructions whose K is
 // exactly the span one scale covers, so no issued multiply is wasted:
@@ -1244,14 +1266,17 @@ hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int
     const int nb = k / 256;
     const u32 max_tiles = (u32)gemm_max_tiles(n_slots, n_experts) + 1; // one more: the block that fills refused slots
     const u32 n_slabs = (u32)((rows_per_expert + kGemmBM - 1) / kGemmBM);
-    // parts: workgroups a tile's 64 slots are shared among (each takes every row slab)
-    auto launch = [&](auto kern, unsigned threads, size_t lds, unsigned parts) {
+    auto launch = [&](auto kern, size_t lds) {
         hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;
-        const u32 n_units = n_slabs * parts;
+        // A workgroup's start (tile, columns, first bytes: a chain of trips to memory, 4 to 5 us) costs more than a super-block, so it
+        // takes several slabs where that leaves enough workgroups to fill the chip's 512 places about four times over (16384 slots:
+        // Q4_K 253 -> 228 us with two of twelve, Q6_K 341 -> 315 us with six of 32).
+        const u32 slabs_max = max_tiles * n_slabs / 2048u, slabs = slabs_max < 1u ? 1u : slabs_max < n_slabs ? slabs_max : n_slabs;
+        const u32 n_units = (n_slabs + slabs - 1) / slabs;
         const unsigned grid = ((max_tiles + 7) / 8) * 8 * n_units;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, L.stream, w, rows_per_expert, nb, act, cols, tiles_dev, n_tiles,
-                           n_units, (u32)slot_div, (u32)n_slots, y);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, w, rows_per_expert, nb, act, cols, tiles_dev, n_tiles, n_units,
+                           (u32)slot_div, (u32)n_slots, y, slabs);
         return hipGetLastError();
     };
     if (bm_takes_q8k(wtype)) {
@@ -1287,12 +1312,9 @@ hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int
         if (wtype == BM_Q5K) return launch_fast(k_gemm_fast<BM_Q5K>, fast_lds_bytes<BM_Q5K>());
         if (wtype == BM_Q6K) return launch_fast(k_gemm_fast<BM_Q6K>, fast_lds_bytes<BM_Q6K>());
     }
-    // 512 threads on 32 slots of a tile for both types (Q4_K 114 registers, Q6_K 121): two workgroups a CU. Measured
-    // against 1024 threads on all 64 slots (Q4_K gate 362 -> 342 us), 512 threads with two slot groups a wave on 64
-    // (Q6_K down 489 -> 407 us), and 256 threads on 16 or 32 slots (slower: the rows are staged once a workgroup).
-    if (wtype == BM_Q4K) return launch(k_gemm<BM_Q4K, 1, 2>, 512, gemm_exact_lds_bytes(32), 2);
-    if (wtype == BM_Q5K) return launch(k_gemm<BM_Q5K, 1, 2>, 512, gemm_exact_lds_bytes(32), 2);
-    if (wtype == BM_Q6K) return launch(k_gemm<BM_Q6K, 1, 2>, 512, gemm_exact_lds_bytes(32), 2);
+    if (wtype == BM_Q4K) return launch(k_gemm<BM_Q4K>, XLds<BM_Q4K>::kBytes);
+    if (wtype == BM_Q5K) return launch(k_gemm<BM_Q5K>, XLds<BM_Q5K>::kBytes);
+    if (wtype == BM_Q6K) return launch(k_gemm<BM_Q6K>, XLds<BM_Q6K>::kBytes);
     return hipErrorInvalidValue;
 }
 

@@ -335,6 +335,41 @@ def test_prefill_refusals_are_named(gpu):
         b.free()
 
 
+@pytest.mark.parametrize("wtype,k", ((bm.Q4_K, 256), (bm.Q4_K, 768), (bm.Q5_K, 512), (bm.Q6_K, 256), (bm.Q6_K, 512)))
+def test_gemm_with_several_slabs_a_workgroup(gpu, wtype, k):
+    """A route of enough tiles that a workgroup takes two row slabs of the seventeen (the last alone, a quarter of it real), with
+    tiles of every length; one refused slot. Sampled slots' rows against the one-column dot, bit for bit."""
+    from test_gpu_decode import random_blocks
+    n_experts, n_slots, rpe = 200, 6000, 1040
+    rng = np.random.default_rng(2700 + k)
+    w = random_blocks(wtype, n_experts * rpe, k, rng)
+    p = 1.0 / np.arange(1, n_experts + 1)
+    ids = rng.choice(n_experts, n_slots, p=p / p.sum()).astype(np.uint32)
+    ids[17] = n_experts
+    x = normal_f32(rng, (n_slots, k))
+    dw, act = gpu.weights(wtype, n_experts * rpe, k, w), gpu.act(wtype, k, n_slots)
+    xd, sel = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32)
+    table = gpu.route(n_slots, n_experts)
+    y = gpu.buffer(np.float32, n_slots * rpe).fill_bytes(0)
+    gpu.fault_clear()
+    gpu.enqueue_quantize(xd, n_slots, act)
+    table.fill(sel, n_slots)
+    gpu.enqueue_gemm(dw, rpe, act, table, 0, y)
+    got = y.download().reshape(n_slots, rpe)
+    assert np.isnan(got[17]).all()
+    rb = ora.row_bytes(wtype, k)
+    counts = np.bincount(ids[ids < n_experts], minlength=n_experts)
+    assert counts.max() > 64 * 9 and counts.min() < 16
+    last = [int(np.flatnonzero(ids == e)[-1]) for e in range(n_experts) if counts[e]]  # each expert's last slot
+    for s in sorted(set(last + list(range(0, n_slots, 61))) - {17}):
+        e = int(ids[s])
+        want = ora.gemv(wtype, w[e * rpe * rb:(e + 1) * rpe * rb], rpe, k, ora.quantize_col(wtype, x[s]), 1)
+        assert_f32(got[s], want, f"slot {s}")
+    gpu.fault_clear()
+    for b in (dw, act, xd, sel, table, y):
+        b.free()
+
+
 def test_gemm_at_the_largest_route(gpu):
     """The route's limits (crates/gpu/src/gemm/mod.rs:97-101): 40960 slots over 1024 experts, one column a slot, with
     runs from empty to many tiles; every slot's 16 rows against the one-column dot, and the table by definition."""
