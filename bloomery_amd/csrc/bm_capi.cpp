@@ -849,8 +849,9 @@ int bm_route_read(bm_ctx *ctx, const bm_route *route, uint32_t *cols_host, uint3
     return rc;
 }
 
-int bm_gemm(bm_ctx *ctx, const bm_weights *w, int rows_per_expert, const bm_act *act, const bm_route *route, int top_k, float *y_dev) {
-    const char *what = "bm_gemm";
+// `second`: a stack of the same type and shape over the same columns, in the same launch.
+static int gemm_over(bm_ctx *ctx, const char *what, const bm_weights *w, int rows_per_expert, const bm_act *act, const bm_route *route,
+                     int top_k, float *y_dev, int mode, const bm_weights *second = nullptr, float *second_y = nullptr) {
     if (!ctx || !w || !act || !route || !y_dev) return fail(ctx, BM_EARG, "%s: NULL argument", what);
     if (!route->filled) return fail(ctx, BM_ESHAPE, "%s: a filled route table (bm_route_fill first)", what);
     if (!bmk::gemm_supported(w->wtype))
@@ -859,9 +860,12 @@ int bm_gemm(bm_ctx *ctx, const bm_weights *w, int rows_per_expert, const bm_act 
     if (rc) return rc;
     if (rows_per_expert <= 0 || rows_per_expert % 16 != 0)
         return fail(ctx, BM_ESHAPE, "%s: rows_per_expert must be a positive multiple of 16, got %d", what, rows_per_expert);
-    if (w->rows != (int64_t)route->n_experts * rows_per_expert)
-        return fail(ctx, BM_ESHAPE, "%s: the stack has %lld rows, the route %d experts of %d rows", what, (long long)w->rows,
-                    route->n_experts, rows_per_expert);
+    if (second) rc = check_pair(ctx, what, second, act);
+    if (rc) return rc;
+    for (const bm_weights *s : {w, second})
+        if (s && s->rows != (int64_t)route->n_experts * rows_per_expert)
+            return fail(ctx, BM_ESHAPE, "%s: the stack has %lld rows, the route %d experts of %d rows", what, (long long)s->rows,
+                        route->n_experts, rows_per_expert);
     const int n_slots = route->filled;
     int slot_div = 1;
     if (top_k > 0) {
@@ -878,7 +882,12 @@ int bm_gemm(bm_ctx *ctx, const bm_weights *w, int rows_per_expert, const bm_act 
         return fail(ctx, BM_ESHAPE, "%s: %d columns of k = %d or %d rows an expert pass 4 GiB, the kernels' offset range", what,
                     n_slots / slot_div, act->k, rows_per_expert);
     return driver(ctx, what, bmk::gemm(launch_of(ctx), w->wtype, w->dev, route->n_experts, rows_per_expert, w->k, act->dev, route->cols,
-                                       route->tiles, route->n_tiles, n_slots, slot_div, y_dev, ctx->gemm_mode));
+                                       route->tiles, route->n_tiles, n_slots, slot_div, y_dev, mode, second ? second->dev : nullptr, second_y));
+}
+
+int bm_gemm(bm_ctx *ctx, const bm_weights *w, int rows_per_expert, const bm_act *act, const bm_route *route, int top_k, float *y_dev) {
+    if (!ctx) return fail(ctx, BM_EARG, "bm_gemm: NULL argument");
+    return gemm_over(ctx, "bm_gemm", w, rows_per_expert, act, route, top_k, y_dev, ctx->gemm_mode);
 }
 
 // ------------------------------------------------------------------------- one entry for every batch size
@@ -1024,7 +1033,8 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     if (m < 1 || m > s->max_tokens) return fail(ctx, BM_ESHAPE, "%s: m = %d tokens, the scratch holds 1..=%d", what, m, s->max_tokens);
     const int spt = s->spt, n_slots = m * spt, hidden = s->hidden, ff = s->ff, n_experts = s->n_experts;
     const bool down_q8k = act_form(s->down_type) != 0;
-    switch (bm_scratch_path_for(s, m)) {
+    int path = bm_scratch_path_for(s, m), mode = ctx->gemm_mode;
+    switch (path) {
     case BM_PATH_PER_SLOT:
         return bm_moe_decode(ctx, wg, wu, wd, x_dev, sel_dev, w_dev, resid_dev, spt, m, rule, s->act_h, nullptr,
                              down_q8k ? s->g : nullptr, y_dev);
@@ -1061,10 +1071,9 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     }
     default: {
         int rc = bm_route_fill_quantize(ctx, sel_dev, n_slots, s->route, x_dev, m, s->act_x);
-        if (!rc) rc = bm_gemm(ctx, wg, ff, s->act_x, s->route, spt, s->g);
-        if (!rc) rc = bm_gemm(ctx, wu, ff, s->act_x, s->route, spt, s->u);
+        if (!rc) rc = gemm_over(ctx, "bm_gemm", wg, ff, s->act_x, s->route, spt, s->g, mode, wu, s->u);
         if (!rc) rc = bm_swiglu_quant_sel(ctx, s->g, s->u, sel_dev, n_experts, n_slots, rule, s->act_h);
-        if (!rc) rc = bm_gemm(ctx, wd, hidden, s->act_h, s->route, 0, s->down);
+        if (!rc) rc = gemm_over(ctx, "bm_gemm", wd, hidden, s->act_h, s->route, 0, s->down, mode);
         if (rc) return rc;
         break;
     }

@@ -17,6 +17,16 @@ struct GemmLds {
 __device__ __forceinline__ u32 tile_of_block(u32 b, u32 n_slabs) { return ((b >> 3) / n_slabs) * 8 + (b & 7); }
 __device__ __forceinline__ u32 slab_of_block(u32 b, u32 n_slabs) { return (b >> 3) % n_slabs; }
 
+// A unit of a tile's work is a run of row slabs. With a second stack (an up beside a gate: the same shape, columns and tiles) its
+// units follow the first's, so that the two fill the chip as one launch.
+__device__ __forceinline__ u32 take_stack(u32 unit, u32 n_units, const uint8_t *&w, float *&y, const uint8_t *w_second, float *y_second) {
+    const u32 half = n_units / 2;
+    if (!w_second || unit < half) return unit;
+    w = w_second;
+    y = y_second;
+    return unit - half;
+}
+
 } // namespace bmk
 
 #endif // BM_GEMM_HPP

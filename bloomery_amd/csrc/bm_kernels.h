@@ -137,10 +137,15 @@ bool gemm_supported(int wtype);
 // slot_div: slots a token when every slot of a token reads the token's column, 1 when each slot reads its own.
 // mode 0: the CPU path's eight-accumulator f32 order (bit-identical to the row dots); 1: one accumulator a value, int8
 // matrix instructions; 2: one accumulator, f16 matrix instructions with the scales in the operands (Q4_K; else as 1).
+// w_second, y_second: a second stack of the same shape over the same columns (an up beside a gate), in the same launch.
 hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int rows_per_expert, int k,
                 const uint8_t *act, const uint32_t *cols, const uint32_t *tiles, const uint32_t *n_tiles, int n_slots,
-                int slot_div, float *y, int mode);
+                int slot_div, float *y, int mode, const uint8_t *w_second = nullptr, float *y_second = nullptr);
 
+// The tolerance mode of IQ2_XXS stacks (bm_gemm_iq2.hip): gemm()'s numbers but for the order of the f32 sums.
+hipError_t gemm_iq2_fast(const Launch &L, const uint8_t *w, int n_experts, int rows_per_expert, int k, const uint8_t *act,
+                         const uint32_t *cols, const uint32_t *tiles_dev, const uint32_t *n_tiles, int n_slots, int slot_div, float *y,
+                         const uint8_t *w_second, float *y_second);
 // The tolerance mode on f16 matrix instructions with both scales folded into the operands (bm_gemm_half.hip): gemm()'s
 // mode 2 where a type has that form; mode 1 is the int8 form.
 bool gemm_half_supported(int wtype);

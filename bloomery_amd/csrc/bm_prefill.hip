@@ -257,13 +257,14 @@ __device__ __forceinline__ u32 and_or(u32 x, u32 mask, u32 bits) {
 template <int WT>
 __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
                                                  const u32 *tiles, const u32 *n_tiles, u32 n_units, u32 slot_div,
-                                                 u32 n_slots, float *y, u32 slabs) {
+                                                 u32 n_slots, float *y, u32 slabs, const uint8_t *w_second, float *y_second) {
     using X = XLds<WT>;
     extern __shared__ __align__(16) uint8_t lds[];
     GemmLds *tab = reinterpret_cast<GemmLds *>(lds + 4 * kXCodes + X::kFactors);
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const u32 g = tile_of_block(blockIdx.x, n_units);
-    int row0 = (int)(slab_of_block(blockIdx.x, n_units) * slabs) * kGemmBM; // of the slabs a workgroup takes one after the other
+    // the first of the slabs the workgroup takes one after the other
+    int row0 = (int)(take_stack(slab_of_block(blockIdx.x, n_units), n_units, w, y, w_second, y_second) * slabs) * kGemmBM;
     const u32 count = n_tiles[0];
     if (g > count) return;
     if (g == count) { // the refused slots' rows: NaN (crates/gpu/src/gemm/grouped.rs:2283-2287)
@@ -603,8 +604,8 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 
 template <int WT>
 __global__ __launch_bounds__(kFastThreads, 2) void k_gemm_fast(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
-                                                      const u32 *tiles, const u32 *n_tiles, u32 n_slabs, u32 slot_div,
-                                                      u32 n_slots, float *y) {
+                                                      const u32 *tiles, const u32 *n_tiles, u32 n_units, u32 slot_div,
+                                                      u32 n_slots, float *y, const uint8_t *w_second, float *y_second) {
     constexpr bool kQ45 = WT == BM_Q4K || WT == BM_Q5K;
     constexpr int kStride = fast_code_stride<WT>(), kUnitsSb = fast_units<WT>(), kBlock = bm_block_bytes<WT>();
     constexpr int kOp = kQ45 ? 16 : 8; // operand bytes a lane
@@ -617,8 +618,8 @@ __global__ __launch_bounds__(kFastThreads, 2) void k_gemm_fast(const uint8_t *w,
     float *my_t = reinterpret_cast<float *>(sv_t + kUnitsSb * kFastRowLine);         // Q4_K, Q5_K only, as is mn_t
     float *mn_t = my_t + 8 * kFastColLine;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const u32 g = tile_of_block(blockIdx.x, n_slabs);
-    const int row0 = (int)slab_of_block(blockIdx.x, n_slabs) * kFastRows;
+    const u32 g = tile_of_block(blockIdx.x, n_units);
+    const int row0 = (int)take_stack(slab_of_block(blockIdx.x, n_units), n_units, w, y, w_second, y_second) * kFastRows;
     const u32 count = n_tiles[0];
     if (g > count) return;
     if (g == count) { // the refused slots' rows: NaN (crates/gpu/src/gemm/grouped.rs:2283-2287)
@@ -866,18 +867,15 @@ __global__ __launch_bounds__(kFastThreads, 2) void k_gemm_fast(const uint8_t *w,
 // 31 * 86 = 2666: too wide for an int8 operand, so each is split into two signed bytes, 256 h + lo with lo = the low byte
 // read as signed and h = (term + 128) >> 8 (0 .. 10), and the dot is two v_mfma_i32_32x32x32_i8 whose sums meet as
 // (H << 8) + L, exactly. The LDS copy of a row's (and a column's) super-block is laid out lane-major, [l][b][i], so a matrix
-// operand is 16 consecutive bytes. With EXACT the eight accumulators and their order are the CPU path's, bit for bit
-// (the value bm_gemv_sel gives); without it one accumulator takes d dy times the super-block's whole sum
-// sum_b (2 s_b + 1) sum_n (u - 43) a, the 43s taken out in integers through two more matrix instructions over the
-// column's 32-value sums (split into two bytes the same way): f32 rounding is the only difference.
+// operand is 16 consecutive bytes. The eight accumulators and
+// their order are the CPU path's, bit for bit (the value bm_gemv_sel gives).
 // A workgroup of four waves takes 64 rows and a tile's 64 slots, a wave 32 x 32 of them.
 constexpr int kIqRows = 64;
 constexpr int kIqStride = 256 + 16; // bytes a row's or a column's 256 codes take in LDS
 constexpr int kIqLine = 64 + 4;     // floats a line of the per-lane tables
-template <int WT, bool EXACT>
+template <int WT>
 __host__ __device__ constexpr size_t gemm_iq_lds_bytes() {
-    return sizeof(GemmLds) + (size_t)tab_bytes<WT>() + 3 * (size_t)64 * kIqStride + 2 * 64 * sizeof(float) +
-           (EXACT ? 2 * 8 * kIqLine * sizeof(float) : 3 * 64 * 16);
+    return sizeof(GemmLds) + (size_t)tab_bytes<WT>() + 3 * (size_t)64 * kIqStride + 2 * 64 * sizeof(float) + 2 * 8 * kIqLine * sizeof(float);
 }
 
 // (2 s + 1) u for the four code bytes of `u`, each product split into the signed low byte (lo) and what is left over 256
@@ -908,7 +906,7 @@ __device__ __forceinline__ void iq_planes_signed(u32 v, int sc, u32 &hi, u32 &lo
 //     (crates/qdot/src/lib.rs:11171-11173);
 //   Q3_K: terms scale x (u - 4) over the sixteen 16-value groups, one integer a super-block and one accumulator, the float step
 //     acc + (dcol d) sum with every operation rounded on its own (crates/qdot/src/lib.rs:2223-2245).
-// EXACT only for the three added types: the tolerance mode runs them in this order too.
+// (The tolerance mode has a kernel of its own for IQ2_XXS and runs the three others in this order too.)
 template <int WT>
 struct IqGemm {
     static constexpr bool kFold = WT == BM_IQ2XXS || WT == BM_IQ3XXS;
@@ -917,11 +915,10 @@ struct IqGemm {
     static constexpr int kBlock = WT == BM_IQ2XXS ? BM_IQ2XXS_BLOCK : WT == BM_IQ3XXS ? BM_IQ3XXS_BLOCK : WT == BM_IQ4XS ? BM_IQ4XS_BLOCK : BM_Q3K_BLOCK;
 };
 
-template <int WT, bool EXACT>
+template <int WT>
 __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
-                                                    const u32 *tiles, const u32 *n_tiles, u32 n_slabs, u32 slot_div,
-                                                    u32 n_slots, float *y) {
-    static_assert(EXACT || WT == BM_IQ2XXS, "the one-accumulator form is IQ2_XXS's");
+                                                    const u32 *tiles, const u32 *n_tiles, u32 n_units, u32 slot_div,
+                                                    u32 n_slots, float *y, const uint8_t *w_second, float *y_second) {
     using G = IqGemm<WT>;
     extern __shared__ __align__(16) uint8_t lds[];
     GemmLds *tab = reinterpret_cast<GemmLds *>(lds);
@@ -931,14 +928,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     uint8_t *w_lo = w_hi + 64 * kIqStride;
     float *dy_t = reinterpret_cast<float *>(w_lo + 64 * kIqStride); // [slot]
     float *d_t = dy_t + 64;                                          // [row]
-    float *bs_t = d_t + 64;                                          // EXACT: [l][slot] the 32-value sums, as floats
-    float *sc_t = bs_t + 8 * kIqLine;                                // EXACT: [l][row] the scales 2 s + 1, as floats
-    uint8_t *x_sc = reinterpret_cast<uint8_t *>(d_t + 64);           // else: [row][16] the scales as bytes, zeros behind
-    uint8_t *x_bl = x_sc + 64 * 16;                                  // [slot][16] the sums' low bytes, zeros behind
-    uint8_t *x_bh = x_bl + 64 * 16;                                  // [slot][16] what is left of the sums over 256
+    float *bs_t = d_t + 64;                                          // [l][slot] the 32-value sums, as floats
+    float *sc_t = bs_t + 8 * kIqLine;                                // [l][row] the scales 2 s + 1, as floats
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const u32 g = tile_of_block(blockIdx.x, n_slabs);
-    const int row0 = (int)slab_of_block(blockIdx.x, n_slabs) * kIqRows;
+    const u32 g = tile_of_block(blockIdx.x, n_units);
+    const int row0 = (int)take_stack(slab_of_block(blockIdx.x, n_units), n_units, w, y, w_second, y_second) * kIqRows;
     const u32 count = n_tiles[0];
     if (g > count) return;
     if (g == count) { // the refused slots' rows: NaN (crates/gpu/src/gemm/grouped.rs:2283-2287)
@@ -1032,27 +1026,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
         if (tid < 64) {
             dy_t[tid] = cdy;
             const u32 bw[8] = {cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y, cb1.z, cb1.w};
-            u32 bl[2] = {0, 0}, bh[2] = {0, 0};
 #pragma unroll
             for (int l = 0; l < 8; l++) { // the two 16-value sums of sub-block l
                 const int bs = (int)(short)(bw[l] & 0xffffu) + (int)(short)(bw[l] >> 16);
-                if constexpr (EXACT) {
-                    if constexpr (G::kFold) bs_t[l * kIqLine + tid] = (float)bs;
-                } else { // 256 hi + lo with lo the low byte read as signed
-                    bl[l >> 2] |= ((u32)bs & 0xffu) << (8 * (l & 3));
-                    bh[l >> 2] |= ((u32)((bs + 128) >> 8) & 0xffu) << (8 * (l & 3));
-                }
-            }
-            if constexpr (!EXACT) {
-                *reinterpret_cast<uint4 *>(x_bl + 16 * tid) = make_uint4(bl[0], bl[1], 0u, 0u);
-                *reinterpret_cast<uint4 *>(x_bh + 16 * tid) = make_uint4(bh[0], bh[1], 0u, 0u);
+                if constexpr (G::kFold) bs_t[l * kIqLine + tid] = (float)bs;
             }
         }
         if (wq == 0) {
             const float dh = bm_half_to_f32((unsigned short)rd);
             d_t[wr] = WT == BM_IQ2XXS ? 0.125f * dh : WT == BM_IQ3XXS ? 0.25f * dh : dh;
         }
-        [[maybe_unused]] u32 scs[2] = {0, 0};
 #pragma unroll
         for (int e2 = 0; e2 < 2; e2++) {
             const int b = 2 * wq + e2;
@@ -1065,8 +1048,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
             if constexpr (WT == BM_IQ2XXS || WT == BM_IQ3XXS) {
                 const u32 aux = WT == BM_IQ2XXS ? (e2 ? rq.w : rq.y) : (e2 ? rx.y : rx.x);
                 const u32 sc = 2u * (aux >> 28) + 1u;
-                scs[e2] = sc;
-                if constexpr (EXACT) sc_t[b * kIqLine + wr] = (float)sc;
+                sc_t[b * kIqLine + wr] = (float)sc;
 #pragma unroll
                 for (int q = 0; q < 4; q++) { // values 8 q .. 8 q + 7: lanes 2 q and 2 q + 1
                     u32 c_lo, c_hi;
@@ -1121,10 +1103,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
                 }
             }
         }
-        if constexpr (!EXACT) { // the row's eight scales as bytes: the thread of sub-blocks 2 wq, 2 wq + 1 writes its two
-            *reinterpret_cast<unsigned short *>(x_sc + 16 * wr + 2 * wq) = (unsigned short)(scs[0] | (scs[1] << 8));
-            if (wq == 0) *reinterpret_cast<uint2 *>(x_sc + 16 * wr + 8) = make_uint2(0u, 0u);
-        }
     };
 
     // this lane in its wave's 32 x 32 product: operand row / slot lane % 32, terms 16 (lane / 32) .. of the 32; result v
@@ -1136,7 +1114,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     const uint8_t *my_a = a_codes + (wslot + l32) * kIqStride + 16 * kh;
     const bool live = wslot < len; // else none of this wave's slots is real
     const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    constexpr int kAcc = EXACT ? G::kLanes : 1;
+    constexpr int kAcc = G::kLanes;
     v16f acc[kAcc];
 #pragma unroll
     for (int l = 0; l < kAcc; l++)
@@ -1146,7 +1124,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     // (the columns' bytes too where the registers allow: the exact forms of the types with eight accumulators a value have few
     // to spare - with everything held over they spilled and ran 6 % slower - so there only the rows' bytes, which come from
     // HBM, are asked for ahead, and the columns', which the cache holds, when their turn comes)
-    constexpr bool kColsAhead = !EXACT || G::kLanes == 1;
+    constexpr bool kColsAhead = G::kLanes == 1;
     fetch_rows(0);
     if constexpr (kColsAhead) fetch_cols(0);
     for (int i = 0; i < nb; i++) {
@@ -1169,7 +1147,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
             dd[4 * q4 + 2] = d4.z;
             dd[4 * q4 + 3] = d4.w;
         }
-        if constexpr (EXACT && G::kLanes == 1) {
+        if constexpr (G::kLanes == 1) {
             // Q3_K: one integer a super-block, then acc + (dcol d) sum, each operation rounded on its own
             v16i hs = z, ls = z;
 #pragma unroll
@@ -1181,7 +1159,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
 #pragma unroll
             for (int v = 0; v < 16; v++)
                 acc[0][v] = __fadd_rn(acc[0][v], __fmul_rn(__fmul_rn(dy, dd[v]), (float)(hs[v] * 256 + ls[v])));
-        } else if constexpr (EXACT) {
+        } else {
             if constexpr (G::kFold) {
                 // the fold of the offsets first: accumulator l takes sub-block l's scale on its two sums
                 // (crates/qdot/src/lib.rs:8691-8694); the product of the two small integers is exact in f32
@@ -1208,26 +1186,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[l][v] = fmaf(dd[v] * dy, (float)(hs[v] * 256 + ls[v]), acc[l][v]);
             }
-        } else {
-            v16i hs = z, ls = z;
-#pragma unroll
-            for (int l = 0; l < 8; l++) {
-                const v4i b = *reinterpret_cast<const v4i *>(my_a + 32 * l);
-                hs = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_h + 32 * l), b, hs, 0, 0, 0);
-                ls = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_l + 32 * l), b, ls, 0, 0, 0);
-            }
-            // sum_b (2 s_b + 1) (the sub-block's sum of a): the scales against the sums' two bytes, terms 8 .. 31 zero
-            const v4i zero4 = {0, 0, 0, 0};
-            const v4i xs = kh ? zero4 : *reinterpret_cast<const v4i *>(x_sc + 16 * (wrow + l32));
-            const v4i xl = kh ? zero4 : *reinterpret_cast<const v4i *>(x_bl + 16 * (wslot + l32));
-            const v4i xh = kh ? zero4 : *reinterpret_cast<const v4i *>(x_bh + 16 * (wslot + l32));
-            const v16i ml = __builtin_amdgcn_mfma_i32_32x32x32_i8(xs, xl, z, 0, 0, 0);
-            const v16i mh = __builtin_amdgcn_mfma_i32_32x32x32_i8(xs, xh, z, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int total = ((hs[v] << 8) + ls[v]) - 43 * ((mh[v] << 8) + ml[v]);
-                acc[0][v] = fmaf(dd[v] * dy, (float)total, acc[0][v]);
-            }
         }
     }
     const int n = wslot + l32;
@@ -1241,7 +1199,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int v = 4 * q4 + k;
-                    if constexpr (EXACT && G::kLanes == 8) { // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order)
+                    if constexpr (G::kLanes == 8) { // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order)
                         const float t0 = acc[0][v] + acc[4][v], t1 = acc[1][v] + acc[5][v];
                         const float t2 = acc[2][v] + acc[6][v], t3 = acc[3][v] + acc[7][v];
                         r[k] = (t0 + t2) + (t1 + t3);
@@ -1262,59 +1220,47 @@ bool gemm_supported(int wtype) {
 
 hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int rows_per_expert, int k,
                 const uint8_t *act, const uint32_t *cols, const uint32_t *tiles_dev, const uint32_t *n_tiles, int n_slots,
-                int slot_div, float *y, int mode) {
+                int slot_div, float *y, int mode, const uint8_t *w_second, float *y_second) {
     const int nb = k / 256;
     const u32 max_tiles = (u32)gemm_max_tiles(n_slots, n_experts) + 1; // one more: the block that fills refused slots
-    const u32 n_slabs = (u32)((rows_per_expert + kGemmBM - 1) / kGemmBM);
-    auto launch = [&](auto kern, size_t lds) {
+    const u32 stacks = w_second ? 2 : 1;
+    auto launch = [&](auto kern, int threads, int slab_rows, size_t lds, auto... more) {
         hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;
-        // A workgroup's start (tile, columns, first bytes: a chain of trips to memory, 4 to 5 us) costs more than a super-block, so it
-        // takes several slabs where that leaves enough workgroups to fill the chip's 512 places about four times over (16384 slots:
-        // Q4_K 253 -> 228 us with two of twelve, Q6_K 341 -> 315 us with six of 32).
-        const u32 slabs_max = max_tiles * n_slabs / 2048u, slabs = slabs_max < 1u ? 1u : slabs_max < n_slabs ? slabs_max : n_slabs;
-        const u32 n_units = (n_slabs + slabs - 1) / slabs;
+        const u32 n_units = stacks * (u32)((rows_per_expert + slab_rows - 1) / slab_rows);
         const unsigned grid = ((max_tiles + 7) / 8) * 8 * n_units;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, w, rows_per_expert, nb, act, cols, tiles_dev, n_tiles, n_units,
-                           (u32)slot_div, (u32)n_slots, y, slabs);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, L.stream, w, rows_per_expert, nb, act, cols, tiles_dev, n_tiles, n_units,
+                           (u32)slot_div, (u32)n_slots, y, more..., w_second, y_second);
         return hipGetLastError();
     };
-    if (bm_takes_q8k(wtype)) {
-        auto launch_iq = [&](auto kern, size_t lds) {
-            hipError_t e = allow_lds(kern, lds);
-            if (e != hipSuccess) return e;
-            const u32 n_slabs_q = (u32)((rows_per_expert + kIqRows - 1) / kIqRows);
-            const unsigned grid = ((max_tiles + 7) / 8) * 8 * n_slabs_q;
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, w, rows_per_expert, nb, act, cols, tiles_dev, n_tiles,
-                               n_slabs_q, (u32)slot_div, (u32)n_slots, y);
-            return hipGetLastError();
-        };
-        if (wtype == BM_IQ3XXS) return launch_iq(k_gemm_iq<BM_IQ3XXS, true>, gemm_iq_lds_bytes<BM_IQ3XXS, true>());
-        if (wtype == BM_IQ4XS) return launch_iq(k_gemm_iq<BM_IQ4XS, true>, gemm_iq_lds_bytes<BM_IQ4XS, true>());
-        if (wtype == BM_Q3K) return launch_iq(k_gemm_iq<BM_Q3K, true>, gemm_iq_lds_bytes<BM_Q3K, true>());
-        if (wtype != BM_IQ2XXS) return hipErrorInvalidValue;
-        if (mode != 0) return launch_iq(k_gemm_iq<BM_IQ2XXS, false>, gemm_iq_lds_bytes<BM_IQ2XXS, false>());
-        return launch_iq(k_gemm_iq<BM_IQ2XXS, true>, gemm_iq_lds_bytes<BM_IQ2XXS, true>());
+    if (wtype == BM_IQ3XXS) return launch(k_gemm_iq<BM_IQ3XXS>, 256, kIqRows, gemm_iq_lds_bytes<BM_IQ3XXS>());
+    if (wtype == BM_IQ4XS) return launch(k_gemm_iq<BM_IQ4XS>, 256, kIqRows, gemm_iq_lds_bytes<BM_IQ4XS>());
+    if (wtype == BM_Q3K) return launch(k_gemm_iq<BM_Q3K>, 256, kIqRows, gemm_iq_lds_bytes<BM_Q3K>());
+    if (wtype == BM_IQ2XXS) {
+        if (mode != 0)
+            return gemm_iq2_fast(L, w, n_experts, rows_per_expert, k, act, cols, tiles_dev, n_tiles, n_slots, slot_div, y, w_second, y_second);
+        return launch(k_gemm_iq<BM_IQ2XXS>, 256, kIqRows, gemm_iq_lds_bytes<BM_IQ2XXS>());
     }
-    if (mode == 2 && gemm_half_supported(wtype)) // the f16 form of the tolerance mode, where the type has one
-        return gemm_half(L, wtype, w, n_experts, rows_per_expert, k, act, cols, tiles_dev, n_tiles, n_slots, slot_div, y);
+    if (mode == 2 && gemm_half_supported(wtype)) { // the f16 form of the tolerance mode, where the type has one
+        hipError_t e = gemm_half(L, wtype, w, n_experts, rows_per_expert, k, act, cols, tiles_dev, n_tiles, n_slots, slot_div, y);
+        if (e == hipSuccess && w_second)
+            e = gemm_half(L, wtype, w_second, n_experts, rows_per_expert, k, act, cols, tiles_dev, n_tiles, n_slots, slot_div, y_second);
+        return e;
+    }
     if (mode == 1 || mode == 2) {
-        auto launch_fast = [&](auto kern, size_t lds) {
-            hipError_t e = allow_lds(kern, lds);
-            if (e != hipSuccess) return e;
-            const u32 n_slabs_f = (u32)((rows_per_expert + kFastRows - 1) / kFastRows);
-            const unsigned grid = ((max_tiles + 7) / 8) * 8 * n_slabs_f;
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(kFastThreads), lds, L.stream, w, rows_per_expert, nb, act, cols, tiles_dev, n_tiles,
-                               n_slabs_f, (u32)slot_div, (u32)n_slots, y);
-            return hipGetLastError();
-        };
-        if (wtype == BM_Q4K) return launch_fast(k_gemm_fast<BM_Q4K>, fast_lds_bytes<BM_Q4K>());
-        if (wtype == BM_Q5K) return launch_fast(k_gemm_fast<BM_Q5K>, fast_lds_bytes<BM_Q5K>());
-        if (wtype == BM_Q6K) return launch_fast(k_gemm_fast<BM_Q6K>, fast_lds_bytes<BM_Q6K>());
+        if (wtype == BM_Q4K) return launch(k_gemm_fast<BM_Q4K>, kFastThreads, kFastRows, fast_lds_bytes<BM_Q4K>());
+        if (wtype == BM_Q5K) return launch(k_gemm_fast<BM_Q5K>, kFastThreads, kFastRows, fast_lds_bytes<BM_Q5K>());
+        if (wtype == BM_Q6K) return launch(k_gemm_fast<BM_Q6K>, kFastThreads, kFastRows, fast_lds_bytes<BM_Q6K>());
     }
-    if (wtype == BM_Q4K) return launch(k_gemm<BM_Q4K>, XLds<BM_Q4K>::kBytes);
-    if (wtype == BM_Q5K) return launch(k_gemm<BM_Q5K>, XLds<BM_Q5K>::kBytes);
-    if (wtype == BM_Q6K) return launch(k_gemm<BM_Q6K>, XLds<BM_Q6K>::kBytes);
+    // A workgroup's start (tile, columns, first bytes: a chain of trips to memory, 4 to 5 us) costs more than a super-block, so it
+    // takes several slabs where that leaves enough workgroups to fill the chip's 512 places about four times over (16384 slots:
+    // Q4_K 253 -> 228 us with two of twelve, Q6_K 341 -> 315 us with six of 32).
+    const u32 n_slabs = (u32)((rows_per_expert + kGemmBM - 1) / kGemmBM), slabs_max = stacks * max_tiles * n_slabs / 2048u;
+    const u32 slabs = slabs_max < 1u ? 1u : slabs_max < n_slabs ? slabs_max : n_slabs;
+    const int run = kGemmBM * (int)slabs;
+    if (wtype == BM_Q4K) return launch(k_gemm<BM_Q4K>, 256, run, XLds<BM_Q4K>::kBytes, slabs);
+    if (wtype == BM_Q5K) return launch(k_gemm<BM_Q5K>, 256, run, XLds<BM_Q5K>::kBytes, slabs);
+    if (wtype == BM_Q6K) return launch(k_gemm<BM_Q6K>, 256, run, XLds<BM_Q6K>::kBytes, slabs);
     return hipErrorInvalidValue;
 }
 

@@ -331,7 +331,7 @@ int bm_gemm(bm_ctx *ctx, const bm_weights *w, int rows_per_expert, const bm_act 
 /* How bm_gemm sums in f32 (the integer block sums are exact either way):
  *   BM_GEMM_EXACT (default): the CPU path's eight accumulators and closing order; bit-identical to bm_gemv_sel;
  *   BM_GEMM_FAST: one accumulator a value, blocks in increasing k; differs from the exact value by f32 rounding
- *     only (observed below 1e-6 of the row's largest magnitude; the contract's tolerance is 1e-4), about 1.9x the
+ *     only (observed below 1e-6 of the row's largest magnitude; the contract's tolerance is 1e-4), about 1.4x the
  *     speed of a Q4_K / Q6_K layer step. No counterpart in the reference, whose grouped GEMM has one order (gemm/grouped.rs:33-58).
  *     IQ3_XXS, IQ4_XS and Q3_K stacks have the exact order only and run in it under every mode.
  *   BM_GEMM_FAST_F16: the tolerance mode with both scales folded into f16 matrix operands (the sub-scale times the 4-bit
@@ -375,8 +375,8 @@ int bm_swiglu_quant_sel(bm_ctx *ctx, const float *g_dev, const float *u_dev, con
  *   BM_PATH_PER_SLOT  bm_moe_decode: two launches, every slot streams its expert's rows (repeats come from the caches);
  *   BM_PATH_GROUPED   bm_tables_quantize, bm_gate_up_tiles (bm_quantize_ord for a down stack on Q8_K columns),
  *                     bm_gemv_tiles, the slots' sum: an expert's rows are read once for all of its slots;
- *   BM_PATH_GEMM      bm_route_fill_quantize, bm_gemm twice, bm_swiglu_quant_sel, bm_gemm, the slots' sum: the int8 matrix
- *                     cores (in the f32 order bm_set_gemm_mode sets; every stack type bm_gemm takes).
+ *   BM_PATH_GEMM      bm_route_fill_quantize, bm_gemm over the gate and the up, bm_swiglu_quant_sel, bm_gemm, the slots' sum: the
+ *                     matrix cores (in the f32 order bm_set_gemm_mode sets; every stack type bm_gemm takes).
  * In the exact mode all three give the same bits in y_dev. bm_scratch holds what the paths need between their launches for
  * up to max_tokens tokens (made at load time and shared by every layer of the same shape, as the reference's Q8Act scratch
  * is): max_tokens * n_slots_per_token <= 40960. BM_PATH_AUTO (the default) takes the per-slot path below grouped_from

@@ -370,6 +370,40 @@ def test_gemm_with_several_slabs_a_workgroup(gpu, wtype, k):
         b.free()
 
 
+@pytest.mark.parametrize("rpe,k,counts", ((16, 256, (1, 64)), (560, 512, (31, 32, 33)), (1040, 768, (65, 5, 0, 97)), (512, 1792, (63, 2)),
+                                          (1536, 256, (40,) * 190)))
+def test_gemm_fast_iq2xxs_at_the_edges(gpu, rpe, k, counts):
+    """The tolerance mode's IQ2_XXS kernel where its splits change: tiles of one and of two slot groups, rows that end inside a wave's
+    64 or a workgroup's 512, one super-block, odd and even counts of them, several slabs a workgroup; against the exact order."""
+    from common import max_abs_normalised
+    from test_gpu_decode import random_blocks
+    n_experts, n_slots = len(counts), sum(counts)
+    rng = np.random.default_rng(2800 + rpe)
+    w = random_blocks(bm.IQ2_XXS, n_experts * rpe, k, rng)
+    ids = rng.permutation(np.repeat(np.arange(n_experts), counts)).astype(np.uint32)
+    x = normal_f32(rng, (n_slots, k))
+    dw, act = gpu.weights(bm.IQ2_XXS, n_experts * rpe, k, w), gpu.act(bm.IQ2_XXS, k, n_slots)
+    xd, sel = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32)
+    table = gpu.route(n_slots, n_experts)
+    y = gpu.buffer(np.float32, n_slots * rpe)
+    gpu.enqueue_quantize(xd, n_slots, act)
+    table.fill(sel, n_slots)
+    got = {}
+    for mode in (bm.GEMM_EXACT, bm.GEMM_FAST):
+        y.fill_bytes(0xFF)
+        gpu.set_gemm_mode(mode)
+        try:
+            gpu.enqueue_gemm(dw, rpe, act, table, 0, y)
+            got[mode] = y.download().reshape(n_slots, rpe)
+        finally:
+            gpu.set_gemm_mode(bm.GEMM_EXACT)
+    assert np.isfinite(got[bm.GEMM_FAST]).all()
+    for s in range(n_slots):
+        assert max_abs_normalised(got[bm.GEMM_FAST][s], got[bm.GEMM_EXACT][s]) <= 1e-5, f"slot {s}"
+    for b in (dw, act, xd, sel, table, y):
+        b.free()
+
+
 def test_gemm_at_the_largest_route(gpu):
     """The route's limits (crates/gpu/src/gemm/mod.rs:97-101): 40960 slots over 1024 experts, one column a slot, with
     runs from empty to many tiles; every slot's 16 rows against the one-column dot, and the table by definition."""
