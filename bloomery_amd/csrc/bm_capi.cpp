@@ -900,6 +900,7 @@ struct bm_scratch {
     uint32_t *order, *start, *tiles; // the grouped table
     bm_route *route;               // the GEMM path's table
     int path, grouped_from, gemm_from, gemm_from_fast;
+    bool own_cut; // gemm_from set by the caller
 };
 
 void bm_scratch_destroy(bm_scratch *s) {
@@ -943,7 +944,7 @@ int bm_scratch_create(bm_ctx *ctx, int gate_type, int down_type, int hidden, int
     //    192      580       246        370          214
     //    256      767       296        392          230
     //    512     1491       534        481          289
-    s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 448, s->gemm_from_fast = 96;
+    s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 448, s->gemm_from_fast = 96, s->own_cut = false;
     // a gate/up stack on Q8_K columns (Q3_K, IQ2_XXS, IQ3_XXS, IQ4_XS): its tile launchers are bound by the type's decode, which
     // the GEMM does once a row and super-block for all of a tile's slots, so the exact GEMM is ahead much earlier (same layer
     // shape, us a step, grouped / GEMM: IQ4_XS 48 tokens 180 / 170, 96 tokens 265 / 185, 2048 tokens 3202 / 907; IQ2_XXS 64
@@ -993,7 +994,7 @@ int bm_scratch_set_path(bm_scratch *s, int path, int grouped_from, int gemm_from
         return fail(s->ctx, BM_ESHAPE, "%s: the crossovers are token counts (0: keep), got %d and %d", what, grouped_from, gemm_from);
     s->path = path;
     if (grouped_from) s->grouped_from = grouped_from;
-    if (gemm_from) s->gemm_from = s->gemm_from_fast = gemm_from;
+    if (gemm_from) s->gemm_from = s->gemm_from_fast = gemm_from, s->own_cut = true;
     return BM_OK;
 }
 
@@ -1034,6 +1035,14 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     const int spt = s->spt, n_slots = m * spt, hidden = s->hidden, ff = s->ff, n_experts = s->n_experts;
     const bool down_q8k = act_form(s->down_type) != 0;
     int path = bm_scratch_path_for(s, m), mode = ctx->gemm_mode;
+    // The grouped range's upper part, where it is the default cut's: from 12 slots an expert, or 192 tokens with at least four, the
+    // GEMM's launches in the exact order give the same bits sooner (us a layer, tile launches / GEMM: hidden 2048, ff 768, top-8 of 128
+    // Q4_K 128 tokens 192 / 210, 192: 240 / 236, 333: 368 / 275; hidden 4096, ff 1536, top-2 of 32, 192: 292 / 216; hidden 2048, ff
+    // 1024, top-2 of 8, 64: 63 / 57; hidden 3072, ff 512, top-6 of 256, 128: 240 / 266, 192: 277 / 270, 256: 340 / 278).
+    const bool gemm_ahead = n_slots >= 12 * n_experts || (m >= 192 && n_slots >= 4 * n_experts);
+    if (path == BM_PATH_GROUPED && s->path == BM_PATH_AUTO && !s->own_cut && gemm_ahead && bmk::gemm_supported(s->gate_type) &&
+        bmk::gemm_supported(s->down_type))
+        path = BM_PATH_GEMM, mode = BM_GEMM_EXACT;
     switch (path) {
     case BM_PATH_PER_SLOT:
         return bm_moe_decode(ctx, wg, wu, wd, x_dev, sel_dev, w_dev, resid_dev, spt, m, rule, s->act_h, nullptr,
