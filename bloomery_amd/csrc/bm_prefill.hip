@@ -875,7 +875,7 @@ constexpr int kIqStride = 256 + 16; // bytes a row's or a column's 256 codes tak
 constexpr int kIqLine = 64 + 4;     // floats a line of the per-lane tables
 template <int WT>
 __host__ __device__ constexpr size_t gemm_iq_lds_bytes() {
-    return sizeof(GemmLds) + (size_t)tab_bytes<WT>() + 3 * (size_t)64 * kIqStride + 2 * 64 * sizeof(float) + 2 * 8 * kIqLine * sizeof(float);
+    return sizeof(GemmLds) + (size_t)tab_bytes<WT>() + (WT == BM_Q3K ? 2 : 3) * (size_t)64 * kIqStride + 2 * 64 * sizeof(float) + 2 * 8 * kIqLine * sizeof(float);
 }
 
 // (2 s + 1) u for the four code bytes of `u`, each product split into the signed low byte (lo) and what is left over 256
@@ -887,14 +887,30 @@ __device__ __forceinline__ void iq2_planes(u32 u, u32 sc, u32 &hi, u32 &lo) {
     hi = __builtin_amdgcn_perm(po + 0x00800080u, pe + 0x00800080u, 0x07030501u);
 }
 
-// The same split for a product of four signed bytes with a signed scale (|product| <= 4064): lo the low byte read as signed,
-// hi what is left over 256.
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+
+// Four bytes, each plus `more`, times a signed scale as two pairs of 16-bit products (bytes 0 and 2, bytes 1 and 3), two products an
+// instruction: |product| <= 4064, so sixteen bits hold them.
+__device__ __forceinline__ void iq_products(u32 bytes, int more, int sc, v2us &even, v2us &odd) {
+    const unsigned short s = (unsigned short)sc, m = (unsigned short)(more * sc);
+    const v2us scale = {s, s}, add = {m, m};
+    even = __builtin_bit_cast(v2us, __builtin_amdgcn_perm(0u, bytes, 0x0c020c00u)) * scale + add;
+    odd = __builtin_bit_cast(v2us, __builtin_amdgcn_perm(0u, bytes, 0x0c030c01u)) * scale + add;
+}
+// The low bytes of four such products, in the bytes' order.
+__device__ __forceinline__ u32 iq_low_bytes(v2us even, v2us odd) {
+    return __builtin_amdgcn_perm(__builtin_bit_cast(u32, odd), __builtin_bit_cast(u32, even), 0x06020400u);
+}
+
+// The same split for a product of four signed bytes with a signed scale: lo the low byte read as signed, hi what is left over 256.
+// (Ten instructions. Byte by byte it took some thirty, and the staging was over half of the kernel's vector work: a layer of 777
+// tokens, top-8 of 128 experts of 768 x 2048 IQ4_XS, 428 -> 391 us.)
 __device__ __forceinline__ void iq_planes_signed(u32 v, int sc, u32 &hi, u32 &lo) {
-    const int p0 = bm_mul24(__builtin_amdgcn_sbfe((int)v, 0, 8), sc), p1 = bm_mul24(__builtin_amdgcn_sbfe((int)v, 8, 8), sc);
-    const int p2 = bm_mul24(__builtin_amdgcn_sbfe((int)v, 16, 8), sc), p3 = bm_mul24(__builtin_amdgcn_sbfe((int)v, 24, 8), sc);
-    lo = ((u32)p0 & 0xffu) | (((u32)p1 & 0xffu) << 8) | (((u32)p2 & 0xffu) << 16) | ((u32)p3 << 24);
-    hi = ((u32)((p0 + 128) >> 8) & 0xffu) | (((u32)((p1 + 128) >> 8) & 0xffu) << 8) | (((u32)((p2 + 128) >> 8) & 0xffu) << 16) |
-         ((u32)((p3 + 128) >> 8) << 24);
+    v2us even, odd;
+    iq_products(v ^ 0x80808080u, -128, sc, even, odd);
+    const v2us half = {128, 128};
+    lo = iq_low_bytes(even, odd);
+    hi = __builtin_amdgcn_perm(__builtin_bit_cast(u32, odd + half), __builtin_bit_cast(u32, even + half), 0x07030501u);
 }
 
 // The types that dot against Q8_K columns (crates/gpu/src/gemm/kernels.rs:867 gemm_iq2xxs, :759 gemm_q3k, :1139 gemm_iq3xxs,
@@ -904,14 +920,16 @@ __device__ __forceinline__ void iq_planes_signed(u32 v, int sc, u32 &hi, u32 &lo
 //     eight accumulators, d = f16 / 8 and f16 / 4;
 //   IQ4_XS: terms scale x level (scale -32 .. 31, the sixteen levels), eight accumulators, one multiply-add a super-block each
 //     (crates/qdot/src/lib.rs:11171-11173);
-//   Q3_K: terms scale x (u - 4) over the sixteen 16-value groups, one integer a super-block and one accumulator, the float step
-//     acc + (dcol d) sum with every operation rounded on its own (crates/qdot/src/lib.rs:2223-2245).
+//   Q3_K: terms scale x (u - 4) over the sixteen 16-value groups, -124 .. 128 and so, negated, one signed byte: one plane and one
+//     product instead of two (with the products above: the same layer in Q3_K / Q4_K 367 -> 300 us). One integer a super-block and
+//     one accumulator, the float step acc + (dcol d) sum with every operation rounded on its own (crates/qdot/src/lib.rs:2223-2245).
 // (The tolerance mode has a kernel of its own for IQ2_XXS and runs the three others in this order too.)
 template <int WT>
 struct IqGemm {
     static constexpr bool kFold = WT == BM_IQ2XXS || WT == BM_IQ3XXS;
     static constexpr int kOff = WT == BM_IQ2XXS ? 43 : 64;
     static constexpr int kLanes = WT == BM_Q3K ? 1 : 8;
+    static constexpr int kPlanes = WT == BM_Q3K ? 1 : 2; // signed bytes a weight-side term takes
     static constexpr int kBlock = WT == BM_IQ2XXS ? BM_IQ2XXS_BLOCK : WT == BM_IQ3XXS ? BM_IQ3XXS_BLOCK : WT == BM_IQ4XS ? BM_IQ4XS_BLOCK : BM_Q3K_BLOCK;
 };
 
@@ -925,7 +943,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     [[maybe_unused]] const Iq2Tables tb = stage_tables<WT>(lds + sizeof(GemmLds));
     uint8_t *a_codes = lds + sizeof(GemmLds) + tab_bytes<WT>();
     uint8_t *w_hi = a_codes + 64 * kIqStride;
-    uint8_t *w_lo = w_hi + 64 * kIqStride;
+    uint8_t *w_lo = w_hi + (G::kPlanes - 1) * 64 * kIqStride; // (the one plane where there is one)
     float *dy_t = reinterpret_cast<float *>(w_lo + 64 * kIqStride); // [slot]
     float *d_t = dy_t + 64;                                          // [row]
     float *bs_t = d_t + 64;                                          // [l][slot] the 32-value sums, as floats
@@ -1096,10 +1114,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
                 for (int t = 0; t < 8; t++) { // cells 4 t .. 4 t + 3: lane t
                     const int sc = (int)((sword >> (8 * (2 * (f & 1) + (t >> 2)))) & 0xffu) - 32;
                     const u32 low = (qs[t] >> (2 * f)) & 0x03030303u, high = (hm[t] >> (4 * j + f)) & 0x01010101u;
-                    const u32 v = __builtin_amdgcn_perm(0x03020100u, 0xfffefdfcu, (high << 2) | low); // u - 4
-                    u32 h, lo;
-                    iq_planes_signed(v, sc, h, lo);
-                    put(t, h, lo);
+                    v2us even, odd;
+                    iq_products((high << 2) | low, -4, -sc, even, odd);
+                    *reinterpret_cast<u32 *>(w_lo + wr * kIqStride + 32 * t + 4 * b) = iq_low_bytes(even, odd);
                 }
             }
         }
@@ -1149,16 +1166,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
         }
         if constexpr (G::kLanes == 1) {
             // Q3_K: one integer a super-block, then acc + (dcol d) sum, each operation rounded on its own
-            v16i hs = z, ls = z;
+            v16i neg = z;
 #pragma unroll
-            for (int l = 0; l < 8; l++) {
-                const v4i b = *reinterpret_cast<const v4i *>(my_a + 32 * l);
-                hs = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_h + 32 * l), b, hs, 0, 0, 0);
-                ls = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_l + 32 * l), b, ls, 0, 0, 0);
-            }
+            for (int l = 0; l < 8; l++)
+                neg = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_l + 32 * l),
+                                                            *reinterpret_cast<const v4i *>(my_a + 32 * l), neg, 0, 0, 0);
 #pragma unroll
             for (int v = 0; v < 16; v++)
-                acc[0][v] = __fadd_rn(acc[0][v], __fmul_rn(__fmul_rn(dy, dd[v]), (float)(hs[v] * 256 + ls[v])));
+                acc[0][v] = __fadd_rn(acc[0][v], __fmul_rn(__fmul_rn(dy, dd[v]), (float)-neg[v]));
         } else {
             if constexpr (G::kFold) {
                 // the fold of the offsets first: accumulator l takes sub-block l's scale on its two sums

@@ -404,6 +404,46 @@ def test_gemm_fast_iq2xxs_at_the_edges(gpu, rpe, k, counts):
         b.free()
 
 
+@pytest.mark.parametrize("wtype", (bm.Q3_K, bm.IQ4_XS))
+def test_gemm_terms_at_the_ends_of_their_range(gpu, wtype):
+    """The weight-side terms of the grouped GEMM at the ends of their range: rows whose scales are all -32 or all 31 against codes
+    that are all the lowest, all the highest or any (Q3_K: -4 x -32 = 128 is the one term that a signed byte holds only negated),
+    with columns of one sign and of both."""
+    from test_gpu_decode import random_blocks
+    rpe, k, n_experts, n_slots = 96, 512, 2, 40
+    rng = np.random.default_rng(2950)
+    bb = ora.BLOCK_BYTES[wtype]
+    w = random_blocks(wtype, n_experts * rpe, k, rng).reshape(n_experts * rpe, k // 256, bb)
+    scales = slice(96, 108) if wtype == bm.Q3_K else slice(2, 8)
+    codes = slice(0, 96) if wtype == bm.Q3_K else slice(8, 136)
+    for r in range(n_experts * rpe):
+        if r % 3:
+            w[r, :, scales] = (0, 255)[r % 3 - 1]
+        if r // 3 % 3:
+            w[r, :, codes] = (0, 255)[r // 3 % 3 - 1]
+    w = w.reshape(-1)
+    ids = rng.integers(0, n_experts, n_slots).astype(np.uint32)
+    x = normal_f32(rng, (n_slots, k))
+    x[:8] = np.sign(x[:8])
+    x[8:16] = 1.0
+    x[16:24] = -1.0
+    dw, act = gpu.weights(wtype, n_experts * rpe, k, w), gpu.act(wtype, k, n_slots)
+    xd, sel = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32)
+    table = gpu.route(n_slots, n_experts)
+    y = gpu.buffer(np.float32, n_slots * rpe).fill_bytes(0xFF)
+    gpu.enqueue_quantize(xd, n_slots, act)
+    table.fill(sel, n_slots)
+    gpu.enqueue_gemm(dw, rpe, act, table, 0, y)
+    got = y.download().reshape(n_slots, rpe)
+    rb = ora.row_bytes(wtype, k)
+    for s in range(n_slots):
+        e = int(ids[s])
+        want = ora.gemv(wtype, w[e * rpe * rb:(e + 1) * rpe * rb], rpe, k, ora.quantize_col(wtype, x[s]), 1)
+        assert_f32(got[s], want, f"slot {s}")
+    for b in (dw, act, xd, sel, table, y):
+        b.free()
+
+
 def test_gemm_at_the_largest_route(gpu):
     """The route's limits (crates/gpu/src/gemm/mod.rs:97-101): 40960 slots over 1024 experts, one column a slot, with
     runs from empty to many tiles; every slot's 16 rows against the one-column dot, and the table by definition."""
