@@ -80,16 +80,17 @@ __global__ __launch_bounds__(256) void k_quantize_q82x4(const float *x, int m, i
     q82_store(act + (size_t)col * (k / 256) * BM_Q82_SB_EXT, k / 256, blk, lane32, code, hd, s16);
 }
 
-// x: m columns of k values -> Q8_K columns (crates/qdot/src/lib.rs:1787-1809). One workgroup a 256-value block.
+// x: m columns of k values -> Q8_K columns (crates/qdot/src/lib.rs:1787-1809). A wave a 256-value block.
 // sel (optional): column c belongs to slot c; a slot whose id names no expert of the stack (served elsewhere, or refused) keeps
 // its column as it stands and raises nothing here: its rows of x need not hold anything.
 __global__ __launch_bounds__(256) void k_quantize_q8k(const float *x, int m, int k, uint8_t *act, const u32 *live,
                                                       const u32 *sel, u32 n_experts, u32 *fault, u32 layer) {
-    const int bpc = k / 256;
-    const int col = blockIdx.x / bpc, blk = blockIdx.x % bpc;
-    if (live && (u32)col >= *live) return;
+    const u32 bpc = (u32)k / 256u, gblk = blockIdx.x * 4u + (u32)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (gblk >= (u32)m * bpc) return;
+    const u32 col = gblk / bpc, lane = threadIdx.x & 63;
+    if (live && col >= *live) return;
     if (sel && sel[col] >= n_experts) return;
-    q8k_block_by_workgroup(x[(size_t)col * k + 256 * blk + threadIdx.x], act + ((size_t)col * bpc + blk) * BM_Q8K_STRIDE, fault, layer);
+    q8k_wave_block(bm_ld4f(x + (size_t)gblk * 256 + 4 * lane), act + (size_t)gblk * BM_Q8K_STRIDE, (int)lane, fault, layer);
 }
 
 // The same columns with eight values a thread, a block a quad of lanes (two 16-byte loads a thread, fewer and fatter
@@ -118,7 +119,7 @@ hipError_t quantize(const Launch &L, int wtype, const float *x, int m, int k, ui
         return hipGetLastError();
     }
     if (bm_takes_q8k(wtype)) {
-        hipLaunchKernelGGL(k_quantize_q8k, dim3((unsigned)(m * (k / 256))), dim3(256), 0, L.stream, x, m, k, act,
+        hipLaunchKernelGGL(k_quantize_q8k, dim3(((unsigned)m * (unsigned)(k / 256) + 3) / 4), dim3(256), 0, L.stream, x, m, k, act,
                            live, sel, n_experts, L.fault, L.layer);
     } else {
         const long blocks = (long)m * (k / 32);

@@ -444,6 +444,29 @@ def test_gemm_terms_at_the_ends_of_their_range(gpu, wtype):
         b.free()
 
 
+@pytest.mark.parametrize("m,k", ((1, 256), (3, 768), (5, 1792), (130, 512)))
+@pytest.mark.parametrize("shift", (0, 1, 3))
+def test_q8k_columns_at_any_f32_address(gpu, m, k, shift):
+    """The Q8_K quantizers where their split ends: block counts that are no multiple of a workgroup's four, rows that start at any f32
+    address, the first of equal magnitudes, an all-zero block: the bytes of the oracle."""
+    rng = np.random.default_rng(2960 + m)
+    x = normal_f32(rng, (m, k))
+    x[0, 7], x[0, 200] = -9.0, 9.0
+    x[m - 1, k - 256:] = 0.0
+    pad = lambda a: gpu.upload(np.concatenate([np.zeros(shift, np.float32), a.reshape(-1)]), np.float32)
+    xd, ones = pad(x), pad(np.ones_like(x))
+    act, act_h = gpu.act(bm.IQ4_XS, k, m), gpu.act(bm.IQ4_XS, k, m)
+    gpu.enqueue_quantize(xd.ptr + 4 * shift, m, act)
+    # silu(x) x 1, and the same values through the quantizer alone
+    gpu.enqueue_swiglu_quant(xd.ptr + 4 * shift, ones.ptr + 4 * shift, m, act_h)
+    h = ora.swiglu(x.reshape(-1), np.ones(m * k, np.float32)).reshape(m, k)
+    for c in range(m):
+        assert bytes(act.download(c)) == bytes(ora.quantize_col(bm.IQ4_XS, x[c])), f"column {c}"
+        assert bytes(act_h.download(c)) == bytes(ora.quantize_col(bm.IQ4_XS, h[c])), f"column {c} of h"
+    for b in (xd, ones, act, act_h):
+        b.free()
+
+
 def test_gemm_at_the_largest_route(gpu):
     """The route's limits (crates/gpu/src/gemm/mod.rs:97-101): 40960 slots over 1024 experts, one column a slot, with
     runs from empty to many tiles; every slot's 16 rows against the one-column dot, and the table by definition."""
