@@ -1039,7 +1039,14 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     // GEMM's launches in the exact order give the same bits sooner (us a layer, tile launches / GEMM: hidden 2048, ff 768, top-8 of 128
     // Q4_K 128 tokens 192 / 210, 192: 240 / 236, 333: 368 / 275; hidden 4096, ff 1536, top-2 of 32, 192: 292 / 216; hidden 2048, ff
     // 1024, top-2 of 8, 64: 63 / 57; hidden 3072, ff 512, top-6 of 256, 128: 240 / 266, 192: 277 / 270, 256: 340 / 278).
-    const bool gemm_ahead = n_slots >= 12 * n_experts || (m >= 192 && n_slots >= 4 * n_experts);
+    // A gate on Q8_K columns of a type whose GEMM unpacks in few instructions, from 24 tokens on: from four slots an expert (Q3_K) or
+    // eight (IQ4_XS, IQ3_XXS), a down stack of these types counted likewise (hidden 2048, ff 768, top-8 of 128, Q3_K / Q4_K, 64 tokens
+    // 182 / 170, 80: 235 / 178, IQ4_XS 80: 270 / 245, 95: 235 / 247; hidden 4096, ff 1024, top-2 of 24, 48 tokens Q3_K / Q4_K 135 / 120,
+    // IQ4_XS 146 / 157, 95: IQ4_XS 199 / 165, IQ3_XXS / IQ4_XS 231 / 194; hidden 7168, ff 2048, top-8 of 32, IQ4_XS 32 tokens 761 / 561).
+    auto q8k_slots = [](int t) { return t == BM_TYPE_IQ4_XS || t == BM_TYPE_IQ3_XXS ? 8 : t == BM_TYPE_IQ2_XXS ? 12 : 4; };
+    const bool q8k_ahead = act_form(s->gate_type) != 0 && m >= 24 &&
+                           n_slots >= (q8k_slots(s->gate_type) > q8k_slots(s->down_type) ? q8k_slots(s->gate_type) : q8k_slots(s->down_type)) * n_experts;
+    const bool gemm_ahead = n_slots >= 12 * n_experts || (m >= 192 && n_slots >= 4 * n_experts) || q8k_ahead;
     if (path == BM_PATH_GROUPED && s->path == BM_PATH_AUTO && !s->own_cut && gemm_ahead && bmk::gemm_supported(s->gate_type) &&
         bmk::gemm_supported(s->down_type))
         path = BM_PATH_GEMM, mode = BM_GEMM_EXACT;

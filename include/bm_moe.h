@@ -385,7 +385,8 @@ int bm_swiglu_quant_sel(bm_ctx *ctx, const float *g_dev, const float *u_dev, con
  * either mode where the gate/up stack dots against Q8_K columns: Q3_K, IQ2_XXS, IQ3_XXS, IQ4_XS; where the down stack does so
  * too and hidden x ff is 2^23 or more, the grouped path from the first token). On the grouped path a batch with no more slots
  * than experts whose h crosses in f32 rows takes the per-slot gate . up launch (over columns made in the tables' launch) and
- * the tile launch for down; one of at least 12 slots an expert (or of 192 tokens and 4 slots an expert), where the crossovers are
+ * the tile launch for down; one of at least 12 slots an expert (or of 192 tokens and 4 slots an expert,
+ * or, with a gate of Q3_K, IQ3_XXS or IQ4_XS, of 24 tokens and 4 or 8 slots an expert), where the crossovers are
  * the defaults, takes the GEMM's launches in the exact order.
  * bm_scratch_set_path sets others (0 keeps a value; gemm_from then holds for both modes) or forces one path.
  * bm_scratch_path_for: the path a call with m tokens takes. A slot whose id names no expert of the stack adds nothing to

@@ -55,6 +55,34 @@ def test_every_path_gives_the_oracles_bits(gpu, types, hidden, ff, n_experts, to
         L.free()
 
 
+@pytest.mark.parametrize("types,n_experts,top_k,tokens", (
+    ((bm.Q3_K, bm.Q3_K, bm.Q4_K), 24, 4, (23, 24, 25)),           # four slots an expert
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 13, 4, (24, 25, 26, 39)),  # eight
+    ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 12, 3, (24, 31, 32)),         # the down stack's eight
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 8, 3, (24, 31, 32)),       # twelve
+))
+def test_the_automatic_choice_gives_the_oracles_bits_where_it_changes(gpu, types, n_experts, top_k, tokens):
+    hidden, ff, m = 512, 768, max(tokens)
+    L = Layer(gpu, types, hidden, ff, n_experts, 5300)
+    rng = np.random.default_rng(5301)
+    x = normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    want, _ = L.oracle(x, ids, wts, top_k)
+    xd, sel, wd = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.upload(wts, np.float32)
+    y = gpu.buffer(np.float32, m * hidden)
+    sc = gpu.scratch(types[0], types[2], hidden, ff, n_experts, top_k, m)
+    try:
+        for n in tokens:
+            y.fill_bytes(0xFF)
+            gpu.enqueue_moe_forward(sc, L.dg, L.du, L.dd, xd, sel, wd, None, n, y)
+            assert_f32(y.download()[:n * hidden], want.reshape(-1)[:n * hidden], f"{n} tokens")
+    finally:
+        sc.free()
+        for b in (xd, sel, wd, y):
+            b.free()
+        L.free()
+
+
 def test_the_automatic_choice_follows_the_crossovers(gpu):
     sc = gpu.scratch(bm.Q4_K, bm.Q6_K, 2048, 768, 128, 8, 4096)
     try:
