@@ -5,6 +5,13 @@
 // f16, so is a, so one v_mfma_f32_32x32x16_f16 does what takes two int8 products on split bytes, and the sum stays in its f32
 // accumulators for the whole super-block: one multiply-add a (row, slot, super-block) is all that is left of the scaling.
 //
+// The sum is the exact integer, rounded once where it becomes the multiply-add's operand, as an int32 sum would be. An f32 accumulator
+// holds it exactly while every partial sum is at most 2^24, which sum |a| <= 2^24 / 1333 over the column's block guarantees: the
+// staging adds the |a| up beside its conversions, and a super-block with a column past that (about one in 2 x 10^5 blocks of normal
+// values, every block whose values have one magnitude) is summed again by `wide_block`, which closes into integers every
+// 64 terms (64 x 1333 x 128 < 2^24). The guard is some twenty of 750 vector instructions a super-block: 2 to 5 % of the kernel, 2.3 %
+// of the layer below (2.28 -> 2.33 ms).
+//
 // Bound by the vector ALU, which makes the terms, 17 instructions for eight values a lane, with LDS (the grid, the columns) and the
 // weights' scattered lines close behind: an expert has about as many slots as one tile, so every weight is unpacked about once
 // and used for one 32- or 64-slot product. So:
@@ -27,6 +34,7 @@
 namespace bmk {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -44,8 +52,10 @@ struct IqLds {
     uint8_t grid[kGridBytes];
     uint8_t cols[2][kIqCols];
     float dy[2][64];
+    u32 mag[2][4][64]; // sum |a| of a column's block, in as many parts as thread quads stage it
     GemmLds tab;
 };
+constexpr u32 kIqMagMax = (1u << 24) / (31u * 43u);
 
 // (x & mask) | bits in one instruction; from the plain expression the compiler makes two.
 __device__ __forceinline__ u32 iq_and_or(u32 x, u32 mask, u32 bits) {
@@ -65,15 +75,17 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
     const u32 row_bytes = (u32)nb * BM_IQ2XXS_BLOCK, col_bytes = (u32)nb * BM_Q8K_STRIDE;
     // What a thread stages of a super-block: one or two runs of sixteen codes of one column.
     const int sc = NCT == 2 ? (tid >> 2) & 63 : (tid >> 2) & 31, sq = (tid & 3) + 4 * (NCT == 2 ? tid >> 8 : tid >> 7);
-    const u32 src = L->tab.col[sc] * col_bytes + 8u + 16u * (u32)sq, src_dy = L->tab.col[sc] * col_bytes;
+    const u32 src = L->tab.col[sc] * col_bytes + 8u + 16u * (u32)sq;
     const LdsB my_put = (LdsB)lds + kGridBytes + sc * kIqColStride + 32 * sq;
+    constexpr int kMagParts = 4 / NCT;
+    u32 mag; // sum |a| of what this thread stages
     constexpr int kPieces = NCT; // of sixteen codes: NCT 2: pieces sq and sq + 8 of the sixteen, NCT 1: piece sq
     v4u ra[kPieces];
     float cdy = 0.0f;
     auto fetch_cols = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < kPieces; q++) __builtin_memcpy(&ra[q], act + (src + (u32)i * BM_Q8K_STRIDE) + 128 * q, 16);
-        cdy = *reinterpret_cast<const float *>(act + (src_dy + (u32)i * BM_Q8K_STRIDE));
+        cdy = *reinterpret_cast<const float *>(act + (src + (u32)i * BM_Q8K_STRIDE) - 8); // (the block's scale where sq is 0, else unused)
     };
     const u32 k1024 = 0x64006400u, m8 = 0x00ff00ffu, msign = 0x80008000u;
     auto less_1152 = [](u32 x) {
@@ -82,8 +94,20 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
     };
     auto stash_word = [&](int at, int k) __attribute__((always_inline)) { // of 4 kPieces; `at`: the buffer
         const u32 u = ra[k >> 2][k & 3] ^ 0x80808080u;
+        mag = __builtin_amdgcn_sad_u8(u, 0x80808080u, k ? mag : 0u);
         *(__attribute__((address_space(3))) v2u *)(my_put + at + 256 * (k >> 2) + 8 * (k & 3)) =
             (v2u){less_1152(iq_and_or(u, m8, k1024)), less_1152(iq_and_or(u >> 8, m8, k1024))};
+    };
+
+    auto mag_quad = [&]() __attribute__((always_inline)) { // over the quad of lanes, 64 or 128 codes of one column
+        mag += (u32)__builtin_amdgcn_mov_dpp((int)mag, 0xb1, 0xf, 0xf, true); // lane ^ 1
+        mag += (u32)__builtin_amdgcn_mov_dpp((int)mag, 0x4e, 0xf, 0xf, true); // lane ^ 2
+    };
+    auto stash_ends = [&](int buf) __attribute__((always_inline)) { // the sum, and the column's scale
+        if ((sq & 3) == 0) {
+            L->mag[buf][sq >> 2][sc] = mag;
+            if (sq == 0) L->dy[buf][sc] = cdy;
+        }
     };
 
     const int l32 = lane & 31, kh = lane >> 5;
@@ -117,39 +141,104 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
         d[0] = kh ? other : mine;
         d[1] = kh ? mine : other;
     };
-    // step t of sixteen: eight values of index byte t % 4 of the lane's sub-block t / 4
-    auto lookup = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const u32 at = __builtin_amdgcn_perm(raw[r][t >> 3][2 * ((t >> 2) & 1)], my_copy, 0x0c0c0000u | ((4u + (u32)(t & 3)) << 8));
-            gr[r][0] = *(LdsV2)((LdsB)lds + at);
-            gr[r][1] = *(LdsV2)((LdsB)lds + at + 128);
-        }
+    // The eight values that byte j of an index word stands for: the grid's magnitudes, and with signs and scale from the other word.
+    auto grid_of = [&](u32 index, int j, v2u(&half)[2]) __attribute__((always_inline)) {
+        const u32 at = __builtin_amdgcn_perm(index, my_copy, 0x0c0c0000u | ((4u + (u32)j) << 8));
+        half[0] = *(LdsV2)((LdsB)lds + at);
+        half[1] = *(LdsV2)((LdsB)lds + at + 128);
     };
-    auto scale_of = [&](int t, int r) __attribute__((always_inline)) {
-        const u32 s = raw[r][t >> 3][2 * ((t >> 2) & 1) + 1] >> 28;
-        // 1024 + 2 s + 1 less 1024
-        const u32 x = (2u * s) | 0x6401u, b = x | (x << 16);
+    auto scale_of = [&](u32 aux) __attribute__((always_inline)) { // 1024 + 2 s + 1 less 1024
+        const u32 x = (2u * (aux >> 28)) | 0x6401u, b = x | (x << 16);
         const _Float16 k = (_Float16)1024.0f;
-        scale[r] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, b) - (v2h){k, k});
+        return __builtin_bit_cast(u32, __builtin_bit_cast(v2h, b) - (v2h){k, k});
     };
-    auto make = [&](int t, int r) __attribute__((always_inline)) {
-        if ((t & 3) == 0) scale_of(t, r);
-        const u32 aux = raw[r][t >> 3][2 * ((t >> 2) & 1) + 1];
-        const u32 v = (aux >> (7 * (t & 3))) & 127u;
+    auto terms_of = [&](u32 aux, int j, const v2u(&half)[2], u32 scale_pair) __attribute__((always_inline)) {
+        const u32 v = (aux >> (7 * j)) & 127u;
         const u32 v8 = v | ((u32)__builtin_popcount(v) << 7); // bit 7: the parity
         u32 s = v8 | (v8 << 14); // bits 0, 1, 4, 5 and sixteen on: the signs of values 0, 1, 4, 5 and 2, 3, 6, 7
         __asm__("" : "+v"(s));   // (else the shifts below become multiplications, four times as slow)
-        const u32 m[4] = {iq_and_or(s << 15, msign, gr[r][0].x), iq_and_or(s << 14, msign, gr[r][0].y), iq_and_or(s << 11, msign, gr[r][1].x),
-                          iq_and_or(s << 10, msign, gr[r][1].y)};
+        const u32 m[4] = {iq_and_or(s << 15, msign, half[0].x), iq_and_or(s << 14, msign, half[0].y), iq_and_or(s << 11, msign, half[1].x),
+                          iq_and_or(s << 10, msign, half[1].y)};
+        v4u out;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-            term[t & 1][r][k] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, m[k]) * __builtin_bit_cast(v2h, scale[r]));
+        for (int k = 0; k < 4; k++) out[k] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, m[k]) * __builtin_bit_cast(v2h, scale_pair));
+        return out;
+    };
+    // step t of sixteen: eight values of index byte t % 4 of the lane's sub-block t / 4
+    auto lookup = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) grid_of(raw[r][t >> 3][2 * ((t >> 2) & 1)], t & 3, gr[r]);
+    };
+    auto make = [&](int t, int r) __attribute__((always_inline)) {
+        const u32 aux = raw[r][t >> 3][2 * ((t >> 2) & 1) + 1];
+        if ((t & 3) == 0) scale[r] = scale_of(aux);
+        term[t & 1][r] = terms_of(aux, t & 3, gr[r], scale[r]);
     };
     auto read_col = [&](int at, int t, int c) __attribute__((always_inline)) {
         const LdsB p = my_col + at + 32 * kIqColStride * c + 16 * t;
         const v2u a = *(LdsV2)p, b = *(LdsV2)(p + 8);
         colv[c] = (v4u){a.x, a.y, b.x, b.y};
+    };
+
+    // A super-block's rows asked for and made ready, none of it in the shade of products: a slab's first one, and around a wide one.
+    auto rows_of = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 5; n++) fetch_raw(i, n);
+        deal(0);
+        deal(1);
+        lookup(0);
+        make(0, 0);
+        make(0, 1);
+        lookup(1);
+    };
+    // the super-block's scaled sums into the accumulators of slot group c
+    auto scale_sums = [&](int buf, int c) __attribute__((always_inline)) {
+        const float *dy = L->dy[buf];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const v4f y4 = *reinterpret_cast<const v4f *>(dy + 32 * c + 8 * q + 4 * kh);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int r = 0; r < 2; r++) acc[r][c][4 * q + k] = fmaf(d[r] * y4[k], sum[r][c][4 * q + k], acc[r][c][4 * q + k]);
+        }
+    };
+    u32 mag_all; // sum |a| of a column of the super-block at hand
+    auto read_mag = [&](int buf) __attribute__((always_inline)) {
+        const int col = NCT == 2 ? lane : l32;
+        mag_all = L->mag[buf][0][col];
+#pragma unroll
+        for (int p = 1; p < kMagParts; p++) mag_all += L->mag[buf][p][col];
+    };
+    // The sums of such a super-block, closed into integers every 64 terms. (A loop that stays one: unrolled, what its passes have in
+    // common was kept in registers that the products behind it do not leave.)
+    auto wide_block = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < NCT; c++)
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                v16i whole = {};
+#pragma nounroll
+                for (int n = 0; n < 4; n++) {
+                    const v4u words = n < 2 ? raw[r][0] : raw[r][1];
+                    const u32 index = n & 1 ? words.z : words.x, aux = n & 1 ? words.w : words.y, by = scale_of(aux);
+                    const LdsB col = my_col + buf * kIqCols + 32 * kIqColStride * c + 64 * n;
+                    v16f part = {};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        v2u half[2];
+                        grid_of(index, j, half);
+                        const v2u a0 = *(LdsV2)(col + 16 * j), a1 = *(LdsV2)(col + 16 * j + 8);
+                        const v4u a = {a0.x, a0.y, a1.x, a1.y}, b = terms_of(aux, j, half, by);
+                        part = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), part, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; v++) whole[v] += (int)part[v];
+                }
+#pragma unroll
+                for (int v = 0; v < 16; v++) sum[r][c][v] = (float)whole[v];
+                __builtin_amdgcn_sched_barrier(0);
+            }
     };
 
     for (int left = (int)slabs; left > 0 && row0 < rpe; left--, row0 += kIqWgRows) {
@@ -164,18 +253,12 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[r][c][v] = 0.0f;
         }
-#pragma unroll
-        for (int n = 0; n < 5; n++) fetch_raw(0, n);
         fetch_cols(0);
-        deal(0);
-        deal(1);
-        lookup(0);
-        make(0, 0);
-        make(0, 1);
-        lookup(1);
+        rows_of(0);
 #pragma unroll
         for (int k = 0; k < 4 * kPieces; k++) stash_word(0, k);
-        if (sq == 0) L->dy[0][sc] = cdy;
+        mag_quad();
+        stash_ends(0);
         __syncthreads();
         for (int i = 0; i < nb; i++) {
             const int next = i + 1 < nb ? i + 1 : i, now_at = (i & 1) * kIqCols, next_at = kIqCols - now_at; // the last one's staging has no reader
@@ -200,7 +283,6 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
                 if (t < 15) read_col(now_at, t + 1, 0);
                 if (t < 5) fetch_raw(next, t); // (one a step: a run of them fills the address unit's queue and stops the wave)
                 if (t >= 16 - 4 * kPieces) stash_word(next_at, t - (16 - 4 * kPieces));
-                if (t == 15 && sq == 0) L->dy[(i + 1) & 1][sc] = cdy;
                 __builtin_amdgcn_sched_barrier(0);
                 if (NCT == 2) product(0, NCT - 1);
                 make((t + 1) & 15, 1);
@@ -210,20 +292,21 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
                 // (a half's words are done with when step 6, or 14, has made the last terms of them)
                 if (t == 12) deal(0);
                 if (t == 15) deal(1);
+                if (t == 14) read_mag(i & 1);
                 lookup((t + 2) & 15);
+                if (t == 15) {
+                    mag_quad();
+                    stash_ends((i + 1) & 1);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            const float *dy = L->dy[i & 1];
+            if (__ballot(mag_all > kIqMagMax)) { // a column whose sums may have passed 2^24: the same answer in every wave
+                rows_of(i);
+                wide_block(i & 1);
+                rows_of(next);
+            }
 #pragma unroll
-            for (int c = 0; c < NCT; c++)
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const v4f y4 = *reinterpret_cast<const v4f *>(dy + 32 * c + 8 * q + 4 * kh);
-#pragma unroll
-                    for (int k = 0; k < 4; k++)
-#pragma unroll
-                        for (int r = 0; r < 2; r++) acc[r][c][4 * q + k] = fmaf(d[r] * y4[k], sum[r][c][4 * q + k], acc[r][c][4 * q + k]);
-                }
+            for (int c = 0; c < NCT; c++) scale_sums(i & 1, c);
             __syncthreads();
         }
 #pragma unroll

@@ -404,6 +404,73 @@ def test_gemm_fast_iq2xxs_at_the_edges(gpu, rpe, k, counts):
         b.free()
 
 
+def fma_f32(a, b, c):
+    """fl32(a b + c) with one rounding: the product of two f32 is exact in f64, the sum is rounded to odd there, which f32 rounding sees through."""
+    p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)
+    s = p + c
+    t = s - p
+    err = (p - (s - t)) + (c - t)
+    to_odd = (err != 0) & ((s.view(np.int64) & 1) == 0)
+    return np.where(to_odd, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s).astype(np.float32)
+
+
+@pytest.mark.parametrize("rpe,k,counts", ((80, 256, (40, 70)), (1040, 768, (2,) * 66 + (64, 40)), (576, 1792, (1, 30, 33))))
+def test_gemm_fast_iq2xxs_block_sums_are_exact(gpu, rpe, k, counts):
+    """The tolerance mode's sum over a super-block is the exact integer rounded to f32 once, whatever its size: rows of large terms of
+    one sign against columns of large codes of one sign (sums to 4e7, past the 2^24 that an f32 accumulator counts to), columns whose
+    codes are large and of both signs, one such super-block among ordinary ones, and ordinary columns beside them in the same tile.
+    The value is then fma(fl(d / 8 dy), fl(sum), acc) in the super-blocks' order, bit for bit."""
+    from test_gpu_decode import random_blocks
+    n_experts, n_slots, nb = len(counts), sum(counts), k // 256
+    rng = np.random.default_rng(2900 + rpe)
+    w = random_blocks(bm.IQ2_XXS, n_experts * rpe, k, rng).reshape(n_experts, rpe, nb, 66)
+    grid = np.zeros((8, 66), np.uint8)
+    grid[:, :2] = np.array([8.0], np.float16).view(np.uint8)  # d / 8 = 1: a value is its integer term
+    grid[:, 2:].reshape(8, 8, 8)[..., :4] = np.arange(256).reshape(8, 8, 4)
+    big = np.argsort(ora.dequant_row(bm.IQ2_XXS, grid.reshape(-1), 2048).reshape(256, 8).sum(1))[-64:].astype(np.uint8)
+    large = w[:, ::2, :, 2:].reshape(n_experts, -1, nb, 8, 8)
+    large[..., :4] = rng.choice(big, large[..., :4].shape)  # the grid's largest entries
+    large[..., 4:7] = 0                                     # no signs
+    large[..., 7] = 0xF0                                    # scale 31
+    w[:, ::2, :, 2:] = large.reshape(n_experts, -1, nb, 64)
+    ids = rng.permutation(np.repeat(np.arange(n_experts), counts)).astype(np.uint32)
+    x = normal_f32(rng, (n_slots, k))
+    even = rng.uniform(0.9, 1.0, (n_slots, k)).astype(np.float32)
+    x[1::4] = even[1::4] * np.sign(x[1::4, :1])
+    x[2::4] = even[2::4] * np.sign(x[2::4])
+    x[3::4, -256:] = even[3::4, -256:]
+    dw, act = gpu.weights(bm.IQ2_XXS, n_experts * rpe, k, w.reshape(-1)), gpu.act(bm.IQ2_XXS, k, n_slots)
+    xd, sel, y = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.buffer(np.float32, n_slots * rpe)
+    table = gpu.route(n_slots, n_experts)
+    gpu.enqueue_quantize(xd, n_slots, act)
+    table.fill(sel, n_slots)
+    y.fill_bytes(0xFF)
+    gpu.set_gemm_mode(bm.GEMM_FAST)
+    try:
+        gpu.enqueue_gemm(dw, rpe, act, table, 0, y)
+    finally:
+        gpu.set_gemm_mode(bm.GEMM_EXACT)
+    got = y.download().reshape(n_slots, rpe)
+    past = 0
+    for e in sorted(range(n_experts), key=lambda e: counts[e])[-3:]:
+        d8 = w[e, :, :, :2].copy().view(np.float16)[..., 0].astype(np.float32) * np.float32(0.125)
+        unit = w[e].copy()
+        unit[:, :, :2] = grid[0, :2]
+        terms = np.stack([ora.dequant_row(bm.IQ2_XXS, unit[r].reshape(-1), k) for r in range(rpe)]).astype(np.int64)
+        for s in np.flatnonzero(ids == e):
+            blocks = act.download(int(s)).reshape(nb, 296)
+            dy, codes = blocks[:, :4].copy().view(np.float32)[:, 0], blocks[:, 8:264].view(np.int8).astype(np.int64)
+            want = np.zeros(rpe, np.float32)
+            for i in range(nb):
+                total = terms[:, 256 * i:256 * i + 256] @ codes[i]
+                past += int(np.count_nonzero(np.abs(total) > 1 << 24))
+                want = fma_f32(d8[:, i] * dy[i], total.astype(np.float32), want)
+            assert_f32(got[s], want, f"slot {s}")
+    assert past > 0
+    for b in (dw, act, xd, sel, table, y):
+        b.free()
+
+
 @pytest.mark.parametrize("wtype", (bm.Q3_K, bm.IQ4_XS))
 def test_gemm_terms_at_the_ends_of_their_range(gpu, wtype):
     """The weight-side terms of the grouped GEMM at the ends of their range: rows whose scales are all -32 or all 31 against codes
