@@ -1,4 +1,5 @@
-// Prefill, tolerance mode (BM_GEMM_FAST): the grouped expert GEMM of IQ2_XXS stacks on the f16 matrix cores.
+// Prefill, tolerance mode (BM_GEMM_FAST): the grouped expert GEMM of IQ2_XXS stacks on the f16 matrix cores. (Launches too small
+// for its workgroups go to k_gemm_iq's int8 form: the line is in gemm, bm_prefill.hip.)
 //
 // A row against a Q8_K column is, a super-block, (d / 8) dy times sum over the 256 values of ((2 s + 1) g) a: g = +-8, 25 or 43 the
 // grid's value, 2 s + 1 the sub-block's scale, a the column's code. The term (2 s + 1) g is an integer of at most 1333 and exact in

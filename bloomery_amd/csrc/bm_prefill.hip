@@ -10,6 +10,7 @@
 // bm_device.hpp. The integer sums of each 16-value group come out of the matrix cores exactly, and each enters the f32 accumulator
 // of the CPU path's lane that owns it, in the CPU path's order (crates/qdot/src/lib.rs:4363-4447 Q4_K, :4776-4874 Q6_K): eight accumulators a
 // value, the min term first, then the groups in increasing k, and the closing sum (t0 + t2) + (t1 + t3).
+#include <algorithm>
 #include <type_traits>
 
 #include "bm_gemm.hpp"
@@ -877,15 +878,18 @@ __global__ __launch_bounds__(kFastThreads, 2) void k_gemm_fast(const uint8_t *w,
 // 31 * 86 = 2666: too wide for an int8 operand, so each is split into two signed bytes, 256 h + lo with lo = the low byte
 // read as signed and h = (term + 128) >> 8 (0 .. 10), and the dot is two v_mfma_i32_32x32x32_i8 whose sums meet as
 // (H << 8) + L, exactly. The LDS copy of a row's (and a column's) super-block is laid out lane-major, [l][b][i], so a matrix
-// operand is 16 consecutive bytes. The eight accumulators and
-// their order are the CPU path's, bit for bit (the value bm_gemv_sel gives).
+// operand is 16 consecutive bytes. With EXACT the eight accumulators and their order are the CPU path's, bit for bit (the value
+// bm_gemv_sel gives); without it (IQ2_XXS, the tolerance mode's small launches: see gemm below) one accumulator takes d dy times the
+// super-block's whole sum sum_b (2 s_b + 1) sum_n (u - 43) a, the 43s taken out in integers through two more matrix instructions over
+// the column's 32-value sums (split into two bytes the same way).
 // A workgroup of four waves takes 64 rows and a tile's 64 slots, a wave 32 x 32 of them.
 constexpr int kIqRows = 64;
 constexpr int kIqStride = 256 + 16; // bytes a row's or a column's 256 codes take in LDS
 constexpr int kIqLine = 64 + 4;     // floats a line of the per-lane tables
-template <int WT>
+template <int WT, bool EXACT = true>
 __host__ __device__ constexpr size_t gemm_iq_lds_bytes() {
-    return sizeof(GemmLds) + (size_t)tab_bytes<WT>() + (WT == BM_Q3K ? 2 : 3) * (size_t)64 * kIqStride + 2 * 64 * sizeof(float) + 2 * 8 * kIqLine * sizeof(float);
+    return sizeof(GemmLds) + (size_t)tab_bytes<WT>() + (WT == BM_Q3K ? 2 : 3) * (size_t)64 * kIqStride + 2 * 64 * sizeof(float) +
+           (EXACT ? 2 * 8 * kIqLine * sizeof(float) : 3 * 64 * 16);
 }
 
 // (2 s + 1) u for the four code bytes of `u`, each product split into the signed low byte (lo) and what is left over 256
@@ -933,7 +937,7 @@ __device__ __forceinline__ void iq_planes_signed(u32 v, int sc, u32 &hi, u32 &lo
 //   Q3_K: terms scale x (u - 4) over the sixteen 16-value groups, -124 .. 128 and so, negated, one signed byte: one plane and one
 //     product instead of two (with the products above: the same layer in Q3_K / Q4_K 367 -> 300 us). One integer a super-block and
 //     one accumulator, the float step acc + (dcol d) sum with every operation rounded on its own (crates/qdot/src/lib.rs:2223-2245).
-// (The tolerance mode has a kernel of its own for IQ2_XXS and runs the three others in this order too.)
+// (EXACT only for the three others: the tolerance mode runs them in this order too.)
 template <int WT>
 struct IqGemm {
     static constexpr bool kFold = WT == BM_IQ2XXS || WT == BM_IQ3XXS;
@@ -943,10 +947,11 @@ struct IqGemm {
     static constexpr int kBlock = WT == BM_IQ2XXS ? BM_IQ2XXS_BLOCK : WT == BM_IQ3XXS ? BM_IQ3XXS_BLOCK : WT == BM_IQ4XS ? BM_IQ4XS_BLOCK : BM_Q3K_BLOCK;
 };
 
-template <int WT>
+template <int WT, bool EXACT = true>
 __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
                                                     const u32 *tiles, const u32 *n_tiles, u32 n_units, u32 slot_div,
                                                     u32 n_slots, float *y, const uint8_t *w_second, float *y_second) {
+    static_assert(EXACT || WT == BM_IQ2XXS, "the one-accumulator form is IQ2_XXS's");
     using G = IqGemm<WT>;
     extern __shared__ __align__(16) uint8_t lds[];
     GemmLds *tab = reinterpret_cast<GemmLds *>(lds);
@@ -956,8 +961,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     uint8_t *w_lo = w_hi + (G::kPlanes - 1) * 64 * kIqStride; // (the one plane where there is one)
     float *dy_t = reinterpret_cast<float *>(w_lo + 64 * kIqStride); // [slot]
     float *d_t = dy_t + 64;                                          // [row]
-    float *bs_t = d_t + 64;                                          // [l][slot] the 32-value sums, as floats
-    float *sc_t = bs_t + 8 * kIqLine;                                // [l][row] the scales 2 s + 1, as floats
+    float *bs_t = d_t + 64;                                          // EXACT: [l][slot] the 32-value sums, as floats
+    float *sc_t = bs_t + 8 * kIqLine;                                // EXACT: [l][row] the scales 2 s + 1, as floats
+    uint8_t *x_sc = reinterpret_cast<uint8_t *>(d_t + 64);           // else: [row][16] the scales as bytes, zeros behind
+    uint8_t *x_bl = x_sc + 64 * 16;                                  // [slot][16] the sums' low bytes, zeros behind
+    uint8_t *x_bh = x_bl + 64 * 16;                                  // [slot][16] what is left of the sums over 256
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const u32 g = tile_of_block(blockIdx.x, n_units);
     const int row0 = (int)take_stack(slab_of_block(blockIdx.x, n_units), n_units, w, y, w_second, y_second) * kIqRows;
@@ -1054,16 +1062,27 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
         if (tid < 64) {
             dy_t[tid] = cdy;
             const u32 bw[8] = {cb0.x, cb0.y, cb0.z, cb0.w, cb1.x, cb1.y, cb1.z, cb1.w};
+            [[maybe_unused]] u32 bl[2] = {0, 0}, bh[2] = {0, 0};
 #pragma unroll
             for (int l = 0; l < 8; l++) { // the two 16-value sums of sub-block l
                 const int bs = (int)(short)(bw[l] & 0xffffu) + (int)(short)(bw[l] >> 16);
-                if constexpr (G::kFold) bs_t[l * kIqLine + tid] = (float)bs;
+                if constexpr (EXACT) {
+                    if constexpr (G::kFold) bs_t[l * kIqLine + tid] = (float)bs;
+                } else { // 256 hi + lo with lo the low byte read as signed
+                    bl[l >> 2] |= ((u32)bs & 0xffu) << (8 * (l & 3));
+                    bh[l >> 2] |= ((u32)((bs + 128) >> 8) & 0xffu) << (8 * (l & 3));
+                }
+            }
+            if constexpr (!EXACT) {
+                *reinterpret_cast<uint4 *>(x_bl + 16 * tid) = make_uint4(bl[0], bl[1], 0u, 0u);
+                *reinterpret_cast<uint4 *>(x_bh + 16 * tid) = make_uint4(bh[0], bh[1], 0u, 0u);
             }
         }
         if (wq == 0) {
             const float dh = bm_half_to_f32((unsigned short)rd);
             d_t[wr] = WT == BM_IQ2XXS ? 0.125f * dh : WT == BM_IQ3XXS ? 0.25f * dh : dh;
         }
+        [[maybe_unused]] u32 scs[2] = {0, 0};
 #pragma unroll
         for (int e2 = 0; e2 < 2; e2++) {
             const int b = 2 * wq + e2;
@@ -1076,7 +1095,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
             if constexpr (WT == BM_IQ2XXS || WT == BM_IQ3XXS) {
                 const u32 aux = WT == BM_IQ2XXS ? (e2 ? rq.w : rq.y) : (e2 ? rx.y : rx.x);
                 const u32 sc = 2u * (aux >> 28) + 1u;
-                sc_t[b * kIqLine + wr] = (float)sc;
+                if constexpr (EXACT) sc_t[b * kIqLine + wr] = (float)sc;
+                else scs[e2] = sc;
 #pragma unroll
                 for (int q = 0; q < 4; q++) { // values 8 q .. 8 q + 7: lanes 2 q and 2 q + 1
                     u32 c_lo, c_hi;
@@ -1130,6 +1150,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
                 }
             }
         }
+        if constexpr (!EXACT) { // the row's eight scales as bytes: the thread of sub-blocks 2 wq, 2 wq + 1 writes its two
+            *reinterpret_cast<unsigned short *>(x_sc + 16 * wr + 2 * wq) = (unsigned short)(scs[0] | (scs[1] << 8));
+            if (wq == 0) *reinterpret_cast<uint2 *>(x_sc + 16 * wr + 8) = make_uint2(0u, 0u);
+        }
     };
 
     // this lane in its wave's 32 x 32 product: operand row / slot lane % 32, terms 16 (lane / 32) .. of the 32; result v
@@ -1141,7 +1165,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     const uint8_t *my_a = a_codes + (wslot + l32) * kIqStride + 16 * kh;
     const bool live = wslot < len; // else none of this wave's slots is real
     const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    constexpr int kAcc = G::kLanes;
+    constexpr int kAcc = EXACT ? G::kLanes : 1;
     v16f acc[kAcc];
 #pragma unroll
     for (int l = 0; l < kAcc; l++)
@@ -1151,7 +1175,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     // (the columns' bytes too where the registers allow: the exact forms of the types with eight accumulators a value have few
     // to spare - with everything held over they spilled and ran 6 % slower - so there only the rows' bytes, which come from
     // HBM, are asked for ahead, and the columns', which the cache holds, when their turn comes)
-    constexpr bool kColsAhead = G::kLanes == 1;
+    constexpr bool kColsAhead = kAcc == 1;
     fetch_rows(0);
     if constexpr (kColsAhead) fetch_cols(0);
     for (int i = 0; i < nb; i++) {
@@ -1184,6 +1208,26 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
 #pragma unroll
             for (int v = 0; v < 16; v++)
                 acc[0][v] = __fadd_rn(acc[0][v], __fmul_rn(__fmul_rn(dy, dd[v]), (float)-neg[v]));
+        } else if constexpr (!EXACT) {
+            v16i hs = z, ls = z;
+#pragma unroll
+            for (int l = 0; l < 8; l++) {
+                const v4i b = *reinterpret_cast<const v4i *>(my_a + 32 * l);
+                hs = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_h + 32 * l), b, hs, 0, 0, 0);
+                ls = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_l + 32 * l), b, ls, 0, 0, 0);
+            }
+            // sum_b (2 s_b + 1) (the sub-block's sum of a): the scales against the sums' two bytes, terms 8 .. 31 zero
+            const v4i zero4 = {0, 0, 0, 0};
+            const v4i xs = kh ? zero4 : *reinterpret_cast<const v4i *>(x_sc + 16 * (wrow + l32));
+            const v4i xl = kh ? zero4 : *reinterpret_cast<const v4i *>(x_bl + 16 * (wslot + l32));
+            const v4i xh = kh ? zero4 : *reinterpret_cast<const v4i *>(x_bh + 16 * (wslot + l32));
+            const v16i ml = __builtin_amdgcn_mfma_i32_32x32x32_i8(xs, xl, z, 0, 0, 0);
+            const v16i mh = __builtin_amdgcn_mfma_i32_32x32x32_i8(xs, xh, z, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int total = ((hs[v] << 8) + ls[v]) - 43 * ((mh[v] << 8) + ml[v]);
+                acc[0][v] = fmaf(dd[v] * dy, (float)total, acc[0][v]);
+            }
         } else {
             if constexpr (G::kFold) {
                 // the fold of the offsets first: accumulator l takes sub-block l's scale on its two sums
@@ -1224,7 +1268,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const int v = 4 * q4 + k;
-                    if constexpr (G::kLanes == 8) { // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order)
+                    if constexpr (kAcc == 8) { // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order)
                         const float t0 = acc[0][v] + acc[4][v], t1 = acc[1][v] + acc[5][v];
                         const float t2 = acc[2][v] + acc[6][v], t3 = acc[3][v] + acc[7][v];
                         r[k] = (t0 + t2) + (t1 + t3);
@@ -1262,8 +1306,17 @@ hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int
     if (wtype == BM_IQ4XS) return launch(k_gemm_iq<BM_IQ4XS>, 256, kIqRows, gemm_iq_lds_bytes<BM_IQ4XS>());
     if (wtype == BM_Q3K) return launch(k_gemm_iq<BM_Q3K>, 256, kIqRows, gemm_iq_lds_bytes<BM_Q3K>());
     if (wtype == BM_IQ2XXS) {
-        if (mode != 0)
+        // The tolerance mode: 512-row workgroups that unpack in registers, one a compute unit, or, where those leave the chip's places
+        // empty, the int8 form's 64-row workgroups, a sixth as long each. Tiles go to the eight dies in turn, so what counts is the
+        // 64-row workgroups of the fullest die's 32 compute units, here in tiles as ids without a favourite would make them; the
+        // line lies at three and a half a unit (the int8 form / the other, us, one stack; 64: k 512 8.3 / 15.1, k 2048 23.7 / 35.9,
+        // k 7168 73.6 / 117; 96: 14.0 / 18.2, 38.2 / 45.0, 122 / 144; 112: 17.8 / 20.2, 47.3 / 49.1, 148 / 136; 128 with tiles of at
+        // most 32 slots: 15.1 / 15.5, 44.7 / 41.6, 143 / 119; 160: 18.7 / 15.7, 57.2 / 42.5, 183 / 118).
+        const u32 est_tiles = std::max((u32)std::min(n_experts, n_slots), (u32)n_slots / kGemmBN + (u32)n_experts / 2);
+        const u32 die_units = (est_tiles + 7) / 8 * stacks * (u32)((rows_per_expert + kIqRows - 1) / kIqRows);
+        if (mode != 0 && die_units > 112u)
             return gemm_iq2_fast(L, w, n_experts, rows_per_expert, k, act, cols, tiles_dev, n_tiles, n_slots, slot_div, y, w_second, y_second);
+        if (mode != 0) return launch(k_gemm_iq<BM_IQ2XXS, false>, 256, kIqRows, gemm_iq_lds_bytes<BM_IQ2XXS, false>());
         return launch(k_gemm_iq<BM_IQ2XXS>, 256, kIqRows, gemm_iq_lds_bytes<BM_IQ2XXS>());
     }
     if (mode == 2 && gemm_half_supported(wtype)) { // the f16 form of the tolerance mode, where the type has one

@@ -404,6 +404,15 @@ def test_gemm_fast_iq2xxs_at_the_edges(gpu, rpe, k, counts):
         b.free()
 
 
+@pytest.mark.parametrize("rpe,k,counts", ((16, 256, (1,) * 1000 + (64,) + (2,) * 23), (560, 512, (31, 32, 33) + (1,) * 118),
+                                          (1040, 768, (65, 5, 0, 97) + (2,) * 60), (512, 1792, (63, 2) + (1,) * 132),
+                                          (1024, 512, (4,) * 52 + (8,) * 4), (1024, 512, (4,) * 53 + (8,) * 4)))
+def test_gemm_fast_iq2xxs_at_the_edges_of_many_workgroups(gpu, rpe, k, counts):
+    """The same edges in launches large enough for the 512-row workgroups (the int8 form takes the small ones), and a launch on
+    each side of the line between the two."""
+    test_gemm_fast_iq2xxs_at_the_edges(gpu, rpe, k, counts)
+
+
 def fma_f32(a, b, c):
     """fl32(a b + c) with one rounding: the product of two f32 is exact in f64, the sum is rounded to odd there, which f32 rounding sees through."""
     p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)
@@ -418,7 +427,8 @@ def fma_f32(a, b, c):
 def test_gemm_fast_iq2xxs_block_sums_are_exact(gpu, rpe, k, counts):
     """The tolerance mode's sum over a super-block is the exact integer rounded to f32 once, whatever its size: rows of large terms of
     one sign against columns of large codes of one sign (sums to 4e7, past the 2^24 that an f32 accumulator counts to), columns whose
-    codes are large and of both signs, one such super-block among ordinary ones, and ordinary columns beside them in the same tile.
+    codes are large and of both signs, one such super-block among ordinary ones, and ordinary columns beside them in the same tile;
+    the second shape by the f16 form's 512-row workgroups, the others by the int8 form.
     The value is then fma(fl(d / 8 dy), fl(sum), acc) in the super-blocks' order, bit for bit."""
     from test_gpu_decode import random_blocks
     n_experts, n_slots, nb = len(counts), sum(counts), k // 256
