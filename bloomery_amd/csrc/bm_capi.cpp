@@ -1,6 +1,7 @@
 // The C ABI of libbm_moe_hip.so (include/bm_moe.h): handles, the host-side geometry checks the reference's
 // launchers make before a launch (crates/gpu/src/q4k_sel.rs:990-1042 and its siblings), and the calls into the
 // kernels. Refusals carry a message naming the entry point and the lengths, as GpuError::Shape does.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -899,8 +900,7 @@ struct bm_scratch {
     float *g, *u, *down;           // f32 rows: g (also the per-slot and grouped paths' h) and u of slots x ff, down of slots x hidden
     uint32_t *order, *start, *tiles; // the grouped table
     bm_route *route;               // the GEMM path's table
-    int path, grouped_from, gemm_from, gemm_from_fast;
-    bool own_cut; // gemm_from set by the caller
+    int path, grouped_from, gemm_from; // gemm_from: the caller's, 0 for the measured rule (path_choice)
 };
 
 void bm_scratch_destroy(bm_scratch *s) {
@@ -936,21 +936,10 @@ int bm_scratch_create(bm_ctx *ctx, int gate_type, int down_type, int hidden, int
     s->ctx = ctx;
     s->gate_type = gate_type, s->down_type = down_type, s->hidden = hidden, s->ff = ff, s->n_experts = n_experts;
     s->spt = n_slots_per_token, s->max_tokens = max_tokens;
-    // the crossovers measured on MI355X at the Qwen3-30B-A3B layer shape (Q4_K gate/up, Q6_K down, top-8 of 128):
-    // tokens   per slot   grouped   GEMM exact   GEMM tolerance mode   (us a step)
-    //     16       67        86        190          118
-    //     24       92        88        217          130
-    //    128      400       188        336          201
-    //    192      580       246        370          214
-    //    256      767       296        392          230
-    //    512     1491       534        481          289
-    s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 448, s->gemm_from_fast = 96, s->own_cut = false;
-    // a gate/up stack on Q8_K columns (Q3_K, IQ2_XXS, IQ3_XXS, IQ4_XS): its tile launchers are bound by the type's decode, which
-    // the GEMM does once a row and super-block for all of a tile's slots, so the exact GEMM is ahead much earlier (same layer
-    // shape, us a step, grouped / GEMM: IQ4_XS 48 tokens 180 / 170, 96 tokens 265 / 185, 2048 tokens 3202 / 907; IQ2_XXS 64
-    // tokens 168 / 196, 96 tokens 230 / 212, 2048 tokens 2682 / 995; IQ3_XXS 96 tokens 241 / 215; Q3_K 24 tokens 112 / 103)
-    if (act_form(gate_type) != 0) s->gemm_from = 96;
-    // ... and where the down stack is on Q8_K columns too and the experts are large, the grouped step - for few slots an
+    // the per-slot step below 22 tokens (Q4_K gate/up, Q6_K down, top-8 of 128, hidden 2048, ff 768, us a step, per slot / grouped:
+    // 16 tokens 67 / 86, 24: 92 / 88, 128: 400 / 188), then by path_choice
+    s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 0;
+    // Where both stacks are on Q8_K columns and the experts are large, the grouped step - for few slots an
     // expert the per-slot gate . up launch and the down tiles, see bm_moe_forward - is ahead of the per-slot step from the first
     // token: every workgroup of the per-slot down launch encodes all of a token's h rows itself, work that grows with hidden x ff
     // (DeepSeek-V3 shape, hidden 7168, ff 2048, IQ2_XXS, us a step per slot / grouped: 1 token 61.5 / 57.9, 4 tokens 171 / 147,
@@ -994,7 +983,7 @@ int bm_scratch_set_path(bm_scratch *s, int path, int grouped_from, int gemm_from
         return fail(s->ctx, BM_ESHAPE, "%s: the crossovers are token counts (0: keep), got %d and %d", what, grouped_from, gemm_from);
     s->path = path;
     if (grouped_from) s->grouped_from = grouped_from;
-    if (gemm_from) s->gemm_from = s->gemm_from_fast = gemm_from, s->own_cut = true;
+    if (gemm_from) s->gemm_from = gemm_from;
     return BM_OK;
 }
 
@@ -1006,17 +995,66 @@ static bool per_slot_fits(const bm_scratch *s) {
     return lds_a <= (size_t)bmk::kMaxLds && lds_b <= (size_t)bmk::kMaxLds;
 }
 
-int bm_scratch_path_for(const bm_scratch *s, int m) {
-    if (!s || m < 1 || m > s->max_tokens) return BM_ESHAPE;
+// Whether the GEMM's launches (exact order) are ahead of the tile launches for m tokens. With v the weights of one matrix of an expert
+// in 2^20, the tile launches' time goes with v x (half the tiles of eight slots and half an eighth of the slots: a tile's rows are
+// decoded once and dotted with the slots it has), the GEMM's with v x the tiles of 64 slots of the fullest of the eight dies (a tile's
+// workgroups run on one die; an expert of few slots costs it a whole tile), and the GEMM has a constant more for its launches. Tiles
+// are counted as ordinary routes make them: an expert's last one half full, no fewer than one an expert; with about a slot an
+// expert the tile launches are ahead whatever else. Where eight columns are short enough to leave LDS for more workgroups the K types' and
+// Q3_K's tile launches are about a third cheaper; the other types are bound by their decode. The numbers are a fit to 2032 measured pairs (1 to 256 experts, 22 to 3000 tokens, hidden 1024 to 7168,
+// cold weights): the chosen side is 0.5 % behind the better one on average and 35 % at worst, where "from 12 slots an expert, and
+// from 448 or 96 tokens on always" was 6 % behind, and twice as slow for one large expert of few slots (a shared expert). Some
+// of the pairs, us a layer, tile launches / GEMM:
+//   hidden 2048, ff 768, top-8 of 128:  Q4_K 128 tokens 182 / 232, 192: 237 / 252, 256: 282 / 257, 447: 446 / 297
+//                                       Q5_K 128 tokens 204 / 232, 192: 263 / 249; Q6_K 192: 270 / 266
+//                                       IQ4_XS 64 tokens 188 / 194, 95: 214 / 202; Q3_K / Q4_K 24: 96 / 107, 48: 148 / 132
+//                                       IQ2_XXS 128 tokens 240 / 287, 192: 319 / 308; IQ3_XXS 95: 201 / 251, 192: 355 / 293
+//   one expert, hidden 7168, ff 2048:   Q6_K 22 tokens 83 / 169, 64: 146 / 177, 95: 206 / 171, 256: 471 / 173
+//                                       IQ2_XXS 22 tokens 99 / 187, 95: 199 / 197, 192: 339 / 199
+//   hidden 7168, ff 1536, top-4 of 8:   Q4_K 22 tokens 197 / 141, 64: 405 / 145
+//   hidden 7168, ff 2048, top-8 of 256: IQ2_XXS 64 tokens 1762 / 2819, 192: 3546 / 3618
+//   hidden 2048, ff 768, top-2 of 256:  Q4_K 500 tokens 191 / 301, 1500: 437 / 399; IQ2_XXS 230: 143 / 281
+static bool gemm_ahead(const bm_scratch *s, int m) {
+    struct Line {
+        double launches, die, fits; // the GEMM's constant, what a 64-slot tile on the die costs, the factor of short columns
+        double short_hidden;        // up to here whole, gone at half as much again
+    };
+    const Line line = s->gate_type == BM_TYPE_IQ2_XXS    ? Line{6.5, 12.0, 1.0, 2560.0}
+                      : s->gate_type == BM_TYPE_IQ3_XXS   ? Line{0.0, 9.5, 1.0, 2560.0}
+                      : s->gate_type == BM_TYPE_IQ4_XS    ? Line{-9.0, 7.0, 1.0, 2560.0}
+                      : s->gate_type == BM_TYPE_Q3_K      ? Line{0.0, 3.6, 0.73, 4096.0}
+                      : act_form(s->down_type) != 0       ? Line{-6.0, 9.0, 0.85, 2560.0}
+                                                          : Line{3.0, 9.1, s->gate_type == BM_TYPE_Q4_K ? 0.65 : 0.7, 2560.0};
+    const double v = (double)s->hidden * s->ff / (1 << 20), n = (double)m * s->spt, experts = s->n_experts;
+    if (n < 1.5 * experts) return false;
+    const double past = std::min(1.0, std::max(0.0, 2.0 * (s->hidden / line.short_hidden - 1.0)));
+    const double tiles = v * std::max(experts / 2 + n / 16, n / 8 + experts / 4) * (line.fits + (1.0 - line.fits) * past);
+    return tiles > line.launches + line.die * v * std::ceil(std::max(experts, n / 64 + experts / 2) / 8);
+}
+
+// The path a call with m tokens takes, and the f32 order of its GEMMs: the one place where it is chosen.
+struct PathChoice {
+    int path, mode;
+};
+static PathChoice path_choice(const bm_scratch *s, int m) {
     const bool gemm_ok = bmk::gemm_supported(s->gate_type) && bmk::gemm_supported(s->down_type);
     const bool per_slot_ok = m <= bmk::kMaxDecodeTokens && per_slot_fits(s);
-    if (s->path != BM_PATH_AUTO) {
-        if (s->path == BM_PATH_PER_SLOT && !per_slot_ok) return BM_PATH_GROUPED;
-        return s->path;
-    }
-    if (m < s->grouped_from && per_slot_ok) return BM_PATH_PER_SLOT;
-    if (m < (s->ctx->gemm_mode != BM_GEMM_EXACT ? s->gemm_from_fast : s->gemm_from) || !gemm_ok) return BM_PATH_GROUPED;
-    return BM_PATH_GEMM;
+    const int mode = s->ctx->gemm_mode;
+    if (s->path == BM_PATH_PER_SLOT) return {per_slot_ok ? BM_PATH_PER_SLOT : BM_PATH_GROUPED, mode};
+    if (s->path != BM_PATH_AUTO) return {s->path, mode};
+    if (m < s->grouped_from && per_slot_ok) return {BM_PATH_PER_SLOT, mode};
+    if (!gemm_ok) return {BM_PATH_GROUPED, mode};
+    if (s->gemm_from) return {m >= s->gemm_from ? BM_PATH_GEMM : BM_PATH_GROUPED, mode}; // the caller's
+    // The tolerance mode: from 96 tokens on in its own f32 order, and where the gate has kernels of that order (Q4_K, Q5_K, Q6_K,
+    // IQ2_XXS) then always by the GEMM (789 pairs of 95 to 800 tokens: 1.4 % behind the better side on average); below, the exact order.
+    const bool fast = mode != BM_GEMM_EXACT && m >= 96;
+    const bool fast_gate = act_form(s->gate_type) == 0 || s->gate_type == BM_TYPE_IQ2_XXS;
+    return {(fast && fast_gate) || gemm_ahead(s, m) ? BM_PATH_GEMM : BM_PATH_GROUPED, fast ? mode : BM_GEMM_EXACT};
+}
+
+int bm_scratch_path_for(const bm_scratch *s, int m) {
+    if (!s || m < 1 || m > s->max_tokens) return BM_ESHAPE;
+    return path_choice(s, m).path;
 }
 
 int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_weights *wu, const bm_weights *wd,
@@ -1034,23 +1072,8 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     if (m < 1 || m > s->max_tokens) return fail(ctx, BM_ESHAPE, "%s: m = %d tokens, the scratch holds 1..=%d", what, m, s->max_tokens);
     const int spt = s->spt, n_slots = m * spt, hidden = s->hidden, ff = s->ff, n_experts = s->n_experts;
     const bool down_q8k = act_form(s->down_type) != 0;
-    int path = bm_scratch_path_for(s, m), mode = ctx->gemm_mode;
-    // The grouped range's upper part, where it is the default cut's: from 12 slots an expert, or 192 tokens with at least four, the
-    // GEMM's launches in the exact order give the same bits sooner (us a layer, tile launches / GEMM: hidden 2048, ff 768, top-8 of 128
-    // Q4_K 128 tokens 192 / 210, 192: 240 / 236, 333: 368 / 275; hidden 4096, ff 1536, top-2 of 32, 192: 292 / 216; hidden 2048, ff
-    // 1024, top-2 of 8, 64: 63 / 57; hidden 3072, ff 512, top-6 of 256, 128: 240 / 266, 192: 277 / 270, 256: 340 / 278).
-    // A gate on Q8_K columns of a type whose GEMM unpacks in few instructions, from 24 tokens on: from four slots an expert (Q3_K) or
-    // eight (IQ4_XS, IQ3_XXS), a down stack of these types counted likewise (hidden 2048, ff 768, top-8 of 128, Q3_K / Q4_K, 64 tokens
-    // 182 / 170, 80: 235 / 178, IQ4_XS 80: 270 / 245, 95: 235 / 247; hidden 4096, ff 1024, top-2 of 24, 48 tokens Q3_K / Q4_K 135 / 120,
-    // IQ4_XS 146 / 157, 95: IQ4_XS 199 / 165, IQ3_XXS / IQ4_XS 231 / 194; hidden 7168, ff 2048, top-8 of 32, IQ4_XS 32 tokens 761 / 561).
-    auto q8k_slots = [](int t) { return t == BM_TYPE_IQ4_XS || t == BM_TYPE_IQ3_XXS ? 8 : t == BM_TYPE_IQ2_XXS ? 12 : 4; };
-    const bool q8k_ahead = act_form(s->gate_type) != 0 && m >= 24 &&
-                           n_slots >= (q8k_slots(s->gate_type) > q8k_slots(s->down_type) ? q8k_slots(s->gate_type) : q8k_slots(s->down_type)) * n_experts;
-    const bool gemm_ahead = n_slots >= 12 * n_experts || (m >= 192 && n_slots >= 4 * n_experts) || q8k_ahead;
-    if (path == BM_PATH_GROUPED && s->path == BM_PATH_AUTO && !s->own_cut && gemm_ahead && bmk::gemm_supported(s->gate_type) &&
-        bmk::gemm_supported(s->down_type))
-        path = BM_PATH_GEMM, mode = BM_GEMM_EXACT;
-    switch (path) {
+    const PathChoice choice = path_choice(s, m);
+    switch (choice.path) {
     case BM_PATH_PER_SLOT:
         return bm_moe_decode(ctx, wg, wu, wd, x_dev, sel_dev, w_dev, resid_dev, spt, m, rule, s->act_h, nullptr,
                              down_q8k ? s->g : nullptr, y_dev);
@@ -1087,9 +1110,9 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     }
     default: {
         int rc = bm_route_fill_quantize(ctx, sel_dev, n_slots, s->route, x_dev, m, s->act_x);
-        if (!rc) rc = gemm_over(ctx, "bm_gemm", wg, ff, s->act_x, s->route, spt, s->g, mode, wu, s->u);
+        if (!rc) rc = gemm_over(ctx, "bm_gemm", wg, ff, s->act_x, s->route, spt, s->g, choice.mode, wu, s->u);
         if (!rc) rc = bm_swiglu_quant_sel(ctx, s->g, s->u, sel_dev, n_experts, n_slots, rule, s->act_h);
-        if (!rc) rc = gemm_over(ctx, "bm_gemm", wd, hidden, s->act_h, s->route, 0, s->down, mode);
+        if (!rc) rc = gemm_over(ctx, "bm_gemm", wd, hidden, s->act_h, s->route, 0, s->down, choice.mode);
         if (rc) return rc;
         break;
     }

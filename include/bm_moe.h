@@ -380,15 +380,15 @@ int bm_swiglu_quant_sel(bm_ctx *ctx, const float *g_dev, const float *u_dev, con
  * In the exact mode all three give the same bits in y_dev. bm_scratch holds what the paths need between their launches for
  * up to max_tokens tokens (made at load time and shared by every layer of the same shape, as the reference's Q8Act scratch
  * is): max_tokens * n_slots_per_token <= 40960. BM_PATH_AUTO (the default) takes the per-slot path below grouped_from
- * tokens, the grouped path below gemm_from and the GEMM from there; the defaults are the crossovers measured on MI355X at
- * the Qwen3-30B-A3B layer shape: 22 tokens, and 448 tokens in the exact mode of bm_gemm or 96 in its tolerance mode (96 in
- * either mode where the gate/up stack dots against Q8_K columns: Q3_K, IQ2_XXS, IQ3_XXS, IQ4_XS; where the down stack does so
- * too and hidden x ff is 2^23 or more, the grouped path from the first token). On the grouped path a batch with no more slots
- * than experts whose h crosses in f32 rows takes the per-slot gate . up launch (over columns made in the tables' launch) and
- * the tile launch for down; one of at least 12 slots an expert (or of 192 tokens and 4 slots an expert,
- * or, with a gate of Q3_K, IQ3_XXS or IQ4_XS, of 24 tokens and 4 or 8 slots an expert), where the crossovers are
- * the defaults, takes the GEMM's launches in the exact order.
- * bm_scratch_set_path sets others (0 keeps a value; gemm_from then holds for both modes) or forces one path.
+ * tokens: 22, measured on MI355X at the Qwen3-30B-A3B layer shape, or 1 where both stacks dot against Q8_K columns (Q3_K,
+ * IQ2_XXS, IQ3_XXS, IQ4_XS) and hidden x ff is 2^23 or more. From there on it takes the grouped path or the GEMM, whichever a
+ * rule fitted to measurements of both expects to be ahead for the types, the shape, the number of experts and of slots (the
+ * GEMM from 196 tokens at that layer shape, from 76 for one large expert with a slot a token). In the tolerance mode of bm_gemm the
+ * GEMM is taken from 96 tokens on where the gate/up type has kernels of that mode; below 96 tokens a GEMM path runs in the exact order.
+ * On the grouped path a batch with no more slots than experts whose h crosses in f32 rows takes the per-slot gate . up launch (over
+ * columns made in the tables' launch) and the tile launch for down.
+ * bm_scratch_set_path sets crossovers of the caller's own (0 keeps what is; gemm_from then holds for both modes, in the mode's own
+ * f32 order) or forces one path.
  * bm_scratch_path_for: the path a call with m tokens takes. A slot whose id names no expert of the stack adds nothing to
  * the sum and raises BM_SITE_EXPERT_ID unless it is BM_HOST_SLOT, which every path skips silently (the GEMM path's route
  * table does not list it, and its SwiGLU quantizer is bm_swiglu_quant_sel). Calls that share a scratch must not overlap. */

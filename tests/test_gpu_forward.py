@@ -55,11 +55,48 @@ def test_every_path_gives_the_oracles_bits(gpu, types, hidden, ff, n_experts, to
         L.free()
 
 
+@pytest.mark.parametrize("gate,down,hidden,ff,n_experts,top_k,gemm", (
+    (bm.Q4_K, bm.Q6_K, 2048, 768, 128, 8, 196),      # many experts of few slots
+    (bm.Q6_K, bm.Q6_K, 2048, 768, 128, 8, 179),
+    (bm.Q4_K, bm.Q6_K, 3072, 512, 256, 6, 410),
+    (bm.Q6_K, bm.Q6_K, 7168, 2048, 1, 1, 73),        # one large expert: its tiles of 64 slots would leave the chip empty
+    (bm.Q5_K, bm.Q6_K, 2048, 768, 8, 2, 56),
+    (bm.Q4_K, bm.IQ4_XS, 4096, 1024, 24, 2, 79),
+    (bm.IQ3_XXS, bm.IQ4_XS, 4096, 1024, 24, 2, 91),
+    (bm.IQ2_XXS, bm.Q6_K, 2048, 768, 8, 3, 39),
+    (bm.IQ2_XXS, bm.IQ2_XXS, 7168, 2048, 256, 8, 321),
+    (bm.Q4_K, bm.Q6_K, 1024, 512, 256, 1, 3146),
+))
+def test_the_query_names_the_path_that_a_call_takes(gpu, gate, down, hidden, ff, n_experts, top_k, gemm):
+    """bm_scratch_path_for, which is what a call asks, on both sides of the count from which the GEMM's launches are expected ahead, in
+    both modes of the f32 order (the tolerance mode takes the GEMM from 96 tokens on at the latest: these gates have its kernels, but
+    for IQ3_XXS), and where the caller has set a crossover of its own."""
+    sc = gpu.scratch(gate, down, hidden, ff, n_experts, top_k, 4096)
+    first = bm.PATH_PER_SLOT if hidden * ff < 1 << 23 or gate != bm.IQ2_XXS else bm.PATH_GROUPED
+    try:
+        for mode in (bm.GEMM_EXACT, bm.GEMM_FAST):
+            gpu.set_gemm_mode(mode)
+            early = mode == bm.GEMM_FAST and gemm > 96 and gate != bm.IQ3_XXS
+            want = [first, bm.PATH_GROUPED, bm.PATH_GEMM if early else bm.PATH_GROUPED, bm.PATH_GEMM, bm.PATH_GEMM]
+            assert [sc.path_for(m) for m in (21, 22, gemm - 1, gemm, 4096)] == want
+            if early:
+                assert [sc.path_for(m) for m in (95, 96)] == [bm.PATH_GROUPED, bm.PATH_GEMM]
+        sc.set_path(bm.PATH_AUTO, 0, 4000)
+        assert [sc.path_for(m) for m in (22, gemm, 3999, 4000)] == [bm.PATH_GROUPED, bm.PATH_GROUPED, bm.PATH_GROUPED, bm.PATH_GEMM]
+    finally:
+        gpu.set_gemm_mode(bm.GEMM_EXACT)
+        sc.free()
+
+
 @pytest.mark.parametrize("types,n_experts,top_k,tokens", (
     ((bm.Q3_K, bm.Q3_K, bm.Q4_K), 24, 4, (23, 24, 25)),           # four slots an expert
     ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 13, 4, (24, 25, 26, 39)),  # eight
     ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 12, 3, (24, 31, 32)),         # the down stack's eight
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 8, 3, (24, 31, 32)),       # twelve
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 8, 3, (72, 73)),           # where the choice changes
+    ((bm.Q5_K, bm.Q5_K, bm.Q6_K), 8, 2, (89, 90)),
+    ((bm.Q4_K, bm.Q4_K, bm.IQ4_XS), 8, 4, (21, 22)),
+    ((bm.Q6_K, bm.Q6_K, bm.Q6_K), 1, 1, (193, 194)),
 ))
 def test_the_automatic_choice_gives_the_oracles_bits_where_it_changes(gpu, types, n_experts, top_k, tokens):
     hidden, ff, m = 512, 768, max(tokens)
@@ -86,7 +123,7 @@ def test_the_automatic_choice_gives_the_oracles_bits_where_it_changes(gpu, types
 def test_the_automatic_choice_follows_the_crossovers(gpu):
     sc = gpu.scratch(bm.Q4_K, bm.Q6_K, 2048, 768, 128, 8, 4096)
     try:
-        assert [sc.path_for(m) for m in (1, 21, 22, 447, 448, 4096)] == [bm.PATH_PER_SLOT, bm.PATH_PER_SLOT, bm.PATH_GROUPED,
+        assert [sc.path_for(m) for m in (1, 21, 22, 195, 196, 4096)] == [bm.PATH_PER_SLOT, bm.PATH_PER_SLOT, bm.PATH_GROUPED,
                                                                        bm.PATH_GROUPED, bm.PATH_GEMM, bm.PATH_GEMM]
         gpu.set_gemm_mode(bm.GEMM_FAST)  # the tolerance mode's GEMM is faster: its cut comes earlier
         try:
@@ -103,10 +140,11 @@ def test_the_automatic_choice_follows_the_crossovers(gpu):
         assert "bm_scratch_set_path" in str(e.value)
     finally:
         sc.free()
-    # a shape whose slot columns do not fit the per-slot step's LDS (64 slots of ff 2048) goes grouped from the first token
+    # a shape whose slot columns do not fit the per-slot step's LDS (64 slots of ff 2048) goes grouped from the first token (and by
+    # the GEMM from three: 48 slots an expert)
     sc = gpu.scratch(bm.Q4_K, bm.Q6_K, 512, 2048, 4, 64, 8)
     try:
-        assert [sc.path_for(m) for m in (1, 8)] == [bm.PATH_GROUPED, bm.PATH_GROUPED]
+        assert [sc.path_for(m) for m in (1, 2, 3, 8)] == [bm.PATH_GROUPED, bm.PATH_GROUPED, bm.PATH_GEMM, bm.PATH_GEMM]
         sc.set_path(bm.PATH_PER_SLOT)
         assert sc.path_for(1) == bm.PATH_GROUPED
     finally:
@@ -114,8 +152,8 @@ def test_the_automatic_choice_follows_the_crossovers(gpu):
     # every type has a grouped GEMM: the same cut for a layer of the added types
     sc = gpu.scratch(bm.IQ4_XS, bm.Q3_K, 512, 256, 4, 2, 512)
     try:
-        # (a gate/up stack on Q8_K columns: the exact GEMM is ahead from 96 tokens)
-        assert [sc.path_for(m) for m in (21, 95, 96, 500)] == [bm.PATH_PER_SLOT, bm.PATH_GROUPED, bm.PATH_GEMM, bm.PATH_GEMM]
+        # (a gate/up stack on Q8_K columns, four experts: the exact GEMM is ahead from where the per-slot step ends)
+        assert [sc.path_for(m) for m in (21, 22, 95, 96, 500)] == [bm.PATH_PER_SLOT] + 4 * [bm.PATH_GEMM]
         sc.set_path(bm.PATH_GEMM)
         assert sc.path_for(3) == bm.PATH_GEMM
     finally:
