@@ -223,7 +223,8 @@ struct XLds {
     static constexpr int kScales = kMins ? 4 : 8;           // lines of scale products a half
     static constexpr int kHalf = (kScales + 4) * kXLine;    // a half's factors: the scale products, and four lines of d8
     static constexpr int kMinsAt = 2 * kHalf;               // and a super-block's: eight lines of mins, eight of d8 isum
-    static constexpr int kFactors = kMinsAt + (kMins ? 16 * kXLine : 0);
+    static constexpr int kHeadsAt = kMinsAt + (kMins ? 16 * kXLine : 0); // a word a staging thread: the heads of its blocks, or-ed
+    static constexpr int kFactors = kHeadsAt + (kMins ? 4 * kXLine : 0);
     static constexpr size_t kBytes = 4 * (size_t)kXCodes + kFactors + sizeof(GemmLds);
 };
 
@@ -252,13 +253,51 @@ __device__ __forceinline__ u32 and_or(u32 x, u32 mask, u32 bits) {
     return r;
 }
 
+// One value of a Q4_K or Q5_K row against a column as a plain walk: see k_gemm.
+template <int WT>
+__device__ __forceinline__ float q45_value(const uint8_t *row, const uint8_t *col, int nb) {
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma nounroll
+    for (int i = 0; i < nb; i++) {
+        const uint8_t *blk = row + (size_t)i * bm_block_bytes<WT>(), *sc = blk + 4, *codes = blk + (WT == BM_Q5K ? 48 : 16);
+        const float *pair = reinterpret_cast<const float *>(col + (size_t)nb * BM_Q82_SB_REF + 64 * (size_t)i); // d8, d8 isum of a block
+        const float d = bm_half_to_f32((unsigned short)bm_ld2u(blk)), dmin = bm_half_to_f32((unsigned short)bm_ld2u(blk + 2));
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const int m = b < 4 ? sc[b + 4] & 63 : (sc[b + 4] >> 4) | ((sc[b] >> 6) << 4);
+            acc[b] = fmaf(pair[2 * b + 1], -(dmin * (float)m), acc[b]);
+        }
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            const int s = b < 4 ? sc[b] & 63 : (sc[b + 4] & 15) | ((sc[b - 4] >> 6) << 4);
+            const float scale = d * (float)s * pair[2 * b];
+            const int8_t *a = reinterpret_cast<const int8_t *>(col + (size_t)(2 * i + (b >> 2)) * BM_Q82X4_STRIDE + 16 + 32 * (b & 3));
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                int sum = 0;
+#pragma nounroll
+                for (int n = 16 * h; n < 16 * h + 16; n++) {
+                    const int low = (codes[32 * (b >> 1) + n] >> (4 * (b & 1))) & 15;
+                    sum += (WT == BM_Q5K ? low | (((blk[16 + n] >> b) & 1) << 4) : low) * a[n];
+                }
+                acc[4 * h + (b & 3)] = fmaf(scale, (float)sum, acc[4 * h + (b & 3)]);
+            }
+        }
+    }
+    return ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7]));
+}
+
 // A workgroup of four waves takes a slab of 64 rows and a tile's 64 slots, a wave 32 x 32 of them.
 // Per (row, slot, 16-value group) the contract is acc[l] = fma(fl(scale d8), sum, acc[l]) over eight accumulators, one fused
 // multiply-add that only the vector ALU can do. The rest is on the matrix cores: the group's integer sum comes out of
 // v_mfma_f32_32x32x16_f16 as a float (codes of at most eight bits, sums below 2^24: exact, where an int8 product needs a
 // conversion a sum), fl(scale d8) over the tile is the outer product v_mfma_f32_32x32x1_2b_f32 (two blocks, or Q6_K's two
 // groups, an instruction; a product plus zero is the product's rounding), and a min term fma(d8 isum, min, acc) is the same
-// instruction with the accumulators as its addend.
+// instruction with the accumulators as its addend. (Subnormal factors and products come out as fmaf gives them. The added zero
+// is +0, so a product of -0, which takes a scale of -0, comes out as +0; that shows where all eight accumulators of a value are
+// zeros, one of them a -0 that a min term has underflowed to: the value's sign. A super-block's d with its sign bit set is
+// what it takes, so a workgroup that has staged one, which no quantizer makes, walks its values of zero again by themselves.
+// Q6_K, without mins, never has an accumulator of -0.)
 // Bound by the vector ALU (the f32 matrix instructions run on it too, 64 cycles each; the f16 ones beside it): 32 multiply-adds a
 // wave and 32 x 32 x 32 values, 16 multiply-adds' worth of outer products and about 30 instructions of staging, 300 of the 490
 // cycles measured. The staging of a half (bytes to f16, the factors) is cut in eight pieces between the groups of the half before
@@ -386,6 +425,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
         if constexpr (kQ45 && j == 0) { // crates/gguf/src/quant.rs:620-628 get_scale_min_k4
             const float d = bm_half_to_f32((unsigned short)(rh.x & 0xffffu)), dmin = bm_half_to_f32((unsigned short)(rh.x >> 16));
             const u32 b0 = (rh.y >> (8 * p)) & 0xffu, b4 = (rh.z >> (8 * p)) & 0xffu, b8 = (rh.w >> (8 * p)) & 0xffu;
+            atomicOr((u32 *)(my_factor + X::kHeadsAt), rh.x); // (its own word: an LDS instruction in place of a register that there is not)
             factor(0, d * (float)(b0 & 63u));
             r4 = d * (float)((b8 & 15u) | ((b0 >> 6) << 4));
             factor(X::kMinsAt, -(dmin * (float)(b4 & 63u)));
@@ -501,8 +541,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
 #pragma unroll
         for (int st = 0; st < 8; st++) stash(half, st, now, next);
     };
+    const int first_row = row0;
     int left = (rpe - row0 + kGemmBM - 1) / kGemmBM; // slabs to do
     left = left < (int)slabs ? left : (int)slabs;
+    if constexpr (kQ45) factor(X::kHeadsAt, 0.0f);
     At now = {row_at(row0), 0};
     fetch_row(now, kFirst);
     fetch_col(0, kFirst, 0);
@@ -551,6 +593,22 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
 #pragma unroll
             for (int l = 0; l < 4; l++) acc[l][v] = acc[l][16 + v] = 0.0f;
         }
+    }
+    if constexpr (kQ45) {
+        u32 heads = 0u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) heads |= *(const u32 *)(lds + 4 * kXCodes + X::kHeadsAt + 4 * lane + q * kXLine);
+        if (__ballot((heads & 0x8000u) != 0u) == 0) return; // (see above)
+        const int end = row0 < rpe ? row0 : rpe;
+#pragma nounroll
+        for (int row = first_row + wrow0 + l32; row < end; row += kGemmBM)
+#pragma nounroll
+            for (int v = 0; v < 16; v++) {
+                const int n = wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
+                if (n >= len) continue;
+                float *out = y + (size_t)tab->slot[n] * rpe + row;
+                if (*out == 0.0f) *out = q45_value<WT>(we + (size_t)row * row_bytes, act + (size_t)tab->col[n] * col_bytes, nb);
+            }
     }
 }
 

@@ -521,6 +521,59 @@ def test_gemm_terms_at_the_ends_of_their_range(gpu, wtype):
         b.free()
 
 
+@pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K))
+def test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype):
+    """The exact GEMM's outer products on the matrix cores where a scale product is subnormal, underflows to zero or is a zero of either
+    sign (subnormal, zero, negative and negative-zero block scales, zero scale codes, columns at the smallest scale the quantizer
+    makes), and where a min term underflows to a negative zero: bit for bit, the sign of a zero included."""
+    from test_gpu_decode import random_blocks
+    rpe, k, n_experts, n_slots = 80, 768, 2, 70
+    rng = np.random.default_rng(2960)
+    bb, nb = ora.BLOCK_BYTES[wtype], k // 256
+    rows = n_experts * rpe
+    w = random_blocks(wtype, rows, k, rng).reshape(rows, nb, bb)
+    d_at = 208 if wtype == bm.Q6_K else 0
+    d = rng.integers(0, 1024, (rows, nb)).astype(np.uint16) | (rng.integers(0, 2, (rows, nb)).astype(np.uint16) << 15)
+    d[::4] &= 0x8001  # the smallest subnormal and zero, of either sign
+    d[1::8] = 0x8000
+    w[:, :, d_at:d_at + 2] = d[..., None].view(np.uint8).reshape(rows, nb, 2)
+    if wtype == bm.Q6_K:
+        w[::3, :, 192:208] &= 1  # scale codes 0 and 1
+    else:
+        w[:, :, 2:4] = (rng.integers(0, 3, (rows, nb)).astype(np.uint16))[..., None].view(np.uint8).reshape(rows, nb, 2)
+        w[::2, :, 4:8] = rng.integers(0, 2, (rows // 2, nb, 4))   # scale codes 0 and 1, min codes 1
+        w[::2, :, 8:12] = 1
+        w[::2, :, 12:16] = 0x10 | rng.integers(0, 2, (rows // 2, nb, 4))
+        w[1::8, :, 4:8] = 0
+        w[1::8, :, 8:12] = 1
+        w[1::8, :, 12:16] = 0x10                                  # d = -0, scale codes 0, min codes 1:
+        w[1::8, :, 2:4] = (1, 0)                                  # dmin the smallest subnormal
+        w[1::16, :, 16:] = 0
+    # (Q6_K: no subnormal d8 but the exact one below, whose rounding makes codes of -128; the CPU path counts those with the wrong sign)
+    lowest = -116 if wtype == bm.Q6_K else -128
+    x = normal_f32(rng, (n_slots, k)) * (2.0 ** rng.uniform(lowest, -100, (n_slots, 1))).astype(np.float32)
+    for s in range(0, n_slots, 3):  # blocks of sum 1 at the smallest scale: the min terms' products round to zero
+        x[s] = 0.0
+        x[s, ::32], x[s, 1::32] = np.float32(127 * 2.0 ** -127), np.float32(-126 * 2.0 ** -127)
+    x[5] = 0.0
+    ids = rng.integers(0, n_experts, n_slots).astype(np.uint32)
+    dw, act = gpu.weights(wtype, rows, k, w.reshape(-1)), gpu.act(wtype, k, n_slots)
+    xd, sel, y = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.buffer(np.float32, n_slots * rpe)
+    table = gpu.route(n_slots, n_experts)
+    gpu.enqueue_quantize(xd, n_slots, act)
+    table.fill(sel, n_slots)
+    y.fill_bytes(0xFF)
+    gpu.enqueue_gemm(dw, rpe, act, table, 0, y)
+    got, rowwise = y.download().reshape(n_slots, rpe), w.reshape(n_experts, -1)
+    want = np.stack([ora.gemv(wtype, rowwise[ids[s]], rpe, k, ora.quantize_col(wtype, x[s]), 1) for s in range(n_slots)])
+    tiny = np.abs(want) < np.finfo(np.float32).tiny
+    assert (tiny & (want != 0)).any() and (want == 0).any() and (wtype == bm.Q6_K or (np.signbit(want) & (want == 0)).any())
+    for s in range(n_slots):
+        assert_f32(got[s], want[s], f"slot {s}")
+    for b in (dw, act, xd, sel, table, y):
+        b.free()
+
+
 @pytest.mark.parametrize("m,k", ((1, 256), (3, 768), (5, 1792), (130, 512)))
 @pytest.mark.parametrize("shift", (0, 1, 3))
 def test_q8k_columns_at_any_f32_address(gpu, m, k, shift):
