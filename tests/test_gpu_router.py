@@ -326,6 +326,34 @@ def test_many_tokens_take_the_tiles_with_the_same_bits(gpu, n_experts, hidden, m
             b.free()
 
 
+@pytest.mark.parametrize("n_experts,hidden,m", ((33, 520, 650), (130, 2048, 1100), (65, 264, 4096)))
+def test_tiles_of_subnormal_products_and_signed_zeros(gpu, n_experts, hidden, m):
+    """The tiles' f32 matrix instructions where a chain of fused multiply-adds has subnormal terms and sums, underflows to either zero, or
+    adds zeros of either sign: the logits bit for bit, the sign of a zero included, against the oracle."""
+    rng = np.random.default_rng(4000 + m)
+    def small(shape):
+        return (rng.choice([-1.0, 1.0], shape) * 2.0 ** rng.uniform(-85, -62, shape)).astype(np.float32)
+    router, x = small((n_experts, hidden)), small((m, hidden))
+    router[::5] *= np.float32(2.0 ** 8)
+    x[::7] *= np.float32(2.0 ** -30)  # all of a row's products round to a zero,
+    x[::14] = -np.abs(x[::14])        # of one sign
+    router[::6] = np.abs(router[::6])
+    x[1::11] = 0.0
+    x[2::11] = -0.0
+    router[1::9] = -0.0
+    router[2::9, 8:] = 0.0
+    x[rng.random((m, hidden)) < 0.2] *= np.float32(-0.0)
+    rd, xd = gpu.upload(router, np.float32), gpu.upload(x, np.float32)
+    logits = gpu.buffer(np.float32, m * n_experts).fill_bytes(0xFF)
+    gpu.enqueue_router_logits(rd, xd, None, 1e-6, m, n_experts, hidden, None, logits)
+    _, want = ora.router_logits(router, x)
+    tiny = np.abs(want) < np.finfo(np.float32).tiny
+    assert (tiny & (want != 0)).any() and (np.signbit(want) & (want == 0)).any()
+    assert np.array_equal(logits.download().view(np.uint32), want.reshape(-1).view(np.uint32))
+    for b in (rd, xd, logits):
+        b.free()
+
+
 @pytest.mark.parametrize("n_experts,top_k", ((128, 8), (200, 6), (40, 4), (300, 8)))
 def test_norm_route_picks_among_equal_probabilities(gpu, n_experts, top_k):
     """Router rows that repeat give logits that are equal bit for bit: the fused launch's picks (by counting, for up to 256
