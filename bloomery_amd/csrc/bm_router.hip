@@ -683,8 +683,9 @@ __global__ __launch_bounds__(256) void k_norm_rows(const float *x, const float *
 // (five chunks ahead), LDS stores and LDS reads stand one by one between the matrix instructions, in whose shadow they issue.
 // Without RAGGED the loop has no branch: a branch round an LDS store (for the padding of a last chunk) cost 55 ns a store, as
 // much as four matrix instructions, so rows that are whole groups of four chunks have a form of their own.
-// Bound: LDS traffic (16-byte reads and stores run at 64 to 80 bytes a cycle; a step of 32 values moves 26 KB a workgroup, 370 cycles,
-// against 256 of matrix instructions). Two tiles of experts a wave, which halve the reads of a matrix instruction, were no faster
+// No unit is full (2048 tokens: one wave a SIMD, matrix cores busy 40 % of the cycles, LDS 23 %, vector ALU 12 %, waiting 23 %; 4096:
+// 52, 31, 15, 19 %): a wave's chain of matrix instructions, 256 cycles a step of 32 values, is stretched by the LDS accesses that stand
+// between them (26 KB a step and workgroup). Two tiles of experts a wave, which halve the reads of a matrix instruction, were no faster
 // (39.1 against 39.8 us at 4096 tokens: half the workgroups). Measured, with the norm's launch: 4096 tokens x 128 experts x 2048 values
 // 827 -> 40 us, 2048 tokens 416 -> 25, 333 tokens 71 -> 13.7, 64 tokens 16.7 -> 11.1; 1024 tokens x 256 experts x 7168 values
 // 2867 -> 64 us. The one-token workgroups of k_router_logits read and lay out the router's rows once a token.

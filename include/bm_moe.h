@@ -324,8 +324,8 @@ int bm_route_read(bm_ctx *ctx, const bm_route *route, uint32_t *cols_host, uint3
  * gemm_iq3xxs, :1248 gemm_iq4xs, :759 gemm_q3k) against Q8_K columns:
  * y_dev[s * rows_per_expert + r] = row r of expert e(s) . column c(s) of act for every slot s of the table's last
  * fill; c(s) = s / top_k (GemmInput::Shared) or s when top_k is 0 (GemmInput::PerSlot). rows_per_expert a
- * multiple of 16. Every value is bm_gemv_sel's for that slot, bit for bit; the integer sums are formed on the int8
- * matrix cores. A refused slot gets NaN in every row. */
+ * multiple of 16. Every value is bm_gemv_sel's for that slot, bit for bit; the integer sums are formed on the matrix
+ * cores, exactly (int8 products, or f16 products of integers whose sums stay below 2^24). A refused slot gets NaN in every row. */
 int bm_gemm(bm_ctx *ctx, const bm_weights *w, int rows_per_expert, const bm_act *act, const bm_route *route, int top_k,
             float *y_dev);
 /* How bm_gemm sums in f32 (the integer block sums are exact either way):
