@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256) void k_gate_up_tiles(const uint8_t *wg, const 
     const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
     const uint8_t *wrow = (which ? wu : wg) + ((size_t)t.e * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     float *hbuf = reinterpret_cast<float *>(cols + (size_t)MC * col_bytes); // [MC][32]
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256) void k_gate_up_tiles(const uint8_t *wg, const 
     for (int c0 = 0; c0 < (PASSES ? t.m : 1); c0 += MC) { // one pass, but for a tile wider than MC under PASSES
         const int mc = !PASSES ? t.m : t.m - c0 < MC ? t.m - c0 : MC;
         if (PASSES) __syncthreads(); // s_entry is written; the pass before is done with cols, hbuf and bad
-        if (PASSES && c0) preload<WT, U>(b, wrow, q);
+        if (PASSES && c0) preload<WT, U>(b, wrow, n, q);
         if (tid < MC) {
             const u32 s = tid < mc ? (PASSES ? s_entry[c0 + tid] : t.entry) : 0;
             const bool none = tid < mc && (s >= n_slots || (int)(s / slots_per_col) >= act_cols);
@@ -283,14 +283,14 @@ __global__ __launch_bounds__(256) void k_gemv_tiles(const uint8_t *w, u32 n_expe
     const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
     const uint8_t *wrow = w + ((size_t)t.e * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     u32 *slot_of = reinterpret_cast<u32 *>(cols + (size_t)MC * col_bytes); // [MC]
     for (int c0 = 0; c0 < (PASSES ? t.m : 1); c0 += MC) { // one pass, but for a tile wider than MC under PASSES
         const int mc = !PASSES ? t.m : t.m - c0 < MC ? t.m - c0 : MC;
         if (PASSES) __syncthreads(); // s_entry is written; the pass before is done with cols and slot_of
-        if (PASSES && c0) preload<WT, U>(b, wrow, q);
+        if (PASSES && c0) preload<WT, U>(b, wrow, n, q);
         if (tid < MC) {
             const u32 s = tid < mc ? (PASSES ? s_entry[c0 + tid] : t.entry) : 0;
             if (tid < mc && s >= n_slots && t.row_block == 0) bm_raise(fault, layer, kSiteExpertId);
@@ -359,7 +359,7 @@ hipError_t gate_up_tiles(const Launch &L, int wtype, const uint8_t *wg, const ui
         if (split) BM_TILE_LAUNCH(kTileNarrow, 0, false)                                                               \
         BM_TILE_LAUNCH(kTileCols, split ? kTileNarrow : 0, false)                                                      \
     }
-    BM_DISPATCH(wtype, nb)
+    BM_DISPATCH_COLS(wtype, nb)
 #undef CALL_BODY
 #undef BM_TILE_LAUNCH
     return hipGetLastError();
@@ -387,7 +387,7 @@ hipError_t gemv_tiles(const Launch &L, int wtype, const uint8_t *w, int n_expert
         if (split) BM_TILE_LAUNCH(kTileNarrow, 0, false)                                                               \
         BM_TILE_LAUNCH(kTileCols, split ? kTileNarrow : 0, false)                                                      \
     }
-    BM_DISPATCH(wtype, nb)
+    BM_DISPATCH_COLS(wtype, nb)
 #undef CALL_BODY
 #undef BM_TILE_LAUNCH
     return hipGetLastError();

@@ -176,7 +176,7 @@ __global__ __launch_bounds__(T) void k_gemv(const uint8_t *w, long rows, int nb,
     Stage<(T == 64 ? 5 : 2), T> st;
     st.load(act + (size_t)col0 * col_bytes, m * col_bytes);
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT, T>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     st.store(cols, act + (size_t)col0 * col_bytes, m * col_bytes);
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256) void k_gate_up(const uint8_t *wg, const uint8_
     Blk<WT> b[U];
     // (behind the wait for the id; nothing reads them before the column stands in LDS)
     const GateUpColLate late = bm_kernarg_at<GateUpColLate>(offsetof(GateUpColArgs, late));
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *col = lds + tab_bytes<WT>();
     st.store(col, act_col, col_bytes);
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void k_gemv_sel(const uint8_t *w, u32 n_expert
     const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
     const uint8_t *wrow = w + ((size_t)id * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *col = lds + tab_bytes<WT>();
     st.store(col, act_col, col_bytes);
@@ -488,7 +488,7 @@ __device__ __forceinline__ void down_combine_body(uint8_t *lds, const uint8_t *w
     // behind the wait for the ids, and nothing reads them before the barrier: their way through memory runs under the columns'
     __builtin_amdgcn_sched_barrier(0);
     const DownLate late = bm_kernarg_at<DownLate>(offsetof(DownArgs, late));
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     BM_TICK(t_asked, tid);
     BM_TICK(t_cols, st.v[4].x);
     st.store(cols, act_cols, spt * col_bytes);
@@ -657,7 +657,7 @@ __device__ __forceinline__ void gate_up_x_body(uint8_t *lds, const float *x, con
     // behind the wait for the id, and nothing reads them before the token's column stands in LDS: their way through memory runs
     // under the quantizer's work
     const GateUpLate late = bm_kernarg_at<GateUpLate>(offsetof(GateUpArgs, late));
-    preload<WA, UA>(b, wrow, q);
+    preload<WA, UA>(b, wrow, na, q);
     bool bad = false;
 #pragma unroll
     for (int p = 0; p < kPasses; p++) {
@@ -805,7 +805,7 @@ __global__ __launch_bounds__(256) void k_gate_up_xq(const float *x, const uint8_
     const size_t row_bytes = (size_t)na * bm_block_bytes<WA>();
     const uint8_t *wrow = (which ? wu : wg) + ((size_t)id * ff + r) * row_bytes;
     Blk<WA> b[UA];
-    preload<WA, UA>(b, wrow, q);
+    preload<WA, UA>(b, wrow, na, q);
     const Iq2Tables tb = stage_tables<WA>(lds);
     uint8_t *col = lds + tab_bytes<WA>();
     const int col_bytes = bm_act_col_bytes<WA>(na);
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
         __builtin_amdgcn_sched_barrier(0);
     }
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *col = lds + tab_bytes<WT>();
     if constexpr (bm_takes_q8k(WT)) {
@@ -906,7 +906,7 @@ __global__ __launch_bounds__(256) void k_down_combine_hq(const uint8_t *w, u32 n
     const int col_bytes = bm_act_col_bytes<WT>(n);
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
@@ -959,7 +959,7 @@ __global__ __launch_bounds__(64) void k_block_sums(const uint8_t *wrow, int nb, 
     __syncthreads();
     if (tid >= 4) return;
     Blk<WT> b[U];
-    preload<WT, U>(b, wrow, q);
+    preload<WT, U>(b, wrow, n, q);
     float v[1];
     row_dot<WT, U, NB, 1>(b, wrow, col, col_bytes, 1, n, q, tb, v, StoreTap{out});
     if constexpr (WT == BM_IQ2XXS || WT == BM_IQ3XXS) {
@@ -995,22 +995,26 @@ hipError_t gemv(const Launch &L, int wtype, const uint8_t *w, int64_t rows, int 
                 int col0, int m, float *y) {
     const int nb = k / 256;
     const size_t lds = tab_bytes_rt(wtype) + (size_t)m * act_col_bytes(wtype, k);
-    const bool few = m == 1 && (rows + 63) / 64 < (int64_t)kCardUnits; // one column of a matrix whose 64-row blocks do not fill the card
+    if (m == 1) {
+        const bool few = (rows + 63) / 64 < (int64_t)kCardUnits; // a matrix whose 64-row blocks do not fill the card
 #define CALL_BODY                                                                                                      \
-    if (few) {                                                                                                         \
-        auto kern = k_gemv<WT, U, NB, 1, 64>;                                                                          \
-        hipError_t e = allow_lds(kern, lds);                                                                           \
-        if (e != hipSuccess) return e;                                                                                 \
-        hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 15) / 16)), dim3(64), lds, L.stream, w, (long)rows, nb, act,  \
-                           m_total, col0, m, y);                                                                       \
-    } else {                                                                                                           \
-        auto kern = m == 1 ? k_gemv<WT, U, NB, 1> : k_gemv<WT, U, NB, 8>;                                              \
-        hipError_t e = allow_lds(kern, lds);                                                                           \
-        if (e != hipSuccess) return e;                                                                                 \
-        hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 63) / 64)), dim3(256), lds, L.stream, w, (long)rows, nb, act, \
-                           m_total, col0, m, y);                                                                       \
+    auto kern = few ? k_gemv<WT, U, NB, 1, 64> : k_gemv<WT, U, NB, 1>;                                                 \
+    hipError_t e = allow_lds(kern, lds);                                                                               \
+    if (e != hipSuccess) return e;                                                                                     \
+    const int T = few ? 64 : 256, per = T / 4;                                                                         \
+    hipLaunchKernelGGL(kern, dim3((unsigned)((rows + per - 1) / per)), dim3(T), lds, L.stream, w, (long)rows, nb, act, \
+                       m_total, col0, m, y);
+        BM_DISPATCH(wtype, nb)
+#undef CALL_BODY
+        return hipGetLastError();
     }
-    BM_DISPATCH(wtype, nb)
+#define CALL_BODY                                                                                                      \
+    auto kern = k_gemv<WT, U, NB, 8>;                                                                                  \
+    hipError_t e = allow_lds(kern, lds);                                                                               \
+    if (e != hipSuccess) return e;                                                                                     \
+    hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 63) / 64)), dim3(256), lds, L.stream, w, (long)rows, nb, act,     \
+                       m_total, col0, m, y);
+    BM_DISPATCH_COLS(wtype, nb)
 #undef CALL_BODY
     return hipGetLastError();
 }
@@ -1133,13 +1137,12 @@ hipError_t gate_up_x(const Launch &L, int gate_type, const float *x, const uint8
     }
     if (gate_type == BM_Q4K) {
         if (nba == 8) BM_GUX(BM_Q4K, kRingQ4K, 8)
-        else BM_GUX(BM_Q4K, 1, 0)
+        else BM_GUX(BM_Q4K, kRing, 0)
     } else if (gate_type == BM_Q5K) {
         if (nba == 8) BM_GUX(BM_Q5K, kRingQ5K, 8)
         else BM_GUX(BM_Q5K, 1, 0)
     } else if (gate_type == BM_Q6K) {
-        if (nba % 2 == 0) BM_GUX(BM_Q6K, 2, 0)
-        else BM_GUX(BM_Q6K, 1, 0)
+        BM_GUX(BM_Q6K, kRing, 0)
     } else if (bm_takes_q8k(gate_type)) {
         const int nb = nba;
         const size_t lds_q = tab_bytes_rt(gate_type) + (size_t)act_col_bytes(gate_type, hidden) + 32 * sizeof(float);

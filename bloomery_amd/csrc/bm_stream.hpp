@@ -8,7 +8,7 @@
 // read once, straight from the file's block bytes.
 //
 // Variants: a kernel is instantiated per weight type and per (U, NB): U the ring's size in super-blocks, NB the
-// row's super-block count when it is known at compile time (0: a run-time count that U divides). The hot shapes
+// row's super-block count when it is known at compile time (0: a run-time count). The hot shapes
 // (Q4_K rows of 2048 values, Q6_K rows of 768) have NB set and their stages unrolled.
 #ifndef BM_STREAM_HPP
 #define BM_STREAM_HPP
@@ -127,9 +127,9 @@ struct Stage {
 // arrived and only then starts to compute; with the ring the requests trickle out between the stages and the
 // arithmetic runs under the stream.
 template <int WT, int U>
-__device__ __forceinline__ void preload(Blk<WT> (&b)[U], const uint8_t *wrow, int q) {
+__device__ __forceinline__ void preload(Blk<WT> (&b)[U], const uint8_t *wrow, int n, int q) {
 #pragma unroll
-    for (int u = 0; u + 1 < U; u++) b[u] = bm_load_blk<WT>(wrow, u, q);
+    for (int u = 0; u + 1 < U; u++) b[u] = bm_load_blk<WT>(wrow, u < n ? u : n - 1, q);
 }
 
 // One stage: request super-block `ahead` into its ring slot, read the next stage's activation operands from LDS,
@@ -152,7 +152,8 @@ __device__ __forceinline__ void stage_one(Blk<WT> (&b)[U], int slot, int fill, c
 }
 
 // Row `wrow` against `m` <= M columns (LDS, `col_stride` apart); b holds the ring, preloaded.
-// NB > 0: the row has NB super-blocks, the stages are unrolled; NB == 0: it has nb, a multiple of U.
+// NB > 0: the row has NB super-blocks, the stages are unrolled; NB == 0: it has nb, of which with M = 1 the stages behind the
+// last whole ring take what U leaves over; with M > 1 nb is a multiple of U (a remainder's stages beside the loop's slowed the loop by 1 to 2 %).
 // Indices past the row's end are clamped onto its last super-block: a redundant read, no branch in the stream.
 template <int WT, int U, int NB, int M, class Tap>
 __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, const uint8_t *cols, int col_stride,
@@ -175,7 +176,8 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
                                  a0[0], a1[0], tap, i + U - 1 < NB); // the count is known here: nothing is asked for past the end
             }
         } else {
-            for (int i0 = 0; i0 < n; i0 += U) {
+            int i0 = 0;
+            for (; i0 + U <= n; i0 += U) {
 #pragma unroll
                 for (int u = 0; u < U; u++) {
                     const int i = i0 + u;
@@ -184,6 +186,11 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
                                      a0[0], a1[0], tap);
                 }
             }
+#pragma unroll
+            for (int u = 0; u + 1 < U; u++) // what U leaves over stands in the ring
+                if (i0 + u < n)
+                    stage_one<WT, U>(b, u, u, wrow, 0, av[0], i0 + u, i0 + u + 1 < n ? i0 + u + 1 : i0 + u, q, tb, cur, a0[0], a1[0], tap,
+                                     false);
         }
     } else {
         // several columns: the same ring for the weights, the activation operands read where they are used
@@ -709,50 +716,53 @@ static hipError_t allow_lds(K kernel, size_t lds) {
 }
 
 // Picks the kernel variant for a row of nb super-blocks and runs CALL_BODY with WT, U and NB as constants. Each
-// type lists the hot shape first (its count known at compile time, stages unrolled), then a ring of two for even
-// counts, then one super-block at a time, which divides every row.
-constexpr int kRingQ4K = 4, kRingQ5K = 4, kRingQ6K = 3;
+// type lists the hot shape first (its count known at compile time, stages unrolled), then a ring of two for any other count: the
+// super-block left over by an odd one stands in the ring when the loop ends. (Odd counts used to go one super-block at a
+// time, nothing asked for ahead: a layer of 1792 x 768 IQ2_XXS, 16 tokens, 91 -> 85 us; rings of three or four measure 1 to 10 % slower.)
+// The kernels of several columns take BM_DISPATCH_COLS: a ring of two for even counts, one super-block at a time else.
+constexpr int kRingQ4K = 4, kRingQ5K = 4, kRingQ6K = 3, kRing = 2;
 #define BM_VARIANT(T, UU, NN)                                                                                          \
     {                                                                                                                  \
         constexpr int WT = T, U = UU, NB = NN;                                                                         \
         CALL_BODY;                                                                                                     \
     }
-#define BM_DISPATCH(wtype, nb)                                                                                         \
+#define BM_DISPATCH_BY(wtype, nb, REST)                                                                                \
     switch (wtype) {                                                                                                   \
     case BM_Q3K:                                                                                                       \
-        if ((nb) % 2 == 0) BM_VARIANT(BM_Q3K, 2, 0)                                                                    \
-        else BM_VARIANT(BM_Q3K, 1, 0)                                                                                  \
+        REST(BM_Q3K, nb)                                                                                               \
         break;                                                                                                         \
     case BM_Q4K:                                                                                                       \
         if ((nb) == 8) BM_VARIANT(BM_Q4K, kRingQ4K, 8)                                                                 \
-        else if ((nb) % 2 == 0) BM_VARIANT(BM_Q4K, 2, 0)                                                               \
-        else BM_VARIANT(BM_Q4K, 1, 0)                                                                                  \
+        else REST(BM_Q4K, nb)                                                                                          \
         break;                                                                                                         \
     case BM_Q5K:                                                                                                       \
         if ((nb) == 8) BM_VARIANT(BM_Q5K, kRingQ5K, 8)                                                                 \
-        else if ((nb) % 2 == 0) BM_VARIANT(BM_Q5K, 2, 0)                                                                    \
-        else BM_VARIANT(BM_Q5K, 1, 0)                                                                                  \
+        else REST(BM_Q5K, nb)                                                                                          \
         break;                                                                                                         \
     case BM_Q6K:                                                                                                       \
         if ((nb) == 3) BM_VARIANT(BM_Q6K, kRingQ6K, 3)                                                                 \
-        else if ((nb) % 2 == 0) BM_VARIANT(BM_Q6K, 2, 0)                                                               \
-        else BM_VARIANT(BM_Q6K, 1, 0)                                                                                  \
+        else REST(BM_Q6K, nb)                                                                                          \
         break;                                                                                                         \
     case BM_IQ2XXS:                                                                                                    \
-        if ((nb) % 2 == 0) BM_VARIANT(BM_IQ2XXS, 2, 0)                                                                 \
-        else BM_VARIANT(BM_IQ2XXS, 1, 0)                                                                               \
+        REST(BM_IQ2XXS, nb)                                                                                            \
         break;                                                                                                         \
     case BM_IQ3XXS:                                                                                                    \
-        if ((nb) % 2 == 0) BM_VARIANT(BM_IQ3XXS, 2, 0)                                                                 \
-        else BM_VARIANT(BM_IQ3XXS, 1, 0)                                                                               \
+        REST(BM_IQ3XXS, nb)                                                                                            \
         break;                                                                                                         \
     case BM_IQ4XS:                                                                                                     \
-        if ((nb) % 2 == 0) BM_VARIANT(BM_IQ4XS, 2, 0)                                                                  \
-        else BM_VARIANT(BM_IQ4XS, 1, 0)                                                                                \
+        REST(BM_IQ4XS, nb)                                                                                             \
         break;                                                                                                         \
     default:                                                                                                           \
         return hipErrorInvalidValue;                                                                                   \
     }
+#define BM_REST_ANY(T, nb) BM_VARIANT(T, kRing, 0)
+#define BM_REST_COLS(T, nb)                                                                                            \
+    {                                                                                                                  \
+        if ((nb) % 2 == 0) BM_VARIANT(T, 2, 0)                                                                         \
+        else BM_VARIANT(T, 1, 0)                                                                                       \
+    }
+#define BM_DISPATCH(wtype, nb) BM_DISPATCH_BY(wtype, nb, BM_REST_ANY)
+#define BM_DISPATCH_COLS(wtype, nb) BM_DISPATCH_BY(wtype, nb, BM_REST_COLS)
 
 static inline int tab_bytes_rt(int wtype) { return wtype == BM_IQ2XXS ? kTabBytes : wtype == BM_IQ3XXS ? kTabBytes3 : 0; }
 
