@@ -3,6 +3,7 @@
 // its fused forms, and the block-sum verification kernel.
 #include "bm_kernels.h"
 
+#include <algorithm>
 #include <atomic>
 
 #include "bm_stream.hpp"
@@ -187,6 +188,53 @@ __global__ __launch_bounds__(T) void k_gemv(const uint8_t *w, long rows, int nb,
 #pragma unroll
         for (int c = 0; c < M; c++)
             if (c < m) y[(size_t)row * m_total + col0 + c] = out[c];
+    }
+}
+
+// The same product of m > 1 columns where 64 rows a workgroup leave most of the card idle: a wave takes 16 rows and C of the
+// columns. What bounds it is a wave's own instruction stream (some 150 instructions a super-block and column, five to six cycles each
+// while a SIMD has one wave), so the columns go side by side instead of one after the other; a workgroup's waves, `rgs` row
+// groups of `cgs` column groups each, share the staged columns and, through the vector cache, the rows' lines. inv: 256 / cgs rounded
+// up, T: the workgroup's threads. (Where a column group is not whole, its last columns are skipped.)
+template <int WT, int U, int NB, int C>
+__global__ __launch_bounds__(1024) void k_gemv_cols(const uint8_t *w, long rows, int nb, const uint8_t *act, int m_total, int col0, int m,
+                                                    float *y, int cgs, int rgs, int inv, int T) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int tid = threadIdx.x, q = tid & 3, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = (wv * inv) >> 8, cg = wv - rg * cgs; // (wv below 16, cgs at most 8: the quotient wv / cgs)
+    const int n = NB > 0 ? NB : nb;
+    const long row = ((long)blockIdx.x * rgs + rg) * 16 + ((tid & 63) >> 2);
+    const bool active = row < rows;
+    const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
+    const int col_bytes = bm_act_col_bytes<WT>(n), bytes = m * col_bytes;
+    const uint8_t *wrow = w + (size_t)(active ? row : 0) * row_bytes;
+    const uint8_t *src = act + (size_t)col0 * col_bytes;
+    uint2 v[4]; // the columns' first bytes in front of the rows, as k_gemv
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int o = (r * T + tid) * 8;
+        v[r] = *reinterpret_cast<const uint2 *>(src + (o < bytes ? o : bytes - 8));
+    }
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    Blk<WT> b[U];
+    preload<WT, U>(b, wrow, n, q);
+    const Iq2Tables tb = stage_tables_by<WT>(lds, T);
+    uint8_t *cols = lds + tab_bytes<WT>();
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int o = (r * T + tid) * 8;
+        if (o < bytes) *reinterpret_cast<uint2 *>(cols + o) = v[r];
+    }
+    for (int o = (4 * T + tid) * 8; o < bytes; o += T * 8) *reinterpret_cast<uint2 *>(cols + o) = *reinterpret_cast<const uint2 *>(src + o);
+    __syncthreads();
+    const int c0 = cg * C, mc = m - c0 < C ? m - c0 : C;
+    float out[C];
+    row_dot<WT, U, NB, C>(b, wrow, cols + (size_t)c0 * col_bytes, col_bytes, mc, n, q, tb, out, NoTap{});
+    if (q == 0 && active) {
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            if (c < mc) y[(size_t)row * m_total + col0 + c0 + c] = out[c];
     }
 }
 
@@ -1006,6 +1054,35 @@ hipError_t gemv(const Launch &L, int wtype, const uint8_t *w, int64_t rows, int 
                        m_total, col0, m, y);
         BM_DISPATCH(wtype, nb)
 #undef CALL_BODY
+        return hipGetLastError();
+    }
+    // Several columns of a matrix whose rows do not fill the card: the columns are dealt to waves as well, one a wave up to about a wave a
+    // SIMD, two (which unpack a row once for both) beyond; row groups share a workgroup, and the columns it stages, where there
+    // are more of them than compute units. us, one launch, k_gemv / one column a wave / two: Q6_K 7168 x 2048, 2 columns
+    // 7.5 / 5.5 / 6.4, 4 columns 9.4 / 8.6 / 6.9, 8 columns 13.5 / 15 / 9.5; Q4_K 768 x 2048, 4 columns 7.3 / 3.9 / 5.6; Q5_K
+    // 2048 x 7168, 8 columns 36 / 19 / 20; IQ2_XXS 16384 x 4096, 8 columns 32 / 43 / 29. From 32768 rows on rows alone are enough waves
+    // (Q6_K of 2048, 4 columns 14.5 / 27 / 16, 8 columns 21 / 54 / 29).
+    const int64_t groups = (rows + 15) / 16;
+    if (groups <= 1024) {
+        const int per = groups * m <= 1280 ? 1 : 2, cgs = (m + per - 1) / per;
+        const int rgs = (int)std::max<int64_t>(1, std::min<int64_t>((groups + kCardUnits - 1) / kCardUnits, 16 / cgs));
+        const int T = 64 * rgs * cgs;
+#define BM_COLS_LAUNCH(C)                                                                                              \
+    auto kern = k_gemv_cols<WT, U, NB, C>;                                                                             \
+    hipError_t e = allow_lds(kern, lds);                                                                               \
+    if (e != hipSuccess) return e;                                                                                     \
+    hipLaunchKernelGGL(kern, dim3((unsigned)((groups + rgs - 1) / rgs)), dim3(T), lds, L.stream, w, (long)rows, nb,    \
+                       act, m_total, col0, m, y, cgs, rgs, (256 + cgs - 1) / cgs, T);
+#define CALL_BODY BM_COLS_LAUNCH(1)
+        if (per == 1) {
+            BM_DISPATCH(wtype, nb)
+            return hipGetLastError();
+        }
+#undef CALL_BODY
+#define CALL_BODY BM_COLS_LAUNCH(2)
+        BM_DISPATCH_COLS(wtype, nb)
+#undef CALL_BODY
+#undef BM_COLS_LAUNCH
         return hipGetLastError();
     }
 #define CALL_BODY                                                                                                      \

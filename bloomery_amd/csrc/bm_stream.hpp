@@ -48,9 +48,10 @@ __device__ __forceinline__ uint2 iq_sign_masks(int t) {
     return make_uint2(m[0], m[1]);
 }
 
-// (T: the workgroup's thread count, a constant: blockDim.x is a load from the dispatch packet, in front of whatever comes next)
-template <int WT, int T = 256>
-__device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds) {
+// (T: how many of the workgroup's threads write them, no call to the built-in: blockDim.x is a load from the dispatch packet, in
+// front of whatever comes next)
+template <int WT>
+__device__ __forceinline__ Iq2Tables stage_tables_by(uint8_t *lds, int T) {
     Iq2Tables tb{nullptr, nullptr, nullptr};
     if constexpr (WT == BM_IQ2XXS) {
         // a grid point as eight byte selectors over the three magnitudes (8, 25, 43 -> 0, 1, 2), a sign index as eight bytes
@@ -82,6 +83,11 @@ __device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds) {
         tb.signs = signs;
     }
     return tb;
+}
+
+template <int WT, int T = 256>
+__device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds) {
+    return stage_tables_by<WT>(lds, T);
 }
 
 // `bytes` (a multiple of 8) from 8-byte aligned global memory to 8-byte aligned LDS, by the whole workgroup of T threads.

@@ -228,6 +228,29 @@ def test_gemv_matches_dot_row(gpu, wtype, rows, k):
         b.free()
 
 
+# Row groups and column groups of the several-column form: one and two columns a wave, one to four row groups a workgroup, a last row
+# group and a last column group that are not whole, rows on either side of where it gives way to 64 rows a workgroup.
+@pytest.mark.parametrize("wtype,rows,k", ((bm.Q4_K, 2570, 512), (bm.Q6_K, 4100, 768), (bm.IQ2_XXS, 8200, 256), (bm.Q3_K, 16381, 256),
+                                          (bm.Q5_K, 16400, 256), (bm.IQ4_XS, 17, 7168), (bm.IQ3_XXS, 4500, 768)))
+def test_gemv_deals_columns_to_waves(gpu, wtype, rows, k):
+    rng = np.random.default_rng(40 + rows)
+    w = stack(wtype, rows, k, 41 + rows)
+    x = normal_f32(rng, (8, k))
+    wd, act, xd = gpu.weights(wtype, rows, k, w), gpu.act(wtype, k, 8), gpu.upload(x, np.float32)
+    gpu.enqueue_quantize(xd, 8, act)
+    cols = np.concatenate([ora.quantize_col(wtype, x[c]) for c in range(8)])
+    want = ora.gemv(wtype, w, rows, k, cols, 8).reshape(rows, 8)
+    for m in range(2, 9):
+        y = gpu.buffer(np.float32, rows * m + 4).fill_bytes(0xFF)
+        gpu.enqueue_gemv(wd, act, m, y)
+        got = y.download()
+        assert_f32(got[:rows * m], np.ascontiguousarray(want[:, :m]).reshape(-1), f"gemv type {wtype} {rows}x{k} m={m}")
+        assert np.isnan(got[rows * m:]).all(), f"m={m}: wrote past the last row"
+        y.free()
+    for b in (wd, act, xd):
+        b.free()
+
+
 @pytest.mark.parametrize("wtype,rows,k", ((bm.Q4_K, 768, 2048), (bm.Q6_K, 2048, 768), (bm.Q5_K, 67, 1280), (bm.Q4_K, 70, 4352),
                                           (bm.IQ2_XXS, 33, 7168), (bm.IQ4_XS, 66, 768), (bm.IQ3_XXS, 40, 1280),
                                           (bm.Q3_K, 150, 2048)))
