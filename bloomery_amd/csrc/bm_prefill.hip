@@ -347,7 +347,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     const int wr = tid >> 2, p = tid & 3;
     const uint8_t *we = w + (size_t)e * rpe * row_bytes;
     auto row_at = [&](int first_row) { return (u32)(first_row + wr < rpe ? first_row + wr : rpe - 1) * row_bytes; };
-    const u32 acol = tab->col[wr] * col_bytes + 16 + 16 * p, apair = acol + (u32)nb * BM_Q82_SB_REF - 16 - 8 * p;
+    // (of at most 32 slots: of column tid / 8 the codes 16 (tid % 8) ..)
+    const bool narrow = len <= 32;
+    const u32 apair = tab->col[wr] * col_bytes + 8 * p + (u32)nb * BM_Q82_SB_REF;
+    const u32 acol = narrow ? tab->col[tid >> 3] * col_bytes + 16 + 16 * (tid & 7) : tab->col[wr] * col_bytes + 16 + 16 * p;
     v4u rw, rq = {0, 0, 0, 0}, rh = {0, 0, 0, 0}, ra[2] = {};
     float d8, y0 = 0.0f, y4 = 0.0f;
     auto ld16 = [](const uint8_t *at) {
@@ -384,7 +387,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     typedef const volatile __attribute__((address_space(3))) v2u *LdsV2;
     typedef const volatile __attribute__((address_space(3))) float *LdsVF;
     const LdsB my_put = (LdsB)lds + wr * kXStride + 32 * p, my_factor = (LdsB)lds + 4 * kXCodes + 4 * wr + kXLine * p;
-    auto put = [&](int at, u32 a, u32 b) { *(__attribute__((address_space(3))) v2u *)(my_put + at) = (v2u){a, b}; };
+    const LdsB my_put_few = (LdsB)lds + (tid >> 3) * kXStride + 32 * (tid & 7);
+    auto put = [&](LdsB to, int at, u32 a, u32 b) { *(__attribute__((address_space(3))) v2u *)(to + at) = (v2u){a, b}; };
     auto factor = [&](int at, float v) { *(LdsF)(my_factor + at) = v; };
     // Word k of the sixteen code bytes of the row. Four codes a word become f16 in the order 0, 2, 1, 3 (rows and columns alike: a
     // sum's terms may come in any order). Low nibbles: group p of the buffer's first four; high nibbles: of its second four (Q6_K:
@@ -408,16 +412,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
             h1 = and_or(t8, my, h1);
         }
         constexpr float kOff = kQ45 ? 0.0f : 32.0f;
-        put(j * kXCodes + 8 * k, h2_less(l0, 1024.0f + kOff), h2_less(l1, 1024.0f + kOff));
-        put(j * kXCodes + 128 + 8 * k, h2_16th(h0, kOff), h2_16th(h1, kOff));
+        put(my_put, j * kXCodes + 8 * k, h2_less(l0, 1024.0f + kOff), h2_less(l1, 1024.0f + kOff));
+        put(my_put, j * kXCodes + 128 + 8 * k, h2_16th(h0, kOff), h2_16th(h1, kOff));
     };
     // Words 2 h and 2 h + 1 of the column's sixteen codes q.
-    auto stash_col = [&](auto half, int q, int h) __attribute__((always_inline)) {
+    auto stash_col = [&](auto few, auto half, int q, int h) __attribute__((always_inline)) {
         constexpr int j = decltype(half)::value;
 #pragma unroll
         for (int k = 2 * h; k < 2 * h + 2; k++) {
             const u32 u = ra[q][k] ^ 0x80808080u;
-            put((2 + j) * kXCodes + 128 * q + 8 * k, h2_less(and_or(u, m8, k1024), 1152.0f), h2_less(and_or(u >> 8, m8, k1024), 1152.0f));
+            put(decltype(few)::value ? my_put_few : my_put, (2 + j) * kXCodes + 128 * q + 8 * k, h2_less(and_or(u, m8, k1024), 1152.0f),
+                h2_less(and_or(u >> 8, m8, k1024), 1152.0f));
         }
     };
     float r4 = 0.0f; // Q4_K, Q5_K: the scale product of block 4 + p, kept for the second half
@@ -460,14 +465,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     };
     // Step st of eight of a half's staging. The codes of the half after it (super-block `next`) are asked for where a register's last
     // word is done with, seven steps before its first use; the half's own factors at step 1, for step 7.
-    auto stash = [&](auto half, int st, At now, At next) __attribute__((always_inline)) {
+    auto stash = [&](auto few, auto half, int st, At now, At next) __attribute__((always_inline)) {
         constexpr std::integral_constant<int, 1 - decltype(half)::value> after{};
+        constexpr int kPieces = decltype(few)::value ? 1 : 2; // of a column's codes
         if (st == 0) fetch_factors(now, half);
         if (st < 4) {
             stash_row(half, st);
             if (st == 3) fetch_row(next, after);
-        } else {
-            stash_col(half, (st - 4) >> 1, st & 1);
+        } else if (st < 4 + 2 * kPieces) {
+            stash_col(few, half, (st - 4) >> 1, st & 1);
             if (st & 1) fetch_col(next.i, after, (st - 4) >> 1);
         }
         if (st == 7) stash_factors(half);
@@ -476,135 +482,164 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     // this lane in its wave's 32 x 32 products: operand slot and row lane % 32, eight of a group's sixteen values by lane / 32;
     // result v is slot 8 (v / 4) + 4 (lane / 32) + v % 4 of row lane % 32
     const int l32 = lane & 31, kh = lane >> 5;
-    const int wrow0 = 32 * (wv & 1), wslot0 = 32 * (wv >> 1);
-    const bool live = wslot0 < len;
-    v32f acc[4]; // accumulator l: [l / 2], results 16 (l % 2) ..
+    const int wrow0 = 32 * (wv & 1), wslot0 = narrow ? 0 : 32 * (wv >> 1);
+    const int gh = wv >> 1; // the half of the accumulators a wave of a narrow tile keeps
 
     constexpr std::integral_constant<int, 0> kFirst{};
     constexpr std::integral_constant<int, 1> kSecond{};
-    const LdsB my_row = (LdsB)lds + (wrow0 + l32) * kXStride + 16 * kh, my_col = (LdsB)lds + 2 * kXCodes + (wslot0 + l32) * kXStride + 16 * kh;
-    // the factors of an outer product's two blocks, or of a block's two groups (Q6_K: one d8 for both): a half of the lanes each
-    const LdsB my_sr = (LdsB)lds + 4 * kXCodes + 4 * (wrow0 + l32) + kh * kXLine;
-    const LdsB my_sc = (LdsB)lds + 4 * kXCodes + 4 * (wslot0 + l32) + (kQ45 ? kh : 0) * kXLine + X::kScales * kXLine;
-    const LdsB my_mr = my_sr + X::kMinsAt, my_mc = my_sc + X::kMinsAt + (8 - X::kScales) * kXLine;
-    // A half's arithmetic, a step a 16-value group, and in the shade of each step's outer product a piece of the staging of the half
-    // after it (super-block i1).
-    auto arithmetic = [&](auto half, At now, At next) __attribute__((always_inline)) {
-        constexpr int j = decltype(half)::value;
-        const v16f z16 = {};
-        const v32f z32 = {};
-        v4u a, b;
-        v16f sum;
-        v32f pd;
-        auto rd = [&](int gr) { // group gr of the half's eight
-            const int at = j * kXCodes + 32 * (kQ45 ? 4 * ((gr >> 1) & 1) + 2 * (gr >> 2) + (gr & 1) : gr), ct = j * kXCodes + 32 * gr;
-            const v2u a0 = *(LdsV2)(my_row + at), a1 = *(LdsV2)(my_row + at + 8), b0 = *(LdsV2)(my_col + ct), b1 = *(LdsV2)(my_col + ct + 8);
-            a = (v4u){a0.x, a0.y, a1.x, a1.y};
-            b = (v4u){b0.x, b0.y, b1.x, b1.y};
-        };
-        auto product = [&]() {
-            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, b), __builtin_bit_cast(v8h, a), z16, 0, 0, 0);
-        };
-        // Q4_K, Q5_K: one scale a block; Q6_K: one a group (crates/qdot/src/lib.rs:4403-4440, :4794-4809)
-        auto scale = [&](int gr) {
-            const float fc = *(LdsVF)(my_sc + j * X::kHalf + (gr >> 1) * kXLine), fr = *(LdsVF)(my_sr + j * X::kHalf + (kQ45 ? gr >> 1 : gr) * kXLine);
-            pd = __builtin_amdgcn_mfma_f32_32x32x1f32(fc, fr, z32, 0, 0, 0);
-        };
-        // the min terms come before a super-block's products: accumulator l takes sub-block l's (crates/qdot/src/lib.rs:4389-4394)
-        auto min_term = [&](int s) {
-            acc[s] = __builtin_amdgcn_mfma_f32_32x32x1f32(*(LdsVF)(my_mc + 2 * s * kXLine), *(LdsVF)(my_mr + 2 * s * kXLine), acc[s], 0, 0, 0);
-        };
-        rd(0);
-        if constexpr (kQ45 && j == 0) {
-            min_term(0);
-            min_term(2);
-        }
-#pragma unroll
-        for (int gr = 0; gr < 8; gr++) {
-            const int bk = gr >> 1, h = gr & 1, l = 4 * h + bk, al = 16 * (l & 1), pb = 16 * (kQ45 ? bk & 1 : h);
-            product();
-            if ((gr & (kQ45 ? 3 : 1)) == 0) scale(gr);
-            if constexpr (kQ45 && j == 0) {
-                if (gr == 1) min_term(1);
-                if (gr == 3) min_term(3);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (gr + 1 < 8) rd(gr + 1);
-            stash(std::integral_constant<int, 1 - j>{}, gr, now, next);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[l >> 1][al + v] = fmaf(pd[pb + v], sum[v], acc[l >> 1][al + v]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-
-    auto stash_all = [&](auto half, At now, At next) __attribute__((always_inline)) {
-#pragma unroll
-        for (int st = 0; st < 8; st++) stash(half, st, now, next);
-    };
     const int first_row = row0;
     int left = (rpe - row0 + kGemmBM - 1) / kGemmBM; // slabs to do
     left = left < (int)slabs ? left : (int)slabs;
-    if constexpr (kQ45) factor(X::kHeadsAt, 0.0f);
-    At now = {row_at(row0), 0};
-    fetch_row(now, kFirst);
-    fetch_col(0, kFirst, 0);
-    fetch_col(0, kFirst, 1);
-    stash_all(kFirst, now, now);
-    __syncthreads();
-    // the super-block after `at`, in the next slab behind a slab's last (the very last: itself, staged for no reader)
-    auto following = [&](At at) {
-        if (at.i + 1 < nb) return At{at.row, at.i + 1};
-        return left > 1 ? At{row_at(row0 + kGemmBM), 0} : at;
-    };
-    // (a half's last readers passed the barrier that ended the half before)
-    if (!live) { // none of this wave's slots is real: it stages only
-        for (; left > 0; left--, row0 += kGemmBM)
+    auto run = [&](auto few) __attribute__((always_inline)) {
+        constexpr bool kFew = decltype(few)::value;
+        constexpr int kPairs = kFew ? 2 : 4;
+        const int up = kFew ? gh : 0;
+        const LdsB my_row = (LdsB)lds + (wrow0 + l32) * kXStride + 16 * kh + 32 * up;
+        const LdsB my_col = (LdsB)lds + 2 * kXCodes + ((kFew ? 0 : wslot0) + l32) * kXStride + 16 * kh + 32 * up;
+        // the factors of an outer product's two blocks, or of a block's two groups (Q6_K in a wide tile: one d8 for both; in a narrow
+        // one two blocks' groups of the wave's half): a half of the lanes each
+        const LdsB my_fr = (LdsB)lds + 4 * kXCodes + 4 * (wrow0 + l32), my_fc = (LdsB)lds + 4 * kXCodes + 4 * ((kFew ? 0 : wslot0) + l32);
+        const LdsB my_sr = my_fr + (kQ45 || !kFew ? kh : up + 2 * kh) * kXLine;
+        const LdsB my_sc = my_fc + (kQ45 || kFew ? kh : 0) * kXLine + X::kScales * kXLine;
+        const LdsB my_mr = my_fr + (kh + 4 * up) * kXLine + X::kMinsAt, my_mc = my_fc + (kh + 4 * up) * kXLine + X::kMinsAt + 8 * kXLine;
+        v32f acc[kPairs]; // accumulator l (a narrow tile: l + 4 gh): [l / 2], results 16 (l % 2) ..
+        // A half's arithmetic, a step a 16-value group, and in the shade of each step's outer product a piece of the staging of the half
+        // after it (super-block i1).
+        auto arithmetic = [&](auto half, At now, At next) __attribute__((always_inline)) {
+            constexpr int j = decltype(half)::value, kSteps = kFew ? 4 : 8;
+            const v16f z16 = {};
+            const v32f z32 = {};
+            v4u a, b;
+            v16f sum;
+            v32f pd;
+            auto rd = [&](int step) { // a step's group of the half's eight
+                const int gr = kFew ? 2 * step : step; // (and the wave's half of the groups on top, where the tile is narrow)
+                const int at = j * kXCodes + 32 * (kQ45 ? 4 * ((gr >> 1) & 1) + 2 * (gr >> 2) + (gr & 1) : gr), ct = j * kXCodes + 32 * gr;
+                const v2u a0 = *(LdsV2)(my_row + at), a1 = *(LdsV2)(my_row + at + 8), b0 = *(LdsV2)(my_col + ct), b1 = *(LdsV2)(my_col + ct + 8);
+                a = (v4u){a0.x, a0.y, a1.x, a1.y};
+                b = (v4u){b0.x, b0.y, b1.x, b1.y};
+            };
+            auto product = [&]() {
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, b), __builtin_bit_cast(v8h, a), z16, 0, 0, 0);
+            };
+            // Q4_K, Q5_K: one scale a block; Q6_K: one a group (crates/qdot/src/lib.rs:4403-4440, :4794-4809)
+            auto scale = [&](int bk, int gr) {
+                const float fc = *(LdsVF)(my_sc + j * X::kHalf + bk * kXLine), fr = *(LdsVF)(my_sr + j * X::kHalf + (kQ45 ? bk : gr) * kXLine);
+                pd = __builtin_amdgcn_mfma_f32_32x32x1f32(fc, fr, z32, 0, 0, 0);
+            };
+            // the min terms come before a super-block's products: accumulator l takes sub-block l's (crates/qdot/src/lib.rs:4389-4394)
+            auto min_term = [&](int s) {
+                acc[s] = __builtin_amdgcn_mfma_f32_32x32x1f32(*(LdsVF)(my_mc + 2 * s * kXLine), *(LdsVF)(my_mr + 2 * s * kXLine), acc[s], 0, 0, 0);
+            };
+            rd(0);
+            if constexpr (kQ45 && j == 0) {
+                min_term(0);
+                if constexpr (!kFew) min_term(2);
+            }
+#pragma unroll
+            for (int step = 0; step < kSteps; step++) {
+                const int bk = kFew ? step : step >> 1, h = kFew ? 0 : step & 1, l = 4 * h + bk, al = 16 * (l & 1), pb = 16 * (kQ45 || kFew ? bk & 1 : h);
+                product();
+                if (kFew ? (step & 1) == 0 : (step & (kQ45 ? 3 : 1)) == 0) scale(bk, kFew ? 2 * step : step);
+                if constexpr (kQ45 && j == 0) {
+                    if (step == (kFew ? 0 : 1)) min_term(1);
+                    if (!kFew && step == 3) min_term(kPairs - 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                if (step + 1 < kSteps) rd(step + 1);
+#pragma unroll
+                for (int st = 8 / kSteps * step; st < 8 / kSteps * (step + 1); st++) stash(few, std::integral_constant<int, 1 - j>{}, st, now, next);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[l >> 1][al + v] = fmaf(pd[pb + v], sum[v], acc[l >> 1][al + v]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        if constexpr (kQ45) factor(X::kHeadsAt, 0.0f);
+        At now = {row_at(row0), 0};
+        fetch_row(now, kFirst);
+        fetch_col(0, kFirst, 0);
+        if constexpr (!kFew) fetch_col(0, kFirst, 1);
+#pragma unroll
+        for (int st = 0; st < 8; st++) stash(few, kFirst, st, now, now);
+        __syncthreads();
+        // the super-block after `at`, in the next slab behind a slab's last (the very last: itself, staged for no reader)
+        auto following = [&](At at) {
+            if (at.i + 1 < nb) return At{at.row, at.i + 1};
+            return left > 1 ? At{row_at(row0 + kGemmBM), 0} : at;
+        };
+        // (a half's last readers passed the barrier that ended the half before)
+#pragma unroll
+        for (int l = 0; l < kPairs; l++)
+#pragma unroll
+            for (int v = 0; v < 32; v++) acc[l][v] = 0.0f;
+        for (; left > 0; left--, row0 += kGemmBM) {
             for (int i = 0; i < nb; i++) {
                 const At next = following(now);
-                stash_all(kSecond, now, next);
+                arithmetic(kFirst, now, next);
                 __syncthreads();
-                stash_all(kFirst, next, next);
+                arithmetic(kSecond, next, next);
                 __syncthreads();
                 now = next;
             }
-        return;
-    }
+            // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order) and the store
+            const int row = row0 + wrow0 + l32;
+            auto store = [&](int v, float t0, float t1, float t2, float t3) {
+                const int n = wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
+                if (row < rpe && n < len) y[(size_t)tab->slot[n] * rpe + row] = (t0 + t2) + (t1 + t3);
+            };
+            if constexpr (kFew) {
+                // a wave sums eight of a lane's sixteen results and has the other wave's accumulators of them through LDS (the half 1
+                // buffers: half 0's hold the next slab's first codes)
+                float *const swap = reinterpret_cast<float *>(lds + (wrow0 ? 3 : 1) * kXCodes);
+                auto give = [&](auto from) __attribute__((always_inline)) { // accumulators of results `from` .. of the other wave
 #pragma unroll
-    for (int l = 0; l < 4; l++)
+                    for (int l = 0; l < 4; l++)
 #pragma unroll
-        for (int v = 0; v < 32; v++) acc[l][v] = 0.0f;
-    for (; left > 0; left--, row0 += kGemmBM) {
-        for (int i = 0; i < nb; i++) {
-            const At next = following(now);
-            arithmetic(kFirst, now, next);
-            __syncthreads();
-            arithmetic(kSecond, next, next);
-            __syncthreads();
-            now = next;
+                        for (int v = 0; v < 8; v++) swap[((gh * 4 + l) * 8 + v) * 64 + lane] = acc[l >> 1][16 * (l & 1) + decltype(from)::value + v];
+                };
+                auto take = [&](auto from) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int v = 0; v < 8; v++) {
+                        float t[4];
+#pragma unroll
+                        for (int l = 0; l < 4; l++)
+                            t[l] = acc[l >> 1][16 * (l & 1) + decltype(from)::value + v] + swap[(((1 - gh) * 4 + l) * 8 + v) * 64 + lane];
+                        store(decltype(from)::value + v, t[0], t[1], t[2], t[3]);
+                    }
+                };
+                constexpr std::integral_constant<int, 0> kLow{};
+                constexpr std::integral_constant<int, 8> kHigh{};
+                if (gh) give(kLow);
+                else give(kHigh);
+                __syncthreads();
+                if (gh) take(kHigh);
+                else take(kLow);
+                __syncthreads();
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                    store(v, acc[0][v] + acc[kPairs - 2][v], acc[0][16 + v] + acc[kPairs - 2][16 + v], acc[1][v] + acc[kPairs - 1][v],
+                          acc[1][16 + v] + acc[kPairs - 1][16 + v]);
+            }
+#pragma unroll
+            for (int l = 0; l < kPairs; l++)
+#pragma unroll
+                for (int v = 0; v < 32; v++) acc[l][v] = 0.0f;
         }
-        // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order) and the store
-        const int row = row0 + wrow0 + l32;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int n = wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
-            const float t0 = acc[0][v] + acc[2][v], t1 = acc[0][16 + v] + acc[2][16 + v];
-            const float t2 = acc[1][v] + acc[3][v], t3 = acc[1][16 + v] + acc[3][16 + v];
-            if (row < rpe && n < len) y[(size_t)tab->slot[n] * rpe + row] = (t0 + t2) + (t1 + t3);
-#pragma unroll
-            for (int l = 0; l < 4; l++) acc[l][v] = acc[l][16 + v] = 0.0f;
-        }
-    }
+    };
+    if (narrow) run(std::true_type{});
+    else run(std::false_type{});
     if constexpr (kQ45) {
         u32 heads = 0u;
 #pragma unroll
         for (int q = 0; q < 4; q++) heads |= *(const u32 *)(lds + 4 * kXCodes + X::kHeadsAt + 4 * lane + q * kXLine);
         if (__ballot((heads & 0x8000u) != 0u) == 0) return; // (see above)
-        const int end = row0 < rpe ? row0 : rpe;
+        const int end = row0 < rpe ? row0 : rpe, first = narrow ? 8 * gh : 0, last = narrow ? first + 8 : 16; // the results this wave stored
 #pragma nounroll
         for (int row = first_row + wrow0 + l32; row < end; row += kGemmBM)
 #pragma nounroll
-            for (int v = 0; v < 16; v++) {
+            for (int v = first; v < last; v++) {
                 const int n = wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
                 if (n >= len) continue;
                 float *out = y + (size_t)tab->slot[n] * rpe + row;

@@ -336,11 +336,11 @@ def test_prefill_refusals_are_named(gpu):
 
 
 @pytest.mark.parametrize("wtype,k", ((bm.Q4_K, 256), (bm.Q4_K, 768), (bm.Q5_K, 512), (bm.Q6_K, 256), (bm.Q6_K, 512)))
-def test_gemm_with_several_slabs_a_workgroup(gpu, wtype, k):
+def test_gemm_with_several_slabs_a_workgroup(gpu, wtype, k, rpe=1040):
     """A route of enough tiles that a workgroup takes two row slabs of the seventeen (the last alone, a quarter of it real), with
     tiles of every length; one refused slot. Sampled slots' rows against the one-column dot, bit for bit."""
     from test_gpu_decode import random_blocks
-    n_experts, n_slots, rpe = 200, 6000, 1040
+    n_experts, n_slots = 200, 6000
     rng = np.random.default_rng(2700 + k)
     w = random_blocks(wtype, n_experts * rpe, k, rng)
     p = 1.0 / np.arange(1, n_experts + 1)
@@ -522,12 +522,12 @@ def test_gemm_terms_at_the_ends_of_their_range(gpu, wtype):
 
 
 @pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K))
-def test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype):
+def test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype, n_slots=70):
     """The exact GEMM's outer products on the matrix cores where a scale product is subnormal, underflows to zero or is a zero of either
     sign (subnormal, zero, negative and negative-zero block scales, zero scale codes, columns at the smallest scale the quantizer
     makes), and where a min term underflows to a negative zero: bit for bit, the sign of a zero included."""
     from test_gpu_decode import random_blocks
-    rpe, k, n_experts, n_slots = 80, 768, 2, 70
+    rpe, k, n_experts = 80, 768, 2
     rng = np.random.default_rng(2960)
     bb, nb = ora.BLOCK_BYTES[wtype], k // 256
     rows = n_experts * rpe
@@ -572,6 +572,43 @@ def test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype):
         assert_f32(got[s], want[s], f"slot {s}")
     for b in (dw, act, xd, sel, table, y):
         b.free()
+
+
+# Tiles of at most 32 slots, whose accumulators are split between two waves, beside wide ones: every edge of the two, a slab that is
+# not whole, one super-block and an odd count of them; bit for bit against the one-column dot.
+@pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K))
+@pytest.mark.parametrize("rpe,k,counts", ((80, 256, (1, 32, 33, 64, 65)), (16, 768, (31, 2, 96, 97)), (144, 1792, (17, 0, 128, 5))))
+def test_gemm_of_narrow_and_wide_tiles(gpu, wtype, rpe, k, counts):
+    from test_gpu_decode import random_blocks
+    n_experts, n_slots = len(counts), sum(counts)
+    rng = np.random.default_rng(2980 + rpe)
+    w = random_blocks(wtype, n_experts * rpe, k, rng)
+    ids = rng.permutation(np.repeat(np.arange(n_experts), counts)).astype(np.uint32)
+    x = normal_f32(rng, (n_slots, k))
+    dw, act = gpu.weights(wtype, n_experts * rpe, k, w), gpu.act(wtype, k, n_slots)
+    xd, sel, table = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.route(n_slots, n_experts)
+    y = gpu.buffer(np.float32, n_slots * rpe).fill_bytes(0xFF)
+    gpu.enqueue_quantize(xd, n_slots, act)
+    table.fill(sel, n_slots)
+    gpu.enqueue_gemm(dw, rpe, act, table, 0, y)
+    got, rb = y.download().reshape(n_slots, rpe), ora.row_bytes(wtype, k)
+    for s in range(n_slots):
+        e = int(ids[s])
+        want = ora.gemv(wtype, w[e * rpe * rb:(e + 1) * rpe * rb], rpe, k, ora.quantize_col(wtype, x[s]), 1)
+        assert_f32(got[s], want, f"slot {s}")
+    for b in (dw, act, xd, sel, table, y):
+        b.free()
+
+
+@pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K))
+def test_gemm_of_narrow_tiles_underflow_and_signed_zeros(gpu, wtype):
+    test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype, n_slots=40)
+
+
+@pytest.mark.parametrize("wtype,k", ((bm.Q4_K, 256), (bm.Q5_K, 768), (bm.Q6_K, 512)))
+def test_gemm_with_several_slabs_of_narrow_and_wide_tiles(gpu, wtype, k):
+    """Thirty-three slabs an expert: a workgroup takes two of them, the last one alone."""
+    test_gemm_with_several_slabs_a_workgroup(gpu, wtype, k, rpe=2064)
 
 
 @pytest.mark.parametrize("m,k", ((1, 256), (3, 768), (5, 1792), (130, 512)))
