@@ -287,7 +287,11 @@ __device__ __forceinline__ float q45_value(const uint8_t *row, const uint8_t *co
     return ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7]));
 }
 
-// A workgroup of four waves takes a slab of 64 rows and a tile's 64 slots, a wave 32 x 32 of them.
+// A workgroup of four waves takes a slab of 64 rows and a tile's 64 slots, a wave 32 x 32 of them. Of a tile of at most 32 slots, which
+// is most tiles of a short prompt, a wave takes 32 rows and all the slots but four of the eight accumulators, i.e. every second
+// group (Q4_K: group h of a block goes to accumulators 4 h ..), and the two waves of a row group meet in the closing sum: with the
+// wide split two waves of such a workgroup had no slots, and the two SIMDs with the others did all the arithmetic (top-8 of 128 experts, Q4_K /
+// Q6_K, us a layer: 256 tokens 251 -> 223, 333 tokens 269 -> 241, 1024 tokens 464 -> 433).
 // Per (row, slot, 16-value group) the contract is acc[l] = fma(fl(scale d8), sum, acc[l]) over eight accumulators, one fused
 // multiply-add that only the vector ALU can do. The rest is on the matrix cores: the group's integer sum comes out of
 // v_mfma_f32_32x32x16_f16 as a float (codes of at most eight bits, sums below 2^24: exact, where an int8 product needs a
@@ -504,7 +508,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
         const LdsB my_mr = my_fr + (kh + 4 * up) * kXLine + X::kMinsAt, my_mc = my_fc + (kh + 4 * up) * kXLine + X::kMinsAt + 8 * kXLine;
         v32f acc[kPairs]; // accumulator l (a narrow tile: l + 4 gh): [l / 2], results 16 (l % 2) ..
         // A half's arithmetic, a step a 16-value group, and in the shade of each step's outer product a piece of the staging of the half
-        // after it (super-block i1).
+        // after it.
         auto arithmetic = [&](auto half, At now, At next) __attribute__((always_inline)) {
             constexpr int j = decltype(half)::value, kSteps = kFew ? 4 : 8;
             const v16f z16 = {};
@@ -1424,10 +1428,12 @@ hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int
         if (wtype == BM_Q5K) return launch(k_gemm_fast<BM_Q5K>, kFastThreads, kFastRows, fast_lds_bytes<BM_Q5K>());
         if (wtype == BM_Q6K) return launch(k_gemm_fast<BM_Q6K>, kFastThreads, kFastRows, fast_lds_bytes<BM_Q6K>());
     }
-    // A workgroup's start (tile, columns, first bytes: a chain of trips to memory, 4 to 5 us) costs more than a super-block, so it
-    // takes several slabs where that leaves enough workgroups to fill the chip's 512 places about four times over (16384 slots:
-    // Q4_K 253 -> 228 us with two of twelve, Q6_K 341 -> 315 us with six of 32).
-    const u32 n_slabs = (u32)((rows_per_expert + kGemmBM - 1) / kGemmBM), slabs_max = stacks * max_tiles * n_slabs / 2048u;
+    // A workgroup's start (tile, columns, first bytes: a chain of trips to memory, 4 to 5 us) costs more than a super-block, so where rows
+    // are short it takes several slabs, up to about sixteen super-blocks, and no more than leaves some 2400 workgroups: with fewer the
+    // tiles, which differ by half in cost, fill the dies unevenly (top-8 of 128 experts, us a layer, one slab / two / four: down of 2048 rows of
+    // 768 Q6_K, 333 tokens 247 / 241 / 247, 2048 tokens 706 / 684 / 680, with six 708; gate and up of 768 rows of 2048 Q4_K, 333 tokens
+    // 241 / 248 / 282, 2048 tokens 684 / 681 / 697).
+    const u32 n_slabs = (u32)((rows_per_expert + kGemmBM - 1) / kGemmBM), slabs_max = std::min(16u / (u32)nb, stacks * max_tiles * n_slabs / 2400u);
     const u32 slabs = slabs_max < 1u ? 1u : slabs_max < n_slabs ? slabs_max : n_slabs;
     const int run = kGemmBM * (int)slabs;
     if (wtype == BM_Q4K) return launch(k_gemm<BM_Q4K>, 256, run, XLds<BM_Q4K>::kBytes, slabs);
