@@ -356,6 +356,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     const u32 apair = tab->col[wr] * col_bytes + 8 * p + (u32)nb * BM_Q82_SB_REF;
     const u32 acol = narrow ? tab->col[tid >> 3] * col_bytes + 16 + 16 * (tid & 7) : tab->col[wr] * col_bytes + 16 + 16 * p;
     v4u rw, rq = {0, 0, 0, 0}, rh = {0, 0, 0, 0}, ra[2] = {};
+    u32 q6d = 0, q6s = 0, q6t = 0; // (Q6_K; words of their own: as parts of a vector they were moved, and waited for, as they came)
     float d8, y0 = 0.0f, y4 = 0.0f;
     auto ld16 = [](const uint8_t *at) {
         v4u v;
@@ -445,9 +446,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
         } else if constexpr (kQ45) {
             factor(X::kHalf, r4);
         } else { // groups p and 4 + p of the half
-            const float d = bm_half_to_f32((unsigned short)rh.x);
-            factor(j * X::kHalf, d * (float)(int)(signed char)(rh.y & 0xffu));
-            factor(j * X::kHalf + 4 * kXLine, d * (float)(int)(signed char)(rh.z & 0xffu));
+            const float d = bm_half_to_f32((unsigned short)q6d);
+            factor(j * X::kHalf, d * (float)(int)(signed char)q6s);
+            factor(j * X::kHalf + 4 * kXLine, d * (float)(int)(signed char)q6t);
         }
         factor(j * X::kHalf + X::kScales * kXLine, d8);
     };
@@ -457,9 +458,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
         if constexpr (kQ45) {
             if constexpr (j == 0) rh = ld16(blk); // d, dmin, the twelve scale bytes
         } else {
-            rh.x = bm_ld2u(blk + 208);         // d
-            rh.y = blk[192 + 8 * j + p];       // the scales of groups p
-            rh.z = blk[192 + 8 * j + 4 + p];   // and 4 + p
+            q6d = bm_ld2u(blk + 208);       // d
+            q6s = blk[192 + 8 * j + p];     // the scales of groups p
+            q6t = blk[192 + 8 * j + 4 + p]; // and 4 + p
         }
         d8 = *reinterpret_cast<const float *>(act + (apair + 64 * (u32)at.i) + 32 * j); // of block 4 j + p
         if constexpr (kQ45 && j == 0) { // d8 isum of blocks p and 4 + p
@@ -564,8 +565,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
         fetch_row(now, kFirst);
         fetch_col(0, kFirst, 0);
         if constexpr (!kFew) fetch_col(0, kFirst, 1);
+        // (the loads in the loop's order, kept by the fences: the loop's first wait counts the loads behind the one it waits for, and
+        // where this way into the loop has fewer it waits for all)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int st = 0; st < 8; st++) stash(few, kFirst, st, now, now);
+        for (int st = 0; st < 8; st++) {
+            stash(few, kFirst, st, now, now);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         __syncthreads();
         // the super-block after `at`, in the next slab behind a slab's last (the very last: itself, staged for no reader)
         auto following = [&](At at) {
