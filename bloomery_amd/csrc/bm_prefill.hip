@@ -1155,7 +1155,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
             rd = tail.w >> 16;
         }
     };
-    auto stage = [&]() {
+    auto stage_cols = [&]() {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             uint8_t *dst = a_codes + a_dst + 16 * j * kIqStride;
@@ -1183,6 +1183,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
                 *reinterpret_cast<uint4 *>(x_bh + 16 * tid) = make_uint4(bh[0], bh[1], 0u, 0u);
             }
         }
+    };
+    auto stage_rows = [&]() {
         if (wq == 0) {
             const float dh = bm_half_to_f32((unsigned short)rd);
             d_t[wr] = WT == BM_IQ2XXS ? 0.125f * dh : WT == BM_IQ3XXS ? 0.25f * dh : dh;
@@ -1285,8 +1287,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     if constexpr (kColsAhead) fetch_cols(0);
     for (int i = 0; i < nb; i++) {
         if (i) __syncthreads(); // the readers of the super-block before are done
-        if constexpr (!kColsAhead) fetch_cols(i);
-        stage();
+        if constexpr (!kColsAhead) {
+            fetch_cols(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        stage_rows();
+        __builtin_amdgcn_sched_barrier(0);
+        stage_cols();
         if (i + 1 < nb) {
             fetch_rows(i + 1);
             if constexpr (kColsAhead) fetch_cols(i + 1);
