@@ -1119,9 +1119,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     u32 rd = 0, ra2 = 0;
     float cdy = 0.0f;
     uint4 cb0 = make_uint4(0, 0, 0, 0), cb1 = cb0;
-    auto fetch_cols = [&](int i) {
+    auto fetch_cols = [&](auto few, int i) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) __builtin_memcpy(&ra[j], act + (src_a[j] + (u32)i * BM_Q8K_STRIDE), 16);
+        for (int j = 0; j < (decltype(few)::value ? 2 : 4); j++) __builtin_memcpy(&ra[j], act + (src_a[j] + (u32)i * BM_Q8K_STRIDE), 16);
         if (tid < 64) {
             const uint8_t *cs = act + (src_c + (u32)i * BM_Q8K_STRIDE);
             cdy = *reinterpret_cast<const float *>(cs);
@@ -1155,9 +1155,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
             rd = tail.w >> 16;
         }
     };
-    auto stage_cols = [&]() {
+    auto stage_cols = [&](auto few) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < (decltype(few)::value ? 2 : 4); j++) {
             uint8_t *dst = a_codes + a_dst + 16 * j * kIqStride;
             *reinterpret_cast<u32 *>(dst) = ra[j].x;
             *reinterpret_cast<u32 *>(dst + 32) = ra[j].y;
@@ -1266,40 +1266,49 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     // this lane in its wave's 32 x 32 product: operand row / slot lane % 32, terms 16 (lane / 32) .. of the 32; result v
     // is row 8 (v / 4) + 4 (lane / 32) + v % 4 of slot lane % 32
     const int l32 = lane & 31, kh = lane >> 5;
-    const int wrow = 32 * (wv & 1), wslot = 32 * (wv >> 1);
+    const int wrow = 32 * (wv & 1);
     const uint8_t *my_h = w_hi + (wrow + l32) * kIqStride + 16 * kh;
     const uint8_t *my_l = w_lo + (wrow + l32) * kIqStride + 16 * kh;
-    const uint8_t *my_a = a_codes + (wslot + l32) * kIqStride + 16 * kh;
-    const bool live = wslot < len; // else none of this wave's slots is real
     const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     constexpr int kAcc = EXACT ? G::kLanes : 1;
-    v16f acc[kAcc];
+    // A tile of at most 32 slots, where there are eight accumulators a value: a wave takes 32 rows, all the slots and four of the
+    // accumulators, and the two waves of a row group meet in the closing sum. (With slots for two of the four waves only, the two SIMDs
+    // with those did all the arithmetic: top-8 of 128 experts, us a layer, IQ4_XS 200 tokens 232 -> 205, 777 tokens 387 -> 363;
+    // 400 tokens of IQ2_XXS, hidden 3072, 402 -> 361.)
+    auto run = [&](auto few) __attribute__((always_inline)) {
+    constexpr bool kFew = decltype(few)::value;
+    constexpr int kMine = kFew ? kAcc / 2 : kAcc;
+    const int wslot = kFew ? 0 : 32 * (wv >> 1);
+    const int l0 = kFew ? kMine * __builtin_amdgcn_readfirstlane(wv >> 1) : 0; // the wave's first accumulator
+    const uint8_t *my_a = a_codes + (wslot + l32) * kIqStride + 16 * kh;
+    const bool live = wslot < len; // else none of this wave's slots is real
+    v16f acc[kMine];
 #pragma unroll
-    for (int l = 0; l < kAcc; l++)
+    for (int l = 0; l < kMine; l++)
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[l][v] = 0.0f;
 
     // (the columns' bytes too where the registers allow: the exact forms of the types with eight accumulators a value have few
     // to spare - with everything held over they spilled and ran 6 % slower - so there only the rows' bytes, which come from
     // HBM, are asked for ahead, and the columns', which the cache holds, when their turn comes)
-    constexpr bool kColsAhead = kAcc == 1;
+    constexpr bool kColsAhead = kMine <= 4;
     fetch_rows(0);
-    if constexpr (kColsAhead) fetch_cols(0);
+    if constexpr (kColsAhead) fetch_cols(few, 0);
     for (int i = 0; i < nb; i++) {
         if (i) __syncthreads(); // the readers of the super-block before are done
         if constexpr (!kColsAhead) {
-            fetch_cols(i);
+            fetch_cols(few, i);
             __builtin_amdgcn_sched_barrier(0);
         }
         stage_rows();
         __builtin_amdgcn_sched_barrier(0);
-        stage_cols();
+        stage_cols(few);
         if (i + 1 < nb) {
             fetch_rows(i + 1);
-            if constexpr (kColsAhead) fetch_cols(i + 1);
+            if constexpr (kColsAhead) fetch_cols(few, i + 1);
         }
         __syncthreads();
-        if (!live) continue;
+        if (!kFew && !live) continue;
         const float dy = dy_t[wslot + l32];
         float dd[16];
 #pragma unroll
@@ -1345,11 +1354,11 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
                 // the fold of the offsets first: accumulator l takes sub-block l's scale on its two sums
                 // (crates/qdot/src/lib.rs:8691-8694); the product of the two small integers is exact in f32
 #pragma unroll
-                for (int l = 0; l < 8; l++) {
-                    const float bs = bs_t[l * kIqLine + wslot + l32];
+                for (int l = 0; l < kMine; l++) {
+                    const float bs = bs_t[(l0 + l) * kIqLine + wslot + l32];
 #pragma unroll
                     for (int q4 = 0; q4 < 4; q4++) {
-                        const float4 s4 = *reinterpret_cast<const float4 *>(sc_t + l * kIqLine + wrow + 8 * q4 + 4 * kh);
+                        const float4 s4 = *reinterpret_cast<const float4 *>(sc_t + (l0 + l) * kIqLine + wrow + 8 * q4 + 4 * kh);
                         const float sv[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
                         for (int k = 0; k < 4; k++) {
@@ -1360,38 +1369,73 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
                 }
             }
 #pragma unroll
-            for (int l = 0; l < 8; l++) {
-                const v4i b = *reinterpret_cast<const v4i *>(my_a + 32 * l);
-                const v16i hs = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_h + 32 * l), b, z, 0, 0, 0);
-                const v16i ls = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_l + 32 * l), b, z, 0, 0, 0);
+            for (int l = 0; l < kMine; l++) {
+                const int at = 32 * (l0 + l);
+                const v4i b = *reinterpret_cast<const v4i *>(my_a + at);
+                const v16i hs = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_h + at), b, z, 0, 0, 0);
+                const v16i ls = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(my_l + at), b, z, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 16; v++) acc[l][v] = fmaf(dd[v] * dy, (float)(hs[v] * 256 + ls[v]), acc[l][v]);
             }
         }
     }
+    // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order), four rows a store
     const int n = wslot + l32;
-    if (live && n < len) {
-        float *out = y + (size_t)tab->slot[n] * rpe + row0 + wrow + 4 * kh;
+    float *const out = y + (size_t)(live ? tab->slot[wslot + l32] : 0) * rpe + row0 + wrow + 4 * kh;
+    auto store = [&](int q4, float r0, float r1, float r2, float r3) {
+        // rows_per_expert is a multiple of 16 and these four rows start at a multiple of 4: all inside or all outside
+        if (live && n < len && row0 + wrow + 4 * kh + 8 * q4 < rpe) *reinterpret_cast<float4 *>(out + 8 * q4) = make_float4(r0, r1, r2, r3);
+    };
+    if constexpr (kFew) {
+        // a wave closes eight of a lane's sixteen results and has the other wave's accumulators of them through LDS
+        __syncthreads();
+        float *const swap = reinterpret_cast<float *>(a_codes) + 4096 * (wv & 1) + lane;
+        const int h = __builtin_amdgcn_readfirstlane(wv >> 1);
+        auto close = [&](auto from) __attribute__((always_inline)) {
+            constexpr int mine = decltype(from)::value, other = 8 - mine;
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-            // rows_per_expert is a multiple of 16 and these four rows start at a multiple of 4: all inside or all outside
-            if (row0 + wrow + 4 * kh + 8 * q4 < rpe) {
+            for (int l = 0; l < kMine; l++)
+#pragma unroll
+                for (int v = 0; v < 8; v++) swap[64 * ((h * kMine + l) * 8 + v)] = acc[l][other + v];
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
                 float r[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const int v = 4 * q4 + k;
-                    if constexpr (kAcc == 8) { // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order)
-                        const float t0 = acc[0][v] + acc[4][v], t1 = acc[1][v] + acc[5][v];
-                        const float t2 = acc[2][v] + acc[6][v], t3 = acc[3][v] + acc[7][v];
-                        r[k] = (t0 + t2) + (t1 + t3);
-                    } else {
-                        r[k] = acc[0][v];
-                    }
+                    float t[kMine];
+#pragma unroll
+                    for (int l = 0; l < kMine; l++) t[l] = acc[l][mine + 4 * q + k] + swap[64 * (((1 - h) * kMine + l) * 8 + 4 * q + k)];
+                    r[k] = (t[0] + t[2]) + (t[1] + t[3]);
                 }
-                *reinterpret_cast<float4 *>(out + 8 * q4) = make_float4(r[0], r[1], r[2], r[3]);
+                store(mine / 4 + q, r[0], r[1], r[2], r[3]);
             }
+        };
+        if (h) close(std::integral_constant<int, 8>{});
+        else close(std::integral_constant<int, 0>{});
+    } else {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) {
+            float r[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int v = 4 * q4 + k;
+                if constexpr (kMine == 8) {
+                    const float t0 = acc[0][v] + acc[4][v], t1 = acc[1][v] + acc[5][v];
+                    const float t2 = acc[2][v] + acc[6][v], t3 = acc[3][v] + acc[7][v];
+                    r[k] = (t0 + t2) + (t1 + t3);
+                } else {
+                    r[k] = acc[0][v];
+                }
+            }
+            store(q4, r[0], r[1], r[2], r[3]);
         }
     }
+    };
+    if constexpr (kAcc == 8) {
+        if (len <= 32) return run(std::true_type{});
+    }
+    run(std::false_type{});
 }
 
 bool gemm_supported(int wtype) {

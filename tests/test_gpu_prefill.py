@@ -576,7 +576,7 @@ def test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype, n_slots=70):
 
 # Tiles of at most 32 slots, whose accumulators are split between two waves, beside wide ones: every edge of the two, a slab that is
 # not whole, one super-block and an odd count of them; bit for bit against the one-column dot.
-@pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K))
+@pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K, bm.Q3_K, bm.IQ2_XXS, bm.IQ3_XXS, bm.IQ4_XS))
 @pytest.mark.parametrize("rpe,k,counts", ((80, 256, (1, 32, 33, 64, 65)), (16, 768, (31, 2, 96, 97)), (144, 1792, (17, 0, 128, 5))))
 def test_gemm_of_narrow_and_wide_tiles(gpu, wtype, rpe, k, counts):
     from test_gpu_decode import random_blocks
