@@ -231,7 +231,9 @@ struct XLds {
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef u32 v2u __attribute__((ext_vector_type(2)));
 typedef u32 v4u __attribute__((ext_vector_type(4)));
 
@@ -351,10 +353,12 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     const int wr = tid >> 2, p = tid & 3;
     const uint8_t *we = w + (size_t)e * rpe * row_bytes;
     auto row_at = [&](int first_row) { return (u32)(first_row + wr < rpe ? first_row + wr : rpe - 1) * row_bytes; };
-    // (of at most 32 slots: of column tid / 8 the codes 16 (tid % 8) ..)
-    const bool narrow = len <= 32;
+    // (of at most 32 slots: of column tid / 8 the codes 16 (tid % 8) ..; of at most 16: of column tid / 16 the codes 8 (tid % 16) ..)
+    const bool narrow = len <= 32, thin = kQ45 && len <= 16;
     const u32 apair = tab->col[wr] * col_bytes + 8 * p + (u32)nb * BM_Q82_SB_REF;
-    const u32 acol = narrow ? tab->col[tid >> 3] * col_bytes + 16 + 16 * (tid & 7) : tab->col[wr] * col_bytes + 16 + 16 * p;
+    const u32 acol = thin ? tab->col[tid >> 4] * col_bytes + 16 + 8 * (tid & 15)
+                     : narrow ? tab->col[tid >> 3] * col_bytes + 16 + 16 * (tid & 7)
+                              : tab->col[wr] * col_bytes + 16 + 16 * p;
     v4u rw, rq = {0, 0, 0, 0}, rh = {0, 0, 0, 0}, ra[2] = {};
     u32 q6d = 0, q6s = 0, q6t = 0; // (Q6_K; words of their own: as parts of a vector they were moved, and waited for, as they came)
     float d8, y0 = 0.0f, y4 = 0.0f;
@@ -398,19 +402,19 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
     // Word k of the sixteen code bytes of the row. Four codes a word become f16 in the order 0, 2, 1, 3 (rows and columns alike: a
     // sum's terms may come in any order). Low nibbles: group p of the buffer's first four; high nibbles: of its second four (Q6_K:
     // the values' own order).
-    auto stash_row = [&](auto half, int k) __attribute__((always_inline)) {
+    auto stash_word = [&](auto half, int k, u32 x, [[maybe_unused]] u32 high) __attribute__((always_inline)) {
         constexpr int j = decltype(half)::value;
-        const u32 x = rw[k], x8 = x >> 8;
+        const u32 x8 = x >> 8;
         u32 l0 = and_or(x, m4l, k1024), l1 = and_or(x8, m4l, k1024), h0 = and_or(x, m4h, k1024), h1 = and_or(x8, m4h, k1024);
         if constexpr (WT == BM_Q5K) { // the fifth bits of blocks 4 j + 2 (p / 2) and the one after
-            const u32 t = rq[k] >> (4 * j + 2 * (p >> 1));
+            const u32 t = high >> (4 * j + 2 * (p >> 1));
             l0 = and_or(t << 4, mx, l0);
             l1 = and_or(t >> 4, mx, l1);
             h0 = and_or(t << 7, my, h0);
             h1 = and_or(t >> 1, my, h1);
         }
         if constexpr (WT == BM_Q6K) { // the two high bits of quarters p / 2 and p / 2 + 2
-            const u32 t = rq[k] >> (2 * (p >> 1)), t4 = t << 4, t8 = t >> 4;
+            const u32 t = high >> (2 * (p >> 1)), t4 = t << 4, t8 = t >> 4;
             l0 = and_or(t4, mx, l0);
             l1 = and_or(t8, mx, l1);
             h0 = and_or(t4, my, h0);
@@ -475,7 +479,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
         constexpr int kPieces = decltype(few)::value ? 1 : 2; // of a column's codes
         if (st == 0) fetch_factors(now, half);
         if (st < 4) {
-            stash_row(half, st);
+            stash_word(half, st, rw[st], rq[st]);
             if (st == 3) fetch_row(next, after);
         } else if (st < 4 + 2 * kPieces) {
             stash_col(few, half, (st - 4) >> 1, st & 1);
@@ -639,19 +643,158 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int 
                 for (int v = 0; v < 32; v++) acc[l][v] = 0.0f;
         }
     };
-    if (narrow) run(std::true_type{});
+    // A tile of at most 16 slots: a wave takes 16 rows, all the slots and all the accumulators; products and outer products are the
+    // 16 x 16 forms (one of scales four blocks at a time), half the multiply-adds of a 32 x 32 tile's padding. Lane: row (operand: slot, row)
+    // lane % 16, four of a group's sixteen values by lane / 16; result r: slot 4 (lane / 16) + r of row lane % 16.
+    // So little arithmetic a byte that it is the bytes on their way that bound it: whole super-blocks are asked for two ahead, into a ring
+    // of three sets of registers. (Top-8 of 128 experts Q4_K, us a layer: 256 tokens 217 -> 209, 512 tokens 280 -> 275; top-8 of 64 of
+    // 7168 x 1536, 300 tokens 890 -> 828. Q6_K, whose bytes come in more and smaller requests, was 2 to 5 % slower this way.)
+    [[maybe_unused]] auto run_thin = [&]() __attribute__((always_inline)) {
+        const int l16 = lane & 15, kq = lane >> 4;
+        const LdsB my_row = (LdsB)lds + (16 * wv + l16) * kXStride + 8 * kq, my_col = (LdsB)lds + 2 * kXCodes + l16 * kXStride + 8 * kq;
+        const LdsB my_fr = (LdsB)lds + 4 * kXCodes + 4 * (16 * wv + l16), my_fc = (LdsB)lds + 4 * kXCodes + 4 * l16;
+        const LdsB my_sr = my_fr + kq * kXLine, my_sc = my_fc + (X::kScales + kq) * kXLine;
+        const LdsB my_mr = my_fr + kq * kXLine + X::kMinsAt, my_mc = my_fc + kq * kXLine + X::kMinsAt + 8 * kXLine;
+        // what a thread stages of a column: of column tid / 16 the codes 8 (tid % 16) .., of column tid / 8 % 16 the factors of block tid % 8
+        const int wc = (tid >> 3) & 15, wb = tid & 7;
+        const u32 col_pair = tab->col[wc] * col_bytes + 8 * wb + (u32)nb * BM_Q82_SB_REF;
+        const LdsB put_col = (LdsB)lds + 2 * kXCodes + (tid >> 4) * kXStride + 16 * (tid & 15);
+        // (a block of the half that is not being staged goes to a slot that nobody reads)
+        const LdsB put_d8[2] = {(LdsB)lds + 4 * kXCodes + (X::kScales + (wb & 3)) * kXLine + 4 * (wc + (wb < 4 ? 0 : 16)),
+                                (LdsB)lds + 4 * kXCodes + (X::kScales + (wb & 3)) * kXLine + 4 * (wc + (wb < 4 ? 16 : 0)) + X::kHalf};
+        const LdsB put_isum = (LdsB)lds + 4 * kXCodes + X::kMinsAt + (8 + wb) * kXLine + 4 * wc;
+        struct Sb { // a super-block's bytes
+            v4u w[2], q, head;
+            v2u col[2], pair;
+        } ring[3];
+        auto fetch = [&](Sb &b, At at) __attribute__((always_inline)) {
+            const uint8_t *blk = we + (at.row + (u32)at.i * kBlock);
+            b.head = ld16(blk);
+            b.pair = *reinterpret_cast<const v2u *>(act + (col_pair + 64 * (u32)at.i));
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                b.w[j] = ld16(blk + kCodesAt + 64 * j + 16 * p);
+                b.col[j] = *reinterpret_cast<const v2u *>(act + (acol + (u32)(2 * at.i + j) * BM_Q82X4_STRIDE));
+            }
+            b.q = WT == BM_Q5K ? ld16(blk + 16 + 16 * (p & 1)) : (v4u){0, 0, 0, 0};
+        };
+        auto stage = [&](const Sb &b, auto half) __attribute__((always_inline)) {
+            constexpr int j = decltype(half)::value;
+#pragma unroll
+            for (int k = 0; k < 4; k++) stash_word(half, k, b.w[j][k], b.q[k]);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const u32 u = b.col[j][k] ^ 0x80808080u;
+                put(put_col, j * kXCodes + 8 * k, h2_less(and_or(u, m8, k1024), 1152.0f), h2_less(and_or(u >> 8, m8, k1024), 1152.0f));
+            }
+            // crates/gguf/src/quant.rs:620-628 get_scale_min_k4
+            const float d = bm_half_to_f32((unsigned short)(b.head.x & 0xffffu)), dmin = bm_half_to_f32((unsigned short)(b.head.x >> 16));
+            const u32 b0 = (b.head.y >> (8 * p)) & 0xffu, b4 = (b.head.z >> (8 * p)) & 0xffu, b8 = (b.head.w >> (8 * p)) & 0xffu;
+            if constexpr (j == 0) {
+                atomicOr((u32 *)(my_factor + X::kHeadsAt), b.head.x);
+                factor(0, d * (float)(b0 & 63u));
+                factor(X::kMinsAt, -(dmin * (float)(b4 & 63u)));
+                factor(X::kMinsAt + 4 * kXLine, -(dmin * (float)((b8 >> 4) | ((b4 >> 6) << 4))));
+                *(LdsF)put_isum = bm_bits_f32(b.pair.y);
+            } else {
+                factor(X::kHalf, d * (float)((b8 & 15u) | ((b0 >> 6) << 4)));
+            }
+            *(LdsF)put_d8[j] = bm_bits_f32(b.pair.x);
+        };
+        v16f acc[2]; // accumulator 4 h + block: [h], results 4 block ..
+        auto arithmetic = [&](auto half, const Sb &staged) __attribute__((always_inline)) {
+            constexpr int j = decltype(half)::value;
+            const v16f z16 = {};
+            const v4f z4 = {};
+            v4f sum[8];
+            const v16f pd = __builtin_amdgcn_mfma_f32_16x16x1f32(*(LdsVF)(my_sc + j * X::kHalf), *(LdsVF)(my_sr + j * X::kHalf), z16, 0, 0, 0);
+            // the min terms come before a super-block's products: accumulator l takes sub-block l's (crates/qdot/src/lib.rs:4389-4394)
+            if constexpr (j == 0)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    acc[h] = __builtin_amdgcn_mfma_f32_16x16x1f32(*(LdsVF)(my_mc + 4 * h * kXLine), *(LdsVF)(my_mr + 4 * h * kXLine), acc[h], 0, 0, 0);
+#pragma unroll
+            for (int gr = 0; gr < 8; gr++) {
+                const int at = j * kXCodes + 32 * (4 * ((gr >> 1) & 1) + 2 * (gr >> 2) + (gr & 1)), ct = j * kXCodes + 32 * gr;
+                const v2u a = *(LdsV2)(my_row + at), b = *(LdsV2)(my_col + ct);
+                sum[gr] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, b), __builtin_bit_cast(v4h, a), z4, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            stage(staged, std::integral_constant<int, 1 - j>{});
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int gr = 0; gr < 8; gr++) {
+                const int bk = gr >> 1, h = gr & 1;
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[h][4 * bk + r] = fmaf(pd[4 * bk + r], sum[gr][r], acc[h][4 * bk + r]);
+            }
+        };
+        factor(X::kHeadsAt, 0.0f);
+        int far_left = left, far_row0 = row0; // of the super-block asked for last
+        At far = {row_at(row0), 0};
+        auto advance = [&]() { // to the super-block after it, in the next slab behind a slab's last (the very last: itself, for no reader)
+            if (far.i + 1 < nb) far.i++;
+            else if (far_left > 1) far_left--, far_row0 += kGemmBM, far = At{row_at(far_row0), 0};
+        };
+        fetch(ring[0], far);
+        advance();
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(ring[1], far);
+        advance();
+        __builtin_amdgcn_sched_barrier(0);
+        stage(ring[0], kFirst);
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[0][v] = acc[1][v] = 0.0f;
+        int todo = left * nb, i = 0;
+        auto step = [&](auto at) __attribute__((always_inline)) { // the super-block in the ring's place `at`
+            constexpr int c = decltype(at)::value;
+            fetch(ring[(c + 2) % 3], far);
+            advance();
+            __builtin_amdgcn_sched_barrier(0);
+            arithmetic(kFirst, ring[c]);
+            __syncthreads();
+            arithmetic(kSecond, ring[(c + 1) % 3]);
+            __syncthreads();
+            if (++i < nb) return;
+            i = 0;
+            // the closing sum of the eight lanes (crates/qdot/src/lib.rs:4128 hsum_float_8's order) and the store
+            const int row = row0 + 16 * wv + l16;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int n = 4 * kq + r;
+                const float t0 = acc[0][r] + acc[1][r], t1 = acc[0][4 + r] + acc[1][4 + r], t2 = acc[0][8 + r] + acc[1][8 + r], t3 = acc[0][12 + r] + acc[1][12 + r];
+                if (row < rpe && n < len) y[(size_t)tab->slot[n] * rpe + row] = (t0 + t2) + (t1 + t3);
+            }
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[0][v] = acc[1][v] = 0.0f;
+            row0 += kGemmBM;
+        };
+        for (;;) {
+            step(std::integral_constant<int, 0>{});
+            if (--todo == 0) break;
+            step(std::integral_constant<int, 1>{});
+            if (--todo == 0) break;
+            step(std::integral_constant<int, 2>{});
+            if (--todo == 0) break;
+        }
+    };
+    if (thin) {
+        if constexpr (kQ45) run_thin();
+    } else if (narrow) run(std::true_type{});
     else run(std::false_type{});
     if constexpr (kQ45) {
         u32 heads = 0u;
 #pragma unroll
         for (int q = 0; q < 4; q++) heads |= *(const u32 *)(lds + 4 * kXCodes + X::kHeadsAt + 4 * lane + q * kXLine);
         if (__ballot((heads & 0x8000u) != 0u) == 0) return; // (see above)
-        const int end = row0 < rpe ? row0 : rpe, first = narrow ? 8 * gh : 0, last = narrow ? first + 8 : 16; // the results this wave stored
+        // the results this lane stored
+        const int end = row0 < rpe ? row0 : rpe, first = narrow && !thin ? 8 * gh : 0, last = thin ? 4 : narrow ? first + 8 : 16;
 #pragma nounroll
-        for (int row = first_row + wrow0 + l32; row < end; row += kGemmBM)
+        for (int row = first_row + (thin ? 16 * wv + (lane & 15) : wrow0 + l32); row < end; row += kGemmBM)
 #pragma nounroll
             for (int v = first; v < last; v++) {
-                const int n = wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
+                const int n = thin ? 4 * (lane >> 4) + v : wslot0 + 8 * (v >> 2) + 4 * kh + (v & 3);
                 if (n >= len) continue;
                 float *out = y + (size_t)tab->slot[n] * rpe + row;
                 if (*out == 0.0f) *out = q45_value<WT>(we + (size_t)row * row_bytes, act + (size_t)tab->col[n] * col_bytes, nb);

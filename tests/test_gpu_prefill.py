@@ -574,10 +574,11 @@ def test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype, n_slots=70):
         b.free()
 
 
-# Tiles of at most 32 slots, whose accumulators are split between two waves, beside wide ones: every edge of the two, a slab that is
-# not whole, one super-block and an odd count of them; bit for bit against the one-column dot.
+# Tiles of at most 32 slots, whose accumulators are split between two waves, and of at most 16, which have 16 x 16 products (Q4_K, Q5_K) and
+# a ring of three super-blocks, beside wide ones: every edge of them, a slab that is not whole, one super-block and an odd count of them; bit for bit against the one-column dot.
 @pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K, bm.Q3_K, bm.IQ2_XXS, bm.IQ3_XXS, bm.IQ4_XS))
-@pytest.mark.parametrize("rpe,k,counts", ((80, 256, (1, 32, 33, 64, 65)), (16, 768, (31, 2, 96, 97)), (144, 1792, (17, 0, 128, 5))))
+@pytest.mark.parametrize("rpe,k,counts", ((80, 256, (1, 32, 33, 64, 65)), (16, 768, (31, 2, 96, 97)), (144, 1792, (17, 0, 128, 5)),
+                                          (272, 512, (15, 16, 17, 80))))
 def test_gemm_of_narrow_and_wide_tiles(gpu, wtype, rpe, k, counts):
     from test_gpu_decode import random_blocks
     n_experts, n_slots = len(counts), sum(counts)
@@ -601,8 +602,9 @@ def test_gemm_of_narrow_and_wide_tiles(gpu, wtype, rpe, k, counts):
 
 
 @pytest.mark.parametrize("wtype", (bm.Q4_K, bm.Q5_K, bm.Q6_K))
-def test_gemm_of_narrow_tiles_underflow_and_signed_zeros(gpu, wtype):
-    test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype, n_slots=40)
+@pytest.mark.parametrize("n_slots", (20, 40))
+def test_gemm_of_narrow_tiles_underflow_and_signed_zeros(gpu, wtype, n_slots):
+    test_gemm_scales_that_underflow_and_signed_zeros(gpu, wtype, n_slots=n_slots)
 
 
 @pytest.mark.parametrize("wtype,k", ((bm.Q4_K, 256), (bm.Q5_K, 768), (bm.Q6_K, 512)))
