@@ -516,6 +516,35 @@ def test_fused_step_matches_the_chain_and_the_oracle(gpu, types, hidden, ff, n_e
     L.free()
 
 
+# Both orders of the fused step's workgroups (by dies from 64 slots on): slot counts that are powers of two and that are not, rows whose
+# last eight of blocks is not whole, repeated experts, types on either column form.
+@pytest.mark.parametrize("types,hidden,ff,m,top_k", (
+    ((bm.Q4_K, bm.Q4_K, bm.Q6_K), 768, 256, 9, 8),
+    ((bm.Q4_K, bm.Q4_K, bm.Q4_K), 256, 512, 13, 5),
+    ((bm.Q6_K, bm.Q6_K, bm.Q6_K), 1280, 256, 10, 7),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 512, 768, 16, 4),
+    ((bm.Q3_K, bm.Q3_K, bm.IQ2_XXS), 768, 256, 11, 6),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 256, 256, 63, 1),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 256, 256, 64, 1),
+))
+def test_fused_step_in_either_order(gpu, types, hidden, ff, m, top_k):
+    L = Layer(gpu, types, hidden, ff, 8, 650 + hidden + ff)
+    rng = np.random.default_rng(651)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, 8, top_k)
+    gpu.fault_clear()
+    y, h, act_h, act_x = run_fused_step(gpu, L, x, ids, wts, top_k, resid)
+    want_y, want_h = L.oracle(x, ids, wts, top_k)
+    for t in range(m):
+        assert np.array_equal(act_x[t], ora.quantize_col(types[0], x[t])), f"act_x token {t}"
+    assert_f32(h, want_h, "h")
+    for s in range(m * top_k):
+        assert np.array_equal(act_h[s], ora.quantize_col(types[2], want_h[s * ff:(s + 1) * ff])), f"act_h slot {s}"
+    assert_f32(y, (want_y.reshape(m, hidden) + resid).astype(np.float32).reshape(-1), "y + resid")
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    L.free()
+
+
 def test_fused_step_at_the_token_limit(gpu):
     """bm_moe_decode takes 1..=1024 tokens a launch: the limit itself against the oracle, one more refused by name."""
     L = Layer(gpu, (bm.Q4_K, bm.Q4_K, bm.Q6_K), 256, 256, 9, 650)
