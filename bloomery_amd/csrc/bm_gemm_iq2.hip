@@ -18,13 +18,18 @@
 // and used for one 32- or 64-slot product. So:
 //   * a wave takes 64 rows and all slots of the tile: no weight is unpacked twice, none goes through LDS, a column operand serves two
 //     row groups;
-//   * a lane owns a row (lane % 32) and one half of every super-block (lane / 32), 32 contiguous bytes of the file;
+//   * a lane owns a row (lane % 32) and sixteen bytes (lane / 32) of each 32 of a super-block in the file, so that two lanes next to
+//     each other ask for 32 contiguous bytes of a row;
 //   * a grid entry is two eight-byte halves of f16 values, in sixteen copies that start on sixteen different bank pairs: the lookups
 //     of a wave, 64 different entries, never collide (a single copy collides about three deep). An entry's address is one byte
 //     permute of the index and the lane's copy;
 //   * signs are shifted out of the seven-bit field and its parity straight into the f16 sign bits;
 //   * the terms of a 16-value step are made between the matrix instructions of the step before, and a super-block's bytes are asked for
-//     a whole super-block ahead;
+//     a whole super-block ahead, one request every second step (one a step: 1 to 2 % slower; a wave's request covers 32 rows, and
+//     eight waves asking at once fill the address unit's queue);
+//   * a row group's lookups go out as soon as its last terms are made, half a step earlier than both groups' at the step's end. That, the
+//     order of the requests and three vector instructions less a lookup (the LDS base, a multiplication by 2^14 + 1 and its wait state):
+//     600 tokens of 64 experts 265 -> 255 us a layer, 192 tokens of 7168 values 497 -> 472, 1024 tokens of the large layer 2.34 -> 2.29 ms;
 //   * tiles of at most 32 slots leave the second slot group out; a gate and an up are one launch, whose last round of workgroups
 //     is then half as much of the whole.
 // 133 KB of LDS, one workgroup of eight waves a CU. 8192 slots of 256 experts, gate and up of 2048 rows of 7168 values:
@@ -64,6 +69,18 @@ constexpr u32 kIqMagMax = (1u << 24) / (31u * 43u);
 __device__ __forceinline__ u32 iq_and_or(u32 x, u32 mask, u32 bits) {
     u32 r;
     __asm__("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(bits));
+    return r;
+}
+// x | x << 14. (Left to the compiler it becomes a multiplication and a wait state behind it.)
+__device__ __forceinline__ u32 iq_twice14(u32 x) {
+    u32 r;
+    __asm__("v_lshl_or_b32 %0, %1, 14, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+// Bits 0 and 16 of x into the sign bits of a pair of f16 values that have none: a product modulo 2^16 and a sum.
+__device__ __forceinline__ u32 iq_low_bit_sign(u32 x, u32 pair) {
+    u32 r;
+    __asm__("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(0x80008000u), "v"(pair));
     return r;
 }
 __device__ __forceinline__ u32 iq_f16_pair(float a, float b) {
@@ -115,20 +132,20 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
 
     const int l32 = lane & 31, kh = lane >> 5;
     const u32 my_copy = 8u * (u32)(lane & 15);
-    const LdsB my_col = (LdsB)lds + kGridBytes + l32 * kIqColStride + 256 * kh;
+    const LdsB my_col = (LdsB)lds + kGridBytes + l32 * kIqColStride + 128 * kh;
     v16f acc[2][NCT], sum[2][NCT]; // [row group][slot group]; result v: slot 8 (v / 4) + 4 kh + v % 4, row l32
-    v4u raw[2][2], ahead[2][2]; // [row group][sub-blocks 4 kh and the next, the two after]: index word, sign/scale word, twice; the next block's
+    v4u raw[2][2], ahead[2][2]; // [row group][q]: sub-blocks 4 q + 2 kh and the next: index word, sign/scale word, twice; the next block's
     u32 rd;                     // the next block's d of row group kh
     u32 wofs[2], dofs; // where this lane's requests for rows start
     v2u gr[2][2];   // [row group][half]: a grid entry
     v4u term[2][2]; // [step % 2][row group]
     v4u colv[NCT];  // [slot group]
     u32 scale[2];   // [row group] (2 s + 1) twice, f16
-    // Two lanes next to each other ask for one row's two halves (they share a line; lanes 32 apart would look it up twice), and the
+    // Two lanes next to each other ask for one row's 32 bytes (they share a line; lanes 32 apart would look it up twice), and the
     // pieces are dealt to the lanes that own them through the LDS crossbar.
     auto fetch_raw = [&](int i, int n) __attribute__((always_inline)) { // request n of five
         const u32 at = (u32)i * BM_IQ2XXS_BLOCK;
-        if (n < 4) __builtin_memcpy(&ahead[n >> 1][n & 1], we + (wofs[n >> 1] + at) + 2 + 16 * (n & 1), 16);
+        if (n < 4) __builtin_memcpy(&ahead[n & 1][n >> 1], we + (wofs[n & 1] + at) + 2 + 32 * (n >> 1), 16);
         else rd = bm_ld2u(we + (dofs + at));
     };
     const int owner = 4 * (2 * l32 + kh);
@@ -147,8 +164,9 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
     // The eight values that byte j of an index word stands for: the grid's magnitudes, and with signs and scale from the other word.
     auto grid_of = [&](u32 index, int j, v2u(&half)[2]) __attribute__((always_inline)) {
         const u32 at = __builtin_amdgcn_perm(index, my_copy, 0x0c0c0000u | ((4u + (u32)j) << 8));
-        half[0] = *(LdsV2)((LdsB)lds + at);
-        half[1] = *(LdsV2)((LdsB)lds + at + 128);
+        // (the grid is where LDS starts: with the array's own address, a zero that only the linker fills in, each lookup would add it)
+        half[0] = *(LdsV2)at;
+        half[1] = *(LdsV2)(at + 128u);
     };
     auto scale_of = [&](u32 aux) __attribute__((always_inline)) { // 1024 + 2 s + 1 less 1024
         const u32 x = (2u * (aux >> 28)) | 0x6401u, b = x | (x << 16);
@@ -158,9 +176,8 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
     auto terms_of = [&](u32 aux, int j, const v2u(&half)[2], u32 scale_pair) __attribute__((always_inline)) {
         const u32 v = (aux >> (7 * j)) & 127u;
         const u32 v8 = v | ((u32)__builtin_popcount(v) << 7); // bit 7: the parity
-        u32 s = v8 | (v8 << 14); // bits 0, 1, 4, 5 and sixteen on: the signs of values 0, 1, 4, 5 and 2, 3, 6, 7
-        __asm__("" : "+v"(s));   // (else the shifts below become multiplications, four times as slow)
-        const u32 m[4] = {iq_and_or(s << 15, msign, half[0].x), iq_and_or(s << 14, msign, half[0].y), iq_and_or(s << 11, msign, half[1].x),
+        const u32 s = iq_twice14(v8); // bits 0, 1, 4, 5 and sixteen on: the signs of values 0, 1, 4, 5 and 2, 3, 6, 7
+        const u32 m[4] = {iq_low_bit_sign(s, half[0].x), iq_and_or(s << 14, msign, half[0].y), iq_and_or(s << 11, msign, half[1].x),
                           iq_and_or(s << 10, msign, half[1].y)};
         v4u out;
 #pragma unroll
@@ -168,17 +185,14 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
         return out;
     };
     // step t of sixteen: eight values of index byte t % 4 of the lane's sub-block t / 4
-    auto lookup = [&](int t) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < 2; r++) grid_of(raw[r][t >> 3][2 * ((t >> 2) & 1)], t & 3, gr[r]);
-    };
+    auto lookup = [&](int t, int r) __attribute__((always_inline)) { grid_of(raw[r][t >> 3][2 * ((t >> 2) & 1)], t & 3, gr[r]); };
     auto make = [&](int t, int r) __attribute__((always_inline)) {
         const u32 aux = raw[r][t >> 3][2 * ((t >> 2) & 1) + 1];
         if ((t & 3) == 0) scale[r] = scale_of(aux);
         term[t & 1][r] = terms_of(aux, t & 3, gr[r], scale[r]);
     };
     auto read_col = [&](int at, int t, int c) __attribute__((always_inline)) {
-        const LdsB p = my_col + at + 32 * kIqColStride * c + 16 * t;
+        const LdsB p = my_col + at + 32 * kIqColStride * c + 256 * (t >> 3) + 16 * (t & 7);
         const v2u a = *(LdsV2)p, b = *(LdsV2)(p + 8);
         colv[c] = (v4u){a.x, a.y, b.x, b.y};
     };
@@ -189,10 +203,12 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
         for (int n = 0; n < 5; n++) fetch_raw(i, n);
         deal(0);
         deal(1);
-        lookup(0);
+        lookup(0, 0);
+        lookup(0, 1);
         make(0, 0);
         make(0, 1);
-        lookup(1);
+        lookup(1, 0);
+        lookup(1, 1);
     };
     // the super-block's scaled sums into the accumulators of slot group c
     auto scale_sums = [&](int buf, int c) __attribute__((always_inline)) {
@@ -225,7 +241,7 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
                 for (int n = 0; n < 4; n++) {
                     const v4u words = n < 2 ? raw[r][0] : raw[r][1];
                     const u32 index = n & 1 ? words.z : words.x, aux = n & 1 ? words.w : words.y, by = scale_of(aux);
-                    const LdsB col = my_col + buf * kIqCols + 32 * kIqColStride * c + 64 * n;
+                    const LdsB col = my_col + buf * kIqCols + 32 * kIqColStride * c + 256 * (n >> 1) + 64 * (n & 1);
                     v16f part = {};
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
@@ -249,7 +265,7 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
         for (int r = 0; r < 2; r++) {
             const int row = row0 + 64 * wv + 32 * r + l32;
             const int asked = row0 + 64 * wv + 32 * r + (lane >> 1);
-            wofs[r] = (u32)(asked < rpe ? asked : rpe - 1) * row_bytes + 32u * (u32)(lane & 1);
+            wofs[r] = (u32)(asked < rpe ? asked : rpe - 1) * row_bytes + 16u * (u32)(lane & 1);
             if (r == kh) dofs = (u32)(row < rpe ? row : rpe - 1) * row_bytes;
 #pragma unroll
             for (int c = 0; c < NCT; c++)
@@ -266,7 +282,6 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
         for (int i = 0; i < nb; i++) {
             const int next = i + 1 < nb ? i + 1 : i, now_at = (i & 1) * kIqCols, next_at = kIqCols - now_at; // the last one's staging has no reader
             const v16f z = {};
-            take_d();
             read_col(now_at, 0, 0);
             if (NCT == 2) read_col(now_at, 0, NCT - 1);
             fetch_cols(next); // before the rows' bytes: loads come back in order, and these are waited for first
@@ -281,14 +296,20 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
                 };
                 product(0, 0);
                 make((t + 1) & 15, 0);
+                lookup((t + 2) & 15, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 product(1, 0);
                 if (t < 15) read_col(now_at, t + 1, 0);
-                if (t < 5) fetch_raw(next, t); // (one a step: a run of them fills the address unit's queue and stops the wave)
+                if (t % 2 == 0 && t < 8) fetch_raw(next, t / 2); // (a run of them fills the address unit's queue and stops the wave)
+                if (t == 8) {
+                    take_d();
+                    fetch_raw(next, 4);
+                }
                 if (t >= 16 - 4 * kPieces) stash_word(next_at, t - (16 - 4 * kPieces));
                 __builtin_amdgcn_sched_barrier(0);
                 if (NCT == 2) product(0, NCT - 1);
                 make((t + 1) & 15, 1);
+                lookup((t + 2) & 15, 1);
                 __builtin_amdgcn_sched_barrier(0);
                 if (NCT == 2) product(1, NCT - 1);
                 if (NCT == 2 && t < 15) read_col(now_at, t + 1, NCT - 1);
@@ -296,7 +317,6 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
                 if (t == 12) deal(0);
                 if (t == 15) deal(1);
                 if (t == 14) read_mag(i & 1);
-                lookup((t + 2) & 15);
                 if (t == 15) {
                     mag_quad();
                     stash_ends((i + 1) & 1);
