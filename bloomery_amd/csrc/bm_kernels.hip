@@ -778,12 +778,14 @@ __global__ __launch_bounds__(256) void k_gate_up_x(const float *x, const uint8_t
 // ------------------------------------------------------------- the fused step for the types that take Q8_K columns
 
 // `cols` columns of nb blocks each, f32 rows at x (column c at x + c * nb * 256), into LDS at `dst` by the workgroup's
-// waves, block by block.
+// waves, block by block. T: the workgroup's thread count.
+template <int T = 256>
 __device__ __forceinline__ void q8k_stage_cols(const float *x, uint8_t *dst, int cols, int nb, u32 *fault, u32 layer,
                                                const u32 *ids = nullptr, u32 n_experts = 0) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = 4; // (256 threads: every caller's workgroup)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int n_waves = T / 64;
     const int total = cols * nb;
-    constexpr int kAhead = 6; // blocks whose loads a wave has in flight
+    constexpr int kAhead = T == 256 ? 6 : T == 512 ? 3 : 2; // blocks whose loads a wave has in flight
     for (int b0 = wave; b0 < total; b0 += kAhead * n_waves) {
         float4 x4[kAhead];
 #pragma unroll
@@ -949,9 +951,9 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
 
 // k_down_combine for down stacks that dot against Q8_K columns: the token's slot rows of h (f32) are quantized by
 // every workgroup into LDS; the first workgroup of a token also leaves the columns in act_h.
-template <int WT, int U, int NB>
-__global__ __launch_bounds__(256) void k_down_combine_hq(const uint8_t *w, u32 n_experts, int nb, const float *h,
-                                                         uint8_t *act_h, const u32 *sel, const float *wts,
+template <int WT, int U, int NB, int T>
+__global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_experts, int nb, const float *h,
+                                                       uint8_t *act_h, const u32 *sel, const float *wts,
                                                          const float *resid, int spt_word, int rpe, float *y, u32 *fault,
                                                          u32 layer) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -959,7 +961,7 @@ __global__ __launch_bounds__(256) void k_down_combine_hq(const uint8_t *w, u32 n
     // the grid and spt_word as k_down_combine's
     const int rb = (int)(spt_word & kDownRowMajor ? blockIdx.x : blockIdx.z * kDies + blockIdx.x), t = (int)blockIdx.y;
     const int spt = spt_word & 0xffff, shift = ((spt_word >> 16) & 0xff) - 1;
-    const int D = shift >= 0 ? 64 >> shift : 64 / spt;
+    const int D = shift >= 0 ? (T / 4) >> shift : T / 4 / spt;
     if (rb * D >= rpe) return;
     const int e = shift >= 0 ? quad & (spt - 1) : quad % spt, dl = shift >= 0 ? quad >> shift : quad / spt;
     const int r = rb * D + dl;
@@ -967,7 +969,7 @@ __global__ __launch_bounds__(256) void k_down_combine_hq(const uint8_t *w, u32 n
     const u32 id = sel[t * spt + e];
     // Q8_2_X4 columns: the token's f32 rows of h are asked for before anything that waits for the expert id, so they
     // arrive with it and are encoded while the weight rows are on their way
-    Q82Cols<4, 256> hrows;
+    Q82Cols<4, T> hrows;
     if constexpr (!bm_takes_q8k(WT)) hrows.load(h + (size_t)t * spt * n * 256, spt * n * 32, n * 32, sel + t * spt);
     const int si = tid < spt ? tid : 0;
     const u32 my_sel = sel[t * spt + si];
@@ -981,12 +983,12 @@ __global__ __launch_bounds__(256) void k_down_combine_hq(const uint8_t *w, u32 n
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT>(lds);
+    const Iq2Tables tb = stage_tables<WT, T>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
     float *s_w = part + D * spt;                                              // [spt]
     u32 *s_sel = reinterpret_cast<u32 *>(s_w + spt);                          // [spt]
-    if constexpr (bm_takes_q8k(WT)) q8k_stage_cols(h + (size_t)t * spt * n * 256, cols, spt, n, fault, layer, sel + t * spt, n_experts);
+    if constexpr (bm_takes_q8k(WT)) q8k_stage_cols<T>(h + (size_t)t * spt * n * 256, cols, spt, n, fault, layer, sel + t * spt, n_experts);
     else hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, sel + t * spt, n_experts, fault, layer);
     if (tid < spt) {
         s_w[tid] = my_w;
@@ -995,7 +997,7 @@ __global__ __launch_bounds__(256) void k_down_combine_hq(const uint8_t *w, u32 n
     __syncthreads();
     if (act_h && rb == 0) // the live slots' columns; the others keep what they held
         for (int c = 0; c < spt; c++)
-            if (s_sel[c] < n_experts) stage_bytes(act_h + ((size_t)t * spt + c) * col_bytes, cols + (size_t)c * col_bytes, col_bytes);
+            if (s_sel[c] < n_experts) stage_bytes<T>(act_h + ((size_t)t * spt + c) * col_bytes, cols + (size_t)c * col_bytes, col_bytes);
     float v[1];
     row_dot<WT, U, NB, 1>(b, wrow, cols + (size_t)e * col_bytes, col_bytes, 1, n, q, tb, v, NoTap{});
     if (q == 0 && dl < D) part[dl * spt + e] = v[0];
@@ -1268,24 +1270,42 @@ hipError_t gate_up_x(const Launch &L, int gate_type, const float *x, const uint8
 }
 
 // Down + combine from the f32 rows of h, for a down stack that takes Q8_K columns; act_h (optional) receives them.
+// Every workgroup quantizes the token's slot rows for itself, some 25 instructions a wave and 256 values beside a row dot's 50 a lane and
+// 256: a larger workgroup shares that between more rows. 256 threads where the token's rows are at most eight blocks (top-2 of 768 values:
+// 4.8 us against 5.5 with 512). Else 512, or 1024, of which a compute unit holds one (92 registers a lane): a round of 256 takes 9.3 us
+// where half a round's work takes 5.1 with 512, so 1024 where the last round is more than half full or there are more than five (us with
+// 256 / 512 / 1024 threads, top-8 of 768 values, IQ4_XS, 2048 rows: 1 token 7.7 / 7.3 / 9.0, 2 tokens 10.2 / 8.1 / 9.6, 3 tokens 12.2 /
+// 11.2 / 10.1, 4 tokens 14.8 / 12.0 / 10.8, 6 tokens 20.2 / 17.0 / 18.3, 7 tokens 22.4 / 20.4 / 18.9, 10 tokens 29.3 / 25.5 / 26.8,
+// 16 tokens 47.6 / 40.1 / 37.0; IQ2_XXS, 1536 values, 5120 rows, one token 19.4 / 17.6 / 16.0).
 hipError_t down_combine_hq(const Launch &L, int wtype, const uint8_t *w, int n_experts, int k, const float *h,
                            uint8_t *act_h, const uint32_t *sel, const float *wts, const float *resid,
                            int slots_per_token, int m, int rows_per_expert, float *y) {
     const int nb = k / 256, rpe = rows_per_expert, spt = slots_per_token;
-    const int D = 64 / spt, spt_shift = (spt & (spt - 1)) == 0 ? __builtin_ctz((unsigned)spt) : -1;
-    const size_t lds = down_combine_lds(wtype, k, spt);
+    const int spt_shift = (spt & (spt - 1)) == 0 ? __builtin_ctz((unsigned)spt) : -1;
+    const bool wide = bm_takes_q8k(wtype) && spt * nb > 8; // (Q8_2_X4 columns are encoded from registers, four tasks a thread of 256)
+    const long of_1024 = (long)m * ((rpe + 256 / spt - 1) / (256 / spt)), rounds = (of_1024 + 255) / 256;
+    const int T = !wide ? 256 : (of_1024 + 127) / 128 == 2 * rounds || rounds > 5 ? 1024 : 512;
+    const int D = T / 4 / spt;
+    const size_t lds = down_combine_lds(wtype, k, spt) + (size_t)(D - 64 / spt) * spt * sizeof(float);
     const unsigned blocks = (unsigned)((rpe + D - 1) / D);
     const bool row_major = plain_order(m * spt, eighths(blocks));
+    auto launch = [&](auto kern) {
+        hipError_t e = allow_lds(kern, lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, row_major ? dim3(blocks, (unsigned)m) : dim3(kDies, (unsigned)m, eighths(blocks)), dim3((unsigned)T), lds,
+                           L.stream, w, (u32)n_experts, nb, h, act_h, sel, wts, resid,
+                           spt | ((spt_shift + 1) << 16) | (row_major ? kDownRowMajor : 0), rpe, y, L.fault, L.layer);
+        return hipGetLastError();
+    };
 #define CALL_BODY                                                                                                      \
-    auto kern = k_down_combine_hq<WT, U, NB>;                                                                          \
-    hipError_t e = allow_lds(kern, lds);                                                                               \
-    if (e != hipSuccess) return e;                                                                                     \
-    hipLaunchKernelGGL(kern, row_major ? dim3(blocks, (unsigned)m) : dim3(kDies, (unsigned)m, eighths(blocks)), dim3(256), lds, L.stream,       \
-                       w, (u32)n_experts, nb, h, act_h, sel, wts, resid,                                               \
-                       spt | ((spt_shift + 1) << 16) | (row_major ? kDownRowMajor : 0), rpe, y, L.fault, L.layer);
+    if constexpr (bm_takes_q8k(WT)) {                                                                                  \
+        if (T == 1024) return launch(k_down_combine_hq<WT, U, NB, 1024>);                                              \
+        if (T == 512) return launch(k_down_combine_hq<WT, U, NB, 512>);                                                \
+    }                                                                                                                  \
+    return launch(k_down_combine_hq<WT, U, NB, 256>)
     BM_DISPATCH(wtype, nb)
 #undef CALL_BODY
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t moe_decode(const Launch &L, int gate_type, int down_type, const float *x, const uint8_t *wg, const uint8_t *wu,

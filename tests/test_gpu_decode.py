@@ -545,6 +545,37 @@ def test_fused_step_in_either_order(gpu, types, hidden, ff, m, top_k):
     L.free()
 
 
+# The down half's workgroups on Q8_K columns: 256 threads where a token's rows are at most eight blocks, else 512, or 1024 where the last
+# round of 256 of those is more than half full or there are more than five rounds; rows that are no multiple of a workgroup's.
+@pytest.mark.parametrize("types,hidden,ff,m,top_k", (
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 4, 4),  # 256
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 3, 5),  # 512
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 7, 5),  # 1024
+    ((bm.Q4_K, bm.Q4_K, bm.IQ2_XXS), 512, 768, 18, 3),       # 512
+    ((bm.Q4_K, bm.Q4_K, bm.IQ2_XXS), 512, 768, 19, 3),       # 1024
+    ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 256, 2304, 257, 1),        # 512: two rounds
+    ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 256, 2304, 385, 1),        # 1024
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ3_XXS), 256, 256, 2, 64), # 512: two rows a workgroup
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ3_XXS), 256, 256, 3, 64), # 1024
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ3_XXS), 256, 256, 21, 64), # 1024: more than five rounds, the last one not half full
+))
+def test_fused_step_with_larger_down_workgroups(gpu, types, hidden, ff, m, top_k):
+    n_experts = max(8, top_k)
+    L = Layer(gpu, types, hidden, ff, n_experts, 660 + hidden + ff)
+    rng = np.random.default_rng(661)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    gpu.fault_clear()
+    y, h, act_h, _ = run_fused_step(gpu, L, x, ids, wts, top_k, resid)
+    want_y, want_h = L.oracle(x, ids, wts, top_k)
+    assert_f32(h, want_h, "h")
+    for s in range(m * top_k):
+        assert np.array_equal(act_h[s], ora.quantize_col(types[2], want_h[s * ff:(s + 1) * ff])), f"act_h slot {s}"
+    assert_f32(y, (want_y.reshape(m, hidden) + resid).astype(np.float32).reshape(-1), "y + resid")
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    L.free()
+
+
 def test_fused_step_at_the_token_limit(gpu):
     """bm_moe_decode takes 1..=1024 tokens a launch: the limit itself against the oracle, one more refused by name."""
     L = Layer(gpu, (bm.Q4_K, bm.Q4_K, bm.Q6_K), 256, 256, 9, 650)
