@@ -653,7 +653,22 @@ struct Iq2Tables {
     const uint2 *grid;  // IQ2_XXS: a grid point's eight magnitude selectors (0, 1, 2), a byte each
     const uint2 *grid3; // IQ3_XXS: (64 + magnitudes, 64 - magnitudes) of a four-value grid point
     const uint2 *signs; // IQ2_XXS: 4 in the bytes of the negative values; IQ3_XXS: 0xff there
+    u32 at;             // where they lie in LDS: the grid, and 2048 bytes on the signs
 };
+constexpr u32 kIqSignsAt = 2048;
+
+// The eight bytes at an LDS address. The row dots address the tables by bytes, an index turned to bits 3 .. of a word and masked: two
+// vector instructions, one of them a double-rate one, where an index taken out and added to a base eightfold takes two of the other rate
+// (wave instructions a SIMD takes one every 2.4 cycles of: and, or, xor, add, three-operand logic, right shifts, f32 multiplies and
+// multiply-adds, all from vector registers or literals only; every 4.3 cycles: the others, and any with a scalar operand; a
+// select by VCC every 19.5).
+__device__ __forceinline__ uint2 bm_lds_pair(u32 at) {
+    typedef u32 v2u __attribute__((ext_vector_type(2)));
+    const v2u v = *(const __attribute__((address_space(3))) v2u *)(uintptr_t)at;
+    return make_uint2(v.x, v.y);
+}
+// Bits n .. of x to bits 3 .. (n below 32, not a constant; the bits below wrap around).
+__device__ __forceinline__ u32 bm_to_bit3(u32 x, int n) { return __builtin_rotateright32(x, (u32)(n + 29)); }
 
 // The eight code bytes 43 +- magnitude of an IQ2_XXS group (what the CPU path dots, crates/qdot/src/lib.rs:8677-8724): two
 // 8-byte table reads, a grid point's magnitude selectors and a sign index's bytes of 4, whose sum is a byte selector into the
@@ -661,10 +676,12 @@ struct Iq2Tables {
 // way, crates/gpu/src/iq.rs:473-512). A third less LDS traffic than ready-made code bytes of both signs and half the banks
 // an entry, for two more vector instructions a group.
 constexpr u32 kIq2Plus = 0x00564433u, kIq2Minus = 0x00001223u;
-__device__ __forceinline__ void bm_iq2_codes(const Iq2Tables &tb, u32 grid_idx, u32 sign_idx, u32 &lo, u32 &hi) {
-    const uint2 g = tb.grid[grid_idx], sg = tb.signs[sign_idx];
+__device__ __forceinline__ void bm_iq2_codes_of(uint2 g, uint2 sg, u32 &lo, u32 &hi) {
     lo = __builtin_amdgcn_perm(kIq2Minus, kIq2Plus, g.x | sg.x);
     hi = __builtin_amdgcn_perm(kIq2Minus, kIq2Plus, g.y | sg.y);
+}
+__device__ __forceinline__ void bm_iq2_codes(const Iq2Tables &tb, u32 grid_idx, u32 sign_idx, u32 &lo, u32 &hi) {
+    bm_iq2_codes_of(tb.grid[grid_idx], tb.signs[sign_idx], lo, hi);
 }
 
 template <>
@@ -703,7 +720,8 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int 
             const int sb = 2 * k + e;
             const u32 idx = e ? idx_b : idx_a, aux = e ? aux_b : aux_a;
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
-            bm_iq2_codes(tb, (idx >> (8 * q)) & 0xffu, (aux >> (7 * q)) & 127u, dec.u_lo[sb], dec.u_hi[sb]);
+            bm_iq2_codes_of(bm_lds_pair(tb.at + (bm_to_bit3(idx, 8 * q) & 0x7f8u)), bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u)),
+                            dec.u_lo[sb], dec.u_hi[sb]);
         }
     }
     return dec;
@@ -783,6 +801,8 @@ struct Act<BM_IQ3XXS> : Act<BM_IQ2XXS> {};
 
 __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int q, const Iq2Tables &tb) {
     Iq2Dec dec;
+    u32 upper = (q & 2) ? 0xffffffffu : 0u;
+    asm("" : "+v"(upper)); // (else the picks by it become selects by VCC)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         // sub-blocks 2k and 2k + 1 sit in lane k of the quad; this lane's two index bytes are bytes 2q, 2q + 1 of a
@@ -793,11 +813,11 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int 
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int sb = 2 * k + e;
-            const u32 word = (q & 2) ? (e ? ib1 : ia1) : (e ? ib0 : ia0), aux = e ? aux_b : aux_a;
-            const u32 pair = word >> (16 * (q & 1));
+            const u32 word = e ? bm_iq_pick(ib0, ib1, upper) : bm_iq_pick(ia0, ia1, upper), aux = e ? aux_b : aux_a;
+            const u32 pair = bm_to_bit3(word, 16 * (q & 1));
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
-            const uint2 g0 = tb.grid3[pair & 0xffu], g1 = tb.grid3[(pair >> 8) & 0xffu];
-            const uint2 sg = tb.signs[(aux >> (7 * q)) & 127u];
+            const uint2 g0 = bm_lds_pair(tb.at + (pair & 0x7f8u)), g1 = bm_lds_pair(tb.at + ((pair >> 8) & 0x7f8u));
+            const uint2 sg = bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
             dec.u_lo[sb] = bm_iq_pick(g0.x, g0.y, sg.x);
             dec.u_hi[sb] = bm_iq_pick(g1.x, g1.y, sg.y);
         }
@@ -867,7 +887,7 @@ __device__ __forceinline__ void bm_dot_q3k(const Blk<BM_Q3K> &b, const Act<BM_Q3
     // 2j + f / 2
     const u32 a0 = (b.tail.x >> 16) | (b.tail.y << 16), a1 = (b.tail.y >> 16) | (b.tail.z << 16);
     const u32 a2 = (b.tail.z >> 16) | (b.tail.w << 16);
-    const u32 lo = j ? (a0 >> 4) : a0, lo1 = j ? (a1 >> 4) : a1, hi = a2 >> (4 * j);
+    const u32 lo = a0 >> (4 * j), lo1 = a1 >> (4 * j), hi = a2 >> (4 * j);
     const u32 w0 = (lo & 0x0f0f0f0fu) | ((hi & 0x03030303u) << 4);
     const u32 w1 = (lo1 & 0x0f0f0f0fu) | (((hi >> 2) & 0x03030303u) << 4);
     const u32 qw[4] = {b.qs.x, b.qs.y, b.qs.z, b.qs.w}, hw[4] = {b.hm.x, b.hm.y, b.hm.z, b.hm.w};

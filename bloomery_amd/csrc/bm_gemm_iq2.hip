@@ -165,8 +165,8 @@ __device__ __forceinline__ void iq2_tile(uint8_t *lds, const uint8_t *we, const 
     auto grid_of = [&](u32 index, int j, v2u(&half)[2]) __attribute__((always_inline)) {
         const u32 at = __builtin_amdgcn_perm(index, my_copy, 0x0c0c0000u | ((4u + (u32)j) << 8));
         // (the grid is where LDS starts: with the array's own address, a zero that only the linker fills in, each lookup would add it)
-        half[0] = *(LdsV2)at;
-        half[1] = *(LdsV2)(at + 128u);
+        half[0] = *(LdsV2)(uintptr_t)at;
+        half[1] = *(LdsV2)(uintptr_t)(at + 128u);
     };
     auto scale_of = [&](u32 aux) __attribute__((always_inline)) { // 1024 + 2 s + 1 less 1024
         const u32 x = (2u * (aux >> 28)) | 0x6401u, b = x | (x << 16);

@@ -52,7 +52,7 @@ __device__ __forceinline__ uint2 iq_sign_masks(int t) {
 // front of whatever comes next)
 template <int WT>
 __device__ __forceinline__ Iq2Tables stage_tables_by(uint8_t *lds, int T) {
-    Iq2Tables tb{nullptr, nullptr, nullptr};
+    Iq2Tables tb{nullptr, nullptr, nullptr, 0};
     if constexpr (WT == BM_IQ2XXS) {
         // a grid point as eight byte selectors over the three magnitudes (8, 25, 43 -> 0, 1, 2), a sign index as eight bytes
         // of 4 where the value is negative: their sum picks a value's code byte 43 +- magnitude out of six (bm_iq2_codes)
@@ -85,9 +85,13 @@ __device__ __forceinline__ Iq2Tables stage_tables_by(uint8_t *lds, int T) {
     return tb;
 }
 
-template <int WT, int T = 256>
+// LDS of a kernel that has no array of fixed size starts at address 0, which then drops out of the lookups' addresses (`at` stays 0).
+// AFTER_FIXED: the kernel has some.
+template <int WT, int T = 256, bool AFTER_FIXED = false>
 __device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds) {
-    return stage_tables_by<WT>(lds, T);
+    Iq2Tables tb = stage_tables_by<WT>(lds, T);
+    if constexpr (AFTER_FIXED) tb.at = (u32)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    return tb;
 }
 
 // `bytes` (a multiple of 8) from 8-byte aligned global memory to 8-byte aligned LDS, by the whole workgroup of T threads.
