@@ -638,6 +638,12 @@ __device__ __forceinline__ Blk<BM_IQ2XXS> bm_load_iq2xxs(const uint8_t *wrow, in
 // IQ3_XXS: a grid point of four magnitudes is kept as its four bytes 64 + mag and its four bytes 64 - mag, a sign index as
 // eight byte masks (0xff where the value is negative), and u is a bitwise pick between the two by the mask (one operation a
 // word).
+// (x & mask) | bits, the mask in a vector register (with a scalar one it takes twice the time).
+__device__ __forceinline__ u32 bm_and_or(u32 x, u32 mask, u32 bits) {
+    u32 r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xea" : "=v"(r) : "v"(x), "v"(mask), "v"(bits));
+    return r;
+}
 __device__ __forceinline__ u32 bm_iq_pick(u32 plus, u32 minus, u32 mask) { return (minus & mask) | (plus & ~mask); }
 
 // a * b + c over 24-bit factors as one multiply-add: the empty statement pins the running sum, so the compiler cannot
@@ -892,15 +898,18 @@ __device__ __forceinline__ void bm_dot_q3k(const Blk<BM_Q3K> &b, const Act<BM_Q3
     const u32 w1 = (lo1 & 0x0f0f0f0fu) | (((hi >> 2) & 0x03030303u) << 4);
     const u32 qw[4] = {b.qs.x, b.qs.y, b.qs.z, b.qs.w}, hw[4] = {b.hm.x, b.hm.y, b.hm.z, b.hm.w};
     int sum = 0;
+    u32 h2[4], four = 0x04040404u; // the high bits of field f at bit 2 + f of their bytes
+    asm("" : "+v"(four));
+#pragma unroll
+    for (int t = 0; t < 4; t++) h2[t] = __builtin_rotateright32(hw[t], (u32)(4 * j + 30));
 #pragma unroll
     for (int f = 0; f < 4; f++) {
         int g = 0;
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             const u32 low = (qw[t] >> (2 * f)) & 0x03030303u;
-            const u32 high = (hw[t] >> (4 * j + f)) & 0x01010101u;
             // u = low | high << 2 picks its level: bytes -4, -3, -2, -1 then 0, 1, 2, 3
-            const u32 v = __builtin_amdgcn_perm(0x03020100u, 0xfffefdfcu, (high << 2) | low);
+            const u32 v = __builtin_amdgcn_perm(0x03020100u, 0xfffefdfcu, bm_and_or(h2[t] >> f, four, low));
             const uint2 a = act.a[2 * f + (t >> 1)];
             g = bm_sdot4(v, (t & 1) ? a.y : a.x, g);
         }
