@@ -352,26 +352,45 @@ __device__ __forceinline__ Blk<BM_Q5K> bm_load_q5k(const uint8_t *wrow, int i, i
     return b;
 }
 
+// What the row dots' integer parts are made of, in cycles a SIMD spends on a wave's instruction, two waves or more on it: 2.4 for and, or,
+// xor, add, logic of three operands, right shifts, f32 multiplies and multiply-adds, all from vector registers or literals only;
+// 4.3 for the others (left shifts, byte permutes, field extracts, dots, conversions, packed f16, lane exchanges), and for any with a
+// scalar operand; 19 for a select by VCC.
+// (x & mask) | bits, the mask in a vector register.
+__device__ __forceinline__ u32 bm_and_or(u32 x, u32 mask, u32 bits) {
+    u32 r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xea" : "=v"(r) : "v"(x), "v"(mask), "v"(bits));
+    return r;
+}
+__device__ __forceinline__ u32 bm_vector_const(u32 c) {
+    asm("" : "+v"(c));
+    return c;
+}
+
 struct FifthBit {
     uint4 qh;
-    // `s`: the sub-block of q's low nibbles; its high nibbles are sub-block s + 1
+    int c;
+    // `s`: the sub-block of q's low nibbles, 2c or 2c + 4; its high nibbles are sub-block s + 1
     __device__ __forceinline__ void dot16(uint4 q, int s, uint4 alo, uint4 ahi, int &lo, int &hi) const {
-        const u32 m = 0x0f0f0f0fu, one = 0x01010101u;
-        lo = bm_sdot4((q.x & m) | (((qh.x >> s) & one) << 4), alo.x, 0);
-        lo = bm_sdot4((q.y & m) | (((qh.y >> s) & one) << 4), alo.y, lo);
-        lo = bm_sdot4((q.z & m) | (((qh.z >> s) & one) << 4), alo.z, lo);
-        lo = bm_sdot4((q.w & m) | (((qh.w >> s) & one) << 4), alo.w, lo);
-        hi = bm_sdot4(((q.x >> 4) & m) | (((qh.x >> (s + 1)) & one) << 4), ahi.x, 0);
-        hi = bm_sdot4(((q.y >> 4) & m) | (((qh.y >> (s + 1)) & one) << 4), ahi.y, hi);
-        hi = bm_sdot4(((q.z >> 4) & m) | (((qh.z >> (s + 1)) & one) << 4), ahi.z, hi);
-        hi = bm_sdot4(((q.w >> 4) & m) | (((qh.w >> (s + 1)) & one) << 4), ahi.w, hi);
+        const u32 m = 0x0f0f0f0fu, fifth = bm_vector_const(0x10101010u);
+        // bit s of a byte to its bit 4: (2c is 0 or 2) up by 4 - 2c, or down by 2c
+        auto turned = [&](u32 w) { return s - 2 * c == 0 ? __builtin_rotateright32(w, (u32)(2 * c + 28)) : w >> (2 * c); };
+        const u32 x = turned(qh.x), y = turned(qh.y), z = turned(qh.z), w = turned(qh.w);
+        lo = bm_sdot4(bm_and_or(x, fifth, q.x & m), alo.x, 0);
+        lo = bm_sdot4(bm_and_or(y, fifth, q.y & m), alo.y, lo);
+        lo = bm_sdot4(bm_and_or(z, fifth, q.z & m), alo.z, lo);
+        lo = bm_sdot4(bm_and_or(w, fifth, q.w & m), alo.w, lo);
+        hi = bm_sdot4(bm_and_or(x >> 1, fifth, (q.x >> 4) & m), ahi.x, 0);
+        hi = bm_sdot4(bm_and_or(y >> 1, fifth, (q.y >> 4) & m), ahi.y, hi);
+        hi = bm_sdot4(bm_and_or(z >> 1, fifth, (q.z >> 4) & m), ahi.z, hi);
+        hi = bm_sdot4(bm_and_or(w >> 1, fifth, (q.w >> 4) & m), ahi.w, hi);
     }
 };
 
 template <class Tap>
 __device__ __forceinline__ void bm_dot_q5k(const Blk<BM_Q5K> &b, const Act<BM_Q5K> &a, int i, int c, int h,
                                            float &acc0, float &acc1, const Tap &tap) {
-    bm_dot_q45k(b.hdr, b.qa, b.qb, FifthBit{b.qh}, a, i, c, h, acc0, acc1, tap);
+    bm_dot_q45k(b.hdr, b.qa, b.qb, FifthBit{b.qh, c}, a, i, c, h, acc0, acc1, tap);
 }
 
 // A Q4_K / Q5_K super-block's weight side, formed once and dotted against several columns: the code words as the dot
@@ -399,7 +418,7 @@ __device__ __forceinline__ Q45Dec bm_decode_q45k(uint4 hdr, uint4 qa, uint4 qb, 
     x.w01 = d * (float)((s0 >> 8) & 0xffu);
     x.w10 = d * (float)(s1 & 0xffu);
     x.w11 = d * (float)((s1 >> 8) & 0xffu);
-    const u32 m = 0x0f0f0f0fu, one = 0x01010101u;
+    const u32 m = 0x0f0f0f0fu, fifth = bm_vector_const(0x10101010u);
     const u32 wa[4] = {qa.x, qa.y, qa.z, qa.w}, wb[4] = {qb.x, qb.y, qb.z, qb.w}, wh[4] = {qh.x, qh.y, qh.z, qh.w};
 #pragma unroll
     for (int t = 0; t < 4; t++) {
@@ -408,10 +427,11 @@ __device__ __forceinline__ Q45Dec bm_decode_q45k(uint4 hdr, uint4 qa, uint4 qb, 
         x.lo1[t] = wb[t] & m;
         x.hi1[t] = (wb[t] >> 4) & m;
         if constexpr (Fifth) { // sub-blocks 2c, 2c + 1 of the first word, 4 + 2c, 5 + 2c of the second
-            x.lo0[t] |= ((wh[t] >> (2 * c)) & one) << 4;
-            x.hi0[t] |= ((wh[t] >> (2 * c + 1)) & one) << 4;
-            x.lo1[t] |= ((wh[t] >> (4 + 2 * c)) & one) << 4;
-            x.hi1[t] |= ((wh[t] >> (5 + 2 * c)) & one) << 4;
+            const u32 up = __builtin_rotateright32(wh[t], (u32)(2 * c + 28)), as = wh[t] >> (2 * c); // bits 2c, 2c + 1 at 4, 5; 2c + 4, 2c + 5 there
+            x.lo0[t] = bm_and_or(up, fifth, x.lo0[t]);
+            x.hi0[t] = bm_and_or(up >> 1, fifth, x.hi0[t]);
+            x.lo1[t] = bm_and_or(as, fifth, x.lo1[t]);
+            x.hi1[t] = bm_and_or(as >> 1, fifth, x.hi1[t]);
         }
     }
     return x;
@@ -638,12 +658,6 @@ __device__ __forceinline__ Blk<BM_IQ2XXS> bm_load_iq2xxs(const uint8_t *wrow, in
 // IQ3_XXS: a grid point of four magnitudes is kept as its four bytes 64 + mag and its four bytes 64 - mag, a sign index as
 // eight byte masks (0xff where the value is negative), and u is a bitwise pick between the two by the mask (one operation a
 // word).
-// (x & mask) | bits, the mask in a vector register (with a scalar one it takes twice the time).
-__device__ __forceinline__ u32 bm_and_or(u32 x, u32 mask, u32 bits) {
-    u32 r;
-    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xea" : "=v"(r) : "v"(x), "v"(mask), "v"(bits));
-    return r;
-}
 __device__ __forceinline__ u32 bm_iq_pick(u32 plus, u32 minus, u32 mask) { return (minus & mask) | (plus & ~mask); }
 
 // a * b + c over 24-bit factors as one multiply-add: the empty statement pins the running sum, so the compiler cannot
@@ -663,11 +677,8 @@ struct Iq2Tables {
 };
 constexpr u32 kIqSignsAt = 2048;
 
-// The eight bytes at an LDS address. The row dots address the tables by bytes, an index turned to bits 3 .. of a word and masked: two
-// vector instructions, one of them a double-rate one, where an index taken out and added to a base eightfold takes two of the other rate
-// (wave instructions a SIMD takes one every 2.4 cycles of: and, or, xor, add, three-operand logic, right shifts, f32 multiplies and
-// multiply-adds, all from vector registers or literals only; every 4.3 cycles: the others, and any with a scalar operand; a
-// select by VCC every 19.5).
+// The eight bytes at an LDS address. The row dots address the tables by bytes: an index turned to bits 3 .. of a word and masked, two
+// vector instructions and one of them a fast one, where an index taken out and added to a base eightfold takes two slow ones.
 __device__ __forceinline__ uint2 bm_lds_pair(u32 at) {
     typedef u32 v2u __attribute__((ext_vector_type(2)));
     const v2u v = *(const __attribute__((address_space(3))) v2u *)(uintptr_t)at;
