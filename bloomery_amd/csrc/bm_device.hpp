@@ -355,7 +355,7 @@ __device__ __forceinline__ Blk<BM_Q5K> bm_load_q5k(const uint8_t *wrow, int i, i
 // What the row dots' integer parts are made of, in cycles a SIMD spends on a wave's instruction, two waves or more on it: 2.4 for and, or,
 // xor, add, logic of three operands, right shifts, f32 multiplies and multiply-adds, all from vector registers or literals only;
 // 4.3 for the others (left shifts, byte permutes, field extracts, dots, conversions, packed f16, lane exchanges), and for any with a
-// scalar operand; 19 for a select by VCC.
+// scalar operand; 19 for a select by a VCC that no vector comparison has just written.
 // (x & mask) | bits, the mask in a vector register.
 __device__ __forceinline__ u32 bm_and_or(u32 x, u32 mask, u32 bits) {
     u32 r;
@@ -819,7 +819,7 @@ struct Act<BM_IQ3XXS> : Act<BM_IQ2XXS> {};
 __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int q, const Iq2Tables &tb) {
     Iq2Dec dec;
     u32 upper = (q & 2) ? 0xffffffffu : 0u;
-    asm("" : "+v"(upper)); // (else the picks by it become selects by VCC)
+    asm("" : "+v"(upper)); // (else the picks by it become selects by a VCC kept over the loop, 19 cycles each)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         // sub-blocks 2k and 2k + 1 sit in lane k of the quad; this lane's two index bytes are bytes 2q, 2q + 1 of a

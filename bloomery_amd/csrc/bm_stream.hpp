@@ -393,28 +393,22 @@ __device__ __forceinline__ float4 bm_ld4f(const float *p) {
 // `o` is the block's 296 bytes (LDS or global memory).
 __device__ __forceinline__ void q8k_wave_block(const float4 x4, uint8_t *o, int lane, u32 *fault, u32 layer) {
     const float v[4] = {x4.x, x4.y, x4.z, x4.w};
-    // the largest magnitude: a maximum of the sign-less bit patterns over the wave
-    u32 mine_ab = 0;
+    // the largest magnitude: a maximum of the sign-less bit patterns over the wave; a lane's own, and the first of its four values that
+    // has it, meanwhile
+    u32 a[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const u32 a = bm_f32_bits(v[k]) & 0x7fffffffu;
-        mine_ab = a > mine_ab ? a : mine_ab;
-    }
+    for (int k = 0; k < 4; k++) a[k] = bm_f32_bits(v[k]) & 0x7fffffffu;
+    const u32 a01 = a[0] > a[1] ? a[0] : a[1], a23 = a[2] > a[3] ? a[2] : a[3], mine_ab = a01 > a23 ? a01 : a23;
+    float mine = v[3];
+    mine = a[2] == mine_ab ? v[2] : mine;
+    mine = a[1] == mine_ab ? v[1] : mine;
+    mine = a[0] == mine_ab ? v[0] : mine;
     const u32 half_ab = bm_max32(mine_ab); // over each half of the wave
     const u32 lo_ab = (u32)__builtin_amdgcn_readlane((int)half_ab, 0), hi_ab = (u32)__builtin_amdgcn_readlane((int)half_ab, 32);
     const u32 ab = lo_ab > hi_ab ? lo_ab : hi_ab;
-    // its first holder (value 4 * lane + k): the lowest lane among those that hold it at k, the lowest such value
-    int first = 1 << 20;
-    float max = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const unsigned long long holders = __ballot((bm_f32_bits(v[k]) & 0x7fffffffu) == ab);
-        if (holders) { // uniform over the wave
-            const int at = __builtin_ctzll(holders);
-            const float val = bm_bits_f32((u32)__builtin_amdgcn_readlane((int)bm_f32_bits(v[k]), at));
-            if (4 * at + k < first) first = 4 * at + k, max = val;
-        }
-    }
+    // its first holder is the lowest lane's that has it
+    const int holder = __builtin_ctzll(__ballot(mine_ab == ab));
+    const float max = bm_bits_f32((u32)__builtin_amdgcn_readlane((int)bm_f32_bits(mine), holder));
     float d;
     int code[4] = {0, 0, 0, 0};
     if (ab > 0x7f7fffffu) {
