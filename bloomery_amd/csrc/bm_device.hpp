@@ -725,6 +725,9 @@ struct Iq2Dec {
     int sc[8];
 };
 
+// BY_BYTES: the lookups by LDS addresses (one column's dot; where a decode serves several columns, and registers are what there is
+// least of, the plain form measures the faster: IQ3_XXS tiles of 64 tokens 116 us against 119).
+template <bool BY_BYTES>
 __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int q, const Iq2Tables &tb) {
     Iq2Dec dec;
 #pragma unroll
@@ -737,8 +740,11 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int 
             const int sb = 2 * k + e;
             const u32 idx = e ? idx_b : idx_a, aux = e ? aux_b : aux_a;
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
-            bm_iq2_codes_of(bm_lds_pair(tb.at + (bm_to_bit3(idx, 8 * q) & 0x7f8u)), bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u)),
-                            dec.u_lo[sb], dec.u_hi[sb]);
+            if constexpr (BY_BYTES)
+                bm_iq2_codes_of(bm_lds_pair(tb.at + (bm_to_bit3(idx, 8 * q) & 0x7f8u)),
+                                bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u)), dec.u_lo[sb], dec.u_hi[sb]);
+            else
+                bm_iq2_codes(tb, (idx >> (8 * q)) & 0xffu, (aux >> (7 * q)) & 127u, dec.u_lo[sb], dec.u_hi[sb]);
         }
     }
     return dec;
@@ -789,7 +795,7 @@ __device__ __forceinline__ void bm_dot_iq2xxs_dec(const Blk<BM_IQ2XXS> &b, const
 template <class Tap>
 __device__ __forceinline__ void bm_dot_iq2xxs(const Blk<BM_IQ2XXS> &b, const Act<BM_IQ2XXS> &act, int i, int q,
                                               const Iq2Tables &tb, float &acc0, float &acc1, const Tap &tap) {
-    const Iq2Dec dec = bm_decode_iq2xxs(b, q, tb);
+    const Iq2Dec dec = bm_decode_iq2xxs<true>(b, q, tb);
     bm_dot_iq2xxs_dec(b, dec, act, i, q, acc0, acc1, tap);
 }
 
@@ -816,10 +822,10 @@ __device__ __forceinline__ Blk<BM_IQ3XXS> bm_load_iq3xxs(const uint8_t *wrow, in
 template <>
 struct Act<BM_IQ3XXS> : Act<BM_IQ2XXS> {};
 
+template <bool BY_BYTES> // as bm_decode_iq2xxs
 __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int q, const Iq2Tables &tb) {
     Iq2Dec dec;
-    u32 upper = (q & 2) ? 0xffffffffu : 0u;
-    asm("" : "+v"(upper)); // (else the picks by it become selects by a VCC kept over the loop, 19 cycles each)
+    [[maybe_unused]] const u32 upper = bm_vector_const((q & 2) ? 0xffffffffu : 0u); // (else the picks by it become selects by a VCC kept over the loop, 19 cycles each)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         // sub-blocks 2k and 2k + 1 sit in lane k of the quad; this lane's two index bytes are bytes 2q, 2q + 1 of a
@@ -830,11 +836,18 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int 
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int sb = 2 * k + e;
-            const u32 word = e ? bm_iq_pick(ib0, ib1, upper) : bm_iq_pick(ia0, ia1, upper), aux = e ? aux_b : aux_a;
-            const u32 pair = bm_to_bit3(word, 16 * (q & 1));
+            const u32 aux = e ? aux_b : aux_a;
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
-            const uint2 g0 = bm_lds_pair(tb.at + (pair & 0x7f8u)), g1 = bm_lds_pair(tb.at + ((pair >> 8) & 0x7f8u));
-            const uint2 sg = bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
+            uint2 g0, g1, sg;
+            if constexpr (BY_BYTES) {
+                const u32 pair = bm_to_bit3(e ? bm_iq_pick(ib0, ib1, upper) : bm_iq_pick(ia0, ia1, upper), 16 * (q & 1));
+                g0 = bm_lds_pair(tb.at + (pair & 0x7f8u)), g1 = bm_lds_pair(tb.at + ((pair >> 8) & 0x7f8u));
+                sg = bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
+            } else {
+                const u32 pair = ((q & 2) ? (e ? ib1 : ia1) : (e ? ib0 : ia0)) >> (16 * (q & 1));
+                g0 = tb.grid3[pair & 0xffu], g1 = tb.grid3[(pair >> 8) & 0xffu];
+                sg = tb.signs[(aux >> (7 * q)) & 127u];
+            }
             dec.u_lo[sb] = bm_iq_pick(g0.x, g0.y, sg.x);
             dec.u_hi[sb] = bm_iq_pick(g1.x, g1.y, sg.y);
         }
@@ -852,7 +865,7 @@ __device__ __forceinline__ void bm_dot_iq3xxs_dec(const Blk<BM_IQ3XXS> &b, const
 template <class Tap>
 __device__ __forceinline__ void bm_dot_iq3xxs(const Blk<BM_IQ3XXS> &b, const Act<BM_IQ3XXS> &act, int i, int q,
                                               const Iq2Tables &tb, float &acc0, float &acc1, const Tap &tap) {
-    const Iq2Dec dec = bm_decode_iq3xxs(b, q, tb);
+    const Iq2Dec dec = bm_decode_iq3xxs<true>(b, q, tb);
     bm_dot_iq3xxs_dec(b, dec, act, i, q, acc0, acc1, tap);
 }
 

@@ -200,10 +200,8 @@ __device__ __forceinline__ void stage_tile_cols(uint8_t *cols, const uint8_t *ac
 // launch of the other width (see tile_widths below). PASSES: it takes every tile, MC columns at a pass over the rows
 // (a wider tile's rows are then read and unpacked again for every pass: the form for batches whose tiles are nearly all
 // narrow, where it saves the second launch; a variant of its own, so that the one-pass kernels stay straight-line code).
-// (IQ3_XXS is held to four waves a SIMD, one register less than it would take for itself: 64 tokens of 128 experts, top 8, 208 us a layer
-// -> 201. The K-quants' forms of several passes would spill.)
 template <int WT, int U, int NB, int MC, bool PASSES>
-__global__ __launch_bounds__(256, WT == BM_IQ3XXS ? 4 : 1) void k_gate_up_tiles(const uint8_t *wg, const uint8_t *wu, u32 n_experts, int nb,
+__global__ __launch_bounds__(256) void k_gate_up_tiles(const uint8_t *wg, const uint8_t *wu, u32 n_experts, int nb,
                                                        const uint8_t *act, int act_cols, const u32 *order,
                                                        const u32 *start, const u32 *tiles, u32 n_slots, u32 cap,
                                                        int rpe, int slots_per_col, float *h, uint8_t *act_h, int m_lo,

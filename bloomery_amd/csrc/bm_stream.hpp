@@ -208,7 +208,7 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
             const int ahead = i + U - 1 < n ? i + U - 1 : n - 1;
             if (NB == 0 || U == 1 || i + U - 1 < NB) b[fill] = bm_load_blk<WT>(wrow, U > 1 ? ahead : i, q);
             if constexpr (WT == BM_IQ2XXS) { // the table lookups once, not once a column
-                const Iq2Dec dec = bm_decode_iq2xxs(b[slot], q, tb);
+                const Iq2Dec dec = bm_decode_iq2xxs<false>(b[slot], q, tb);
 #pragma unroll
                 for (int c = 0; c < M; c++)
                     if (c < m) {
@@ -216,7 +216,7 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
                         bm_dot_iq2xxs_dec(b[slot], dec, a, i, q, a0[c], a1[c], tap);
                     }
             } else if constexpr (WT == BM_IQ3XXS) {
-                const Iq2Dec dec = bm_decode_iq3xxs(b[slot], q, tb);
+                const Iq2Dec dec = bm_decode_iq3xxs<false>(b[slot], q, tb);
 #pragma unroll
                 for (int c = 0; c < M; c++)
                     if (c < m) {
