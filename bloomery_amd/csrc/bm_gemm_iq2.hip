@@ -13,7 +13,7 @@
 // 64 terms (64 x 1333 x 128 < 2^24). The guard is some twenty of 750 vector instructions a super-block: 2 to 5 % of the kernel, 2.3 %
 // of the layer below (2.28 -> 2.33 ms).
 //
-// Bound by the vector ALU, which makes the terms, 17 instructions for eight values a lane, with LDS (the grid, the columns) and the
+// Bound by the vector ALU, which makes the terms, 16 instructions for eight values a lane, with LDS (the grid, the columns) and the
 // weights' scattered lines close behind: an expert has about as many slots as one tile, so every weight is unpacked about once
 // and used for one 32- or 64-slot product. So:
 //   * a wave takes 64 rows and all slots of the tile: no weight is unpacked twice, none goes through LDS, a column operand serves two
@@ -34,9 +34,10 @@
 //     is then half as much of the whole.
 // 133 KB of LDS, one workgroup of eight waves a CU. 8192 slots of 256 experts, gate and up of 2048 rows of 7168 values:
 // 2 x 1266 -> 1232 us; down of 7168 rows of 2048: 1266 -> 693 us, against int8 products on split bytes through LDS. The weights alone
-// take 376 and 188 us from memory. Counters of the pair: vector ALU 60 % of the cycles, matrix cores 27 %, LDS 37 % (a third of that
-// bank conflicts), a wave waits 32 % of its time, at the super-block's barrier and for LDS: two waves a SIMD, no unit full. (These times
-// are without the guard above.)
+// take 376 and 188 us from memory. Counters of the pair: vector ALU 62 % of the cycles, matrix cores 29 %, LDS 41 % (a third of that
+// bank conflicts), the address units 58 % (a lane's sixteen bytes lie at odd multiples of two), a wave waits a third of its time, at the
+// super-block's barrier and for LDS: two waves a SIMD, no unit full. Sixteen waves of 32 rows instead, four a SIMD, were 3 to 15 % slower
+// (twice the column reads), a table of spread signs in LDS no faster. (These times are without the guard above.)
 #include "bm_gemm.hpp"
 
 namespace bmk {

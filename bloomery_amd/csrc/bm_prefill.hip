@@ -305,12 +305,14 @@ __device__ __forceinline__ float q45_value(const uint8_t *row, const uint8_t *co
 // what it takes, so a workgroup that has staged one, which no quantizer makes, walks its values of zero again by themselves.
 // Q6_K, without mins, never has an accumulator of -0.)
 // Bound by the vector ALU (the f32 matrix instructions run on it too, 64 cycles each; the f16 ones beside it) as far as two waves a
-// SIMD fill it: gate and up of 16384 slots Q4_K take 837 k cycles, of which vector instructions are 58 % (32 multiply-adds a wave and
-// 32 x 32 x 32 values, about 30 instructions of staging, addresses) and outer products 13 %; a wave waits a quarter of its time. Down in
-// Q6_K: 612 k, 49 % and 9 %, a third. The staging of a half (bytes to f16, the factors) is cut in eight pieces between the groups of the half before
-// it, each behind the group's matrix instruction, and its bytes are asked for a whole half ahead: one barrier a half, no wait in
-// front of it. 80 KB: two workgroups a CU. 16384 slots of 128 experts, 768 rows of 2048 values Q4_K: 293 -> 205 us; 2048 rows of
-// 768 Q6_K: 359 -> 287 us, against int8 products with the scaling, the conversion and the mins on the vector ALU.
+// SIMD fill it: gate and up of 16384 slots Q4_K take 756 k cycles, of which vector instructions are 62 % (32 multiply-adds a wave and
+// 32 x 32 x 32 values, about 30 instructions of staging, addresses) and outer products 14 %; a wave waits a fifth of its time. Down in
+// Q6_K: 514 k, 57 % and 10 %, a quarter. The clock is 2.05 GHz under it, what the card's power leaves: a fifth of the vector
+// instructions less (the columns as f16 brought to LDS directly) took the same time. The staging of a half (bytes to f16, the factors) is cut
+// in eight pieces between the groups of the half before it, each behind the group's matrix instruction, and its codes are asked for seven
+// pieces before their use: one barrier a half. 80 KB: two workgroups a CU. 16384 slots of 128 experts, 768 rows of 2048 values
+// Q4_K and Q6_K down, a layer: 1459 us with int8 products and the scaling, the conversion and the mins on the vector ALU, 725 with the
+// products and scales on the matrix cores, 668 with the waits where they are now and more rows a workgroup.
 template <int WT>
 __global__ __launch_bounds__(256, 2) void k_gemm(const uint8_t *w, int rpe, int nb, const uint8_t *act, const u32 *cols,
                                                  const u32 *tiles, const u32 *n_tiles, u32 n_units, u32 slot_div,
