@@ -367,6 +367,12 @@ __device__ __forceinline__ u32 bm_and_or(u32 x, u32 mask, u32 bits) {
     asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xea" : "=v"(r) : "v"(x), "v"(mask), "v"(bits));
     return r;
 }
+// b where the mask has ones, else a. (From the plain expression the compiler makes a field insert, one of the slower ones.)
+__device__ __forceinline__ u32 bm_pick(u32 a, u32 b, u32 mask) {
+    u32 r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xd8" : "=v"(r) : "v"(a), "v"(b), "v"(mask));
+    return r;
+}
 __device__ __forceinline__ u32 bm_vector_const(u32 c) {
     asm("" : "+v"(c));
     return c;
@@ -845,7 +851,7 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int 
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
             uint2 g0, g1, sg;
             if constexpr (BY_BYTES) {
-                const u32 pair = bm_to_bit3(e ? bm_iq_pick(ib0, ib1, upper) : bm_iq_pick(ia0, ia1, upper), 16 * (q & 1));
+                const u32 pair = bm_to_bit3(e ? bm_pick(ib0, ib1, upper) : bm_pick(ia0, ia1, upper), 16 * (q & 1));
                 g0 = bm_lds_pair(tb.at + (pair & 0x7f8u)), g1 = bm_lds_pair(tb.at + ((pair >> 8) & 0x7f8u));
                 sg = bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
             } else {
@@ -1044,15 +1050,27 @@ __device__ __forceinline__ void bm_dot_iq4xs_dec(const Blk<BM_IQ4XS> &b, const I
         }
         tap.iq4_sub(i, 2 * q + e, sub);
     }
-    // the quad's four shares of each lane sum
+    // The quad's four shares of each lane sum: lane q ends with sums 2q and 2q + 1. In two steps a lane hands over the half of what it has that
+    // is not its own, twelve picks and six exchanges; the sum of all eight in every lane is sixteen exchanges and the picks behind them.
+    int s0, s1;
+    if constexpr (Tap::kActive) {
 #pragma unroll
-    for (int l = 0; l < 8; l++) {
-        lanes[l] += (int)bm_dpp<kDppXor1>((u32)lanes[l]);
-        lanes[l] += (int)bm_dpp<kDppXor2>((u32)lanes[l]);
-        if (q == 0) tap.iq4_lane(i, l, lanes[l]);
+        for (int l = 0; l < 8; l++) {
+            lanes[l] += (int)bm_dpp<kDppXor1>((u32)lanes[l]);
+            lanes[l] += (int)bm_dpp<kDppXor2>((u32)lanes[l]);
+            if (q == 0) tap.iq4_lane(i, l, lanes[l]);
+        }
+        s0 = q == 0 ? lanes[0] : (q == 1 ? lanes[2] : (q == 2 ? lanes[4] : lanes[6]));
+        s1 = q == 0 ? lanes[1] : (q == 1 ? lanes[3] : (q == 2 ? lanes[5] : lanes[7]));
+    } else {
+        const u32 upper = bm_vector_const((q & 2) ? 0xffffffffu : 0u), odd = bm_vector_const((q & 1) ? 0xffffffffu : 0u);
+        u32 half[4];
+#pragma unroll
+        for (int l = 0; l < 4; l++)
+            half[l] = bm_pick((u32)lanes[l], (u32)lanes[4 + l], upper) + bm_dpp<kDppXor2>(bm_pick((u32)lanes[4 + l], (u32)lanes[l], upper));
+        s0 = (int)(bm_pick(half[0], half[2], odd) + bm_dpp<kDppXor1>(bm_pick(half[2], half[0], odd)));
+        s1 = (int)(bm_pick(half[1], half[3], odd) + bm_dpp<kDppXor1>(bm_pick(half[3], half[1], odd)));
     }
-    const int s0 = q == 0 ? lanes[0] : (q == 1 ? lanes[2] : (q == 2 ? lanes[4] : lanes[6]));
-    const int s1 = q == 0 ? lanes[1] : (q == 1 ? lanes[3] : (q == 2 ? lanes[5] : lanes[7]));
     // one fused multiply-add a super-block and lane (crates/qdot/src/lib.rs:11171-11173)
     const float f = bm_half_to_f32(b.hd.x & 0xffffu) * act.dy;
     acc0 = fmaf(f, (float)s0, acc0);
