@@ -1002,7 +1002,7 @@ __device__ __forceinline__ u32 bm_iq4_levels(u32 x) {
     constexpr u32 t0 = bm_iq4_levels_word(0), t1 = bm_iq4_levels_word(1), t2 = bm_iq4_levels_word(2), t3 = bm_iq4_levels_word(3);
     const u32 s = (x >> SHIFT) & 0x07070707u;
     const u32 lo = __builtin_amdgcn_perm(t1, t0, s), hi = __builtin_amdgcn_perm(t3, t2, s);
-    const u32 pick = ((x >> (SHIFT + 1)) & 0x04040404u) | 0x03020100u;
+    const u32 pick = bm_and_or(x >> (SHIFT + 1), bm_vector_const(0x04040404u), bm_vector_const(0x03020100u));
     return __builtin_amdgcn_perm(hi, lo, pick);
 }
 
