@@ -533,8 +533,9 @@ int bm_gate_up_x(bm_ctx *ctx, const bm_weights *wg, const bm_weights *wu, const 
     int rc = check_stack(ctx, what, wg, ff, &n_experts);
     if (rc) return rc;
     if (ff % 256 != 0) return fail(ctx, BM_ESHAPE, "%s: rows_per_expert = %d is not a whole number of 256-value super-blocks", what, ff);
-    if (n_slots_per_token < 1 || m < 1 || m > bmk::kMaxDecodeTokens)
-        return fail(ctx, BM_ESHAPE, "%s: %d slots a token, m = %d tokens (1..=%d)", what, n_slots_per_token, m, bmk::kMaxDecodeTokens);
+    if (n_slots_per_token < 1 || n_slots_per_token > bmk::kMaxGateSlots || m < 1 || m > bmk::kMaxDecodeTokens)
+        return fail(ctx, BM_ESHAPE, "%s: %d slots a token (1..=%d), m = %d tokens (1..=%d)", what, n_slots_per_token, bmk::kMaxGateSlots, m,
+                    bmk::kMaxDecodeTokens);
     if (act_h && (act_form(act_h->wtype) != 0 || act_h->k != ff || (int64_t)act_h->m_cap < (int64_t)m * n_slots_per_token))
         return fail(ctx, BM_ESHAPE,
                     "%s: act_h must hold %d Q8_2_X4 columns of k = %d (the launch folds that quantizer only; pass NULL and h_dev for a "

@@ -66,6 +66,8 @@ hipError_t down_combine(const Launch &L, int wtype, const uint8_t *w, int n_expe
 // The whole decode step: quantize x, gate . up . SwiGLU, quantize h, down, weighted slot sum, in two launches: gate . up
 // with the quantizers folded in, then down + combine.
 constexpr int kMaxDecodeTokens = 1024;
+// Slots a token may have in gate_up_x: each is eight workgroups of 256 threads along the grid's first dimension, which holds less than 2^32 threads.
+constexpr int kMaxGateSlots = (1 << 21) - 1;
 bool moe_decode_supported(int gate_type, int down_type);
 // gate . up . SwiGLU from f32 token rows, the token quantizer folded in: the first launch of moe_decode. act_h
 // (Q8_2_X4 columns, or NULL when the down stack takes Q8_K ones) is quantized in the same launch; h (f32 rows) is

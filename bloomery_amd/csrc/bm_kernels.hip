@@ -249,7 +249,7 @@ __global__ __launch_bounds__(1024) void k_gemv_cols(const uint8_t *w, long rows,
 // 1792, 16 tokens 84.5 / 82.5; Q6_K 6 tokens 56.7 / 57.4, Q5_K of 3072, top-6, 3 tokens 46.6 / 47.1.)
 constexpr unsigned kDies = 8, kMaxGridZ = 65535;
 static inline unsigned eighths(unsigned blocks) { return (blocks + kDies - 1) / kDies; }
-static inline bool plain_order(int slots, unsigned eights) { return slots < 64 || eights > kMaxGridZ; }
+static inline bool plain_order(int64_t slots, unsigned eights) { return slots < 64 || eights > kMaxGridZ; }
 
 // --------------------------------------------------------------------------------- gate . up . SwiGLU
 
@@ -768,7 +768,7 @@ __global__ __launch_bounds__(256) void k_gate_up_x(const float *x, const uint8_t
     // the grid: (dies x slots of a token, tokens, blocks of 32 rows in eights; a slot has 8 nh blocks): no division stands before the
     // workgroup's first request (and no read of the grid's size, which comes from the dispatch packet in memory: spt is an argument, in
     // a register at the start). Bit 30 of spt: (blocks, slots of a token, tokens) instead
-    const int slots = spt & 0xffff;
+    const int slots = spt & ~kGateRowMajor;
     const bool row_major = (spt & kGateRowMajor) != 0;
     const int t = (int)(row_major ? blockIdx.z : blockIdx.y), e = (int)(row_major ? blockIdx.y : blockIdx.x / kDies);
     const int rb = (int)(row_major ? blockIdx.x : blockIdx.z * kDies + blockIdx.x % kDies);
@@ -861,7 +861,7 @@ __global__ __launch_bounds__(256) void k_gate_up_xq(const float *x, const uint8_
     const int tid = threadIdx.x, q = tid & 3, which = (tid >> 2) & 1;
     // the grid as k_gate_up_x's
     const bool row_major = (spt_word & kGateRowMajor) != 0;
-    const int spt = spt_word & 0xffff;
+    const int spt = spt_word & ~kGateRowMajor;
     const int t = (int)(row_major ? blockIdx.z : blockIdx.y), slot = t * spt + (int)(row_major ? blockIdx.y : blockIdx.x / kDies);
     const int rb = (int)(row_major ? blockIdx.x : blockIdx.z * kDies + blockIdx.x % kDies);
     const int na = NBA > 0 ? NBA : nba;
@@ -1233,7 +1233,7 @@ hipError_t gate_up_x(const Launch &L, int gate_type, const float *x, const uint8
                      uint8_t *act_x, uint8_t *act_h, float *h) {
     const int nba = hidden / 256, nbb = ff / 256, spt = slots_per_token;
     const size_t lds_a = (size_t)act_col_bytes(gate_type, hidden) + 32 * sizeof(float);
-    const bool row_major = plain_order(m * spt, (unsigned)nbb);
+    const bool row_major = plain_order((int64_t)m * spt, (unsigned)nbb);
     const dim3 grid_a = row_major ? dim3((unsigned)(ff / 32), (unsigned)spt, (unsigned)m) : dim3(kDies * (unsigned)spt, (unsigned)m, (unsigned)nbb);
 #define BM_GUX(WA, UA, NA)                                                                                             \
     {                                                                                                                  \

@@ -233,7 +233,7 @@ int bm_moe_decode(bm_ctx *ctx, const bm_weights *wg, const bm_weights *wu, const
 /* The first launch of bm_moe_decode on its own: bm_quantize, bm_gate_up and the quantizer of h in one
  * launch, from the f32 token rows (gate and up of one type; rows_per_expert = ff a multiple of 256). act_h: Q8_2_X4
  * columns for the down stack, or NULL; h_dev: the f32 h rows, or NULL; one of the two at least. Ids as bm_gate_up
- * takes them (BM_HOST_SLOT skipped silently). Follow it with
+ * takes them (BM_HOST_SLOT skipped silently). At most 2^21 - 1 slots a token. Follow it with
  * bm_down_combine or bm_gemv_sel over act_h, or bm_down_combine_h over h_dev. */
 int bm_gate_up_x(bm_ctx *ctx, const bm_weights *wg, const bm_weights *wu, const float *x_dev, const uint32_t *sel_dev,
                  int n_slots_per_token, int m, int rows_per_expert, const bm_gate_act *rule, bm_act *act_h, bm_act *act_x,

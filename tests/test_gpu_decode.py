@@ -545,6 +545,34 @@ def test_fused_step_in_either_order(gpu, types, hidden, ff, m, top_k):
     L.free()
 
 
+@pytest.mark.parametrize("wtype", (bm.Q4_K, bm.IQ4_XS))
+@pytest.mark.parametrize("spt", (65535, 65537))
+def test_gate_up_x_of_many_slots_a_token(gpu, wtype, spt):
+    """A slot count of more than sixteen bits, two tokens: every slot's row of h is its own expert's for its own token; the largest count's
+    successor is refused by name."""
+    m, hidden, ff, n_experts = 2, 256, 256, 3
+    L = Layer(gpu, (wtype, wtype, bm.Q4_K), hidden, ff, n_experts, 670)
+    rng = np.random.default_rng(671)
+    x = normal_f32(rng, (m, hidden))
+    every = np.tile(np.arange(n_experts, dtype=np.uint32), (m, 1))
+    of_expert = L.oracle(x, every, np.ones(every.shape, np.float32), n_experts)[1].reshape(m, n_experts, ff)
+    ids = rng.integers(0, n_experts, size=(m, spt)).astype(np.uint32)
+    xd, sel, act_x = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.act(wtype, hidden, m)
+    h = gpu.buffer(np.float32, m * spt * ff).fill_bytes(0xFF)
+    gpu.fault_clear()
+    gpu.enqueue_gate_up_x(L.dg, L.du, xd, sel, spt, m, ff, None, act_x, h)
+    got = h.download().reshape(m, spt, ff)
+    for t in range(m):
+        assert_f32(got[t], of_expert[t][ids[t]], f"h of token {t}")
+        assert np.array_equal(act_x.download(t), ora.quantize_col(wtype, x[t])), f"act_x token {t}"
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    with pytest.raises(bm.GpuError, match="bm_gate_up_x: 2097152 slots a token"):
+        gpu.enqueue_gate_up_x(L.dg, L.du, xd, sel, 1 << 21, 1, ff, None, act_x, h)
+    for b in (xd, sel, act_x, h):
+        b.free()
+    L.free()
+
+
 # The down half's workgroups on Q8_K columns: 256 threads where a token's rows are at most eight blocks, else 512, or 1024 where the last
 # round of 256 of those is more than half full or there are more than five rounds; rows that are no multiple of a workgroup's.
 @pytest.mark.parametrize("types,hidden,ff,m,top_k", (
