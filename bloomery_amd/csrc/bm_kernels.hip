@@ -248,6 +248,7 @@ __global__ __launch_bounds__(1024) void k_gemv_cols(const uint8_t *w, long rows,
 // dies: top-8 of 128 experts Q4_K / Q6_K 16 tokens 75 / 74.5, 20 tokens 89 / 87.7, Q5_K 21 tokens 100.5 / 98.5, IQ2_XXS of
 // 1792, 16 tokens 84.5 / 82.5; Q6_K 6 tokens 56.7 / 57.4, Q5_K of 3072, top-6, 3 tokens 46.6 / 47.1.)
 constexpr unsigned kDies = 8, kMaxGridZ = 65535;
+constexpr int kMaxGridTokens = 65535; // what the grid's second dimension holds
 static inline unsigned eighths(unsigned blocks) { return (blocks + kDies - 1) / kDies; }
 static inline bool plain_order(int64_t slots, unsigned eights) { return slots < 64 || eights > kMaxGridZ; }
 
@@ -1191,6 +1192,13 @@ hipError_t down_combine(const Launch &L, int wtype, const uint8_t *w, int n_expe
                         const uint32_t *sel, const float *wts, const float *resid, int slots_per_token, int m,
                         int rows_per_expert, float *y) {
     const int nb = k / 256, rpe = rows_per_expert, spt = slots_per_token;
+    if (m > kMaxGridTokens) {
+        const size_t slots = (size_t)kMaxGridTokens * spt, rows = (size_t)kMaxGridTokens * rpe;
+        const hipError_t e = down_combine(L, wtype, w, n_experts, k, act, sel, wts, resid, spt, kMaxGridTokens, rpe, y);
+        if (e != hipSuccess) return e;
+        return down_combine(L, wtype, w, n_experts, k, act + slots * act_col_bytes(wtype, k), sel + slots, wts + slots,
+                            resid ? resid + rows : nullptr, spt, m - kMaxGridTokens, rpe, y + rows);
+    }
     const int D = 64 / spt;
     const int spt_shift = (spt & (spt - 1)) == 0 ? __builtin_ctz((unsigned)spt) : -1;
     const size_t lds = down_combine_lds(wtype, k, spt);
@@ -1281,6 +1289,13 @@ hipError_t down_combine_hq(const Launch &L, int wtype, const uint8_t *w, int n_e
                            uint8_t *act_h, const uint32_t *sel, const float *wts, const float *resid,
                            int slots_per_token, int m, int rows_per_expert, float *y) {
     const int nb = k / 256, rpe = rows_per_expert, spt = slots_per_token;
+    if (m > kMaxGridTokens) {
+        const size_t slots = (size_t)kMaxGridTokens * spt, rows = (size_t)kMaxGridTokens * rpe;
+        const hipError_t e = down_combine_hq(L, wtype, w, n_experts, k, h, act_h, sel, wts, resid, spt, kMaxGridTokens, rpe, y);
+        if (e != hipSuccess) return e;
+        return down_combine_hq(L, wtype, w, n_experts, k, h + slots * k, act_h ? act_h + slots * act_col_bytes(wtype, k) : nullptr, sel + slots,
+                               wts + slots, resid ? resid + rows : nullptr, spt, m - kMaxGridTokens, rpe, y + rows);
+    }
     const int spt_shift = (spt & (spt - 1)) == 0 ? __builtin_ctz((unsigned)spt) : -1;
     const bool wide = bm_takes_q8k(wtype) && spt * nb > 8; // (Q8_2_X4 columns are encoded from registers, four tasks a thread of 256)
     const long of_1024 = (long)m * ((rpe + 256 / spt - 1) / (256 / spt)), rounds = (of_1024 + 255) / 256;

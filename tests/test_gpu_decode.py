@@ -573,6 +573,38 @@ def test_gate_up_x_of_many_slots_a_token(gpu, wtype, spt):
     L.free()
 
 
+@pytest.mark.parametrize("wtype", (bm.Q6_K, bm.IQ4_XS))
+@pytest.mark.parametrize("entry", ("down_combine", "down_combine_h"))
+def test_down_of_more_tokens_than_a_launch_holds(gpu, wtype, entry):
+    """Tokens are the grid's second dimension, 65535 at most: on either side of it, and one launch more, with a residual."""
+    k, rpe, n_experts, kinds = 256, 16, 3, 37
+    m = 65535 + 6
+    rng = np.random.default_rng(680)
+    w = stack(wtype, n_experts * rpe, k, 681)
+    rows = normal_f32(rng, (kinds, k))
+    ids = rng.integers(0, n_experts, size=m).astype(np.uint32)
+    wts, resid = rng.random(m, dtype=np.float32) + np.float32(0.1), normal_f32(rng, (m, rpe))
+    col_of = [ora.quantize_col(wtype, rows[i]) for i in range(kinds)]
+    dots = np.stack([ora.gemv(wtype, w, n_experts * rpe, k, c, 1).reshape(n_experts, rpe) for c in col_of])
+    kind = np.arange(m) % kinds
+    want = (dots[kind, ids] * wts[:, None] + resid).astype(np.float32) # one slot: a product and a sum, each rounded
+    wd, act = gpu.weights(wtype, n_experts * rpe, k, w), gpu.act(wtype, k, m)
+    h, sel, wt, rd = gpu.upload(rows[kind], np.float32), gpu.upload(ids, np.uint32), gpu.upload(wts, np.float32), gpu.upload(resid, np.float32)
+    y = gpu.buffer(np.float32, m * rpe).fill_bytes(0xFF)
+    gpu.fault_clear()
+    if entry == "down_combine":
+        gpu.enqueue_quantize(h, m, act)
+        gpu.enqueue_down_combine(wd, act, sel, wt, rd, 1, m, rpe, y)
+    else:
+        gpu.enqueue_down_combine_h(wd, h, act, sel, wt, rd, 1, m, rpe, y)
+    assert_f32(y.download(), want.reshape(-1), entry)
+    for t in (0, 65534, 65535, m - 1):
+        assert np.array_equal(act.download(t), col_of[t % kinds]), f"column {t}"
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    for b in (wd, act, h, sel, wt, rd, y):
+        b.free()
+
+
 # The down half's workgroups on Q8_K columns: 256 threads where a token's rows are at most eight blocks, else 512, or 1024 where the last
 # round of 256 of those is more than half full or there are more than five rounds; rows that are no multiple of a workgroup's.
 @pytest.mark.parametrize("types,hidden,ff,m,top_k", (
