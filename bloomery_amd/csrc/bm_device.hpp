@@ -448,8 +448,11 @@ __device__ __forceinline__ Q45Dec bm_decode_q45k(uint4 hdr, uint4 qa, uint4 qb, 
     return x;
 }
 
+// (The dots behind a bm_sdot4_first are another instruction, which waits three cycles for its sum. With scales to form meanwhile that is
+// hidden; Q6_K's several columns, which need the sum at once, take a zero beforehand: 16384 rows of 768, 8 columns 7.1 -> 6.5 us.)
+template <bool ZERO_FIRST = false>
 __device__ __forceinline__ int bm_dot16_words(const u32 (&w)[4], uint4 a) {
-    int s = bm_sdot4_first(w[0], a.x);
+    int s = ZERO_FIRST ? bm_sdot4(w[0], a.x, 0) : bm_sdot4_first(w[0], a.x);
     s = bm_sdot4(w[1], a.y, s);
     s = bm_sdot4(w[2], a.z, s);
     return bm_sdot4(w[3], a.w, s);
@@ -639,8 +642,8 @@ __device__ __forceinline__ void bm_dot_q6k_dec(const Q6Dec &x, const Act<BM_Q6K>
                                                float &acc1, const Tap &tap) {
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-        const int s0 = bm_dot16_words(x.wa[j], a.aa[j]) - 32 * a.sa[j];
-        const int s1 = bm_dot16_words(x.wb[j], a.ab[j]) - 32 * a.sb[j];
+        const int s0 = bm_dot16_words<true>(x.wa[j], a.aa[j]) - 32 * a.sa[j];
+        const int s1 = bm_dot16_words<true>(x.wb[j], a.ab[j]) - 32 * a.sb[j];
         acc0 = fmaf(x.fa[j] * a.d8a[j], (float)s0, acc0);
         acc1 = fmaf(x.fb[j] * a.d8b[j], (float)s1, acc1);
         tap.q6k(i, 8 * j + 2 * c + h, s0);
