@@ -251,6 +251,14 @@ def test_gemv_deals_columns_to_waves(gpu, wtype, rows, k):
         b.free()
 
 
+# 513 to 1024 row groups, where a row's length, its type and the column count choose between the two forms: each column count on short
+# rows, rows of an odd number of super-blocks and longer ones, below and above 768 groups, and one group past the last.
+@pytest.mark.parametrize("wtype,rows,k", ((bm.Q6_K, 8200, 512), (bm.Q6_K, 12300, 2048), (bm.IQ3_XXS, 8200, 768), (bm.IQ3_XXS, 12290, 1280),
+                                          (bm.Q4_K, 12290, 768), (bm.IQ4_XS, 8210, 2304), (bm.Q5_K, 12289, 2048), (bm.Q3_K, 16385, 768)))
+def test_gemv_of_several_columns_where_the_forms_meet(gpu, wtype, rows, k):
+    test_gemv_deals_columns_to_waves(gpu, wtype, rows, k)
+
+
 @pytest.mark.parametrize("wtype,rows,k", ((bm.Q4_K, 768, 2048), (bm.Q6_K, 2048, 768), (bm.Q5_K, 67, 1280), (bm.Q4_K, 70, 4352),
                                           (bm.IQ2_XXS, 33, 7168), (bm.IQ4_XS, 66, 768), (bm.IQ3_XXS, 40, 1280),
                                           (bm.Q3_K, 150, 2048)))
