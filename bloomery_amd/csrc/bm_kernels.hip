@@ -1075,12 +1075,12 @@ int gemv_max_cols(int wtype, int k) {
 // past three). Past 1024 groups k_gemv wins everywhere. us, k_gemv / columns dealt: 16384 rows, 8 columns, Q6_K k 512 5.7 / 7.6, k 768 7.0 / 9.3, k 2304
 // 20.1 / 17.1, IQ3_XXS k 2048 16.9 / 18.1, Q4_K k 2048 13.6 / 11.2; 12288 rows, 8 columns, Q6_K k 512 5.7 / 6.5, k 2048 14.4 / 13.2; 16384
 // rows, 5 columns, Q5_K k 512 4.7 / 5.2, k 2048 11.5 / 10.7. Of 6174 calls from 600 to 16384 rows (seven types, 256 to 4352 values, 2
-// to 8 columns) k_gemv is more than 2 % ahead of the form chosen in 23, by 4.5 % at most.
+// to 8 columns) k_gemv is more than 2 % ahead of the form chosen in 21, by 4.5 % at most.
 static int gemv_cols_from(int wtype, int m, bool far, bool ringless) {
     constexpr int kNever = 1 << 30;
     const bool q8k = bm_takes_q8k(wtype), odd = m % 2 != 0;
     if (m == 2) return 1;
-    if (ringless) return odd && (far ? wtype != BM_Q4K && wtype != BM_Q5K : m == 3 && q8k) ? 9 : 1;
+    if (ringless) return odd && (m == 3 ? q8k : far && wtype != BM_Q3K && wtype != BM_Q4K && wtype != BM_Q5K) ? 9 : 1;
     if (m == 3) {
         if (q8k) return kNever;
         far = true;
@@ -1116,12 +1116,12 @@ hipError_t gemv(const Launch &L, int wtype, const uint8_t *w, int64_t rows, int 
     // 7.5 / 5.5 / 6.4, 4 columns 9.4 / 8.6 / 6.9, 8 columns 13.5 / 15 / 9.5; Q4_K 768 x 2048, 4 columns 7.3 / 3.9 / 5.6; Q5_K
     // 2048 x 7168, 8 columns 36 / 19 / 20. (Q6_K goes over to two a little sooner: 3000 rows of 512, 7 columns
     // 5.2 / 4.6 / 3.8. Rows of an odd number of super-blocks, where two columns a wave have no ring: two columns go one a wave all the way, IQ3_XXS
-    // 12288 x 2304 10.8 / 10.2 / 12.2. Else two a wave past 512 groups.)
+    // 12288 x 2304 10.8 / 10.2 / 12.2. Else two a wave past 512 groups, but for three super-blocks.)
     const int64_t groups = (rows + 15) / 16;
     const bool ringless = nb % 2 != 0 && nb > 3;
     if (groups <= 512 || (groups <= 1024 && nb >= gemv_cols_from(wtype, m, groups > 768, ringless))) {
         const bool one = ringless ? m == 2 || groups * m <= 1280
-                                  : groups <= 512 && (wtype == BM_Q6K ? groups * (m + m % 2) <= 1100 : groups * m <= 1280);
+                         : wtype == BM_Q6K ? groups * (m + m % 2) <= 1024 : groups * m <= 1280 && (groups <= 512 || nb == 3);
         const int per = one ? 1 : 2, cgs = (m + per - 1) / per;
         const int rgs = (int)std::max<int64_t>(1, std::min<int64_t>((groups + kCardUnits - 1) / kCardUnits, 16 / cgs));
         const int T = 64 * rgs * cgs;
