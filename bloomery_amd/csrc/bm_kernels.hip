@@ -195,9 +195,10 @@ __global__ __launch_bounds__(T) void k_gemv(const uint8_t *w, long rows, int nb,
 // columns. What bounds it is a wave's own instruction stream (some 150 instructions a super-block and column, five to six cycles each
 // while a SIMD has one wave), so the columns go side by side instead of one after the other; a workgroup's waves, `rgs` row
 // groups of `cgs` column groups each, share the staged columns and, through the vector cache, the rows' lines. inv: 256 / cgs rounded
-// up, T: the workgroup's threads. (Where a column group is not whole, its last columns are skipped.)
+// up, T: the workgroup's threads, at most 512 of one column a wave (with a bound of 1024 Q5_K spilled three registers:
+// 2000 rows of 2048, 4 columns 4.8 us, 4.5 without). (Where a column group is not whole, its last columns are skipped.)
 template <int WT, int U, int NB, int C>
-__global__ __launch_bounds__(1024) void k_gemv_cols(const uint8_t *w, long rows, int nb, const uint8_t *act, int m_total, int col0, int m,
+__global__ __launch_bounds__(C == 1 ? 512 : 1024) void k_gemv_cols(const uint8_t *w, long rows, int nb, const uint8_t *act, int m_total, int col0, int m,
                                                     float *y, int cgs, int rgs, int inv, int T) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, q = tid & 3, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1123,7 +1124,7 @@ hipError_t gemv(const Launch &L, int wtype, const uint8_t *w, int64_t rows, int 
         const bool one = ringless ? m == 2 || groups * m <= 1280
                          : wtype == BM_Q6K ? groups * (m + m % 2) <= 1024 : groups * m <= 1280 && (groups <= 512 || nb == 3);
         const int per = one ? 1 : 2, cgs = (m + per - 1) / per;
-        const int rgs = (int)std::max<int64_t>(1, std::min<int64_t>((groups + kCardUnits - 1) / kCardUnits, 16 / cgs));
+        const int rgs = (int)std::max<int64_t>(1, std::min<int64_t>((groups + kCardUnits - 1) / kCardUnits, (one ? 8 : 16) / cgs));
         const int T = 64 * rgs * cgs;
 #define BM_COLS_LAUNCH(C)                                                                                              \
     auto kern = k_gemv_cols<WT, U, NB, C>;                                                                             \
