@@ -245,13 +245,21 @@ __global__ __launch_bounds__(C == 1 ? 512 : 1024) void k_gemv_cols(const uint8_t
 // launches give row block b of every slot (or token) to die b % 8 and, on a die, go through all the slots before the next block: the rows of
 // an expert that two slots have are read from memory by the one and found in the L2 by the other, at about the same time. Such a grid's
 // first dimension is eight, or eight times something, and its last counts the blocks in eights. With few slots (or more blocks than a
-// last dimension holds) the plain order: a slot's blocks one after the other, which are neighbours in memory. (us a layer, plain / by
+// last dimension holds) the plain order: a slot's blocks one after the other, which are neighbours in memory. So too where the last eight
+// blocks are not whole: a token's workgroups without a block leave their dies idle, and even with the dies changing places from token to token
+// some compute units get a workgroup more than the others, so that they may be two in a hundred, or eight of a launch that fills the card
+// more than once (1024 workgroups of 256 threads; random down launches of 64 slots or more, by dies over plain: none empty 0.98, below two in a
+// hundred 0.97, up to eight 0.985, but of the smaller launches one in ten then takes 1.08 to 1.2 times as long, beyond thirty 1.07; IQ4_XS of
+// 304 rows, 1536 values, top-3, 34 tokens 12.0 / 22.2 us). (us a layer, plain / by
 // dies: top-8 of 128 experts Q4_K / Q6_K 16 tokens 75 / 74.5, 20 tokens 89 / 87.7, Q5_K 21 tokens 100.5 / 98.5, IQ2_XXS of
 // 1792, 16 tokens 84.5 / 82.5; Q6_K 6 tokens 56.7 / 57.4, Q5_K of 3072, top-6, 3 tokens 46.6 / 47.1.)
 constexpr unsigned kDies = 8, kMaxGridZ = 65535;
 constexpr int kMaxGridTokens = 65535; // what the grid's second dimension holds
 static inline unsigned eighths(unsigned blocks) { return (blocks + kDies - 1) / kDies; }
-static inline bool plain_order(int64_t slots, unsigned eights) { return slots < 64 || eights > kMaxGridZ; }
+static inline bool plain_order(int64_t slots, int tokens, unsigned blocks, int threads = 256) {
+    const unsigned none = kDies * eighths(blocks) - blocks;
+    return slots < 64 || eighths(blocks) > kMaxGridZ || (int64_t)none * ((int64_t)blocks * tokens * threads >= 1024 * 256 ? 12 : 50) > blocks;
+}
 
 // --------------------------------------------------------------------------------- gate . up . SwiGLU
 
@@ -1233,7 +1241,7 @@ hipError_t down_combine(const Launch &L, int wtype, const uint8_t *w, int n_expe
     const int spt_shift = (spt & (spt - 1)) == 0 ? __builtin_ctz((unsigned)spt) : -1;
     const size_t lds = down_combine_lds(wtype, k, spt);
     const unsigned blocks = (unsigned)((rpe + D - 1) / D), grid = (unsigned)m * blocks;
-    const bool row_major = plain_order(m * spt, eighths(blocks));
+    const bool row_major = plain_order((int64_t)m * spt, m, blocks);
     if (L.down_form == 1 && wtype == BM_Q6K && nb == 3 && 64 % spt == 0) { // BM_DOWN_SPLIT where it is built: the super-blocks of a row dealt to the waves
         constexpr int NB = 3;
         const size_t lds_split = (size_t)spt * bm_act_col_bytes<BM_Q6K>(NB) + (64 * (NB - 1) * 32 + D * spt + 2 * spt) * sizeof(float);
@@ -1271,7 +1279,7 @@ hipError_t gate_up_x(const Launch &L, int gate_type, const float *x, const uint8
                      uint8_t *act_x, uint8_t *act_h, float *h) {
     const int nba = hidden / 256, nbb = ff / 256, spt = slots_per_token;
     const size_t lds_a = (size_t)act_col_bytes(gate_type, hidden) + 32 * sizeof(float);
-    const bool row_major = plain_order((int64_t)m * spt, (unsigned)nbb);
+    const bool row_major = plain_order((int64_t)m * spt, m, kDies * (unsigned)nbb);
     const dim3 grid_a = row_major ? dim3((unsigned)(ff / 32), (unsigned)spt, (unsigned)m) : dim3(kDies * (unsigned)spt, (unsigned)m, (unsigned)nbb);
 #define BM_GUX(WA, UA, NA)                                                                                             \
     {                                                                                                                  \
@@ -1307,14 +1315,30 @@ hipError_t gate_up_x(const Launch &L, int gate_type, const float *x, const uint8
     return hipGetLastError();
 }
 
+// How many threads a workgroup of down + combine takes where it quantizes the token's slot rows of h itself: `blocks` blocks of 256 values,
+// some 25 instructions a wave and block beside a row dot's 50 a lane and super-block; a larger workgroup shares that between more rows.
+// 256 threads where the blocks are at most eight, or at most twenty and the launch is a single small round. Else 512, or 1024, of which a
+// compute unit holds one (84 to 102 registers a lane): a round of 256 takes 9.3 us where half a round's work takes 5.1 with 512, so 1024 where
+// its last round is more than half full or there are more than five. 256 again, which end most evenly, where that is not so, the blocks are at
+// most 24 and what 512 have behind a round or two of 512 is less than a quarter of one. (us with 256 / 512 / 1024 threads, top-8 of 768
+// values, IQ4_XS, 2048 rows: 1 token 7.7 / 7.3 / 9.0, 2 tokens 10.2 / 8.1 / 9.6, 3 tokens 12.2 / 11.2 / 10.1, 4 tokens 14.8 / 12.0 / 10.8, 6
+// tokens 20.2 / 17.0 / 18.3, 7 tokens 22.4 / 20.4 / 18.9, 10 tokens 29.3 / 25.5 / 26.8, 16 tokens 47.6 / 40.1 / 37.0; IQ2_XXS, 1536
+// values, 5120 rows, one token 19.4 / 17.6 / 16.0, top-2, 880 rows, 7 tokens 9.1 / 9.9 / 13.3, top-7 of 512, 1824 rows, 11 tokens 18.8 /
+// 20.7 / 20.9. Of 3800 random calls of the four types, 2 to 8 super-blocks a row, 256 to 7200 rows, top-1 to 12, 1 to 40 tokens, the rule is
+// 1.4 % behind the best of the three, 256 threads for all 11 %.)
+static int down_threads(int spt, int m, int rpe, int blocks) {
+    auto units = [&](int T) {
+        const int D = T / 4 / spt;
+        return (int64_t)m * ((rpe + D - 1) / D);
+    };
+    constexpr int64_t kCard = kCardUnits;
+    if (blocks <= 8 || (blocks <= 20 && units(256) <= kCard)) return 256;
+    const int64_t of_1024 = units(1024), rounds = (of_1024 + kCard - 1) / kCard, of_512 = units(512), last = of_512 % (2 * kCard);
+    if ((of_1024 + kCard / 2 - 1) / (kCard / 2) == 2 * rounds || rounds > 5) return 1024;
+    return blocks <= 24 && of_512 > 2 * kCard && of_512 < 6 * kCard && last > 0 && last < kCard / 2 ? 256 : 512;
+}
+
 // Down + combine from the f32 rows of h, for a down stack that takes Q8_K columns; act_h (optional) receives them.
-// Every workgroup quantizes the token's slot rows for itself, some 25 instructions a wave and 256 values beside a row dot's 50 a lane and
-// 256: a larger workgroup shares that between more rows. 256 threads where the token's rows are at most eight blocks (top-2 of 768 values:
-// 4.8 us against 5.5 with 512). Else 512, or 1024, of which a compute unit holds one (92 registers a lane): a round of 256 takes 9.3 us
-// where half a round's work takes 5.1 with 512, so 1024 where the last round is more than half full or there are more than five (us with
-// 256 / 512 / 1024 threads, top-8 of 768 values, IQ4_XS, 2048 rows: 1 token 7.7 / 7.3 / 9.0, 2 tokens 10.2 / 8.1 / 9.6, 3 tokens 12.2 /
-// 11.2 / 10.1, 4 tokens 14.8 / 12.0 / 10.8, 6 tokens 20.2 / 17.0 / 18.3, 7 tokens 22.4 / 20.4 / 18.9, 10 tokens 29.3 / 25.5 / 26.8,
-// 16 tokens 47.6 / 40.1 / 37.0; IQ2_XXS, 1536 values, 5120 rows, one token 19.4 / 17.6 / 16.0).
 hipError_t down_combine_hq(const Launch &L, int wtype, const uint8_t *w, int n_experts, int k, const float *h,
                            uint8_t *act_h, const uint32_t *sel, const float *wts, const float *resid,
                            int slots_per_token, int m, int rows_per_expert, float *y) {
@@ -1327,13 +1351,11 @@ hipError_t down_combine_hq(const Launch &L, int wtype, const uint8_t *w, int n_e
                                wts + slots, resid ? resid + rows : nullptr, spt, m - kMaxGridTokens, rpe, y + rows);
     }
     const int spt_shift = (spt & (spt - 1)) == 0 ? __builtin_ctz((unsigned)spt) : -1;
-    const bool wide = bm_takes_q8k(wtype) && spt * nb > 8; // (Q8_2_X4 columns are encoded from registers, four tasks a thread of 256)
-    const long of_1024 = (long)m * ((rpe + 256 / spt - 1) / (256 / spt)), rounds = (of_1024 + 255) / 256;
-    const int T = !wide ? 256 : (of_1024 + 127) / 128 == 2 * rounds || rounds > 5 ? 1024 : 512;
+    const int T = bm_takes_q8k(wtype) ? down_threads(spt, m, rpe, spt * nb) : 256; // (Q8_2_X4 columns are encoded from registers, four tasks a thread of 256)
     const int D = T / 4 / spt;
     const size_t lds = down_combine_lds(wtype, k, spt) + (size_t)(D - 64 / spt) * spt * sizeof(float);
     const unsigned blocks = (unsigned)((rpe + D - 1) / D);
-    const bool row_major = plain_order(m * spt, eighths(blocks));
+    const bool row_major = plain_order((int64_t)m * spt, m, blocks, T);
     auto launch = [&](auto kern) {
         hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;

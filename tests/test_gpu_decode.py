@@ -524,8 +524,9 @@ def test_fused_step_matches_the_chain_and_the_oracle(gpu, types, hidden, ff, n_e
     L.free()
 
 
-# Both orders of the fused step's workgroups (by dies from 64 slots on): slot counts that are powers of two and that are not, rows whose
-# last eight of blocks is not whole, repeated experts, types on either column form.
+# Both orders of the fused step's workgroups (by dies from 64 slots on; the down half so only where few of a token's last eight blocks do
+# not exist): slot counts that are powers of two and that are not, rows whose last eight of blocks is not whole, repeated experts, types on
+# either column form.
 @pytest.mark.parametrize("types,hidden,ff,m,top_k", (
     ((bm.Q4_K, bm.Q4_K, bm.Q6_K), 768, 256, 9, 8),
     ((bm.Q4_K, bm.Q4_K, bm.Q4_K), 256, 512, 13, 5),
@@ -534,12 +535,17 @@ def test_fused_step_matches_the_chain_and_the_oracle(gpu, types, hidden, ff, n_e
     ((bm.Q3_K, bm.Q3_K, bm.IQ2_XXS), 768, 256, 11, 6),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 256, 256, 63, 1),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 256, 256, 64, 1),
+    ((bm.Q4_K, bm.Q4_K, bm.Q4_K), 1280, 256, 11, 7),         # 143 blocks of nine rows: one of 144 does not exist, by dies
+    ((bm.Q3_K, bm.Q3_K, bm.Q6_K), 768, 256, 6, 12),          # 154 of 160: by dies only past 1023 workgroups
+    ((bm.Q3_K, bm.Q3_K, bm.Q6_K), 768, 256, 14, 12),
+    ((bm.Q3_K, bm.Q3_K, bm.IQ4_XS), 512, 512, 32, 3),        # 25 of 32, quantized in the launch: plain
 ))
 def test_fused_step_in_either_order(gpu, types, hidden, ff, m, top_k):
-    L = Layer(gpu, types, hidden, ff, 8, 650 + hidden + ff)
+    n_experts = max(8, top_k)
+    L = Layer(gpu, types, hidden, ff, n_experts, 650 + hidden + ff)
     rng = np.random.default_rng(651)
     x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
-    ids, wts = route(rng, m, 8, top_k)
+    ids, wts = route(rng, m, n_experts, top_k)
     gpu.fault_clear()
     y, h, act_h, act_x = run_fused_step(gpu, L, x, ids, wts, top_k, resid)
     want_y, want_h = L.oracle(x, ids, wts, top_k)
@@ -613,15 +619,20 @@ def test_down_of_more_tokens_than_a_launch_holds(gpu, wtype, entry):
         b.free()
 
 
-# The down half's workgroups on Q8_K columns: 256 threads where a token's rows are at most eight blocks, else 512, or 1024 where the last
-# round of 256 of those is more than half full or there are more than five rounds; rows that are no multiple of a workgroup's.
+# The down half's workgroups on Q8_K columns: 256 threads where a token's rows are at most eight blocks, or twenty of a small launch, else
+# 512, or 1024 where the last round of 256 of those is more than half full or there are more than five rounds, or 256 where 512 leave a
+# last round less than a quarter full; rows that are no multiple of a workgroup's.
 @pytest.mark.parametrize("types,hidden,ff,m,top_k", (
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 4, 4),  # 256
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 3, 5),  # 512
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 7, 5),  # 1024
     ((bm.Q4_K, bm.Q4_K, bm.IQ2_XXS), 512, 768, 18, 3),       # 512
     ((bm.Q4_K, bm.Q4_K, bm.IQ2_XXS), 512, 768, 19, 3),       # 1024
-    ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 256, 2304, 257, 1),        # 512: two rounds
+    ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 256, 2304, 257, 1),        # 256: two of 512 threads behind a round of 512
+    ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 256, 2304, 340, 1),        # 512: two rounds
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 1280, 512, 2, 10), # 512: twenty blocks, 428 workgroups of 256
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 768, 512, 2, 10),  # 256: twenty blocks, 256 workgroups
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 768, 512, 2, 11),  # 512: twenty-two blocks
     ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 256, 2304, 385, 1),        # 1024
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ3_XXS), 256, 256, 2, 64), # 512: two rows a workgroup
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ3_XXS), 256, 256, 3, 64), # 1024
