@@ -1083,19 +1083,20 @@ int gemv_max_cols(int wtype, int k) {
 // above all) and for the types whose unpacking is dear beside a column's dot. It gains most where k_gemv has no ring (`ringless`: an odd count
 // past three). Past 1024 groups k_gemv wins everywhere. us, k_gemv / columns dealt: 16384 rows, 8 columns, Q6_K k 512 5.7 / 7.6, k 768 7.0 / 9.3, k 2304
 // 20.1 / 17.1, IQ3_XXS k 2048 16.9 / 18.1, Q4_K k 2048 13.6 / 11.2; 12288 rows, 8 columns, Q6_K k 512 5.7 / 6.5, k 2048 14.4 / 13.2; 16384
-// rows, 5 columns, Q5_K k 512 4.7 / 5.2, k 2048 11.5 / 10.7. Of 6174 calls from 600 to 16384 rows (seven types, 256 to 4352 values, 2
-// to 8 columns) k_gemv is more than 2 % ahead of the form chosen in 21, by 4.5 % at most.
+// rows, 5 columns, Q5_K k 512 4.7 / 5.2, k 2048 11.5 / 10.7; of Q6_K's rows the longer ones lose most past 768 groups: 14657 rows of 4096, 8
+// columns 29.2 / 35.3, 4 columns of 4608 21.3 / 24.4. (10193 calls from 600 to 17000 rows, seven types, 256 to 5120 values, 2 to 8 columns.)
 static int gemv_cols_from(int wtype, int m, bool far, bool ringless) {
     constexpr int kNever = 1 << 30;
     const bool q8k = bm_takes_q8k(wtype), odd = m % 2 != 0;
     if (m == 2) return 1;
+    if (wtype == BM_Q6K && (ringless ? far && m == 7 : far || odd)) return kNever;
     if (ringless) return odd && (m == 3 ? q8k : far && wtype != BM_Q3K && wtype != BM_Q4K && wtype != BM_Q5K) ? 9 : 1;
     if (m == 3) {
         if (q8k) return kNever;
         far = true;
     }
-    if (wtype == BM_Q6K) return far ? (odd ? kNever : m == 4 ? 8 : 16) : (odd ? 16 : m == 4 ? 3 : 8);
-    if (!far) return m % 4 == 0 ? 2 : 3;
+    if (wtype == BM_Q6K) return m == 4 ? 3 : 8;
+    if (!far) return m == 8 || (m == 4 && q8k) ? 2 : 3;
     if (wtype == BM_Q3K || wtype == BM_Q4K) return odd ? 8 : 3;
     if (wtype == BM_Q5K) return 8;
     if (wtype == BM_IQ3XXS) return odd ? kNever : 16;
