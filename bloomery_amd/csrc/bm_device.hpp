@@ -687,8 +687,10 @@ struct Iq2Tables {
     const uint2 *grid;  // IQ2_XXS: a grid point's eight magnitude selectors (0, 1, 2), a byte each
     const uint2 *grid3; // IQ3_XXS: (64 + magnitudes, 64 - magnitudes) of a four-value grid point
     const uint2 *signs; // IQ2_XXS: 4 in the bytes of the negative values; IQ3_XXS: 0xff there
-    u32 at;             // where they lie in LDS: the grid, and 2048 bytes on the signs
 };
+// Where the signs lie behind the grid. One column's row dots take both tables to start where LDS does: their kernels have no array of
+// fixed size (a test reads that from the built library), and with the dynamic array's own address, a zero that only the
+// linker fills in, each lookup would add it.
 constexpr u32 kIqSignsAt = 2048;
 
 // The eight bytes at an LDS address. The row dots address the tables by bytes: an index turned to bits 3 .. of a word and masked, two
@@ -739,7 +741,7 @@ struct Iq2Dec {
     int sc[8];
 };
 
-// BY_BYTES: the lookups by LDS addresses (one column's dot; where a decode serves several columns, and registers are what there is
+// BY_BYTES: the lookups by LDS addresses, the tables at the start of LDS (one column's dot; where a decode serves several columns, and registers are what there is
 // least of, the plain form measures the faster: IQ3_XXS tiles of 64 tokens 116 us against 119).
 template <bool BY_BYTES>
 __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int q, const Iq2Tables &tb) {
@@ -755,8 +757,8 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int 
             const u32 idx = e ? idx_b : idx_a, aux = e ? aux_b : aux_a;
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
             if constexpr (BY_BYTES)
-                bm_iq2_codes_of(bm_lds_pair(tb.at + (bm_to_bit3(idx, 8 * q) & 0x7f8u)),
-                                bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u)), dec.u_lo[sb], dec.u_hi[sb]);
+                bm_iq2_codes_of(bm_lds_pair(bm_to_bit3(idx, 8 * q) & 0x7f8u),
+                                bm_lds_pair(kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u)), dec.u_lo[sb], dec.u_hi[sb]);
             else
                 bm_iq2_codes(tb, (idx >> (8 * q)) & 0xffu, (aux >> (7 * q)) & 127u, dec.u_lo[sb], dec.u_hi[sb]);
         }
@@ -855,8 +857,8 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int 
             uint2 g0, g1, sg;
             if constexpr (BY_BYTES) {
                 const u32 pair = bm_to_bit3(e ? bm_pick(ib0, ib1, upper) : bm_pick(ia0, ia1, upper), 16 * (q & 1));
-                g0 = bm_lds_pair(tb.at + (pair & 0x7f8u)), g1 = bm_lds_pair(tb.at + ((pair >> 8) & 0x7f8u));
-                sg = bm_lds_pair(tb.at + kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
+                g0 = bm_lds_pair(pair & 0x7f8u), g1 = bm_lds_pair((pair >> 8) & 0x7f8u);
+                sg = bm_lds_pair(kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
             } else {
                 const u32 pair = ((q & 2) ? (e ? ib1 : ia1) : (e ? ib0 : ia0)) >> (16 * (q & 1));
                 g0 = tb.grid3[pair & 0xffu], g1 = tb.grid3[(pair >> 8) & 0xffu];

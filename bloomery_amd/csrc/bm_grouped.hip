@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void k_gate_up_tiles(const uint8_t *wg, const 
     const uint8_t *wrow = (which ? wu : wg) + ((size_t)t.e * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT, 256, true>(lds);
+    const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     float *hbuf = reinterpret_cast<float *>(cols + (size_t)MC * col_bytes); // [MC][32]
     u32 *bad = reinterpret_cast<u32 *>(hbuf + MC * 32);                      // [MC]: entry names no slot
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(256) void k_gemv_tiles(const uint8_t *w, u32 n_expe
     const uint8_t *wrow = w + ((size_t)t.e * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT, 256, true>(lds);
+    const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
     u32 *slot_of = reinterpret_cast<u32 *>(cols + (size_t)MC * col_bytes); // [MC]
     for (int c0 = 0; c0 < (PASSES ? t.m : 1); c0 += MC) { // one pass, but for a tile wider than MC under PASSES

@@ -178,7 +178,7 @@ __global__ __launch_bounds__(T) void k_gemv(const uint8_t *w, long rows, int nb,
     st.load(act + (size_t)col0 * col_bytes, m * col_bytes);
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT, T>(lds);
+    const Iq2Tables tb = stage_tables<WT>(lds, T);
     uint8_t *cols = lds + tab_bytes<WT>();
     st.store(cols, act + (size_t)col0 * col_bytes, m * col_bytes);
     __syncthreads();
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(C == 1 ? 512 : 1024) void k_gemv_cols(const uint8_t
     __builtin_amdgcn_sched_barrier(0);
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables_by<WT>(lds, T);
+    const Iq2Tables tb = stage_tables<WT>(lds, T);
     uint8_t *cols = lds + tab_bytes<WT>();
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -993,7 +993,7 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT, T>(lds);
+    const Iq2Tables tb = stage_tables<WT>(lds, T);
     uint8_t *cols = lds + tab_bytes<WT>();
     float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
     float *s_w = part + D * spt;                                              // [spt]
@@ -1038,7 +1038,7 @@ __global__ __launch_bounds__(64) void k_block_sums(const uint8_t *wrow, int nb, 
     const int n = NB > 0 ? NB : nb;
     const int col_bytes = bm_act_col_bytes<WT>(n);
     for (int i = tid; i < 16 * n; i += 64) out[i] = 0;
-    const Iq2Tables tb = stage_tables<WT, 64>(lds);
+    const Iq2Tables tb = stage_tables<WT>(lds, 64);
     uint8_t *col = lds + tab_bytes<WT>();
     stage_bytes<64>(col, act_col, col_bytes);
     __threadfence();

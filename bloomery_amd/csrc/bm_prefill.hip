@@ -1205,7 +1205,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
     using G = IqGemm<WT>;
     extern __shared__ __align__(16) uint8_t lds[];
     GemmLds *tab = reinterpret_cast<GemmLds *>(lds);
-    [[maybe_unused]] const Iq2Tables tb = stage_tables<WT, 256, true>(lds + sizeof(GemmLds));
+    [[maybe_unused]] const Iq2Tables tb = stage_tables<WT>(lds + sizeof(GemmLds));
     uint8_t *a_codes = lds + sizeof(GemmLds) + tab_bytes<WT>();
     uint8_t *w_hi = a_codes + 64 * kIqStride;
     uint8_t *w_lo = w_hi + (G::kPlanes - 1) * 64 * kIqStride; // (the one plane where there is one)

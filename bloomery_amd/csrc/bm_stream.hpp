@@ -51,8 +51,8 @@ __device__ __forceinline__ uint2 iq_sign_masks(int t) {
 // (T: how many of the workgroup's threads write them, no call to the built-in: blockDim.x is a load from the dispatch packet, in
 // front of whatever comes next)
 template <int WT>
-__device__ __forceinline__ Iq2Tables stage_tables_by(uint8_t *lds, int T) {
-    Iq2Tables tb{nullptr, nullptr, nullptr, 0};
+__device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds, int T = 256) {
+    Iq2Tables tb{nullptr, nullptr, nullptr};
     if constexpr (WT == BM_IQ2XXS) {
         // a grid point as eight byte selectors over the three magnitudes (8, 25, 43 -> 0, 1, 2), a sign index as eight bytes
         // of 4 where the value is negative: their sum picks a value's code byte 43 +- magnitude out of six (bm_iq2_codes)
@@ -82,15 +82,6 @@ __device__ __forceinline__ Iq2Tables stage_tables_by(uint8_t *lds, int T) {
         tb.grid3 = grid;
         tb.signs = signs;
     }
-    return tb;
-}
-
-// LDS of a kernel that has no array of fixed size starts at address 0, which then drops out of the lookups' addresses (`at` stays 0).
-// AFTER_FIXED: the kernel has some.
-template <int WT, int T = 256, bool AFTER_FIXED = false>
-__device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds) {
-    Iq2Tables tb = stage_tables_by<WT>(lds, T);
-    if constexpr (AFTER_FIXED) tb.at = (u32)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     return tb;
 }
 

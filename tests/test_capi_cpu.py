@@ -3,6 +3,7 @@ host-only entry points answer without a GPU. No kernel is launched here."""
 import ctypes
 import os
 import re
+import struct
 
 import pytest
 
@@ -75,3 +76,46 @@ def test_the_benchmark_refuses_more_than_one_gpu():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert r.returncode != 0 and "one GPU" in r.stderr and r.stdout.strip() == ""
+
+
+def built_kernels():
+    """name -> the compiler's record of every kernel in the built library: its bundles' gfx950 code objects, their metadata notes."""
+    msgpack = pytest.importorskip("msgpack")
+    data, out, at = open(bm.LIB_PATH, "rb").read(), {}, 0
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    while (at := data.find(magic, at)) >= 0:
+        (count,), p = struct.unpack_from("<Q", data, at + len(magic)), at + len(magic) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            triple, p = data[p + 24:p + 24 + length], p + 24 + length
+            if b"gfx950" not in triple:
+                continue
+            elf = data[at + offset:at + offset + size]
+            sections, (entry, n) = struct.unpack_from("<Q", elf, 40)[0], struct.unpack_from("<HH", elf, 58)
+            for s in range(n):
+                kind, = struct.unpack_from("<I", elf, sections + s * entry + 4)
+                if kind != 7:  # SHT_NOTE
+                    continue
+                note, = struct.unpack_from("<Q", elf, sections + s * entry + 24)
+                name_len, desc_len, note_type = struct.unpack_from("<III", elf, note)
+                if note_type == 32:  # NT_AMDGPU_METADATA
+                    desc = note + 12 + (name_len + 3) // 4 * 4
+                    for k in msgpack.unpackb(elf[desc:desc + desc_len])["amdhsa.kernels"]:
+                        out[k[".name"]] = k
+        at += len(magic)
+    return out
+
+
+def test_kernels_that_look_tables_up_at_the_start_of_lds():
+    """The IQ2_XXS and IQ3_XXS tables are read at LDS address 0 by one column's row dots and by the tolerance-mode GEMM: none of those kernels
+    may have LDS of a fixed size, which would come first."""
+    kernels = built_kernels()
+    assert kernels["_ZN3bmk8k_tablesEPKjjjjPjS2_S2_S2_j"][".group_segment_fixed_size"] > 0  # (the reader sees such a size)
+    one_column = r"k_(gemv|gemv_cols|gemv_sel|gemv_x|gate_up|gate_up_xq|down_combine|down_combine_hq|block_sums|gemm_iq2_fast)"
+    seen = set()
+    for name, k in kernels.items():
+        m = re.match(r"_ZN3bmk\d+" + one_column + r"(?:ILi(\d+)|E)", name)
+        if m and (m[1] == "gemm_iq2_fast" or int(m[2]) in (bm.IQ2_XXS, bm.IQ3_XXS)):
+            seen.add(m[1])
+            assert k[".group_segment_fixed_size"] == 0, name
+    assert len(seen) == 10, seen

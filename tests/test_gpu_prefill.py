@@ -609,7 +609,7 @@ def test_gemm_of_narrow_tiles_underflow_and_signed_zeros(gpu, wtype, n_slots):
 
 @pytest.mark.parametrize("wtype,k", ((bm.Q4_K, 256), (bm.Q5_K, 768), (bm.Q6_K, 512)))
 def test_gemm_with_several_slabs_of_narrow_and_wide_tiles(gpu, wtype, k):
-    """Thirty-three slabs an expert: a workgroup takes two of them, the last one alone."""
+    """Thirty-three slabs an expert: a workgroup takes four of them, the last one alone."""
     test_gemm_with_several_slabs_a_workgroup(gpu, wtype, k, rpe=2064)
 
 
