@@ -1445,9 +1445,14 @@ __global__ __launch_bounds__(256, 2) void k_gemm_iq(const uint8_t *w, int rpe, i
             fetch_cols(few, i);
             __builtin_amdgcn_sched_barrier(0);
         }
-        stage_rows();
-        __builtin_amdgcn_sched_barrier(0);
-        stage_cols(few);
+        if constexpr (WT == BM_Q3K) { // (the other way round one in nine of the launches under 60 us takes 3 to 9 % longer)
+            stage_cols(few);
+            stage_rows();
+        } else {
+            stage_rows();
+            __builtin_amdgcn_sched_barrier(0);
+            stage_cols(few);
+        }
         if (i + 1 < nb) {
             fetch_rows(i + 1);
             if constexpr (kColsAhead) fetch_cols(few, i + 1);
