@@ -938,7 +938,7 @@ int bm_scratch_create(bm_ctx *ctx, int gate_type, int down_type, int hidden, int
     s->gate_type = gate_type, s->down_type = down_type, s->hidden = hidden, s->ff = ff, s->n_experts = n_experts;
     s->spt = n_slots_per_token, s->max_tokens = max_tokens;
     // the per-slot step below 22 tokens (Q4_K gate/up, Q6_K down, top-8 of 128, hidden 2048, ff 768, us a step, per slot / grouped:
-    // 16 tokens 67 / 86, 24: 92 / 88, 128: 400 / 188), then by path_choice
+    // 16 tokens 63 / 81, 24: 85 / 84, 128: 328 / 177), then by path_choice
     s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 0;
     // Where both stacks are on Q8_K columns and the experts are large, the grouped step - for few slots an
     // expert the per-slot gate . up launch and the down tiles, see bm_moe_forward - is ahead of the per-slot step from the first
@@ -1002,19 +1002,21 @@ static bool per_slot_fits(const bm_scratch *s) {
 // workgroups run on one die; an expert of few slots costs it a whole tile), and the GEMM has a constant more for its launches. Tiles
 // are counted as ordinary routes make them: an expert's last one half full, no fewer than one an expert; with about a slot an
 // expert the tile launches are ahead whatever else. Where eight columns are short enough to leave LDS for more workgroups the K types' and
-// Q3_K's tile launches are about a third cheaper; the other types are bound by their decode. The numbers are a fit to 2032 measured pairs (1 to 256 experts, 22 to 3000 tokens, hidden 1024 to 7168,
-// cold weights): the chosen side is 0.5 % behind the better one on average and 35 % at worst, where "from 12 slots an expert, and
-// from 448 or 96 tokens on always" was 6 % behind, and twice as slow for one large expert of few slots (a shared expert). Some
-// of the pairs, us a layer, tile launches / GEMM:
-//   hidden 2048, ff 768, top-8 of 128:  Q4_K 128 tokens 182 / 232, 192: 237 / 252, 256: 282 / 257, 447: 446 / 297
-//                                       Q5_K 128 tokens 204 / 232, 192: 263 / 249; Q6_K 192: 270 / 266
-//                                       IQ4_XS 64 tokens 188 / 194, 95: 214 / 202; Q3_K / Q4_K 24: 96 / 107, 48: 148 / 132
-//                                       IQ2_XXS 128 tokens 240 / 287, 192: 319 / 308; IQ3_XXS 95: 201 / 251, 192: 355 / 293
-//   one expert, hidden 7168, ff 2048:   Q6_K 22 tokens 83 / 169, 64: 146 / 177, 95: 206 / 171, 256: 471 / 173
-//                                       IQ2_XXS 22 tokens 99 / 187, 95: 199 / 197, 192: 339 / 199
-//   hidden 7168, ff 1536, top-4 of 8:   Q4_K 22 tokens 197 / 141, 64: 405 / 145
-//   hidden 7168, ff 2048, top-8 of 256: IQ2_XXS 64 tokens 1762 / 2819, 192: 3546 / 3618
-//   hidden 2048, ff 768, top-2 of 256:  Q4_K 500 tokens 191 / 301, 1500: 437 / 399; IQ2_XXS 230: 143 / 281
+// Q3_K's tile launches are about a third cheaper; the other types are bound by their decode. The numbers are a fit to 2032 pairs (1 to 256
+// experts, 22 to 3000 tokens, hidden 1024 to 7168, cold weights) measured when both sides were slower, the GEMM of few slots an expert by
+// more: on 3858 random layers of 22 to 1500 tokens the chosen side is now 1.4 % behind the better one on average, more than 5 % in 8 % of
+// them and 1.9 times as slow at worst, nearly all of it tile launches of the K types that the GEMM has overtaken (of the calls that go to
+// tile launches 4 to 5 % on average; of those that go to the GEMM 0.1 %, Q3_K 1 to 2 %). The per-slot step, which is not asked past its
+// own cut, would be ahead of both below about one slot an expert. Some of the pairs, us a layer, tile launches / GEMM:
+//   hidden 2048, ff 768, top-8 of 128:  Q4_K 128 tokens 179 / 187, 192: 232 / 189, 256: 284 / 200, 447: 444 / 241
+//                                       Q5_K 128 tokens 187 / 201, 192: 243 / 203; Q6_K 192: 271 / 215
+//                                       IQ4_XS 64 tokens 156 / 197, 95: 180 / 198; Q3_K / Q4_K 24: 95 / 143, 48: 143 / 169
+//                                       IQ2_XXS 128 tokens 215 / 242, 192: 286 / 246; IQ3_XXS 95: 176 / 228, 192: 305 / 232
+//   one expert, hidden 7168, ff 2048:   Q6_K 22 tokens 84 / 114, 64: 148 / 157, 95: 208 / 161, 256: 473 / 168
+//                                       IQ2_XXS 22 tokens 94 / 143, 95: 181 / 195, 192: 304 / 199
+//   hidden 7168, ff 1536, top-4 of 8:   Q4_K 22 tokens 213 / 92, 64: 391 / 142
+//   hidden 7168, ff 2048, top-8 of 256: IQ2_XXS 64 tokens 1363 / 3190, 192: 3013 / 3603
+//   hidden 2048, ff 768, top-2 of 256:  Q4_K 500 tokens 222 / 312, 1500: 430 / 342; IQ2_XXS 230: 151 / 391
 static bool gemm_ahead(const bm_scratch *s, int m) {
     struct Line {
         double launches, die, fits; // the GEMM's constant, what a 64-slot tile on the die costs, the factor of short columns
@@ -1047,7 +1049,7 @@ static PathChoice path_choice(const bm_scratch *s, int m) {
     if (!gemm_ok) return {BM_PATH_GROUPED, mode};
     if (s->gemm_from) return {m >= s->gemm_from ? BM_PATH_GEMM : BM_PATH_GROUPED, mode}; // the caller's
     // The tolerance mode: from 96 tokens on in its own f32 order, and where the gate has kernels of that order (Q4_K, Q5_K, Q6_K,
-    // IQ2_XXS) then always by the GEMM (789 pairs of 95 to 800 tokens: 1.4 % behind the better side on average); below, the exact order.
+    // IQ2_XXS) then always by the GEMM (1925 layers of 96 to 800 tokens: 1.7 % behind the better side on average, twice as slow at worst); below, the exact order.
     const bool fast = mode != BM_GEMM_EXACT && m >= 96;
     const bool fast_gate = act_form(s->gate_type) == 0 || s->gate_type == BM_TYPE_IQ2_XXS;
     return {(fast && fast_gate) || gemm_ahead(s, m) ? BM_PATH_GEMM : BM_PATH_GROUPED, fast ? mode : BM_GEMM_EXACT};

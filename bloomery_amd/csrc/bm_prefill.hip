@@ -1617,7 +1617,8 @@ hipError_t gemm(const Launch &L, int wtype, const uint8_t *w, int n_experts, int
         // 64-row workgroups of the fullest die's 32 compute units, here in tiles as ids without a favourite would make them; the
         // line lies at three and a half a unit (the int8 form / the other, us, one stack; 64: k 512 8.3 / 15.1, k 2048 23.7 / 35.9,
         // k 7168 73.6 / 117; 96: 14.0 / 18.2, 38.2 / 45.0, 122 / 144; 112: 17.8 / 20.2, 47.3 / 49.1, 148 / 136; 128 with tiles of at
-        // most 32 slots: 15.1 / 15.5, 44.7 / 41.6, 143 / 119; 160: 18.7 / 15.7, 57.2 / 42.5, 183 / 118).
+        // most 32 slots: 15.1 / 15.5, 44.7 / 41.6, 143 / 119; 160: 18.7 / 15.7, 57.2 / 42.5, 183 / 118. Of 3958 random launches the rule is 1.2 %
+        // behind the better form on average; so are 104 and 128, 80 is 1.8 %).
         const u32 est_tiles = std::max((u32)std::min(n_experts, n_slots), (u32)n_slots / kGemmBN + (u32)n_experts / 2);
         const u32 die_units = (est_tiles + 7) / 8 * stacks * (u32)((rows_per_expert + kIqRows - 1) / kIqRows);
         if (mode != 0 && die_units > 112u)
