@@ -1081,7 +1081,8 @@ int gemv_max_cols(int wtype, int k) {
 // waves. There k_gemv, a wave a group and all columns, has up to a wave a SIMD and its time no longer grows with the rows, while the
 // other form's does: it loses where its start counts (short rows), where half of a wave's last column pair is idle (odd counts, three
 // above all) and for the types whose unpacking is dear beside a column's dot. It gains most where k_gemv has no ring (`ringless`: an odd count
-// past three). Past 1024 groups k_gemv wins everywhere. us, k_gemv / columns dealt: 16384 rows, 8 columns, Q6_K k 512 5.7 / 7.6, k 768 7.0 / 9.3, k 2304
+// past three). Past 1024 groups k_gemv: dealt columns take 1.08 (Q4_K) to 1.38 times (Q6_K) its time on average there, though up to 24000 rows those
+// of rows without a ring would still gain (four columns 0.77 to 0.9). us, k_gemv / columns dealt: 16384 rows, 8 columns, Q6_K k 512 5.7 / 7.6, k 768 7.0 / 9.3, k 2304
 // 20.1 / 17.1, IQ3_XXS k 2048 16.9 / 18.1, Q4_K k 2048 13.6 / 11.2; 12288 rows, 8 columns, Q6_K k 512 5.7 / 6.5, k 2048 14.4 / 13.2; 16384
 // rows, 5 columns, Q5_K k 512 4.7 / 5.2, k 2048 11.5 / 10.7; of Q6_K's rows the longer ones lose most past 768 groups: 14657 rows of 4096, 8
 // columns 29.2 / 35.3, 4 columns of 4608 21.3 / 24.4. (10193 calls from 600 to 17000 rows, seven types, 256 to 5120 values, 2 to 8 columns.)
