@@ -133,7 +133,8 @@ constexpr int kDppXor2 = 0x4E;        // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141; // lane i <-> 7 - i inside each 8
 constexpr int kDppMirror = 0x140;     // lane i <-> 15 - i inside each 16
 constexpr int kDppShl1 = 0x101, kDppShl2 = 0x102, kDppShl4 = 0x104; // lane i reads lane i + n of its row of 16
-constexpr int kDppShr4 = 0x114;                                     // lane i reads lane i - 4
+constexpr int kDppShl7 = 0x107, kDppShl8 = 0x108;
+constexpr int kDppShr1 = 0x111, kDppShr4 = 0x114;                   // lane i reads lane i - n
 
 __device__ __forceinline__ float bm_quad_xor1(float v) { return bm_dppf<kDppXor1>(v); }
 __device__ __forceinline__ float bm_quad_xor2(float v) { return bm_dppf<kDppXor2>(v); }

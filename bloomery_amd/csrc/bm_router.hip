@@ -13,6 +13,8 @@
 //
 // A token with a logit that is not finite has no defined routing: it raises Router on the fault word, gets NaN
 // probabilities and weights, and keeps its ids as they stand (crates/gpu/src/route_softmax.rs:53-62).
+#include <type_traits>
+
 #include "bm_stream.hpp"
 
 namespace bmk {
@@ -20,7 +22,8 @@ namespace bmk {
 // Timeline of the router launch, in measurement builds only (-DBM_TIMELINE, the library bench.py --timeline loads): thread 0 of
 // workgroup b keeps the device's constant-rate counter (100 MHz) in registers at six points of router_logits_body and stores
 // them at its end in row b: start, the token's row arrived, normed, rows and token in LDS (behind the barrier), dots done,
-// the routing done (the workgroup that routes).
+// the routing done (the workgroup that routes: start, maximum known, exponentials summed, probabilities formed, logits held, routed,
+// places found by the second wave).
 #ifdef BM_TIMELINE
 constexpr int kRouterTimelineRows = 1024;
 __device__ unsigned long long g_router_timeline[kRouterTimelineRows * 8];
@@ -47,9 +50,21 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr u32 kSiteRouter = 5; // crates/device/src/fault.rs:84-86
 
-// Sum / maximum over the wave, every lane ending with it: pairs, quads, eights and sixteens by data-parallel-primitive moves
-// (a few cycles each, where a shuffle through the LDS crossbar is a hundred), the two sixteens of a half by one swizzle, the
-// halves by two lane reads. The sum's association: ((pairs) quads) ... halves, lower half first.
+// Sum / maximum over the wave, every lane ending with it: pairs, quads, eights and sixteens by data-parallel-primitive moves, the
+// two sixteens of a half and the two halves by row swaps (a few cycles each, where the LDS crossbar is a hundred). The sum's
+// association: ((pairs) quads) ... halves.
+struct Pair32 {
+    u32 a, b;
+};
+// a: the lower row of sixteen of every half, in both its rows; b: the upper one (wave halves: the lower half, the upper half).
+__device__ __forceinline__ Pair32 rows_of_half(u32 v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {r[0], r[1]};
+}
+__device__ __forceinline__ Pair32 halves(u32 v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {r[0], r[1]};
+}
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
     return __hiloint2double((int)bm_dpp<CTRL>((u32)__double2hiint(v)), (int)bm_dpp<CTRL>((u32)__double2loint(v)));
@@ -59,43 +74,44 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     v += dpp_f64<kDppXor2>(v);
     v += dpp_f64<kDppHalfMirror>(v);
     v += dpp_f64<kDppMirror>(v);
-    v += __hiloint2double((int)bm_swap16((u32)__double2hiint(v)), (int)bm_swap16((u32)__double2loint(v)));
-    const int lo = __double2loint(v), hi = __double2hiint(v);
-    const double a = __hiloint2double(__builtin_amdgcn_readlane(hi, 0), __builtin_amdgcn_readlane(lo, 0));
-    const double b = __hiloint2double(__builtin_amdgcn_readlane(hi, 32), __builtin_amdgcn_readlane(lo, 32));
-    return a + b;
+    const Pair32 h = rows_of_half((u32)__double2hiint(v)), l = rows_of_half((u32)__double2loint(v));
+    v = __hiloint2double((int)h.a, (int)l.a) + __hiloint2double((int)h.b, (int)l.b);
+    const Pair32 hh = halves((u32)__double2hiint(v)), ll = halves((u32)__double2loint(v));
+    return __hiloint2double((int)hh.a, (int)ll.a) + __hiloint2double((int)hh.b, (int)ll.b);
 }
 __device__ __forceinline__ float wave_max_f32(float v) {
     v = fmaxf(v, bm_dppf<kDppXor1>(v));
     v = fmaxf(v, bm_dppf<kDppXor2>(v));
     v = fmaxf(v, bm_dppf<kDppHalfMirror>(v));
     v = fmaxf(v, bm_dppf<kDppMirror>(v));
-    v = fmaxf(v, bm_bits_f32(bm_swap16(bm_f32_bits(v))));
-    const int bits = (int)bm_f32_bits(v);
-    return fmaxf(bm_bits_f32((u32)__builtin_amdgcn_readlane(bits, 0)), bm_bits_f32((u32)__builtin_amdgcn_readlane(bits, 32)));
+    const Pair32 r = rows_of_half(bm_f32_bits(v));
+    v = fmaxf(bm_bits_f32(r.a), bm_bits_f32(r.b));
+    const Pair32 h = halves(bm_f32_bits(v));
+    return fmaxf(bm_bits_f32(h.a), bm_bits_f32(h.b));
 }
 
-// Token t's routing by one wave; lane L owns experts L + 64 j, j < PER. `v`: this lane's logits, expert lane + 64 j in v[j]
-// (-inf past n_exp). First the probabilities (p[j]; stored if asked for): false, with NaN probabilities and weights and
-// BM_SITE_ROUTER raised, when a logit is not finite.
+// Token t's routing; lane L of a wave owns experts L + 64 j, j < PER. `v`: this lane's logits, expert lane + 64 j in v[j] (-inf past
+// n_exp).
 template <int PER>
-__device__ __forceinline__ bool route_probs_wave(const float (&v)[PER], u32 t, u32 n_exp, u32 used, float *probs, float *weights,
-                                                 u32 *fault, u32 layer, float (&p)[PER]) {
-    const u32 lane = threadIdx.x & 63;
+__device__ __forceinline__ bool logits_finite(const float (&v)[PER], u32 n_exp) {
     bool odd = false;
 #pragma unroll
-    for (int j = 0; j < PER; j++) odd |= lane + 64 * j < n_exp && !(fabsf(v[j]) <= 3.402823466e38f);
-    if (__ballot(odd) != 0) {
-        const float nan = bm_bits_f32(0x7fc00000u);
-        if (probs) {
-#pragma unroll
-            for (int j = 0; j < PER; j++)
-                if (lane + 64 * j < n_exp) probs[(size_t)t * n_exp + lane + 64 * j] = nan;
-        }
-        if (lane < used) weights[(size_t)t * used + lane] = nan;
-        if (lane == 0) bm_raise(fault, layer, kSiteRouter);
-        return false;
-    }
+    for (int j = 0; j < PER; j++) odd |= (threadIdx.x & 63) + 64 * j < n_exp && !(fabsf(v[j]) <= 3.402823466e38f);
+    return __ballot(odd) == 0;
+}
+// A token with a logit that is not finite.
+__device__ __forceinline__ void route_refuse(u32 t, u32 n_exp, u32 used, float *probs, float *weights, u32 *fault, u32 layer) {
+    const u32 lane = threadIdx.x & 63;
+    const float nan = bm_bits_f32(0x7fc00000u);
+    if (probs)
+        for (u32 e = lane; e < n_exp; e += 64) probs[(size_t)t * n_exp + e] = nan;
+    if (lane < used) weights[(size_t)t * used + lane] = nan;
+    if (lane == 0) bm_raise(fault, layer, kSiteRouter);
+}
+// The probabilities of finite logits, zero past n_exp.
+template <int PER>
+__device__ __forceinline__ void route_probs_wave(const float (&v)[PER], u32 n_exp, float (&p)[PER]) {
+    const u32 lane = threadIdx.x & 63;
     float mx = -INFINITY;
 #pragma unroll
     for (int j = 0; j < PER; j++) mx = fmaxf(mx, v[j]);
@@ -112,18 +128,23 @@ __device__ __forceinline__ bool route_probs_wave(const float (&v)[PER], u32 t, u
     BM_RTICK(tl_b, sum);
     const float inv = (float)sum;
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        p[j] = p[j] / inv;
-        if (probs && lane + 64 * j < n_exp) probs[(size_t)t * n_exp + lane + 64 * j] = p[j];
-    }
+    for (int j = 0; j < PER; j++) p[j] = p[j] / inv;
     BM_RTICK(tl_c, p[0]);
     BM_RTOCK(1, tl_a);
     BM_RTOCK(2, tl_b);
     BM_RTOCK(3, tl_c);
-    return true;
+}
+template <int PER>
+__device__ __forceinline__ void store_probs(const float (&p)[PER], u32 t, u32 n_exp, float *probs) {
+    if (!probs) return;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const u32 e = (threadIdx.x & 63) + 64 * j;
+        if (e < n_exp) probs[(size_t)t * n_exp + e] = p[j];
+    }
 }
 
-// Then the picks, by the wave alone: `used` rounds of a wave argmax under (probability descending, id ascending): the
+// The picks by the wave alone, where counting (below) has met a tie: `used` rounds of a wave argmax under (probability descending, id ascending): the
 // largest probability left (its bits order as its value: not negative) as one unsigned maximum over the wave, then the
 // smallest id that holds it: expert lane + 64 j, so the first j with a holder and that ballot's lowest lane. The winning
 // lane marks its entry.
@@ -165,104 +186,132 @@ __device__ __forceinline__ void route_pick_rounds(const float (&p)[PER], u32 t, 
     if (lane < used) weights[(size_t)t * used + lane] = renorm ? mine / (float)chosen : mine;
 }
 
+// A token's places (0 .. used, the last one past the picks) and probabilities in LDS.
+constexpr u32 kNoExpert = 0xffffffffu;
 template <int PER>
-__device__ __forceinline__ void route_softmax_wave(const float (&v)[PER], u32 t, u32 n_exp, u32 used, u32 renorm, float *probs,
-                                                   u32 *ids, float *weights, u32 *fault, u32 layer) {
-    float p[PER];
-    if (route_probs_wave<PER>(v, t, n_exp, used, probs, weights, fault, layer, p)) route_pick_rounds<PER>(p, t, n_exp, used, renorm, ids, weights);
+struct PickLds {
+    __align__(16) float value[64]; // the entries that may be among the first, in any order
+    u32 id[64];
+    u32 at[kRouteMaxPicks + 1];
+    float p[64 * PER];
+};
+// (between LDS stores and loads of one wave's lanes, which the LDS takes in order: for the compiler)
+__device__ __forceinline__ void lds_of_wave() { __asm__ volatile("" ::: "memory"); }
+
+// In front of places_by_counting, by its wave.
+template <int PER>
+__device__ __forceinline__ void places_clear(PickLds<PER> &L) {
+    const u32 lane = threadIdx.x & 63;
+    L.value[lane] = -INFINITY;
+    if (lane <= (u32)kRouteMaxPicks) L.at[lane] = kNoExpert;
+    lds_of_wave();
 }
 
-// The same picks by a workgroup of 256 threads for up to 256 experts (n_exp >= used), the probabilities in LDS: an entry's
-// place in the order (probability descending, id ascending) is the number of entries ahead of it, counted by comparing it
-// with every other - independent instructions spread over four waves, where the wave's rounds are a chain of some eighty
-// dependent ones each (2.0 us of a 2.6 us routing at 128 experts, 8 picks). What is counted is the entries not smaller
-// (one compare and one add with carry an entry; probabilities are not negative, so their bits order as signed integers,
-// and the places past n_exp hold -1): without the entry itself that is its place unless another entry has its bits, and then
-// some place below `used` is taken twice or not at all - seen by counting the takers of every place - and the first wave
-// picks by its rounds instead. The entry with `s` ahead of it is pick s: the rounds' ids, and the same weights from the
-// same sums (the chosen probabilities added in pick order).
-// A barrier that waits for the wave's LDS traffic only: the routing workgroup's waves meet over LDS while the first wave's
-// stores to memory (the words armed again, the probabilities) are still on their way, and a barrier that waited for those to
-// be acknowledged cost the routing 1 us.
-__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// The places of the first `used` + 1 entries in descending order of v, by one wave: at[r] = e for the entry e that r others are
+// larger than. Entries of equal value have the same count: they take the same place and leave the next one as it was, so a
+// caller finds out, and picks by rounds; so it does where more than 64 entries pass the bound, which takes equal ones.
+// Not every entry is compared with every other (128 of them: a quarter of it a wave, over LDS, took 0.9 us, and the rounds are a
+// chain of eighty dependent instructions each): an entry below `used` + 1 others' maxima cannot be among the first, so the maxima of
+// sixteen groups of lanes (of the 64 lanes, for more than fifteen picks) give a bound that about as many entries pass as are
+// wanted; those go to LDS, a lane each, and are compared with one another.
+template <int PER>
+__device__ __forceinline__ void places_by_counting(const float (&v)[PER], u32 n_exp, u32 used, PickLds<PER> &L) {
+    const u32 lane = threadIdx.x & 63;
+    float top = -INFINITY; // the lane's largest, then its group's
+#pragma unroll
+    for (int j = 0; j < PER; j++) top = fmaxf(top, lane + 64 * j < n_exp ? v[j] : -INFINITY);
+    u32 above = 0; // groups with a larger maximum
+    auto count_group = [&](u32 g) { above += bm_bits_f32((u32)__builtin_amdgcn_readlane((int)bm_f32_bits(top), (int)g)) > top ? 1u : 0u; };
+    if (used < 16) {
+        top = fmaxf(top, bm_dppf<kDppXor1>(top));
+        top = fmaxf(top, bm_dppf<kDppXor2>(top));
+#pragma unroll
+        for (u32 g = 0; g < 64; g += 4) count_group(g);
+    } else {
+#pragma unroll 16
+        for (u32 g = 0; g < 64; g++) count_group(g);
+    }
+    // the maximum with `used` above it: no entry below it is wanted (none, where maxima are equal or fewer: then every entry may be)
+    const unsigned long long bound_at = __ballot(above == used);
+    const float bound = bound_at ? bm_bits_f32((u32)__builtin_amdgcn_readlane((int)bm_f32_bits(top), __builtin_ctzll(bound_at))) : -INFINITY;
+    u32 n = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const bool in = lane + 64 * j < n_exp && v[j] >= bound;
+        const unsigned long long who = __ballot(in);
+        const u32 to = n + __builtin_amdgcn_mbcnt_hi((u32)(who >> 32), __builtin_amdgcn_mbcnt_lo((u32)who, 0));
+        if (in && to < 64) L.value[to] = v[j], L.id[to] = lane + 64 * j;
+        n += (u32)__builtin_popcountll(who);
+    }
+    if (n > 64) return;
+    lds_of_wave();
+    const float mine = L.value[lane];
+    const u32 id = L.id[lane];
+    u32 ahead = 0;
+    for (u32 c = 0; c < n; c += 16) { // (the list ends in -inf)
+        float4 o[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = *reinterpret_cast<const float4 *>(&L.value[c + 4 * k]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            ahead += o[k].x > mine ? 1u : 0u;
+            ahead += o[k].y > mine ? 1u : 0u;
+            ahead += o[k].z > mine ? 1u : 0u;
+            ahead += o[k].w > mine ? 1u : 0u;
+        }
+    }
+    if (lane < n && ahead <= used) L.at[ahead] = id;
+    lds_of_wave();
+}
 
-struct PickLds {
-    __align__(16) float p[256];      // entry e's probability, -1 past n_exp
-    u32 ahead[256];    // zero on entry
-    u32 takers[32];    // zero on entry
-    u32 pick_id[32];
-    __align__(16) float pick_p[32];
-    u32 ok;
-};
-// Every thread of the workgroup calls it; true: the picks are written; false (first wave: pick by rounds): two entries tie.
-__device__ __forceinline__ bool route_pick_ranks(PickLds &L, u32 t, u32 n_exp, u32 used, u32 renorm, u32 *ids, float *weights) {
-    const u32 tid = threadIdx.x;
-    // the entries padded to 64 << k; a thread an (entry, part of the others): 4 >> k parts of 16 << 2 k entries, a wave's
-    // threads all of one part, so its reads of the others are broadcasts
-    const u32 k = n_exp <= 64 ? 0u : n_exp <= 128 ? 1u : 2u;
-    const u32 n_pad = 64u << k, chunk = 16u << (2 * k);
-    const u32 i = tid & (n_pad - 1), j0 = (tid >> (6 + k)) * chunk;
-    if (i < n_exp) {
-        const int ki = (int)bm_f32_bits(L.p[i]);
-        u32 cnt = 0;
-        for (u32 j = j0; j < j0 + chunk; j += 16) { // sixteen entries' reads in flight, then their compares (chunk: 16, 64 or 256)
-            float4 o[4];
+// The picks of a token whose places and probabilities are in LDS, by one wave: false, with nothing stored, where two of the
+// probabilities that decide are equal (two places' entries, or entries that share a place). Weights from the chosen
+// probabilities added in pick order, as the rounds do.
+template <int PER>
+__device__ __forceinline__ bool picks_from_places(const PickLds<PER> &L, u32 t, u32 n_exp, u32 used, u32 renorm, u32 *ids, float *weights) {
+    const u32 lane = threadIdx.x & 63, s = lane < used ? lane : used - 1;
+    const u32 id = L.at[s], id_next = L.at[s + 1];
+    const bool have_next = s + 1 < n_exp;
+    const float p = L.p[id < n_exp ? id : 0], p_next = have_next ? L.p[id_next < n_exp ? id_next : 0] : -1.0f;
+    if (__ballot(id == kNoExpert || (have_next && id_next == kNoExpert) || !(p > p_next)) != 0) return false;
+    const float term = lane < used ? p : 0.0f;
+    double chosen = 0.0;
+    for (u32 i = 0; i < used; i += 8)
 #pragma unroll
-            for (int k = 0; k < 4; k++) o[k] = *reinterpret_cast<const float4 *>(&L.p[j + 4 * k]);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                cnt += (int)bm_f32_bits(o[k].x) >= ki;
-                cnt += (int)bm_f32_bits(o[k].y) >= ki;
-                cnt += (int)bm_f32_bits(o[k].z) >= ki;
-                cnt += (int)bm_f32_bits(o[k].w) >= ki;
-            }
-        }
-        if (cnt) atomicAdd(&L.ahead[i], cnt);
-    }
-    [[maybe_unused]] unsigned long long tl_cnt = 0, tl_place = 0;
-    BM_RTICK(tl_cnt, tid);
-    lds_barrier();
-    BM_RTICK(tl_place, tid);
-    BM_RTOCK(6, tl_cnt);
-    BM_RTOCK(7, tl_place);
-    if (tid < n_exp) {
-        const u32 r = L.ahead[tid] - 1; // (itself among the counted)
-        if (r < used) {
-            L.pick_id[r] = tid, L.pick_p[r] = L.p[tid];
-            atomicAdd(&L.takers[r], 1u);
-        }
-    }
-    lds_barrier();
-    if (tid >= 64) return true;
-    if (__ballot(tid < used && L.takers[tid] != 1u) != 0) return false;
-    if (tid < used) {
-        double chosen = 0.0;
-        for (u32 s0 = 0; s0 < used; s0 += 8) { // eight reads at a time, then their adds in pick order
-            const float4 a = *reinterpret_cast<const float4 *>(&L.pick_p[s0]), b = *reinterpret_cast<const float4 *>(&L.pick_p[s0 + 4]);
-            const float q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-            for (int k = 0; k < 8; k++)
-                if (s0 + k < used) chosen += (double)q[k];
-        }
-        ids[(size_t)t * used + tid] = L.pick_id[tid];
-        weights[(size_t)t * used + tid] = renorm ? L.pick_p[tid] / (float)chosen : L.pick_p[tid];
+        for (u32 k = 0; k < 8; k++) chosen += (double)bm_bits_f32((u32)__builtin_amdgcn_readlane((int)bm_f32_bits(term), (int)(i + k)));
+    if (lane < used) {
+        ids[(size_t)t * used + lane] = id;
+        weights[(size_t)t * used + lane] = renorm ? p / (float)chosen : p;
     }
     return true;
 }
+
+// A barrier that waits for the wave's LDS traffic only: the routing workgroup's waves meet over LDS while stores to memory are
+// still on their way, and a barrier that waited for those to be acknowledged cost the routing 1 us.
+__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // One wave a token.
 template <int PER>
 __global__ __launch_bounds__(256) void k_route_softmax(const float *logits, u32 n_tok, u32 n_exp, u32 used, u32 renorm,
                                                        float *probs, u32 *ids, float *weights, u32 *fault, u32 layer) {
-    const u32 t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    __shared__ PickLds<PER> s_pick[4];
+    const u32 wave = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), t = blockIdx.x * 4 + wave;
     if (t >= n_tok) return; // whole waves leave
-    float v[PER];
+    PickLds<PER> &L = s_pick[wave];
+    float v[PER], p[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const u32 e = (threadIdx.x & 63) + 64 * j;
         v[j] = e < n_exp ? logits[(size_t)t * n_exp + e] : -INFINITY;
     }
-    route_softmax_wave<PER>(v, t, n_exp, used, renorm, probs, ids, weights, fault, layer);
+    if (!logits_finite<PER>(v, n_exp)) return route_refuse(t, n_exp, used, probs, weights, fault, layer);
+    places_clear(L);
+    route_probs_wave<PER>(v, n_exp, p);
+    store_probs<PER>(p, t, n_exp, probs);
+#pragma unroll
+    for (int j = 0; j < PER; j++) L.p[(threadIdx.x & 63) + 64 * j] = p[j];
+    places_by_counting<PER>(p, n_exp, used, L);
+    if (!picks_from_places(L, t, n_exp, used, renorm, ids, weights)) route_pick_rounds<PER>(p, t, n_exp, used, renorm, ids, weights);
 }
 
 hipError_t route_softmax(const Launch &L, const float *logits, int n_tok, int n_exp, int used, int renorm, float *probs,
@@ -291,10 +340,18 @@ hipError_t route_softmax(const Launch &L, const float *logits, int n_tok, int n_
 // crates/qdot/src/lib.rs:11349-11386: eight lane accumulators (a product, then fused multiply-adds in increasing k) and
 // (l0 + l4 + l2 + l6) + (l1 + l5 + l3 + l7).
 //
-// A workgroup takes one token and R router rows: the token's row is normed into LDS by all 256 threads while the rows'
-// bytes arrive (both requested at once), then eight lanes a row walk it, lane l the accumulator l.
-// Floats a line of the accumulator-major LDS rows.
-__host__ __device__ inline int router_line(int hidden) { return ((hidden / 8 + 3) & ~3) + 8; }
+// A workgroup takes T tokens and R router rows: the tokens' rows are normed into LDS by all 256 threads, then a wave takes a row.
+//
+// A row dot is eight chains of hidden / 8 fused multiply-adds, serial by the order's definition: a chain's steps cost 6 cycles each
+// when their operands stand in registers, and what they cost more than that is the operands' way there (eight lanes a row,
+// reading four steps at a time from LDS: 11 cycles a step, and the rows had to be laid out accumulator-major for it). So a row is
+// spread over the whole wave: lane 8 l + s holds the 32 operands of accumulator l in super-block s of eight (256 values, 32 steps),
+// read by one instruction a step for all the lanes - the router's row from memory, eight lanes of which are 32 consecutive bytes,
+// the token's from LDS, whose super-blocks stand eight floats more than their length apart so that a wave's 64 words fall on 64
+// banks. Then the chains run super-block by super-block: every lane does its 32 steps, only the lanes of the chains' present place
+// with a meaning, and a move to the next lane hands the accumulators on.
+constexpr int kRouterSb = 256 + 8; // floats from one super-block of a token's row in LDS to the next
+__host__ __device__ inline int router_line(int hidden) { return (hidden + 255) / 256 * kRouterSb; }
 
 // (k_norm_route's arguments: what the head of a logits workgroup needs stands in the first fourteen words, which are in registers when a
 // wave starts - m_word is the token count, bit 31 set where the quantized column is asked for - and the rest travels as one
@@ -321,234 +378,273 @@ struct NormRouteArgs { // k_norm_route's argument block
 };
 static_assert(offsetof(NormRouteArgs, late) == 56, "fourteen words in front of the late arguments");
 
-// t: the token; e0: the first of the workgroup's R router rows, or -1 for a workgroup that only norms the token's row into LDS
-// (k_norm_route's quantizer workgroups): no router rows, no logits.
-template <int R, bool COH = false>
-__device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *router, const float *x, const float *gain, float eps,
-                                                   int n_exp, int hidden, float *normed_out, float *logits, int t, int e0) {
-    // The token's row and the R router rows lie accumulator-major in LDS: value k at line k % 8, place k / 8, so that the
-    // lane that owns accumulator l reads four consecutive steps' operands as 16 bytes. A line is hidden / 8 floats, rounded up
-    // to whole 16 bytes, + 8 (the eight lines of a row 8 banks apart), a router row four floats past the one before (rows r
-    // and r + 1 on different banks).
-    const int line = router_line(hidden), wrow_floats = 8 * line + 4;
-    float *xs = reinterpret_cast<float *>(lds);  // [8][line]
-    float *ws = xs + 8 * line;                   // [R][8][line] (+ 4 a row)
-    auto put4 = [&](float *base, int c, const float4 v) { // the four values 4 c .. 4 c + 3 of a row
-        float *at = base + (4 * (c & 1)) * line + (c >> 1);
-        at[0] = v.x, at[line] = v.y, at[2 * line] = v.z, at[3 * line] = v.w;
+// The norm of T rows (of tokens t0 .., the last token's where there are fewer: its numbers again) into LDS, row after row of
+// router_line(hidden) floats, without a barrier behind it; and to normed_out where that is wanted. Without a gain the rows as they are. N4: 16-byte
+// pieces of a row a thread holds in registers (rows of up to 1024 N4 values); 0: rows of any length, through LDS. `behind_requests` is
+// called when the rows have been asked for, `behind_sums` when their squares are summed.
+template <int T, int N4, class F, class G>
+__device__ __forceinline__ void norm_rows(float *xs, double (*s_part)[4], const float *x, const float *gain, float eps, int hidden, float *normed_out,
+                                          int t0, int m, F behind_requests, G behind_sums) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n4 = hidden / 4, line = router_line(hidden);
+    auto in_lds = [&](int tt, int i) { return reinterpret_cast<float4 *>(xs + tt * line + 4 * i + 8 * (i >> 6)); };
+    auto row = [&](int tt) { return (size_t)(t0 + tt < m ? t0 + tt : m - 1) * hidden; };
+    auto squares = [](double &sum, const float4 v) {
+        sum += (double)__fmul_rn(v.x, v.x);
+        sum += (double)__fmul_rn(v.y, v.y);
+        sum += (double)__fmul_rn(v.z, v.z);
+        sum += (double)__fmul_rn(v.w, v.w);
     };
-    __shared__ double s_part[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    [[maybe_unused]] unsigned long long tl_start = 0, tl_row = 0, tl_norm = 0, tl_lds = 0, tl_dots = 0;
-    BM_RTICK(tl_start, tid);
-    const float *xt = x + (size_t)t * hidden;
-    // the rows' bytes on their way first: they do not depend on the norm. Eight 16-byte loads a thread are asked for together
-    // and go to LDS once the token's row has been asked for too and normed
-    const int n4 = hidden / 4;
-    // A thread's pieces of the R rows: row 0's pieces tid, tid + 256, ..., then row 1's, ...: piece n of the thread is (row, place)
-    // by counting on, no division by a length only known at run time in front of the first request.
-    constexpr int kBatch = 8;
-    float4 rv[kBatch];
-    struct Piece {
-        int r, c;
+    auto normed = [](float scale, const float4 g, const float4 v) {
+        return make_float4(__fmul_rn(__fmul_rn(scale, g.x), v.x), __fmul_rn(__fmul_rn(scale, g.y), v.y), __fmul_rn(__fmul_rn(scale, g.z), v.z),
+                           __fmul_rn(__fmul_rn(scale, g.w), v.w));
     };
-    const int rows_here = e0 >= 0 ? R : 0;
-    auto step = [&](Piece &p) {
-        p.c += 256;
-        if (p.c >= n4) p.r++, p.c = tid;
+    auto put = [&](int tt, int i, const float4 v) {
+        *in_lds(tt, i) = v;
+        if (normed_out && t0 + tt < m) reinterpret_cast<float4 *>(normed_out + row(tt))[i] = v;
     };
-    const Piece first = {tid < n4 ? 0 : rows_here, tid};
-    auto ask = [&](Piece p) { // asks for the next kBatch pieces from p on; returns the piece behind them
+    constexpr int kRegs = N4 ? N4 : 1;
+    [[maybe_unused]] float4 xv[T][kRegs], gv[kRegs];
+    [[maybe_unused]] unsigned long long tl_row = 0, tl_norm = 0;
+    double sum[T];
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            if (p.r < rows_here) {
-                const int e = e0 + p.r < n_exp ? e0 + p.r : n_exp - 1;
-                rv[u] = reinterpret_cast<const float4 *>(router + (size_t)e * hidden)[p.c];
-                step(p);
-            }
-        }
-        return p;
-    };
-    auto park = [&](Piece p) {
+    for (int tt = 0; tt < T; tt++) sum[tt] = 0.0;
+    if constexpr (N4 != 0) {
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            if (p.r < rows_here) {
-                put4(ws + (size_t)p.r * wrow_floats, p.c, rv[u]);
-                step(p);
-            }
-        }
-        return p;
-    };
-    ask(first);
-    double sum = 0.0;
-    constexpr int kInRegs = 8; // float4s of the row a thread can hold: rows of up to 8192 values stay in registers
-    if (gain && n4 <= 256 * kInRegs) {
-        // the row and the gain requested together and kept in registers: one pass, no second wait on memory
-        float4 xv[kInRegs], gv[kInRegs];
+        for (int tt = 0; tt < T; tt++)
 #pragma unroll
-        for (int j = 0; j < kInRegs; j++) {
-            const int i = tid + 256 * j;
-            if (i < n4) {
-                xv[j] = reinterpret_cast<const float4 *>(xt)[i];
-                gv[j] = reinterpret_cast<const float4 *>(gain)[i];
-            }
-        }
+            for (int j = 0; j < N4; j++)
+                if (tid + 256 * j < n4) xv[tt][j] = reinterpret_cast<const float4 *>(x + row(tt))[tid + 256 * j];
+        if (gain)
 #pragma unroll
-        for (int j = 0; j < kInRegs; j++)
-            if (tid + 256 * j < n4) {
-                sum += (double)__fmul_rn(xv[j].x, xv[j].x);
-                sum += (double)__fmul_rn(xv[j].y, xv[j].y);
-                sum += (double)__fmul_rn(xv[j].z, xv[j].z);
-                sum += (double)__fmul_rn(xv[j].w, xv[j].w);
-            }
-        BM_RTICK(tl_row, sum);
-        sum = wave_sum_f64(sum);
-        if (lane == 0) s_part[wave] = sum;
-        __syncthreads();
-        const double total = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
-        const float mean = (float)(total / (double)hidden);
-        const float scale = __fdiv_rn(1.0f, bm_sqrt_rn(__fadd_rn(mean, eps)));
-        BM_RTICK(tl_norm, scale);
+            for (int j = 0; j < N4; j++)
+                if (tid + 256 * j < n4) gv[j] = reinterpret_cast<const float4 *>(gain)[tid + 256 * j];
+        behind_requests();
+        if (gain)
 #pragma unroll
-        for (int j = 0; j < kInRegs; j++) {
-            const int i = tid + 256 * j;
-            if (i < n4) {
-                const float4 v = make_float4(__fmul_rn(__fmul_rn(scale, gv[j].x), xv[j].x), __fmul_rn(__fmul_rn(scale, gv[j].y), xv[j].y),
-                                             __fmul_rn(__fmul_rn(scale, gv[j].z), xv[j].z), __fmul_rn(__fmul_rn(scale, gv[j].w), xv[j].w));
-                put4(xs, i, v);
-                if (normed_out && e0 <= 0) reinterpret_cast<float4 *>(normed_out + (size_t)t * hidden)[i] = v;
-            }
-        }
+            for (int tt = 0; tt < T; tt++)
+#pragma unroll
+                for (int j = 0; j < N4; j++)
+                    if (tid + 256 * j < n4) squares(sum[tt], xv[tt][j]);
     } else {
-        for (int i = tid; i < n4; i += 256) {
-            const float4 v = reinterpret_cast<const float4 *>(xt)[i];
-            put4(xs, i, v);
-            if (gain) {
-                sum += (double)__fmul_rn(v.x, v.x);
-                sum += (double)__fmul_rn(v.y, v.y);
-                sum += (double)__fmul_rn(v.z, v.z);
-                sum += (double)__fmul_rn(v.w, v.w);
+        behind_requests();
+        for (int tt = 0; tt < T; tt++)
+            for (int i = tid; i < n4; i += 256) {
+                const float4 v = reinterpret_cast<const float4 *>(x + row(tt))[i];
+                if (gain) {
+                    *in_lds(tt, i) = v;
+                    squares(sum[tt], v);
+                } else {
+                    put(tt, i, v);
+                }
+            }
+        // the steps past a row's end, to a whole super-block: -0, which times +0 leaves a chain as it is
+        for (int tt = 0; tt < T; tt++)
+            for (int k = hidden + tid; k < (hidden + 255) / 256 * 256; k += 256) xs[tt * line + k + 8 * (k >> 8)] = -0.0f;
+    }
+    BM_RTICK(tl_row, sum[0]);
+    BM_RTOCK(1, tl_row);
+    if (!gain) {
+        behind_sums();
+        if constexpr (N4 != 0)
+#pragma unroll
+            for (int tt = 0; tt < T; tt++)
+#pragma unroll
+                for (int j = 0; j < N4; j++)
+                    if (tid + 256 * j < n4) put(tt, tid + 256 * j, xv[tt][j]);
+        return;
+    }
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+        sum[tt] = wave_sum_f64(sum[tt]);
+        if (lane == 0) s_part[tt][wave] = sum[tt];
+    }
+    lds_barrier();
+    double part[T][4];
+#pragma unroll
+    for (int tt = 0; tt < T; tt++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) part[tt][k] = s_part[tt][k];
+    behind_sums();
+    float scale[T];
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+        const double total = (part[tt][0] + part[tt][1]) + (part[tt][2] + part[tt][3]);
+        const float mean = (float)(total / (double)hidden);
+        scale[tt] = __fdiv_rn(1.0f, bm_sqrt_rn(__fadd_rn(mean, eps)));
+    }
+    BM_RTICK(tl_norm, scale[0]);
+    BM_RTOCK(2, tl_norm);
+    if constexpr (N4 != 0) {
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+#pragma unroll
+            for (int j = 0; j < N4; j++)
+                if (tid + 256 * j < n4) put(tt, tid + 256 * j, normed(scale[tt], gv[j], xv[tt][j]));
+    } else {
+        for (int tt = 0; tt < T; tt++)
+            for (int i = tid; i < n4; i += 256) // (a thread's own pieces)
+                put(tt, i, normed(scale[tt], reinterpret_cast<const float4 *>(gain)[i], *in_lds(tt, i)));
+    }
+}
+
+// The logits of tokens t0 .. t0 + T - 1 against router rows e0 .. e0 + R - 1. A wave takes one row and all the
+// tokens, whose chains run side by side. N4: see norm_rows; 0 takes a hidden that is not whole super-blocks too.
+template <int R, int T, int N4, bool COH>
+__device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *router, const float *x, const float *gain, float eps, int n_exp,
+                                                   int hidden, int m, float *normed_out, float *logits, int t0, int e0) {
+    static_assert((R == 1 && T == 1) || R == 4, "a wave takes one row, and all the tokens");
+    float *const xs = reinterpret_cast<float *>(lds);
+    __shared__ double s_part[T][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    [[maybe_unused]] unsigned long long tl_start = 0, tl_lds = 0, tl_dots = 0;
+    BM_RTICK(tl_start, tid);
+    BM_RTOCK(0, tl_start);
+    const int r = wave; // the wave's row
+    const bool has_dot = wave < R;
+    const int acc_l = lane >> 3, sb_l = lane & 7, line = router_line(hidden), sbs = (hidden + 255) / 256, passes = (sbs + 7) / 8;
+    const float *const wrow = router + (size_t)(e0 + r < n_exp ? e0 + r : n_exp - 1) * hidden;
+    struct Row { // a lane's operands of a pass
+        float w[32], x[T][32];
+    };
+    // The router's row comes in whole lines, a super-block an instruction, and goes through the wave's own eight super-blocks of LDS:
+    // asked for straight into the lanes that use it, 32 bytes here and there, it kept the address unit busy for 33 cycles an instruction.
+    float4 *const ws = reinterpret_cast<float4 *>(xs + T * line + wave * (8 * kRouterSb));
+    v4f raw[8];
+    auto ask = [&](int q) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int sb = 8 * q + i < sbs ? 8 * q + i : sbs - 1, at = 256 * sb + 4 * lane; // (past the row's end: its last, for no reader)
+            if constexpr (N4 != 0) {
+                raw[i] = *reinterpret_cast<const v4f *>(wrow + at);
+            } else {
+                const bool in = at < hidden;
+                raw[i] = *reinterpret_cast<const v4f *>(wrow + (in ? at : hidden - 4));
+                if (!in) raw[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
             }
         }
-        if (gain) {
-            sum = wave_sum_f64(sum);
-            if (lane == 0) s_part[wave] = sum;
-            __syncthreads();
-            const double total = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
-            const float mean = (float)(total / (double)hidden);
-            const float scale = __fdiv_rn(1.0f, bm_sqrt_rn(__fadd_rn(mean, eps)));
-            for (int i = tid; i < hidden; i += 256) {
-                float *at = xs + (i & 7) * line + (i >> 3);
-                const float v = __fmul_rn(__fmul_rn(scale, gain[i]), *at); // written before the barrier above
-                *at = v;
-                if (normed_out && e0 <= 0) normed_out[(size_t)t * hidden + i] = v;
-            }
-        }
-    }
-    Piece parked = park(first);
-    while (parked.r < rows_here) { // (no barrier inside: a thread with fewer pieces leaves earlier)
-        ask(parked);
-        parked = park(parked);
-    }
-    __syncthreads();
+    };
+    auto park = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) *reinterpret_cast<v4f *>(ws + (kRouterSb / 4) * i + lane) = raw[i];
+        lds_of_wave();
+    };
+    auto read_row = [&](Row &o) __attribute__((always_inline)) {
+        const float *const from = reinterpret_cast<const float *>(ws) + kRouterSb * sb_l + acc_l;
+#pragma unroll
+        for (int j = 0; j < 32; j++) o.w[j] = from[8 * j];
+        lds_of_wave();
+    };
+    auto read_token = [&](Row &o, int q) __attribute__((always_inline)) {
+        const int sb = 8 * q + sb_l < sbs ? 8 * q + sb_l : sbs - 1;
+        const float *const from = xs + kRouterSb * sb + acc_l;
+#pragma unroll
+        for (int tt = 0; tt < T; tt++)
+#pragma unroll
+            for (int j = 0; j < 32; j++) o.x[tt][j] = from[tt * line + 8 * j];
+    };
+    Row a, b;
+    norm_rows<T, N4>(xs, s_part, x, gain, eps, hidden, e0 == 0 ? normed_out : nullptr, t0, m, [&]() __attribute__((always_inline)) {
+        if (has_dot) ask(0);
+    }, [&]() __attribute__((always_inline)) {
+        if (!has_dot) return;
+        park();
+        if (passes > 1) ask(1);
+        read_row(a);
+    });
+    lds_barrier();
     BM_RTICK(tl_lds, tid);
+    BM_RTOCK(3, tl_lds);
+    if (!has_dot) return;
     // (k_norm_route's hand-over words: an argument behind the preloaded ones, read here, where its way through memory runs under
     // the dots)
     [[maybe_unused]] u32 *hand = nullptr;
     if constexpr (COH) hand = bm_global(bm_kernarg_at<u32 *>(offsetof(NormRouteArgs, late) + offsetof(NormRouteLate, hand)));
-    if (!gain && normed_out && e0 <= 0) // the rows as they are (read after the barrier: other threads staged them)
-        for (int i = tid; i < hidden; i += 256) normed_out[(size_t)t * hidden + i] = xs[(i & 7) * line + (i >> 3)];
-    // every thread that stores a logit below is of the first wave: k_norm_route's hand-over (a device-scope count updated by
-    // thread 0 behind the workgroup's barrier) publishes that wave's stores and relies on it
-    static_assert(8 * R <= 64, "the logits of a workgroup are stored by its first wave");
-    if (e0 >= 0 && tid < 8 * R) {
-        const int r = tid >> 3, l = tid & 7;
-        const float4 *xl = reinterpret_cast<const float4 *>(xs + l * line);
-        const float4 *wl = reinterpret_cast<const float4 *>(ws + (size_t)r * wrow_floats + l * line);
-        // the chain is serial by the order's definition (a product, then fused multiply-adds in increasing k); the reads
-        // are not: sixteen steps' operands, four 16-byte reads a side, a batch
-        const float *xf = xs + l * line, *wf = ws + (size_t)r * wrow_floats + l * line;
-        const int steps = hidden / 8;
-        float acc = __fmul_rn(xf[0], wf[0]);
-        int i = 1;
-        for (; i < 4 && i < steps; i++) acc = fmaf(xf[i], wf[i], acc);
-        auto rd = [&](float4(&a)[4], float4(&b)[4], int at) {
+    float acc[T];
 #pragma unroll
-            for (int u = 0; u < 4; u++) a[u] = xl[at / 4 + u], b[u] = wl[at / 4 + u];
-        };
-        auto chain = [&](const float4(&a)[4], const float4(&b)[4]) {
+    for (int tt = 0; tt < T; tt++) acc[tt] = -0.0f; // (a first product keeps its own sign of zero, as the product that starts the chain does)
+    auto steps = [&](const Row &o) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                acc = fmaf(a[u].x, b[u].x, acc), acc = fmaf(a[u].y, b[u].y, acc);
-                acc = fmaf(a[u].z, b[u].z, acc), acc = fmaf(a[u].w, b[u].w, acc);
-            }
-        };
-        if (i + 16 <= steps) {
-            // two batches a turn in two sets of registers: a batch's operands are read while the batch before runs its chain
-            float4 a0[4], b0[4], a1[4], b1[4];
-            rd(a0, b0, i);
-            for (; i + 48 <= steps; i += 32) {
-                rd(a1, b1, i + 16);
-                __builtin_amdgcn_sched_barrier(0);
-                chain(a0, b0);
-                __builtin_amdgcn_sched_barrier(0);
-                rd(a0, b0, i + 32);
-                __builtin_amdgcn_sched_barrier(0);
-                chain(a1, b1);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            chain(a0, b0);
-            i += 16;
-            for (; i + 16 <= steps; i += 16) {
-                rd(a0, b0, i);
-                chain(a0, b0);
-            }
+        for (int j = 0; j < 32; j++)
+#pragma unroll
+            for (int tt = 0; tt < T; tt++) acc[tt] = fmaf(o.x[tt][j], o.w[j], acc[tt]);
+    };
+    auto pass = [&](const Row &o, int q, auto behind_first) __attribute__((always_inline)) {
+        if (q > 0)
+#pragma unroll
+            for (int tt = 0; tt < T; tt++) acc[tt] = bm_dppf<kDppShl7>(acc[tt]); // from the eighth super-block's lanes to the first's
+        steps(o);
+        behind_first();
+        const int here = sbs - 8 * q < 8 ? sbs - 8 * q : 8;
+#pragma nounroll
+        for (int sb = 1; sb < here; sb++) {
+#pragma unroll
+            for (int tt = 0; tt < T; tt++) acc[tt] = bm_dppf<kDppShr1>(acc[tt]);
+            steps(o);
         }
-        for (; i < steps; i++) acc = fmaf(xf[i], wf[i], acc);
-        // s_l = acc_l + acc_{l+4} on lanes 0..3 of the row's eight, then (s0 + s2) + (s1 + s3)
-        // (lane i reads lane i + n of its sixteen: right for the lanes of the eight whose value is used)
-        const float s = __fadd_rn(acc, bm_dppf<kDppShl4>(acc));
-        const float pair = __fadd_rn(s, bm_dppf<kDppShl2>(s)); // lane 0: s0 + s2, lane 1: s1 + s3
-        const float out = __fadd_rn(pair, bm_dppf<kDppShl1>(pair));
+    };
+    read_token(a, 0);
+    // two sets of operands: a pass's are read, and the bytes of the one after it asked for, while the pass before runs
+    auto prepare = [&](Row &o, int q) __attribute__((always_inline)) {
+        park();
+        if (q + 1 < passes) ask(q + 1);
+        read_row(o);
+        read_token(o, q);
+    };
+    // (behind the pass's first super-block: the counter of LDS reads on their way ends at fifteen, and a wait for the pass's own in
+    // front of its first step would be one for the next pass's)
+    for (int q = 0;; q += 2) {
+        pass(a, q, [&]() __attribute__((always_inline)) {
+            if (q + 1 < passes) prepare(b, q + 1);
+        });
+        if (q + 1 >= passes) break;
+        pass(b, q + 1, [&]() __attribute__((always_inline)) {
+            if (q + 2 < passes) prepare(a, q + 2);
+        });
+        if (q + 2 >= passes) break;
+    }
+    // s_l = acc_l + acc_{l+4}, then (s0 + s2) + (s1 + s3): accumulators 4 apart stand a half of the wave apart, 2 apart a row of
+    // sixteen, neighbours eight lanes
+    const int last = (sbs - 1) & 7; // the lanes of the last super-block hold the sums
+#pragma unroll
+    for (int tt = 0; tt < T; tt++) {
+        const Pair32 h = halves(bm_f32_bits(acc[tt]));
+        const float s = __fadd_rn(bm_bits_f32(h.a), bm_bits_f32(h.b));
+        const Pair32 q = rows_of_half(bm_f32_bits(s));
+        const float pair = __fadd_rn(bm_bits_f32(q.a), bm_bits_f32(q.b));
+        const float out = __fadd_rn(pair, bm_dppf<kDppShl8>(pair));
         BM_RTICK(tl_dots, out);
-        if (l == 0 && e0 + r < n_exp) {
-            logits[(size_t)t * n_exp + e0 + r] = out;
+        const int t = t0 + tt;
+        if (lane == last && e0 + r < n_exp && t < m) {
             // k_norm_route's hand-over: the logit as a device-scope store of its own, into a word that held the armed pattern
             if constexpr (COH) __hip_atomic_store(hand + (size_t)t * n_exp + e0 + r, bm_f32_bits(out), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            logits[(size_t)t * n_exp + e0 + r] = out;
         }
     }
-    BM_RTOCK(0, tl_start);
-    BM_RTOCK(1, tl_row);
-    BM_RTOCK(2, tl_norm);
-    BM_RTOCK(3, tl_lds);
     BM_RTOCK(4, tl_dots);
 }
 
-template <int R>
-__global__ __launch_bounds__(256) void k_router_logits(const float *router, const float *x, const float *gain, float eps,
-                                                       int n_exp, int hidden, float *normed_out, float *logits) {
+template <int R, int T, int N4>
+__global__ __launch_bounds__(256) void k_router_logits(const float *router, const float *x, const float *gain, float eps, int n_exp, int hidden, int m,
+                                                       float *normed_out, float *logits) {
     extern __shared__ __align__(16) uint8_t lds[];
-    const int blocks_per_token = (n_exp + R - 1) / R;
-    router_logits_body<R>(lds, router, x, gain, eps, n_exp, hidden, normed_out, logits, blockIdx.x / blocks_per_token,
-                          (blockIdx.x % blocks_per_token) * R);
+    const int row_blocks = (n_exp + R - 1) / R;
+    router_logits_body<R, T, N4, false>(lds, router, x, gain, eps, n_exp, hidden, m, normed_out, logits, (int)(blockIdx.x / row_blocks) * T,
+                                        (int)(blockIdx.x % row_blocks) * R);
 }
 
-// A normed row as router_logits_body leaves it in LDS (value k at line k % 8, place k / 8) into column t of act_x.
+// A normed row as norm_rows leaves it in LDS into column t of act_x.
 __device__ __forceinline__ void quant_normed_row(const float *xs, int hidden, int t, uint8_t *act_x, int q8k, u32 *fault, u32 layer) {
-    const int line = router_line(hidden), nb = hidden / 256, tid = threadIdx.x;
+    const int nb = hidden / 256, tid = threadIdx.x;
     if (q8k) {
         uint8_t *col = act_x + (size_t)t * nb * BM_Q8K_STRIDE;
-        for (int b = tid >> 6; b < nb; b += 4) { // a wave a 256-value block, four consecutive values a lane
-            const int k = 256 * b + 4 * (tid & 63);
-            const float *at = xs + (k & 7) * line + (k >> 3);
-            q8k_wave_block(make_float4(at[0], at[line], at[2 * line], at[3 * line]), col + (size_t)b * BM_Q8K_STRIDE, tid & 63, fault, layer);
-        }
+        for (int b = tid >> 6; b < nb; b += 4) // a wave a 256-value block, four consecutive values a lane
+            q8k_wave_block(*reinterpret_cast<const float4 *>(xs + kRouterSb * b + 4 * (tid & 63)), col + (size_t)b * BM_Q8K_STRIDE, tid & 63, fault, layer);
     } else {
         uint8_t *col = act_x + (size_t)t * nb * BM_Q82_SB_EXT;
         for (int k = 8 * tid; k < hidden; k += 2048) { // a quad of lanes a 32-value block, eight consecutive values a lane
-            float v8[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) v8[j] = xs[j * line + (k >> 3)];
+            const float4 *at = reinterpret_cast<const float4 *>(xs + k + 8 * (k >> 8));
+            const float4 lo = at[0], hi = at[1];
+            const float v8[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
             q82_quad8(v8, col, nb, k >> 5, tid & 3, fault, layer);
         }
     }
@@ -556,13 +652,15 @@ __device__ __forceinline__ void quant_normed_row(const float *xs, int hidden, in
 
 // Norm, logits and routing in one launch (crates/gpu/src/route_softmax.rs:1667-1674 enqueue_norm_fused; the quantizer of
 // that launch is an option here, see below). The workgroups are k_router_logits's, and behind them in the grid one more a
-// token, whose first wave routes it with k_route_softmax's numbers. The hand-over is one trip through memory: `hand` holds a
+// token, which routes it with k_route_softmax's numbers. The hand-over is one trip through memory: `hand` holds a
 // word a (token, expert) that is armed between launches - kRouteArmed, a signalling NaN pattern, which no arithmetic
 // leaves behind (an operation on it gives the quiet form) - each logit is stored over its word with a device-scope store as
-// soon as it is formed, and the routing wave reads its words with device-scope loads until none is armed, so it has the
-// logits the moment the last one lands: no acknowledgement is waited for, no count is kept, nothing is read back (the form
-// before, a count raised behind acknowledged stores by the last workgroup to finish, which then read the logits back: 10.3
-// us a token against this one's figure in the bench line). The wave arms its words again before it ends, so a graph replay
+// soon as it is formed, and the routing waves read their words with device-scope loads until none is armed, so they have the
+// logits the moment the last one lands: no acknowledgement is waited for, no count is kept, nothing is read back (a count
+// raised behind acknowledged stores by the last workgroup to finish, which then read the logits back, took 2.3 us longer). Two polls are on
+// their way at once (5.5 us a token against 5.7 with one, 5.75 with four). Two waves have the logits: the first forms the probabilities
+// while the second finds the places - by the logits, whose order the probabilities have but where two of them round to the same
+// value, which picks_from_places sees - and the first picks. It arms the words again before it ends, so a graph replay
 // needs no memset. A routing workgroup comes after every workgroup it waits for in the grid, so those are dispatched
 // whatever else the card runs; the wait is bounded all the same (max_polls polls, kRoutePolls = 2^24 or some ten seconds unless the caller says otherwise - an XCD busy with another stream's work may hold some of them back for
 // a while - then BM_SITE_ROUTER and NaN weights), and
@@ -570,78 +668,97 @@ __device__ __forceinline__ void quant_normed_row(const float *xs, int hidden, in
 // With act_x (the reference launch's quantizer, route_softmax.rs:1679): one more workgroup a token, between the two kinds in
 // the grid, norms the token's row the same way and leaves it as the token's quantized column (q8k: a Q8_K column, else a
 // Q8_2_X4 one with its tables), the bytes bm_quantize makes of normed_out. The routing waits for none of it.
-template <int R, int PER>
+// Latency: 1 token x 128 experts x 2048 values 7.9 -> 5.5 us a launch (us after its start: row arrived 0.6, normed 1.2, in LDS 1.4, dots done
+// 2.3 - 2.4, logits held 3.5, routed 4.6; before: 0.9, 1.25, 1.9, 3.5 - 4.0, 5.0, 7.1), 16 tokens 11.0 -> 7.7, 4 tokens x 256 x 7168 22.1 -> 10.9.
+template <int R, int T, int N4, int PER>
 __global__ __launch_bounds__(256) void k_norm_route(const float *router, const float *x, const float *gain, float eps, int n_exp,
                                                     int hidden, u32 m_word, float *normed_out, float *logits, NormRouteLate) {
     extern __shared__ __align__(16) uint8_t lds[];
-    const u32 blocks_per_token = (u32)((n_exp + R - 1) / R);
+    const u32 row_blocks = (u32)((n_exp + R - 1) / R);
     const u32 m = m_word & 0x7fffffffu;
-    const u32 n_logit_blocks = m * blocks_per_token, n_quant_blocks = (m_word >> 31) ? m : 0u;
-    if (blockIdx.x >= n_logit_blocks + n_quant_blocks) { // a routing workgroup: its first wave takes the logits
-        __shared__ PickLds pick;
-        const u32 t = blockIdx.x - n_logit_blocks - n_quant_blocks, lane = threadIdx.x;
+    const u32 n_logit_blocks = (m + T - 1) / T * row_blocks, n_quant_blocks = (m_word >> 31) ? m : 0u;
+    if (blockIdx.x >= n_logit_blocks + n_quant_blocks) { // a routing workgroup: two waves of it
+        const u32 wave = (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        if (wave > 1) return;
+        __shared__ PickLds<PER> pick;
+        const u32 t = blockIdx.x - n_logit_blocks - n_quant_blocks, lane = threadIdx.x & 63;
         const NormRouteLate late = bm_kernarg_at<NormRouteLate>(offsetof(NormRouteArgs, late));
         const u32 used = late.used, renorm = late.renorm, layer = late.layer, max_polls = late.max_polls;
         float *const probs = bm_global(late.probs), *const weights = bm_global(late.weights);
         u32 *const ids = bm_global(late.ids), *const hand = bm_global(late.hand), *const fault = bm_global(late.fault);
-        constexpr bool kRanks = PER <= 4; // up to 256 experts: the picks by the whole workgroup
-        if constexpr (kRanks) {
-            pick.p[threadIdx.x] = -1.0f, pick.ahead[threadIdx.x] = 0;
-            if (threadIdx.x < 32) pick.takers[threadIdx.x] = 0;
-            lds_barrier();
-        } else {
-            if (threadIdx.x >= 64) return;
-        }
-        [[maybe_unused]] float p[PER];
-        if (threadIdx.x < 64) {
-            u32 *mine = hand + (size_t)t * n_exp;
-            [[maybe_unused]] unsigned long long tl_start = 0, tl_seen = 0;
-            BM_RTICK(tl_start, lane);
-            u32 w[PER];
-            bool late = true;
-            for (u32 spin = 0; spin < max_polls && late; spin++) {
-                bool armed = false;
-#pragma unroll
-                for (int j = 0; j < PER; j++) {
-                    const u32 e = lane + 64 * j;
-                    w[j] = e < (u32)n_exp ? __hip_atomic_load(mine + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-                    armed |= w[j] == kRouteArmed;
-                }
-                late = __ballot(armed) != 0;
-            }
-            BM_RTICK(tl_seen, w[0]);
-            BM_RTOCK(0, tl_start);
-            BM_RTOCK(4, tl_seen);
-            float v[PER];
+        u32 *const mine = hand + (size_t)t * n_exp;
+        if (wave == 1) places_clear(pick);
+        [[maybe_unused]] unsigned long long tl_start = 0, tl_seen = 0, tl_places = 0, tl_routed = 0;
+        BM_RTICK(tl_start, lane);
+        // (several polls on their way at once, spread over the time one takes: the logits are seen that much sooner after they are there)
+        constexpr int kPolls = 2;
+        u32 w[kPolls][PER];
+        auto poll = [&](u32(&o)[PER]) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < PER; j++) {
                 const u32 e = lane + 64 * j;
-                // (a word still armed after the last poll: the NaN it is, which the routing refuses as it refuses any)
-                v[j] = e < (u32)n_exp ? bm_bits_f32(w[j]) : -INFINITY;
-                if (e < (u32)n_exp) __hip_atomic_store(mine + e, kRouteArmed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                o[j] = e < (u32)n_exp ? __hip_atomic_load(mine + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
             }
-            if constexpr (!kRanks) route_softmax_wave<PER>(v, t, (u32)n_exp, used, renorm, probs, ids, weights, fault, layer);
-            if constexpr (kRanks) {
-                const bool ok = route_probs_wave<PER>(v, t, (u32)n_exp, used, probs, weights, fault, layer, p);
-                if (lane == 0) pick.ok = ok;
+        };
+        u32 got[PER];
+        bool waiting = true;
 #pragma unroll
-                for (int j = 0; j < PER; j++)
-                    if (ok && lane + 64 * j < (u32)n_exp) pick.p[lane + 64 * j] = p[j];
+        for (int k = 0; k < kPolls; k++) {
+            poll(w[k]);
+            __builtin_amdgcn_s_sleep(4);
+        }
+        for (u32 spin = 0; waiting; spin += kPolls) {
+#pragma unroll
+            for (int k = 0; k < kPolls; k++) {
+                bool armed = false;
+#pragma unroll
+                for (int j = 0; j < PER; j++) {
+                    got[j] = w[k][j];
+                    armed |= got[j] == kRouteArmed;
+                }
+                waiting = __ballot(armed) != 0 && spin + k + 1 < max_polls;
+                if (!waiting) break;
+                poll(w[k]);
             }
         }
-        if constexpr (kRanks) {
-            lds_barrier();
-            if (pick.ok && !route_pick_ranks(pick, t, (u32)n_exp, used, renorm, ids, weights))
-                route_pick_rounds<PER>(p, t, (u32)n_exp, used, renorm, ids, weights); // (the first wave, which holds p)
+        BM_RTICK(tl_seen, got[0]);
+        float v[PER], p[PER];
+#pragma unroll
+        for (int j = 0; j < PER; j++) // (a word still armed after the last poll: the NaN it is, which is refused as any is)
+            v[j] = lane + 64 * j < (u32)n_exp ? bm_bits_f32(got[j]) : -INFINITY;
+        const bool finite = logits_finite<PER>(v, (u32)n_exp);
+        if (wave == 1) {
+            if (finite) places_by_counting<PER>(v, (u32)n_exp, used, pick);
+            BM_RTICK(tl_places, lane);
+        } else {
+            route_probs_wave<PER>(v, (u32)n_exp, p);
+#pragma unroll
+            for (int j = 0; j < PER; j++) pick.p[lane + 64 * j] = p[j];
         }
-        [[maybe_unused]] unsigned long long tl_routed = 0;
+        lds_barrier();
+#ifdef BM_TIMELINE
+        if (wave == 1 && lane == 0 && blockIdx.x < (unsigned)kRouterTimelineRows) g_router_timeline[blockIdx.x * 8 + 6] = tl_places;
+#endif
+        if (wave == 1) return;
+        // (both waves have their logits: the words are armed again)
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+            if (lane + 64 * j < (u32)n_exp) __hip_atomic_store(mine + lane + 64 * j, kRouteArmed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!finite) return route_refuse(t, (u32)n_exp, used, probs, weights, fault, layer);
+        if (!picks_from_places(pick, t, (u32)n_exp, used, renorm, ids, weights))
+            route_pick_rounds<PER>(p, t, (u32)n_exp, used, renorm, ids, weights);
+        store_probs<PER>(p, t, (u32)n_exp, probs);
         BM_RTICK(tl_routed, threadIdx.x);
+        BM_RTOCK(0, tl_start);
+        BM_RTOCK(4, tl_seen);
         BM_RTOCK(5, tl_routed);
         return;
     }
     if (blockIdx.x >= n_logit_blocks) { // a quantizer workgroup
         const int tq = (int)(blockIdx.x - n_logit_blocks);
-        router_logits_body<R>(lds, router, x, gain, eps, n_exp, hidden, nullptr, nullptr, tq, -1);
+        __shared__ double s_part[1][4];
+        norm_rows<1, N4>(reinterpret_cast<float *>(lds), s_part, x, gain, eps, hidden, nullptr, tq, (int)m, []() {}, []() {});
+        lds_barrier();
         const NormRouteLate late = bm_kernarg_at<NormRouteLate>(offsetof(NormRouteArgs, late));
         uint8_t *const act_x = bm_global(late.act_x);
         u32 *const fault = bm_global(late.fault);
@@ -650,20 +767,23 @@ __global__ __launch_bounds__(256) void k_norm_route(const float *router, const f
         quant_normed_row(reinterpret_cast<const float *>(lds), hidden, tq, act_x, q8k, fault, layer);
         return;
     }
-    const u32 t = blockIdx.x / blocks_per_token;
-    router_logits_body<R, true>(lds, router, x, gain, eps, n_exp, hidden, normed_out, logits, (int)t, (int)(blockIdx.x % blocks_per_token) * R);
+    router_logits_body<R, T, N4, true>(lds, router, x, gain, eps, n_exp, hidden, (int)m, normed_out, logits, (int)(blockIdx.x / row_blocks) * T,
+                                       (int)(blockIdx.x % row_blocks) * R);
 }
 
 // ---- many tokens
 
-// The norm of many tokens' rows, a workgroup a token: router_logits_body's row into normed_out and, with act_x, into the token's
-// quantized column.
+// The norm of many tokens' rows, a workgroup a token: into normed_out and, with act_x, into the token's quantized column.
+template <int N4>
 __global__ __launch_bounds__(256) void k_norm_rows(const float *x, const float *gain, float eps, int hidden, float *normed_out, uint8_t *act_x,
                                                    int q8k, u32 *fault, u32 layer) {
     extern __shared__ __align__(16) uint8_t lds[];
+    __shared__ double s_part[1][4];
     const int t = (int)blockIdx.x;
-    router_logits_body<1>(lds, nullptr, x, gain, eps, 0, hidden, normed_out, nullptr, t, -1);
-    if (act_x) quant_normed_row(reinterpret_cast<const float *>(lds), hidden, t, act_x, q8k, fault, layer);
+    norm_rows<1, N4>(reinterpret_cast<float *>(lds), s_part, x, gain, eps, hidden, normed_out, t, t + 1, []() {}, []() {});
+    if (!act_x) return;
+    lds_barrier();
+    quant_normed_row(reinterpret_cast<const float *>(lds), hidden, t, act_x, q8k, fault, layer);
 }
 
 // The logits of many tokens' normed rows: tiles of tokens x experts on the matrix cores. v_mfma_f32_16x16x4_f32 runs four steps of
@@ -823,42 +943,56 @@ __global__ __launch_bounds__(256) void k_router_tiles(const float *router, const
     }
 }
 
-// LDS of a workgroup of R rows: the token's row and the router rows, each as eight lines.
-static size_t router_lds_bytes(int rows, int hidden) {
-    return ((size_t)(rows + 1) * 8 * router_line(hidden) + 4 * (size_t)rows) * sizeof(float);
+// LDS of a workgroup of so many tokens, whose dots take so many waves.
+static size_t router_lds_bytes(int tokens, int waves, int hidden) { return ((size_t)tokens * router_line(hidden) + (size_t)waves * 8 * kRouterSb) * sizeof(float); }
+
+bool router_logits_fits(int hidden) { return 16 * (size_t)(((hidden / 8 + 3) & ~3) + 8) * sizeof(float) + 16 <= (size_t)kMaxLds - 1024; }
+
+// Router rows and tokens a workgroup takes. A row and a token each while that leaves no more workgroups than stand on the card at once at three
+// waves a SIMD (two, where a row takes several passes): a launch of few workgroups is a wave's chain behind the norm of its token's
+// row, and nothing is shorter than one of each. Then four rows a token, a wave each, and from three workgroups a compute unit on two tokens
+// a workgroup, which ask for a row's bytes once - not where two rows of tokens leave a compute unit one workgroup.
+// (us a launch, 1 x 1 / 4 x 1 / 4 x 2, 128 experts: 2048 values 1 token 5.6 / 6.3 / 7.5, 4 tokens 6.0 / 6.4 / 7.6, 8 tokens 7.9 / 6.6 / 7.9, 24 tokens
+// 13.0 / 8.4 / 9.1, 32 tokens 15.9 / 10.5 / 9.6; 4096 values 4 tokens 7.7 / 8.5 / 10.4, 8 tokens 11.9 / 8.8 / 10.7, 24 tokens - / 14.7 / 12.6; 7168 values
+// 4 tokens 9.9 / 10.3 / 13.5, 24 tokens - / 19.6 / 24.3.)
+enum RouterForm { kForm1x1, kForm4x1, kForm4x2 };
+static long router_fours(int m, int n_exp) { return (long)m * ((n_exp + 3) / 4); }
+static RouterForm router_form(int m, int n_exp, int hidden) {
+    if ((long)m * n_exp <= (hidden <= 2048 ? 640 : 512)) return kForm1x1;
+    if (hidden <= 4096 && router_fours(m, n_exp) > (hidden <= 2048 ? 768 : 640)) return kForm4x2;
+    return kForm4x1;
 }
 
-// Rows a workgroup takes: four where they fit the LDS beside the token's row, else two, else one - and no more than leaves
-// a workgroup for every compute unit: a workgroup's time goes to bringing its rows in and laying them out in LDS (the dots of
-// its rows run side by side on one wave), so with few tokens fewer rows a workgroup is the shorter launch.
-static int router_rows(int hidden, int m = 1 << 20, int n_exp = 1 << 20) {
-    int fit = 0;
-    for (int r = 4; r >= 1; r >>= 1)
-        if (router_lds_bytes(r, hidden) <= (size_t)kMaxLds - 1024) {
-            fit = r;
-            break;
-        }
-    while (fit > 1 && (long)m * ((n_exp + fit - 1) / fit) < 256) fit >>= 1;
-    return fit;
+// Calls f with the form's rows and tokens and the pieces of a row a thread holds as constants.
+template <class F>
+static hipError_t with_form(RouterForm form, int hidden, F f) {
+    using std::integral_constant;
+    constexpr integral_constant<int, 1> one{};
+    constexpr integral_constant<int, 2> two{};
+    constexpr integral_constant<int, 4> four{};
+    auto tokens = [&](auto n4) { return form == kForm1x1 ? f(one, one, n4) : form == kForm4x1 ? f(four, one, n4) : f(four, two, n4); };
+    if (hidden % 256 != 0 || hidden > 8192) return tokens(integral_constant<int, 0>{});
+    if (hidden > 2048) return tokens(integral_constant<int, 8>{});
+    return tokens(two);
 }
 
-bool router_logits_fits(int hidden) { return router_rows(hidden) > 0; }
-
-// Whether the norm and the logits go as two launches, rows and then tiles: from ten million products on. Below that the one launch is
-// as short as the tiles' two (logits, one launch / two: 32 tokens x 128 experts x 2048 values 11.0 / 10.8 us, 16 tokens 6.3 / 10.7; 4 tokens x
-// 256 x 7168 13.8 / 25.1 us, 16 tokens 49.1 / 25.6). The tiles read normed rows from memory: a caller that wants none of them stays
-// with the one-token workgroups.
+// Whether the norm and the logits go as two launches, rows and then tiles: from six workgroups of four rows a compute unit on, from five
+// for rows of up to 1024 values, whose tiles are short, and of more than 4096, of which fewer workgroups stand on a compute unit. (us, one launch /
+// the tiles' three, routing included, by such workgroups: 1024 values 1024 of them 7.9 / 10.0, 1536 10.8 / 10.0; 2048 values 1536 12.5 / 13.3, 2048 15.0 /
+// 13.5; 4096 values 1536 18.7 / 20.0, 2048 22.4 / 20.3; 7168 values 1024 23.2 / 28.8, 1536 31.4 / 29.4.) The tiles read
+// normed rows from memory: a caller that wants none of them stays with the workgroups that norm their own.
 static bool router_tiled(int m, int n_exp, int hidden, const float *gain, const float *normed_out) {
-    return (double)m * n_exp * hidden >= (double)(10 << 20) && (!gain || normed_out);
+    return router_fours(m, n_exp) > (hidden > 1024 && hidden <= 4096 ? 1536 : 1280) && (!gain || normed_out);
 }
 
 static hipError_t router_tiles(const Launch &L, const float *router, const float *x, const float *gain, float eps, int m, int n_exp,
                                int hidden, float *normed_out, float *logits, uint8_t *act_x = nullptr, bool q8k = false) {
     if (normed_out || act_x) {
-        const size_t lds = router_lds_bytes(0, hidden);
-        hipError_t e = allow_lds(k_norm_rows, lds);
+        const size_t lds = router_lds_bytes(1, 0, hidden);
+        auto kern = hidden % 256 != 0 || hidden > 8192 ? k_norm_rows<0> : hidden > 2048 ? k_norm_rows<8> : k_norm_rows<2>;
+        hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_norm_rows, dim3((unsigned)m), dim3(256), lds, L.stream, x, gain, eps, hidden, normed_out, act_x, q8k ? 1 : 0, L.fault,
+        hipLaunchKernelGGL(kern, dim3((unsigned)m), dim3(256), lds, L.stream, x, gain, eps, hidden, normed_out, act_x, q8k ? 1 : 0, L.fault,
                            L.layer);
     }
     auto launch = [&](auto kern, unsigned grid, unsigned rows, unsigned kc) {
@@ -878,58 +1012,39 @@ static hipError_t router_tiles(const Launch &L, const float *router, const float
 hipError_t router_logits(const Launch &L, const float *router, const float *x, const float *gain, float eps, int m, int n_exp,
                          int hidden, float *normed_out, float *logits) {
     if (router_tiled(m, n_exp, hidden, gain, normed_out)) return router_tiles(L, router, x, gain, eps, m, n_exp, hidden, normed_out, logits);
-    const int rows = router_rows(hidden, m, n_exp);
-    if (rows == 0) return hipErrorInvalidValue;
-    const size_t lds = router_lds_bytes(rows, hidden);
-    const unsigned grid = (unsigned)m * (unsigned)((n_exp + rows - 1) / rows);
-#define BM_RL(R)                                                                                                       \
-    {                                                                                                                  \
-        auto kern = k_router_logits<R>;                                                                                \
-        hipError_t e = allow_lds(kern, lds);                                                                           \
-        if (e != hipSuccess) return e;                                                                                 \
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, router, x, gain, eps, n_exp, hidden, normed_out, \
-                           logits);                                                                                    \
-    }
-    if (rows == 4) BM_RL(4)
-    else if (rows == 2) BM_RL(2)
-    else BM_RL(1)
-#undef BM_RL
-    return hipGetLastError();
+    if (!router_logits_fits(hidden)) return hipErrorInvalidValue;
+    return with_form(router_form(m, n_exp, hidden), hidden, [&](auto r, auto t, auto n4) {
+        auto kern = k_router_logits<decltype(r)::value, decltype(t)::value, decltype(n4)::value>;
+        const size_t lds = router_lds_bytes(t, r, hidden);
+        hipError_t e = allow_lds(kern, lds);
+        if (e != hipSuccess) return e;
+        const unsigned grid = (unsigned)((m + t - 1) / t) * (unsigned)((n_exp + r - 1) / r);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, router, x, gain, eps, n_exp, hidden, m, normed_out, logits);
+        return hipGetLastError();
+    });
 }
 
 hipError_t norm_route(const Launch &L, const float *router, const float *x, const float *gain, float eps, int m, int n_exp,
                       int hidden, float *normed_out, float *logits, int used, int renorm, float *probs, uint32_t *ids,
                       float *weights, uint32_t *hand, uint8_t *act_x, bool q8k, uint32_t max_polls) {
-    const int rows = router_rows(hidden, m, n_exp);
-    if (rows == 0) return hipErrorInvalidValue;
+    if (!router_logits_fits(hidden)) return hipErrorInvalidValue;
     if (act_x && hidden % 256 != 0) return hipErrorInvalidValue;
     if (router_tiled(m, n_exp, hidden, gain, normed_out)) {
         const hipError_t e = router_tiles(L, router, x, gain, eps, m, n_exp, hidden, normed_out, logits, act_x, q8k);
         return e != hipSuccess ? e : route_softmax(L, logits, m, n_exp, used, renorm, probs, ids, weights);
     }
-    const size_t lds = router_lds_bytes(rows, hidden);
-    const unsigned grid = (unsigned)m * (unsigned)((n_exp + rows - 1) / rows) + (act_x ? (unsigned)m : 0u) + (unsigned)m;
-#define BM_NR(R, PER)                                                                                                  \
-    {                                                                                                                  \
-        auto kern = k_norm_route<R, PER>;                                                                              \
-        hipError_t e = allow_lds(kern, lds);                                                                           \
-        if (e != hipSuccess) return e;                                                                                 \
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, router, x, gain, eps, n_exp, hidden,           \
-                           (u32)m | (act_x ? 0x80000000u : 0u), normed_out, logits,                                    \
-                           NormRouteLate{(u32)used, (u32)renorm, probs, ids, weights, hand, act_x, q8k ? 1 : 0, L.layer, L.fault, max_polls, 0u}); \
-    }
-#define BM_NR_ROWS(PER)                                                                                                \
-    {                                                                                                                  \
-        if (rows == 4) BM_NR(4, PER)                                                                                   \
-        else if (rows == 2) BM_NR(2, PER)                                                                              \
-        else BM_NR(1, PER)                                                                                             \
-    }
-    if (n_exp <= 128) BM_NR_ROWS(2)
-    else if (n_exp <= 256) BM_NR_ROWS(4)
-    else BM_NR_ROWS(16)
-#undef BM_NR_ROWS
-#undef BM_NR
-    return hipGetLastError();
+    return with_form(router_form(m, n_exp, hidden), hidden, [&](auto r, auto t, auto n4) {
+        constexpr int R = decltype(r)::value, T = decltype(t)::value, N4 = decltype(n4)::value;
+        auto kern = n_exp <= 128 ? k_norm_route<R, T, N4, 2> : n_exp <= 256 ? k_norm_route<R, T, N4, 4> : k_norm_route<R, T, N4, 16>;
+        const size_t lds = router_lds_bytes(T, R, hidden);
+        hipError_t e = allow_lds(kern, lds);
+        if (e != hipSuccess) return e;
+        const unsigned grid = (unsigned)((m + T - 1) / T) * (unsigned)((n_exp + R - 1) / R) + (act_x ? (unsigned)m : 0u) + (unsigned)m;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, L.stream, router, x, gain, eps, n_exp, hidden,
+                           (u32)m | (act_x ? 0x80000000u : 0u), normed_out, logits,
+                           NormRouteLate{(u32)used, (u32)renorm, probs, ids, weights, hand, act_x, q8k ? 1 : 0, L.layer, L.fault, max_polls, 0u});
+        return hipGetLastError();
+    });
 }
 
 } // namespace bmk

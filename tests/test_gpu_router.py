@@ -290,6 +290,42 @@ def test_norm_route_is_the_two_launches_in_one(gpu, n_experts, hidden, m, top_k,
             b.free()
 
 
+@pytest.mark.parametrize("n_experts,hidden,m,top_k,with_gain", ((128, 256, 1, 15, True), (5, 2304, 3, 5, True), (127, 2048, 5, 8, True), (641, 2048, 1, 16, True),
+                                                                (130, 1792, 25, 32, False), (98, 2048, 33, 1, True), (257, 4352, 3, 9, True),
+                                                                (66, 4096, 41, 6, True), (131, 7168, 5, 8, True), (64, 8448, 9, 8, True), (70, 264, 3, 16, True),
+                                                                (129, 2312, 7, 17, False), (17, 20256, 33, 3, True)))
+def test_norm_route_forms(gpu, n_experts, hidden, m, top_k, with_gain):
+    """Every form of the fused launch's workgroups (bm_router.hip, router_form: a row and a token, four rows, four rows and two
+    tokens, with a last token by itself and rows left over) over rows of one super-block, of one whole pass of eight and a super-block more, of
+    lengths that are not whole super-blocks and the longest taken: normed rows, logits, ids against the oracle, the weights
+    within its units; picks up to the most there are."""
+    rng = np.random.default_rng(7000 + hidden + m)
+    router = normal_f32(rng, (n_experts, hidden), 0.05)
+    x = normal_f32(rng, (m, hidden)) * (10.0 ** rng.uniform(-2, 2, (m, 1))).astype(np.float32)
+    router[:, :8] *= np.float32(-0.0)
+    gain = (1.0 + normal_f32(rng, hidden, 0.2)).astype(np.float32) if with_gain else None
+    if gain is None:
+        x /= np.sqrt((x ** 2).mean(axis=1, keepdims=True))
+    rd, xd = gpu.upload(router, np.float32), gpu.upload(x, np.float32)
+    gd = gpu.upload(gain, np.float32) if with_gain else None
+    normed, logits = gpu.buffer(np.float32, m * hidden).fill_bytes(0xFF), gpu.buffer(np.float32, m * n_experts).fill_bytes(0xFF)
+    ids, wts = gpu.buffer(np.uint32, m * top_k).fill_bytes(0xEE), gpu.buffer(np.float32, m * top_k).fill_bytes(0xFF)
+    gpu.fault_clear()
+    gpu.enqueue_norm_route(rd, xd, gd, 1e-6, m, n_experts, hidden, top_k, True, normed, logits, None, ids, wts)
+    want_n, want_l = ora.router_logits(router, x, gain, 1e-6)
+    assert_f32(normed.download(), want_n.reshape(-1), "normed rows")
+    assert np.array_equal(logits.download().view(np.uint32), want_l.reshape(-1).view(np.uint32)), "logits"
+    got_ids, got_w = ids.download().reshape(m, top_k), wts.download().reshape(m, top_k)
+    for t in range(m):
+        want_ids, want_w = ora.route_softmax_topk(want_l[t], top_k)
+        assert np.array_equal(got_ids[t], want_ids), f"token {t}"
+        assert_ulp(got_w[t], want_w, f"weights of token {t}", odd_share=1.0)
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    for b in (rd, xd, gd, normed, logits, ids, wts):
+        if b is not None:
+            b.free()
+
+
 @pytest.mark.parametrize("n_experts,hidden,m,with_gain", ((129, 2048, 49, True), (16, 2048, 330, False), (17, 2056, 400, True), (1000, 512, 33, True),
                                                            (33, 520, 650, False), (130, 2048, 1100, True), (70, 2072, 2100, True), (65, 264, 4096, True)))
 def test_many_tokens_take_the_tiles_with_the_same_bits(gpu, n_experts, hidden, m, with_gain):
