@@ -23,6 +23,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 typedef uint32_t u32;
 
@@ -368,6 +369,12 @@ __device__ __forceinline__ u32 bm_and_or(u32 x, u32 mask, u32 bits) {
     asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0xea" : "=v"(r) : "v"(x), "v"(mask), "v"(bits));
     return r;
 }
+// a with the bits of x turned over where the mask has ones.
+__device__ __forceinline__ u32 bm_flip(u32 a, u32 x, u32 mask) {
+    u32 r;
+    asm("v_bitop3_b32 %0, %1, %2, %3 bitop3:0x78" : "=v"(r) : "v"(a), "v"(x), "v"(mask));
+    return r;
+}
 // b where the mask has ones, else a. (From the plain expression the compiler makes a field insert, one of the slower ones.)
 __device__ __forceinline__ u32 bm_pick(u32 a, u32 b, u32 mask) {
     u32 r;
@@ -689,10 +696,22 @@ struct Iq2Tables {
     const uint2 *grid3; // IQ3_XXS: (64 + magnitudes, 64 - magnitudes) of a four-value grid point
     const uint2 *signs; // IQ2_XXS: 4 in the bytes of the negative values; IQ3_XXS: 0xff there
 };
-// Where the signs lie behind the grid. One column's row dots take both tables to start where LDS does: their kernels have no array of
+// The tables' places. One column's row dots take them to start where LDS does: their kernels have no array of
 // fixed size (a test reads that from the built library), and with the dynamic array's own address, a zero that only the
-// linker fills in, each lookup would add it.
-constexpr u32 kIqSignsAt = 2048;
+// linker fills in, each lookup would add it. LDS serves 32 lanes' eight bytes (16 lanes' sixteen) at a time from 32 pairs of banks, and the
+// lookups of a table that lies there once come about three deep: two thirds of the tables' LDS time. Larger workgroups hold the grid in copies,
+// an entry's 256 bytes apart from the next one's and each lane's on banks of its own. That leaves LDS time for entries of sixteen bytes
+// where a code is then one instruction less, and makes an entry's address one byte permute of the index and the lane's copy.
+// (Gate . up of IQ2_XXS, 2048 rows of 7168, 32 slots: LDS 87 % busy with the tables as they are, 46 % in copies, the launch 71 us against 69: what is left
+// is memory, whose rate for rows read 66 bytes at a time from sixteen places is 4.2 TB/s where the same bytes in order come at 5.6. IQ3_XXS, 768
+// rows of 2048, 40 slots: 17.4 against 15.5.)
+template <int WT, bool WIDE>
+struct IqGeom {
+    static constexpr int kEntry = WIDE && WT == BM_IQ2XXS ? 16 : 8;
+    static constexpr int kSignLog = WIDE ? 2 : 0, kSignCopies = 1 << kSignLog, kSignAt = 3 + kSignLog; // kSignAt: a sign index' first bit in an address
+    static constexpr u32 kSignMask = 127u << kSignAt, kSignsAt = WIDE ? 256 * 256 : 256 * 8;
+    static constexpr int kBytes = (int)kSignsAt + 1024 * kSignCopies;
+};
 
 // The eight bytes at an LDS address. The row dots address the tables by bytes: an index turned to bits 3 .. of a word and masked, two
 // vector instructions and one of them a fast one, where an index taken out and added to a base eightfold takes two slow ones.
@@ -701,8 +720,39 @@ __device__ __forceinline__ uint2 bm_lds_pair(u32 at) {
     const v2u v = *(const __attribute__((address_space(3))) v2u *)(uintptr_t)at;
     return make_uint2(v.x, v.y);
 }
-// Bits n .. of x to bits 3 .. (n below 32, not a constant; the bits below wrap around).
-__device__ __forceinline__ u32 bm_to_bit3(u32 x, int n) { return __builtin_rotateright32(x, (u32)(n + 29)); }
+__device__ __forceinline__ uint4 bm_lds_quad(u32 at) {
+    typedef u32 v4u __attribute__((ext_vector_type(4)));
+    const v4u v = *(const __attribute__((address_space(3))) v4u *)(uintptr_t)at;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+// Bits N .. of x to bits TO .. (right shifts and masks are the fast instructions, hence not a field extract and a shift).
+template <int N, int TO>
+__device__ __forceinline__ u32 bm_to_bit(u32 x) {
+    return N < TO ? x << (TO - N & 31) : x >> (N - TO & 31);
+}
+// A lane's lookups: table entries by index fields of a word, at constant places.
+template <int WT, bool WIDE>
+struct IqLookup {
+    using G = IqGeom<WT, WIDE>;
+    u32 grid_copy, sign_mask, sign_copy;
+    __device__ __forceinline__ IqLookup() {
+        if constexpr (WIDE) {
+            grid_copy = (threadIdx.x * G::kEntry) & 255u;
+            sign_mask = bm_vector_const(G::kSignMask), sign_copy = G::kSignsAt | (8 * (threadIdx.x & (G::kSignCopies - 1))); // (too far for a read's own offset)
+        }
+    }
+    template <int BYTE>
+    __device__ __forceinline__ u32 grid_at(u32 word) const {
+        if constexpr (WIDE) return __builtin_amdgcn_perm(word, grid_copy, 0x0c0c0000u | ((4u + BYTE) << 8));
+        return bm_to_bit<8 * BYTE, 3>(word) & 0x7f8u;
+    }
+    template <int N>
+    __device__ __forceinline__ uint2 signs(u32 word) const {
+        const u32 x = bm_to_bit<N, G::kSignAt>(word);
+        if constexpr (WIDE) return bm_lds_pair(bm_and_or(x, sign_mask, sign_copy));
+        return bm_lds_pair(G::kSignsAt + (x & G::kSignMask));
+    }
+};
 
 // The eight code bytes 43 +- magnitude of an IQ2_XXS group (what the CPU path dots, crates/qdot/src/lib.rs:8677-8724): two
 // 8-byte table reads, a grid point's magnitude selectors and a sign index's bytes of 4, whose sum is a byte selector into the
@@ -718,33 +768,90 @@ __device__ __forceinline__ void bm_iq2_codes(const Iq2Tables &tb, u32 grid_idx, 
     bm_iq2_codes_of(tb.grid[grid_idx], tb.signs[sign_idx], lo, hi);
 }
 
+// Two ways to deal a super-block to its quad. The sums over its sub-blocks are integers, so any lane may form any of their terms:
+//   * own, with one column: lane q takes sub-blocks 2q and 2q + 1 whole, whose words it has loaded itself: every field lies at a constant
+//     place, the two scales are the lane's own, and nothing is handed round but, behind the dots, the eight lane sums
+//     (bm_quad_lane_sums): 139 vector instructions a super-block of IQ2_XXS against 151, 115 with the tables in copies;
+//   * across, with several: lane q takes group q of every sub-block and so forms its two lane sums alone, but each word goes round the quad
+//     first, is turned to the lane's field and yields its scale in all four lanes, once whatever the number of columns (the tile
+//     launch of IQ2_XXS 7168 x 2048, tiles of one column: 61 us, own 63).
 template <>
 struct Act<BM_IQ2XXS> {
     float dy;
     uint2 bs;   // bsums 4q .. 4q + 3
-    uint2 a[8]; // values 8q .. 8q + 8 of each of the eight sub-blocks
+    uint2 a[8]; // own: the 64 codes of sub-blocks 2q and 2q + 1; across: values 8q .. 8q + 8 of each of the eight sub-blocks
 };
 
-__device__ __forceinline__ Act<BM_IQ2XXS> bm_act_iq2xxs(const ActView &av, int i, int q) {
+typedef u32 bm_v2u __attribute__((ext_vector_type(2)));
+// volatile: eight-byte reads stay eight bytes (two merged into sixteen, the quad's four, 64 bytes apart, meet in two pairs of banks)
+typedef const volatile __attribute__((address_space(3))) bm_v2u *BmLdsV2;
+template <bool OWN>
+__device__ __forceinline__ Act<BM_IQ2XXS> bm_act_iqx(const ActView &av, int i, int q) {
     const uint8_t *blk = av.col + (size_t)i * BM_Q8K_STRIDE;
     Act<BM_IQ2XXS> a;
     a.dy = *reinterpret_cast<const float *>(blk);
     a.bs = *reinterpret_cast<const uint2 *>(blk + 264 + 8 * q);
 #pragma unroll
-    for (int sb = 0; sb < 8; sb++) a.a[sb] = *reinterpret_cast<const uint2 *>(blk + 8 + 32 * sb + 8 * q);
+    for (int k = 0; k < 8; k++) {
+        if constexpr (OWN) {
+            const bm_v2u v = *(BmLdsV2)(blk + 8 + 64 * q + 8 * k);
+            a.a[k] = make_uint2(v.x, v.y);
+        } else {
+            a.a[k] = *reinterpret_cast<const uint2 *>(blk + 8 + 32 * k + 8 * q);
+        }
+    }
     return a;
 }
 
-// The block's codes as this lane dots them: per sub-block the eight signed grid values (two words) and the
+// The block's codes as a lane dots them, own: sub-block 2q + e, group j.
+struct IqOwnDec {
+    u32 lo[2][4], hi[2][4]; // the bytes +-mag + offset of values 0 .. 3 and 4 .. 7
+    int sc[2];
+};
+
+template <bool WIDE>
+__device__ __forceinline__ IqOwnDec bm_decode_own(const Blk<BM_IQ2XXS> &b) {
+    const IqLookup<BM_IQ2XXS, WIDE> at;
+    IqOwnDec dec;
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const u32 idx = e ? b.q.z : b.q.x, aux = e ? b.q.w : b.q.y;
+        dec.sc[e] = 2 * (int)(aux >> 28) + 1;
+        auto group = [&](int j, u32 entry, uint2 sg) {
+            if constexpr (WIDE) {
+                const uint4 g = bm_lds_quad(entry);
+                dec.lo[e][j] = bm_flip(g.x, g.z, sg.x), dec.hi[e][j] = bm_flip(g.y, g.w, sg.y);
+            } else {
+                bm_iq2_codes_of(bm_lds_pair(entry), sg, dec.lo[e][j], dec.hi[e][j]);
+            }
+        };
+        group(0, at.template grid_at<0>(idx), at.template signs<0>(aux));
+        group(1, at.template grid_at<1>(idx), at.template signs<7>(aux));
+        group(2, at.template grid_at<2>(idx), at.template signs<14>(aux));
+        group(3, at.template grid_at<3>(idx), at.template signs<21>(aux));
+    }
+    return dec;
+}
+
+// The quad's four shares of eight lane sums: lane q ends with sums 2q and 2q + 1. In two steps a lane hands over the half of what it has that
+// is not its own, twelve picks and six exchanges; the sum of all eight in every lane is sixteen exchanges and the picks behind them.
+__device__ __forceinline__ void bm_quad_lane_sums(const int (&lanes)[8], int q, int &s0, int &s1) {
+    const u32 upper = bm_vector_const((q & 2) ? 0xffffffffu : 0u), odd = bm_vector_const((q & 1) ? 0xffffffffu : 0u);
+    u32 half[4];
+#pragma unroll
+    for (int l = 0; l < 4; l++)
+        half[l] = bm_pick((u32)lanes[l], (u32)lanes[4 + l], upper) + bm_dpp<kDppXor2>(bm_pick((u32)lanes[4 + l], (u32)lanes[l], upper));
+    s0 = (int)(bm_pick(half[0], half[2], odd) + bm_dpp<kDppXor1>(bm_pick(half[2], half[0], odd)));
+    s1 = (int)(bm_pick(half[1], half[3], odd) + bm_dpp<kDppXor1>(bm_pick(half[3], half[1], odd)));
+}
+
+// The block's codes as a lane dots them, across: per sub-block the eight signed grid values (two words) and the
 // scale 2s + 1. Decoded once a super-block, whatever the number of columns.
 struct Iq2Dec {
     u32 u_lo[8], u_hi[8]; // the bytes +-mag + 43
     int sc[8];
 };
 
-// BY_BYTES: the lookups by LDS addresses, the tables at the start of LDS (one column's dot; where a decode serves several columns, and registers are what there is
-// least of, the plain form measures the faster: IQ3_XXS tiles of 64 tokens 116 us against 119).
-template <bool BY_BYTES>
 __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int q, const Iq2Tables &tb) {
     Iq2Dec dec;
 #pragma unroll
@@ -757,63 +864,73 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq2xxs(const Blk<BM_IQ2XXS> &b, int 
             const int sb = 2 * k + e;
             const u32 idx = e ? idx_b : idx_a, aux = e ? aux_b : aux_a;
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
-            if constexpr (BY_BYTES)
-                bm_iq2_codes_of(bm_lds_pair(bm_to_bit3(idx, 8 * q) & 0x7f8u),
-                                bm_lds_pair(kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u)), dec.u_lo[sb], dec.u_hi[sb]);
-            else
-                bm_iq2_codes(tb, (idx >> (8 * q)) & 0xffu, (aux >> (7 * q)) & 127u, dec.u_lo[sb], dec.u_hi[sb]);
+            bm_iq2_codes(tb, (idx >> (8 * q)) & 0xffu, (aux >> (7 * q)) & 127u, dec.u_lo[sb], dec.u_hi[sb]);
         }
     }
     return dec;
 }
 
 // The float and integer steps IQ2_XXS and IQ3_XXS share (crates/qdot/src/lib.rs:8677-8724, :7494-7541): the fold of
-// the offset through the column's 16-value sums first, then the scaled sums of offset byte x code. `off`: 43 / 64;
+// the offset through the column's 16-value sums first, then the scaled sums of offset byte x code. OFF: 43 / 64;
 // d: f16 / 8 or f16 / 4; sca, scb: the scales 2s + 1 of the lane's own sub-blocks 2q and 2q + 1.
+template <int OFF>
+__device__ __forceinline__ void bm_fold_iqx(float d, int sca, int scb, const Act<BM_IQ2XXS> &act, float &acc0, float &acc1) {
+    // crates/qdot/src/lib.rs:8691-8694: accumulator l takes sub-block l's scale on its two bsums
+    const uint2 bs = act.bs;
+    const int b0 = (int)(short)(bs.x & 0xffffu), b1 = (int)(short)(bs.x >> 16);
+    const int b2 = (int)(short)(bs.y & 0xffffu), b3 = (int)(short)(bs.y >> 16);
+    const int ma = bm_mad24(sca, b0, bm_mul24(sca, b1)), mb = bm_mad24(scb, b2, bm_mul24(scb, b3)); // bsums: 16 bits
+    const float f = (-d * (float)OFF) * act.dy;
+    acc0 = fmaf(f, (float)ma, acc0);
+    acc1 = fmaf(f, (float)mb, acc1);
+}
+
 template <int OFF, class Tap>
-__device__ __forceinline__ void bm_dot_iqx_dec(float d, int sca, int scb, const Iq2Dec &dec, const Act<BM_IQ2XXS> &act,
-                                               int i, int q, float &acc0, float &acc1, const Tap &tap) {
-    const float dy = act.dy;
-    const float dmin = -d * (float)OFF;
-    // Fold first (crates/qdot/src/lib.rs:8691-8694): accumulator l takes sub-block l's scale on its two bsums.
-    {
-        const uint2 bs = act.bs;
-        const int b0 = (int)(short)(bs.x & 0xffffu), b1 = (int)(short)(bs.x >> 16);
-        const int b2 = (int)(short)(bs.y & 0xffffu), b3 = (int)(short)(bs.y >> 16);
-        const int ma = bm_mad24(sca, b0, bm_mul24(sca, b1)), mb = bm_mad24(scb, b2, bm_mul24(scb, b3)); // bsums: 16 bits
-        const float f = dmin * dy;
-        acc0 = fmaf(f, (float)ma, acc0);
-        acc1 = fmaf(f, (float)mb, acc1);
+__device__ __forceinline__ void bm_dot_own(float d, const IqOwnDec &dec, const Act<BM_IQ2XXS> &act, int i, int q, float &acc0, float &acc1,
+                                           const Tap &tap) {
+    bm_fold_iqx<OFF>(d, dec.sc[0], dec.sc[1], act, acc0, acc1);
+    // the reference sums sc * u * a (the offsets come back out through the fold above); sums within 4 * 126 * 128 and
+    // sc <= 31 lie inside 24 bits
+    int lanes[8];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint2 a = act.a[j], b = act.a[4 + j];
+        const int lo0 = bm_sdot4_first(dec.lo[0][j], a.x), hi0 = bm_sdot4_first(dec.hi[0][j], a.y);
+        const int lo1 = bm_sdot4_first(dec.lo[1][j], b.x), hi1 = bm_sdot4_first(dec.hi[1][j], b.y);
+        lanes[2 * j] = bm_mad24_chain(dec.sc[1], lo1, bm_mul24(dec.sc[0], lo0));
+        lanes[2 * j + 1] = bm_mad24_chain(dec.sc[1], hi1, bm_mul24(dec.sc[0], hi0));
+        if constexpr (Tap::kActive) { // the signed sums: less the offset times the eight codes
+            tap.iq2(i, 2 * q, j, lo0 + hi0 - OFF * (bm_sdot4(0x01010101u, a.x, 0) + bm_sdot4(0x01010101u, a.y, 0)));
+            tap.iq2(i, 2 * q + 1, j, lo1 + hi1 - OFF * (bm_sdot4(0x01010101u, b.x, 0) + bm_sdot4(0x01010101u, b.y, 0)));
+        }
     }
+    int s0, s1;
+    bm_quad_lane_sums(lanes, q, s0, s1);
+    const float f = d * act.dy;
+    acc0 = fmaf(f, (float)s0, acc0);
+    acc1 = fmaf(f, (float)s1, acc1);
+}
+
+template <int OFF>
+__device__ __forceinline__ void bm_dot_iqx_dec(float d, int sca, int scb, const Iq2Dec &dec, const Act<BM_IQ2XXS> &act, float &acc0,
+                                               float &acc1) {
+    bm_fold_iqx<OFF>(d, sca, scb, act, acc0, acc1);
     int sumi0 = 0, sumi1 = 0;
 #pragma unroll
     for (int sb = 0; sb < 8; sb++) {
         const uint2 a = act.a[sb];
-        // the reference sums sc * u * a (the offsets come back out through the fold above); sums within 4 * 126 * 128
-        // and sc <= 31 lie inside 24 bits
-        const int d_lo = bm_sdot4_first(dec.u_lo[sb], a.x), d_hi = bm_sdot4_first(dec.u_hi[sb], a.y);
-        sumi0 = bm_mad24_chain(dec.sc[sb], d_lo, sumi0);
-        sumi1 = bm_mad24_chain(dec.sc[sb], d_hi, sumi1);
-        if constexpr (Tap::kActive) // the signed sum: less the offset times the eight codes
-            tap.iq2(i, sb, q, d_lo + d_hi - OFF * (bm_sdot4(0x01010101u, a.x, 0) + bm_sdot4(0x01010101u, a.y, 0)));
+        sumi0 = bm_mad24_chain(dec.sc[sb], bm_sdot4_first(dec.u_lo[sb], a.x), sumi0);
+        sumi1 = bm_mad24_chain(dec.sc[sb], bm_sdot4_first(dec.u_hi[sb], a.y), sumi1);
     }
-    const float f = d * dy;
+    const float f = d * act.dy;
     acc0 = fmaf(f, (float)sumi0, acc0);
     acc1 = fmaf(f, (float)sumi1, acc1);
 }
 
-template <class Tap>
-__device__ __forceinline__ void bm_dot_iq2xxs_dec(const Blk<BM_IQ2XXS> &b, const Iq2Dec &dec, const Act<BM_IQ2XXS> &act,
-                                                  int i, int q, float &acc0, float &acc1, const Tap &tap) {
-    bm_dot_iqx_dec<43>(0.125f * bm_half_to_f32(b.d), 2 * (int)(b.q.y >> 28) + 1, 2 * (int)(b.q.w >> 28) + 1, dec, act, i, q,
-                       acc0, acc1, tap);
-}
-
-template <class Tap>
-__device__ __forceinline__ void bm_dot_iq2xxs(const Blk<BM_IQ2XXS> &b, const Act<BM_IQ2XXS> &act, int i, int q,
-                                              const Iq2Tables &tb, float &acc0, float &acc1, const Tap &tap) {
-    const Iq2Dec dec = bm_decode_iq2xxs<true>(b, q, tb);
-    bm_dot_iq2xxs_dec(b, dec, act, i, q, acc0, acc1, tap);
+__device__ __forceinline__ float bm_iqx_d(const Blk<BM_IQ2XXS> &b) { return 0.125f * bm_half_to_f32(b.d); }
+__device__ __forceinline__ void bm_dot_iqx_across(const Blk<BM_IQ2XXS> &b, const Iq2Dec &dec, const Act<BM_IQ2XXS> &act, float &acc0,
+                                                  float &acc1) {
+    bm_dot_iqx_dec<43>(bm_iqx_d(b), 2 * (int)(b.q.y >> 28) + 1, 2 * (int)(b.q.w >> 28) + 1, dec, act, acc0, acc1);
 }
 
 // ---- IQ3_XXS (crates/qdot/src/lib.rs:7494-7541): IQ2_XXS's lane map. Lane q owns accumulators 2q and 2q + 1: the
@@ -839,10 +956,29 @@ __device__ __forceinline__ Blk<BM_IQ3XXS> bm_load_iq3xxs(const uint8_t *wrow, in
 template <>
 struct Act<BM_IQ3XXS> : Act<BM_IQ2XXS> {};
 
-template <bool BY_BYTES> // as bm_decode_iq2xxs
+template <bool WIDE>
+__device__ __forceinline__ IqOwnDec bm_decode_own(const Blk<BM_IQ3XXS> &b) {
+    const IqLookup<BM_IQ3XXS, WIDE> at;
+    IqOwnDec dec;
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const u32 first = e ? b.qi.z : b.qi.x, second = e ? b.qi.w : b.qi.y, aux = e ? b.aux.y : b.aux.x;
+        dec.sc[e] = 2 * (int)(aux >> 28) + 1;
+        auto group = [&](int j, u32 lo, u32 hi, uint2 sg) {
+            const uint2 g0 = bm_lds_pair(lo), g1 = bm_lds_pair(hi);
+            dec.lo[e][j] = bm_iq_pick(g0.x, g0.y, sg.x);
+            dec.hi[e][j] = bm_iq_pick(g1.x, g1.y, sg.y);
+        };
+        group(0, at.template grid_at<0>(first), at.template grid_at<1>(first), at.template signs<0>(aux));
+        group(1, at.template grid_at<2>(first), at.template grid_at<3>(first), at.template signs<7>(aux));
+        group(2, at.template grid_at<0>(second), at.template grid_at<1>(second), at.template signs<14>(aux));
+        group(3, at.template grid_at<2>(second), at.template grid_at<3>(second), at.template signs<21>(aux));
+    }
+    return dec;
+}
+
 __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int q, const Iq2Tables &tb) {
     Iq2Dec dec;
-    [[maybe_unused]] const u32 upper = bm_vector_const((q & 2) ? 0xffffffffu : 0u); // (else the picks by it become selects by a VCC kept over the loop, 19 cycles each)
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         // sub-blocks 2k and 2k + 1 sit in lane k of the quad; this lane's two index bytes are bytes 2q, 2q + 1 of a
@@ -853,18 +989,9 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int 
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int sb = 2 * k + e;
-            const u32 aux = e ? aux_b : aux_a;
+            const u32 aux = e ? aux_b : aux_a, pair = ((q & 2) ? (e ? ib1 : ia1) : (e ? ib0 : ia0)) >> (16 * (q & 1));
             dec.sc[sb] = 2 * (int)(aux >> 28) + 1;
-            uint2 g0, g1, sg;
-            if constexpr (BY_BYTES) {
-                const u32 pair = bm_to_bit3(e ? bm_pick(ib0, ib1, upper) : bm_pick(ia0, ia1, upper), 16 * (q & 1));
-                g0 = bm_lds_pair(pair & 0x7f8u), g1 = bm_lds_pair((pair >> 8) & 0x7f8u);
-                sg = bm_lds_pair(kIqSignsAt + (bm_to_bit3(aux, 7 * q) & 0x3f8u));
-            } else {
-                const u32 pair = ((q & 2) ? (e ? ib1 : ia1) : (e ? ib0 : ia0)) >> (16 * (q & 1));
-                g0 = tb.grid3[pair & 0xffu], g1 = tb.grid3[(pair >> 8) & 0xffu];
-                sg = tb.signs[(aux >> (7 * q)) & 127u];
-            }
+            const uint2 g0 = tb.grid3[pair & 0xffu], g1 = tb.grid3[(pair >> 8) & 0xffu], sg = tb.signs[(aux >> (7 * q)) & 127u];
             dec.u_lo[sb] = bm_iq_pick(g0.x, g0.y, sg.x);
             dec.u_hi[sb] = bm_iq_pick(g1.x, g1.y, sg.y);
         }
@@ -872,18 +999,10 @@ __device__ __forceinline__ Iq2Dec bm_decode_iq3xxs(const Blk<BM_IQ3XXS> &b, int 
     return dec;
 }
 
-template <class Tap>
-__device__ __forceinline__ void bm_dot_iq3xxs_dec(const Blk<BM_IQ3XXS> &b, const Iq2Dec &dec, const Act<BM_IQ3XXS> &act,
-                                                  int i, int q, float &acc0, float &acc1, const Tap &tap) {
-    bm_dot_iqx_dec<64>(0.25f * bm_half_to_f32(b.d), 2 * (int)(b.aux.x >> 28) + 1, 2 * (int)(b.aux.y >> 28) + 1, dec, act, i,
-                       q, acc0, acc1, tap);
-}
-
-template <class Tap>
-__device__ __forceinline__ void bm_dot_iq3xxs(const Blk<BM_IQ3XXS> &b, const Act<BM_IQ3XXS> &act, int i, int q,
-                                              const Iq2Tables &tb, float &acc0, float &acc1, const Tap &tap) {
-    const Iq2Dec dec = bm_decode_iq3xxs<true>(b, q, tb);
-    bm_dot_iq3xxs_dec(b, dec, act, i, q, acc0, acc1, tap);
+__device__ __forceinline__ float bm_iqx_d(const Blk<BM_IQ3XXS> &b) { return 0.25f * bm_half_to_f32(b.d); }
+__device__ __forceinline__ void bm_dot_iqx_across(const Blk<BM_IQ3XXS> &b, const Iq2Dec &dec, const Act<BM_IQ2XXS> &act, float &acc0,
+                                                  float &acc1) {
+    bm_dot_iqx_dec<64>(bm_iqx_d(b), 2 * (int)(b.aux.x >> 28) + 1, 2 * (int)(b.aux.y >> 28) + 1, dec, act, acc0, acc1);
 }
 
 // ---- Q3_K (crates/qdot/src/lib.rs:2223-2245, layout crates/gguf/src/quant.rs:671-678): one integer a super-block
@@ -1056,8 +1175,6 @@ __device__ __forceinline__ void bm_dot_iq4xs_dec(const Blk<BM_IQ4XS> &b, const I
         }
         tap.iq4_sub(i, 2 * q + e, sub);
     }
-    // The quad's four shares of each lane sum: lane q ends with sums 2q and 2q + 1. In two steps a lane hands over the half of what it has that
-    // is not its own, twelve picks and six exchanges; the sum of all eight in every lane is sixteen exchanges and the picks behind them.
     int s0, s1;
     if constexpr (Tap::kActive) {
 #pragma unroll
@@ -1068,15 +1185,7 @@ __device__ __forceinline__ void bm_dot_iq4xs_dec(const Blk<BM_IQ4XS> &b, const I
         }
         s0 = q == 0 ? lanes[0] : (q == 1 ? lanes[2] : (q == 2 ? lanes[4] : lanes[6]));
         s1 = q == 0 ? lanes[1] : (q == 1 ? lanes[3] : (q == 2 ? lanes[5] : lanes[7]));
-    } else {
-        const u32 upper = bm_vector_const((q & 2) ? 0xffffffffu : 0u), odd = bm_vector_const((q & 1) ? 0xffffffffu : 0u);
-        u32 half[4];
-#pragma unroll
-        for (int l = 0; l < 4; l++)
-            half[l] = bm_pick((u32)lanes[l], (u32)lanes[4 + l], upper) + bm_dpp<kDppXor2>(bm_pick((u32)lanes[4 + l], (u32)lanes[l], upper));
-        s0 = (int)(bm_pick(half[0], half[2], odd) + bm_dpp<kDppXor1>(bm_pick(half[2], half[0], odd)));
-        s1 = (int)(bm_pick(half[1], half[3], odd) + bm_dpp<kDppXor1>(bm_pick(half[3], half[1], odd)));
-    }
+    } else bm_quad_lane_sums(lanes, q, s0, s1);
     // one fused multiply-add a super-block and lane (crates/qdot/src/lib.rs:11171-11173)
     const float f = bm_half_to_f32(b.hd.x & 0xffffu) * act.dy;
     acc0 = fmaf(f, (float)s0, acc0);
@@ -1154,15 +1263,14 @@ __device__ __forceinline__ Act<WT> bm_load_act(const ActView &av, int i, int q) 
         return bm_act_q3k(av, i, q);
     else if constexpr (WT == BM_IQ3XXS) {
         Act<BM_IQ3XXS> a;
-        static_cast<Act<BM_IQ2XXS> &>(a) = bm_act_iq2xxs(av, i, q);
+        static_cast<Act<BM_IQ2XXS> &>(a) = bm_act_iqx<true>(av, i, q);
         return a;
     } else
-        return bm_act_iq2xxs(av, i, q);
+        return bm_act_iqx<true>(av, i, q);
 }
 
-template <int WT, class Tap>
-__device__ __forceinline__ void bm_dot_blk(const Blk<WT> &b, const Act<WT> &a, int i, int q, const Iq2Tables &tb,
-                                           float &acc0, float &acc1, const Tap &tap) {
+template <int WT, bool WIDE, class Tap>
+__device__ __forceinline__ void bm_dot_blk(const Blk<WT> &b, const Act<WT> &a, int i, int q, float &acc0, float &acc1, const Tap &tap) {
     if constexpr (WT == BM_Q4K)
         bm_dot_q4k(b, a, i, q & 1, q >> 1, acc0, acc1, tap);
     else if constexpr (WT == BM_Q5K)
@@ -1174,9 +1282,9 @@ __device__ __forceinline__ void bm_dot_blk(const Blk<WT> &b, const Act<WT> &a, i
     else if constexpr (WT == BM_Q3K)
         bm_dot_q3k(b, a, i, q, acc0, tap);
     else if constexpr (WT == BM_IQ3XXS)
-        bm_dot_iq3xxs(b, a, i, q, tb, acc0, acc1, tap);
+        bm_dot_own<64>(bm_iqx_d(b), bm_decode_own<WIDE>(b), a, i, q, acc0, acc1, tap);
     else
-        bm_dot_iq2xxs(b, a, i, q, tb, acc0, acc1, tap);
+        bm_dot_own<43>(bm_iqx_d(b), bm_decode_own<WIDE>(b), a, i, q, acc0, acc1, tap);
 }
 
 template <int WT>

@@ -287,15 +287,16 @@ constexpr unsigned kGateUpGridY = 32768; // slots along the grid's second dimens
 
 // The grid: (blocks of 32 rows, slots, slots / kGateUpGridY): no division stands before the workgroup's first request.
 // spc_word: slots_per_col, and above bit 24 one more than its log2 where it is a power of two.
-template <int WT, int U, int NB>
-__global__ __launch_bounds__(256) void k_gate_up(const uint8_t *wg, const uint8_t *wu, u32 n_experts, int nb,
+template <int WT, int U, int NB, int T = 256, bool WIDE = false>
+__global__ __launch_bounds__(T) void k_gate_up(const uint8_t *wg, const uint8_t *wu, u32 n_experts, int nb,
                                                  const uint8_t *act, const u32 *sel, int rpe, int spc_word, u32 n_slots,
                                                  GateUpColLate) {
     extern __shared__ __align__(16) uint8_t lds[];
     const int tid = threadIdx.x, q = tid & 3, which = (tid >> 2) & 1;
     const int slot = (int)(blockIdx.z * kGateUpGridY + blockIdx.y), rb = (int)blockIdx.x;
     if ((u32)slot >= n_slots) return;
-    const int r = rb * 32 + (tid >> 3);
+    const int r0 = rb * (T / 8);
+    const int r = r0 + (tid >> 3);
     const bool active = r < rpe;
     const u32 id = sel[slot];
     const int n = NB > 0 ? NB : nb;
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(256) void k_gate_up(const uint8_t *wg, const uint8_
     const int spc_shift = (spc_word >> 24) - 1;
     const int token = spc_shift >= 0 ? slot >> spc_shift : slot / (spc_word & 0xffffff);
     const uint8_t *act_col = act + (size_t)token * col_bytes;
-    Stage<2> st;
+    Stage<512 / T, T> st;
     st.load(act_col, col_bytes);
     if (id >= n_experts) { // uniform over the workgroup: no weight is read (crates/gpu/src/kquant/sel.rs:22-28)
         if (id == 0xffffffffu) return; // a slot served elsewhere: nothing written, nothing raised (sel.rs:153-161)
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(256) void k_gate_up(const uint8_t *wg, const uint8_
         uint8_t *const act_h = bm_global(late.act_h);
         if (tid == 0) bm_raise(bm_global(late.fault), late.layer, kSiteExpertId);
         if (h && active && (tid & 7) == 0) h[(size_t)slot * rpe + r] = bm_bits_f32(0x7fc00000u);
-        if (act_h && tid < 32) q82_store(act_h + (size_t)slot * nb_h * BM_Q82_SB_EXT, nb_h, rb, tid, 0, Q82Head{0x7fc0u, 0, true}, 0);
+        if (act_h && tid < T / 8 && r0 + tid < rpe) q82_store(act_h + (size_t)slot * nb_h * BM_Q82_SB_EXT, nb_h, (r0 + tid) >> 5, tid & 31, 0, Q82Head{0x7fc0u, 0, true}, 0);
         return;
     }
     const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(256) void k_gate_up(const uint8_t *wg, const uint8_
     // (behind the wait for the id; nothing reads them before the column stands in LDS)
     const GateUpColLate late = bm_kernarg_at<GateUpColLate>(offsetof(GateUpColArgs, late));
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT>(lds);
-    uint8_t *col = lds + tab_bytes<WT>();
+    const Iq2Tables tb = stage_tables_as<WT, WIDE, T>(lds);
+    uint8_t *col = lds + tab_bytes<WT, WIDE>();
     st.store(col, act_col, col_bytes);
     __syncthreads();
     float *const h = bm_global(late.h);
@@ -332,14 +333,14 @@ __global__ __launch_bounds__(256) void k_gate_up(const uint8_t *wg, const uint8_
     const u32 layer = late.layer;
     uint8_t *hcol = act_h ? act_h + (size_t)slot * nb_h * BM_Q82_SB_EXT : nullptr;
     float v[1];
-    row_dot<WT, U, NB, 1>(b, wrow, col, col_bytes, 1, n, q, tb, v, NoTap{});
+    row_dot<WT, U, NB, 1, WIDE>(b, wrow, col, col_bytes, 1, n, q, tb, v, NoTap{});
     const float hv = swiglu_of_pair(v[0], which, late.rule, fault, layer);
     if (h && active && (tid & 7) == 0) h[(size_t)slot * rpe + r] = hv;
     if (act_h) { // rpe is a multiple of 256 here, so every row of the block is live
         float *hbuf = reinterpret_cast<float *>(col + col_bytes);
         if ((tid & 7) == 0) hbuf[tid >> 3] = hv;
         __syncthreads();
-        if (tid < 32) quantize_h_block(hbuf, hcol, nb_h, rb, tid, fault, layer);
+        if (tid < T / 8 && r0 + tid < rpe) quantize_h_block(hbuf + (tid & ~31), hcol, nb_h, (r0 + tid) >> 5, tid & 31, fault, layer);
     }
 }
 
@@ -863,8 +864,8 @@ struct Q82Cols {
 // k_gate_up_x for gate / up stacks that dot against Q8_K columns (Q3_K, IQ2_XXS, IQ3_XXS, IQ4_XS): the token's row is
 // quantized by every workgroup into LDS, h is written as f32 rows, and where the down stack takes Q8_2_X4 columns
 // (act_h given) the workgroup's 32 values also become their block of the slot's column.
-template <int WA, int UA, int NBA>
-__global__ __launch_bounds__(256) void k_gate_up_xq(const float *x, const uint8_t *wg, const uint8_t *wu, u32 n_experts,
+template <int WA, int UA, int NBA, int T = 256, bool WIDE = false>
+__global__ __launch_bounds__(T) void k_gate_up_xq(const float *x, const uint8_t *wg, const uint8_t *wu, u32 n_experts,
                                                     int nba, int nh, const u32 *sel, int spt_word, uint8_t *act_x,
                                                     uint8_t *act_h, float *h, GateRule rule, u32 *fault, u32 layer) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -876,35 +877,36 @@ __global__ __launch_bounds__(256) void k_gate_up_xq(const float *x, const uint8_
     const int rb = (int)(row_major ? blockIdx.x : blockIdx.z * kDies + blockIdx.x % kDies);
     const int na = NBA > 0 ? NBA : nba;
     const int hidden = na * 256, ff = nh * 256;
-    const int r = rb * 32 + (tid >> 3);
+    const int r0 = rb * (T / 8), r = r0 + (tid >> 3);
+    if (T > 256 && r0 >= ff) return; // (by dies, the last eight blocks need not be whole)
     const u32 id = sel[slot];
     uint8_t *hcol = act_h ? act_h + (size_t)slot * nh * BM_Q82_SB_EXT : nullptr;
     if (id >= n_experts) { // uniform over the workgroup
         if (id == 0xffffffffu) return; // a slot served elsewhere: nothing written, nothing raised
         if (tid == 0) bm_raise(fault, layer, kSiteExpertId);
         if (h && (tid & 7) == 0) h[(size_t)slot * ff + r] = bm_bits_f32(0x7fc00000u);
-        if (hcol && tid < 32) q82_store(hcol, nh, rb, tid, 0, Q82Head{0x7fc0u, 0, true}, 0);
+        if (hcol && tid < T / 8) q82_store(hcol, nh, (r0 + tid) >> 5, tid & 31, 0, Q82Head{0x7fc0u, 0, true}, 0);
         return;
     }
     const size_t row_bytes = (size_t)na * bm_block_bytes<WA>();
     const uint8_t *wrow = (which ? wu : wg) + ((size_t)id * ff + r) * row_bytes;
     Blk<WA> b[UA];
     preload<WA, UA>(b, wrow, na, q);
-    const Iq2Tables tb = stage_tables<WA>(lds);
-    uint8_t *col = lds + tab_bytes<WA>();
+    const Iq2Tables tb = stage_tables_as<WA, WIDE, T>(lds);
+    uint8_t *col = lds + tab_bytes<WA, WIDE>();
     const int col_bytes = bm_act_col_bytes<WA>(na);
-    q8k_stage_cols(x + (size_t)t * hidden, col, 1, na, fault, layer);
+    q8k_stage_cols<T>(x + (size_t)t * hidden, col, 1, na, fault, layer);
     __syncthreads();
-    if (act_x && rb == 0 && slot % spt == 0) stage_bytes(act_x + (size_t)t * col_bytes, col, col_bytes);
+    if (act_x && rb == 0 && slot % spt == 0) stage_bytes<T>(act_x + (size_t)t * col_bytes, col, col_bytes);
     float v[1];
-    row_dot<WA, UA, NBA, 1>(b, wrow, col, col_bytes, 1, na, q, tb, v, NoTap{});
+    row_dot<WA, UA, NBA, 1, WIDE>(b, wrow, col, col_bytes, 1, na, q, tb, v, NoTap{});
     const float hv = swiglu_of_pair(v[0], which, rule, fault, layer);
     if (h && (tid & 7) == 0) h[(size_t)slot * ff + r] = hv;
     if (hcol) {
         float *hbuf = reinterpret_cast<float *>(col + col_bytes);
         if ((tid & 7) == 0) hbuf[tid >> 3] = hv;
         __syncthreads();
-        if (tid < 32) quantize_h_block(hbuf, hcol, nh, rb, tid, fault, layer);
+        if (tid < T / 8) quantize_h_block(hbuf + (tid & ~31), hcol, nh, (r0 + tid) >> 5, tid & 31, fault, layer);
     }
 }
 
@@ -961,7 +963,7 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
 
 // k_down_combine for down stacks that dot against Q8_K columns: the token's slot rows of h (f32) are quantized by
 // every workgroup into LDS; the first workgroup of a token also leaves the columns in act_h.
-template <int WT, int U, int NB, int T>
+template <int WT, int U, int NB, int T, bool WIDE = false>
 __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_experts, int nb, const float *h,
                                                        uint8_t *act_h, const u32 *sel, const float *wts,
                                                          const float *resid, int spt_word, int rpe, float *y, u32 *fault,
@@ -993,8 +995,8 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
-    const Iq2Tables tb = stage_tables<WT>(lds, T);
-    uint8_t *cols = lds + tab_bytes<WT>();
+    const Iq2Tables tb = stage_tables_as<WT, WIDE, T>(lds);
+    uint8_t *cols = lds + tab_bytes<WT, WIDE>();
     float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
     float *s_w = part + D * spt;                                              // [spt]
     u32 *s_sel = reinterpret_cast<u32 *>(s_w + spt);                          // [spt]
@@ -1009,7 +1011,7 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
         for (int c = 0; c < spt; c++)
             if (s_sel[c] < n_experts) stage_bytes<T>(act_h + ((size_t)t * spt + c) * col_bytes, cols + (size_t)c * col_bytes, col_bytes);
     float v[1];
-    row_dot<WT, U, NB, 1>(b, wrow, cols + (size_t)e * col_bytes, col_bytes, 1, n, q, tb, v, NoTap{});
+    row_dot<WT, U, NB, 1, WIDE>(b, wrow, cols + (size_t)e * col_bytes, col_bytes, 1, n, q, tb, v, NoTap{});
     if (q == 0 && dl < D) part[dl * spt + e] = v[0];
     __syncthreads();
     if (tid < D && rb * D + tid < rpe) y[(size_t)t * rpe + rb * D + tid] = slot_sum(part + tid * spt, s_w, s_sel, spt, n_experts, resid_v, resid != nullptr);
@@ -1182,11 +1184,28 @@ hipError_t gemv_x(const Launch &L, int wtype, const uint8_t *w, int64_t rows, in
     return hipGetLastError();
 }
 
+// Whether a launch of one-column row dots takes the IQ tables in copies: `lds` bytes with them, `threads` a workgroup. Not where they leave a
+// compute unit fewer than sixteen waves.
+static bool copies_fit(int wtype, size_t lds, int threads) {
+    return (wtype == BM_IQ2XXS || wtype == BM_IQ3XXS) && (size_t)kMaxLds / lds * (size_t)threads >= 16 * 64;
+}
+#define BM_WITH_TABLES(PLAIN, WIDE)                                                                                    \
+    {                                                                                                                  \
+        if constexpr (WT == BM_IQ2XXS || WT == BM_IQ3XXS)                                                              \
+            if (wide) return launch(WIDE);                                                                             \
+        return launch(PLAIN);                                                                                          \
+    }
+// A gate . up launch of `blocks` workgroups of 32 row pairs as one of workgroups of 64 that hold the tables in copies: from more blocks than
+// compute units on, where two of the smaller ones would share a unit (below, a unit's only workgroup then takes twice as long: 700 random
+// layers of IQ2_XXS and IQ3_XXS, 1 to 24 tokens: up to 256 blocks 1.03, from there to 1024 0.97, past that 0.975 and 0.96; at worst 1.07).
+static bool gate_up_in_copies(int wtype, int k, int64_t blocks) {
+    return blocks > kCardUnits && copies_fit(wtype, tab_bytes_rt(wtype, true) + (size_t)act_col_bytes(wtype, k) + 64 * sizeof(float), 512);
+}
+
 hipError_t gate_up(const Launch &L, int wtype, const uint8_t *wg, const uint8_t *wu, int n_experts, int k,
                    const uint8_t *act, const uint32_t *sel, int n_slots, int rows_per_expert, int slots_per_col,
                    float *h, uint8_t *act_h) {
     const int nb = k / 256, rpe = rows_per_expert;
-    const size_t lds = tab_bytes_rt(wtype) + (size_t)act_col_bytes(wtype, k) + 32 * sizeof(float);
     if (n_slots <= 0 || slots_per_col <= 0) return hipErrorInvalidValue;
     if (slots_per_col > 0xffffff) { // (more slots a column than there are slots: column 0 either way)
         if (n_slots > 0xffffff) return hipErrorInvalidValue;
@@ -1195,16 +1214,20 @@ hipError_t gate_up(const Launch &L, int wtype, const uint8_t *wg, const uint8_t 
     const unsigned grid_y = (unsigned)n_slots < kGateUpGridY ? (unsigned)n_slots : kGateUpGridY;
     const unsigned grid_z = ((unsigned)n_slots + kGateUpGridY - 1) / kGateUpGridY;
     const int spc_shift = (slots_per_col & (slots_per_col - 1)) == 0 ? __builtin_ctz((unsigned)slots_per_col) : -1;
-#define CALL_BODY                                                                                                      \
-    auto kern = k_gate_up<WT, U, NB>;                                                                                  \
-    hipError_t e = allow_lds(kern, lds);                                                                               \
-    if (e != hipSuccess) return e;                                                                                     \
-    hipLaunchKernelGGL(kern, dim3((unsigned)((rpe + 31) / 32), grid_y, grid_z), dim3(256), lds, L.stream, wg, wu, (u32)n_experts, nb, \
-                       act, sel, rpe, slots_per_col | ((spc_shift + 1) << 24), (u32)n_slots,                           \
-                       GateUpColLate{h, act_h, L.rule, L.fault, L.layer});
+    const bool wide = gate_up_in_copies(wtype, k, (int64_t)n_slots * ((rpe + 31) / 32));
+    const int T = wide ? 512 : 256;
+    const size_t bytes = tab_bytes_rt(wtype, wide) + (size_t)act_col_bytes(wtype, k) + T / 8 * sizeof(float);
+    auto launch = [&](auto kern) {
+        hipError_t e = allow_lds(kern, bytes);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((rpe + T / 8 - 1) / (T / 8)), grid_y, grid_z), dim3(T), bytes, L.stream, wg, wu, (u32)n_experts, nb,
+                           act, sel, rpe, slots_per_col | ((spc_shift + 1) << 24), (u32)n_slots, GateUpColLate{h, act_h, L.rule, L.fault, L.layer});
+        return hipGetLastError();
+    };
+#define CALL_BODY BM_WITH_TABLES((k_gate_up<WT, U, NB>), (k_gate_up<WT, U, NB, 512, true>))
     BM_DISPATCH(wtype, nb)
 #undef CALL_BODY
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t gemv_sel(const Launch &L, int wtype, const uint8_t *w, int n_experts, int k, const uint8_t *act,
@@ -1301,13 +1324,21 @@ hipError_t gate_up_x(const Launch &L, int gate_type, const float *x, const uint8
         BM_GUX(BM_Q6K, kRing, 0)
     } else if (bm_takes_q8k(gate_type)) {
         const int nb = nba;
-        const size_t lds_q = tab_bytes_rt(gate_type) + (size_t)act_col_bytes(gate_type, hidden) + 32 * sizeof(float);
-#define CALL_BODY                                                                                                      \
-    auto kern = k_gate_up_xq<WT, U, NB>;                                                                               \
-    hipError_t e = allow_lds(kern, lds_q);                                                                             \
-    if (e != hipSuccess) return e;                                                                                     \
-    hipLaunchKernelGGL(kern, grid_a, dim3(256), lds_q, L.stream, x, wg, wu, (u32)n_experts, nba, nbb, sel,             \
-                       spt | (row_major ? kGateRowMajor : 0), act_x, act_h, h, L.rule, L.fault, L.layer);
+        const int wtype = gate_type;
+        const bool wide = gate_up_in_copies(wtype, hidden, (int64_t)m * spt * (ff / 32));
+        const int T = wide ? 512 : 256;
+        const size_t bytes = tab_bytes_rt(wtype, wide) + (size_t)act_col_bytes(gate_type, hidden) + T / 8 * sizeof(float);
+        const unsigned blocks = (unsigned)(ff / (T / 8));
+        const bool row_major = plain_order((int64_t)m * spt, m, blocks, T);
+        auto launch = [&](auto kern) {
+            hipError_t e = allow_lds(kern, bytes);
+            if (e != hipSuccess) return e;
+            const dim3 grid = row_major ? dim3(blocks, (unsigned)spt, (unsigned)m) : dim3(kDies * (unsigned)spt, (unsigned)m, eighths(blocks));
+            hipLaunchKernelGGL(kern, grid, dim3(T), bytes, L.stream, x, wg, wu, (u32)n_experts, nba, nbb, sel,
+                               spt | (row_major ? kGateRowMajor : 0), act_x, act_h, h, L.rule, L.fault, L.layer);
+            return hipGetLastError();
+        };
+#define CALL_BODY BM_WITH_TABLES((k_gate_up_xq<WT, U, NB>), (k_gate_up_xq<WT, U, NB, 512, true>))
         BM_DISPATCH(gate_type, nb)
 #undef CALL_BODY
     } else {
@@ -1358,18 +1389,21 @@ hipError_t down_combine_hq(const Launch &L, int wtype, const uint8_t *w, int n_e
     const size_t lds = down_combine_lds(wtype, k, spt) + (size_t)(D - 64 / spt) * spt * sizeof(float);
     const unsigned blocks = (unsigned)((rpe + D - 1) / D);
     const bool row_major = plain_order((int64_t)m * spt, m, blocks, T);
+    // (from 512 threads on: of 256 a compute unit holds too few beside the copies; 450 random launches 0.95 to 0.99, at worst 1.03)
+    const bool wide = copies_fit(wtype, lds + (size_t)(tab_bytes_rt(wtype, true) - tab_bytes_rt(wtype)), T);
+    const size_t bytes = lds + (size_t)(tab_bytes_rt(wtype, wide) - tab_bytes_rt(wtype));
     auto launch = [&](auto kern) {
-        hipError_t e = allow_lds(kern, lds);
+        hipError_t e = allow_lds(kern, bytes);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, row_major ? dim3(blocks, (unsigned)m) : dim3(kDies, (unsigned)m, eighths(blocks)), dim3((unsigned)T), lds,
+        hipLaunchKernelGGL(kern, row_major ? dim3(blocks, (unsigned)m) : dim3(kDies, (unsigned)m, eighths(blocks)), dim3((unsigned)T), bytes,
                            L.stream, w, (u32)n_experts, nb, h, act_h, sel, wts, resid,
                            spt | ((spt_shift + 1) << 16) | (row_major ? kDownRowMajor : 0), rpe, y, L.fault, L.layer);
         return hipGetLastError();
     };
 #define CALL_BODY                                                                                                      \
     if constexpr (bm_takes_q8k(WT)) {                                                                                  \
-        if (T == 1024) return launch(k_down_combine_hq<WT, U, NB, 1024>);                                              \
-        if (T == 512) return launch(k_down_combine_hq<WT, U, NB, 512>);                                                \
+        if (T == 1024) BM_WITH_TABLES((k_down_combine_hq<WT, U, NB, 1024>), (k_down_combine_hq<WT, U, NB, 1024, true>)) \
+        if (T == 512) BM_WITH_TABLES((k_down_combine_hq<WT, U, NB, 512>), (k_down_combine_hq<WT, U, NB, 512, true>)) \
     }                                                                                                                  \
     return launch(k_down_combine_hq<WT, U, NB, 256>)
     BM_DISPATCH(wtype, nb)

@@ -26,14 +26,11 @@ constexpr u32 kSiteQuantColumn = 1; // crates/device/src/fault.rs:73-76
 constexpr u32 kSiteExpertId = 7;    // crates/device/src/fault.rs:89
 constexpr u32 kSiteF32Product = 21; // crates/device/src/fault.rs:151-155: a gate or up sum that is not finite under a clamp
 
-// LDS bytes of the IQ2_XXS tables: 256 grid entries of 8 + 128 sign entries of 8.
-constexpr int kTabBytes = 256 * 8 + 128 * 8;
-
-constexpr int kTabBytes3 = 256 * 8 + 128 * 8; // IQ3_XXS: 256 grid entries of 8 + 128 sign entries of 8
-
-template <int WT>
+// LDS bytes of the IQ tables: 256 grid entries of 8 and 128 sign entries of 8, each in its copies (IqGeom).
+template <int WT, bool WIDE = false>
 __host__ __device__ constexpr int tab_bytes() {
-    return WT == BM_IQ2XXS ? kTabBytes : WT == BM_IQ3XXS ? kTabBytes3 : 0;
+    if constexpr (WT == BM_IQ2XXS || WT == BM_IQ3XXS) return IqGeom<WT, WIDE>::kBytes;
+    return 0;
 }
 
 // A sign index's eight signs as two words of byte masks: 0xff where the value is negative.
@@ -46,6 +43,38 @@ __device__ __forceinline__ uint2 iq_sign_masks(int t) {
                   ((nib & 8) ? 0xff000000u : 0u);
     }
     return make_uint2(m[0], m[1]);
+}
+
+// Four magnitudes of an IQ2_XXS grid point as selectors, a byte each: 0x08 -> 0, 0x19 -> 1, 0x2b -> 2 (bit 0 of the byte is 1 for 0x19 and
+// 0x2b, bit 1 for 0x2b only).
+__device__ __forceinline__ u32 iq2_selectors(u32 g) { return (g & 0x01010101u) + ((g >> 1) & 0x01010101u); }
+
+// The tables in their copies (IqGeom). A thread writes an entry's in an order of its own, so that lanes that store together reach different banks.
+template <int WT, int T>
+__device__ __forceinline__ void stage_wide_tables(uint8_t *lds) {
+    using G = IqGeom<WT, true>;
+    static_assert(T >= 256 && T % 256 == 0, "whole threads an entry");
+    constexpr u32 kParts = T / 256, kUnits = 16 / kParts; // threads an entry, and how many of its sixteen times sixteen bytes each writes
+    const u32 t = threadIdx.x / kParts, part = threadIdx.x % kParts;
+    uint4 v;
+    if constexpr (WT == BM_IQ2XXS) {
+        // the codes 43 + magnitude, and what turns each into 43 - magnitude (0x33, 0x44, 0x56 into 0x23, 0x12, 0x00)
+        const uint64_t g = BM_IQ2XXS_GRID[t];
+        const u32 s_lo = iq2_selectors((u32)g), s_hi = iq2_selectors((u32)(g >> 32));
+        v = make_uint4(__builtin_amdgcn_perm(0, kIq2Plus, s_lo), __builtin_amdgcn_perm(0, kIq2Plus, s_hi),
+                       __builtin_amdgcn_perm(0, kIq2Plus ^ kIq2Minus, s_lo), __builtin_amdgcn_perm(0, kIq2Plus ^ kIq2Minus, s_hi));
+    } else {
+        const u32 g = BM_IQ3XXS_GRID[t], plus = 0x40404040u + g, minus = 0x40404040u - g; // bytes 4 .. 62: both stay inside a byte
+        v = make_uint4(plus, minus, plus, minus);
+    }
+#pragma unroll
+    for (u32 c = 0; c < kUnits; c++) *reinterpret_cast<uint4 *>(lds + 256 * t + 16 * ((kUnits * part + c) ^ (t & 15))) = v;
+    if (threadIdx.x < 128) {
+        const uint2 m = iq_sign_masks((int)threadIdx.x);
+#pragma unroll
+        for (u32 c = 0; c < (u32)G::kSignCopies; c++)
+            *reinterpret_cast<uint2 *>(lds + G::kSignsAt + 8 * (threadIdx.x * G::kSignCopies + (c ^ ((threadIdx.x >> 3) % G::kSignCopies)))) = m;
+    }
 }
 
 // (T: how many of the workgroup's threads write them, no call to the built-in: blockDim.x is a load from the dispatch packet, in
@@ -61,8 +90,7 @@ __device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds, int T = 256) {
         for (int t = threadIdx.x; t < 256; t += T) {
             const uint64_t g = BM_IQ2XXS_GRID[t];
             const u32 lo = (u32)g, hi = (u32)(g >> 32);
-            // 0x08 -> 0, 0x19 -> 1, 0x2b -> 2: bit 0 of the byte is 1 for 0x19 and 0x2b, bit 1 for 0x2b only
-            grid[t] = make_uint2(((lo & 0x01010101u) + ((lo >> 1) & 0x01010101u)), ((hi & 0x01010101u) + ((hi >> 1) & 0x01010101u)));
+            grid[t] = make_uint2(iq2_selectors(lo), iq2_selectors(hi));
         }
         for (int t = threadIdx.x; t < 128; t += T) {
             const uint2 m = iq_sign_masks(t);
@@ -83,6 +111,16 @@ __device__ __forceinline__ Iq2Tables stage_tables(uint8_t *lds, int T = 256) {
         tb.signs = signs;
     }
     return tb;
+}
+
+template <int WT, bool WIDE, int T>
+__device__ __forceinline__ Iq2Tables stage_tables_as(uint8_t *lds) {
+    if constexpr (WIDE) {
+        stage_wide_tables<WT, T>(lds);
+        return Iq2Tables{nullptr, nullptr, nullptr};
+    } else {
+        return stage_tables<WT>(lds, T);
+    }
 }
 
 // `bytes` (a multiple of 8) from 8-byte aligned global memory to 8-byte aligned LDS, by the whole workgroup of T threads.
@@ -136,17 +174,17 @@ __device__ __forceinline__ void preload(Blk<WT> (&b)[U], const uint8_t *wrow, in
 // One stage: request super-block `ahead` into its ring slot, read the next stage's activation operands from LDS,
 // then the arithmetic of super-block i (ring slot `slot`). The asm statements pin that order: the compiler may
 // neither hoist the reads of later stages nor sink this stage's sums past them.
-template <int WT, int U, class Tap>
+template <int WT, int U, bool WIDE, class Tap>
 __device__ __forceinline__ void stage_one(Blk<WT> (&b)[U], int slot, int fill, const uint8_t *wrow, int ahead,
-                                          const ActView &av, int i, int act_next, int q, const Iq2Tables &tb,
-                                          Act<WT> &cur, float &a0, float &a1, const Tap &tap, bool fetch = true) {
+                                          const ActView &av, int i, int act_next, int q, Act<WT> &cur, float &a0,
+                                          float &a1, const Tap &tap, bool fetch = true) {
     __asm__ volatile("" ::: "memory");
     if (U > 1 && fetch) b[fill] = bm_load_blk<WT>(wrow, ahead, q);
     const Act<WT> next = bm_load_act<WT, Tap::kActive>(av, act_next, q);
     __asm__ volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     if (U == 1) b[0] = bm_load_blk<WT>(wrow, i, q);
-    bm_dot_blk<WT>(b[slot], cur, i, q, tb, a0, a1, tap);
+    bm_dot_blk<WT, WIDE>(b[slot], cur, i, q, a0, a1, tap);
     __asm__ volatile("" : "+v"(a0), "+v"(a1)::"memory");
     __builtin_amdgcn_sched_barrier(0);
     cur = next;
@@ -156,7 +194,8 @@ __device__ __forceinline__ void stage_one(Blk<WT> (&b)[U], int slot, int fill, c
 // NB > 0: the row has NB super-blocks, the stages are unrolled; NB == 0: it has nb, of which with M = 1 the stages behind the
 // last whole ring take what U leaves over; with M > 1 nb is a multiple of U (a remainder's stages beside the loop's slowed the loop by 1 to 2 %).
 // Indices past the row's end are clamped onto its last super-block: a redundant read, no branch in the stream.
-template <int WT, int U, int NB, int M, class Tap>
+// WIDE: the IQ tables lie in LDS in copies (IqGeom; one column only).
+template <int WT, int U, int NB, int M, bool WIDE = false, class Tap>
 __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, const uint8_t *cols, int col_stride,
                                         int m, int nb, int q, const Iq2Tables &tb, float (&out)[M], const Tap &tap) {
     float a0[M], a1[M];
@@ -173,7 +212,7 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
 #pragma unroll
             for (int i = 0; i < NB; i++) {
                 const int ahead = i + U - 1 < NB ? i + U - 1 : NB - 1;
-                stage_one<WT, U>(b, i % U, (i + U - 1) % U, wrow, ahead, av[0], i, i + 1 < NB ? i + 1 : i, q, tb, cur,
+                stage_one<WT, U, WIDE>(b, i % U, (i + U - 1) % U, wrow, ahead, av[0], i, i + 1 < NB ? i + 1 : i, q, cur,
                                  a0[0], a1[0], tap, i + U - 1 < NB); // the count is known here: nothing is asked for past the end
             }
         } else {
@@ -183,14 +222,14 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
                 for (int u = 0; u < U; u++) {
                     const int i = i0 + u;
                     const int ahead = i + U - 1 < n ? i + U - 1 : n - 1;
-                    stage_one<WT, U>(b, u, (u + U - 1) % U, wrow, ahead, av[0], i, i + 1 < n ? i + 1 : i, q, tb, cur,
+                    stage_one<WT, U, WIDE>(b, u, (u + U - 1) % U, wrow, ahead, av[0], i, i + 1 < n ? i + 1 : i, q, cur,
                                      a0[0], a1[0], tap);
                 }
             }
 #pragma unroll
             for (int u = 0; u + 1 < U; u++) // what U leaves over stands in the ring
                 if (i0 + u < n)
-                    stage_one<WT, U>(b, u, u, wrow, 0, av[0], i0 + u, i0 + u + 1 < n ? i0 + u + 1 : i0 + u, q, tb, cur, a0[0], a1[0], tap,
+                    stage_one<WT, U, WIDE>(b, u, u, wrow, 0, av[0], i0 + u, i0 + u + 1 < n ? i0 + u + 1 : i0 + u, q, cur, a0[0], a1[0], tap,
                                      false);
         }
     } else {
@@ -198,22 +237,13 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
         auto stage = [&](int slot, int fill, int i) {
             const int ahead = i + U - 1 < n ? i + U - 1 : n - 1;
             if (NB == 0 || U == 1 || i + U - 1 < NB) b[fill] = bm_load_blk<WT>(wrow, U > 1 ? ahead : i, q);
-            if constexpr (WT == BM_IQ2XXS) { // the table lookups once, not once a column
-                const Iq2Dec dec = bm_decode_iq2xxs<false>(b[slot], q, tb);
+            if constexpr (WT == BM_IQ2XXS || WT == BM_IQ3XXS) { // the table lookups once, not once a column
+                Iq2Dec dec;
+                if constexpr (WT == BM_IQ2XXS) dec = bm_decode_iq2xxs(b[slot], q, tb);
+                else dec = bm_decode_iq3xxs(b[slot], q, tb);
 #pragma unroll
                 for (int c = 0; c < M; c++)
-                    if (c < m) {
-                        const Act<WT> a = bm_load_act<WT, Tap::kActive>(av[c], i, q);
-                        bm_dot_iq2xxs_dec(b[slot], dec, a, i, q, a0[c], a1[c], tap);
-                    }
-            } else if constexpr (WT == BM_IQ3XXS) {
-                const Iq2Dec dec = bm_decode_iq3xxs<false>(b[slot], q, tb);
-#pragma unroll
-                for (int c = 0; c < M; c++)
-                    if (c < m) {
-                        const Act<WT> a = bm_load_act<WT, Tap::kActive>(av[c], i, q);
-                        bm_dot_iq3xxs_dec(b[slot], dec, a, i, q, a0[c], a1[c], tap);
-                    }
+                    if (c < m) bm_dot_iqx_across(b[slot], dec, bm_act_iqx<false>(av[c], i, q), a0[c], a1[c]);
             } else if constexpr (WT == BM_IQ4XS) { // likewise the level permutes
                 const Iq4Dec dec = bm_decode_iq4xs(b[slot], q);
 #pragma unroll
@@ -245,7 +275,7 @@ __device__ __forceinline__ void row_dot(Blk<WT> (&b)[U], const uint8_t *wrow, co
                 for (int c = 0; c < M; c++)
                     if (c < m) {
                         const Act<WT> a = bm_load_act<WT, Tap::kActive>(av[c], i, q);
-                        bm_dot_blk<WT>(b[slot], a, i, q, tb, a0[c], a1[c], tap);
+                        bm_dot_blk<WT, false>(b[slot], a, i, q, a0[c], a1[c], tap);
                     }
             }
         };
@@ -759,7 +789,11 @@ constexpr int kRingQ4K = 4, kRingQ5K = 4, kRingQ6K = 3, kRing = 2;
 #define BM_DISPATCH(wtype, nb) BM_DISPATCH_BY(wtype, nb, BM_REST_ANY)
 #define BM_DISPATCH_COLS(wtype, nb) BM_DISPATCH_BY(wtype, nb, BM_REST_COLS)
 
-static inline int tab_bytes_rt(int wtype) { return wtype == BM_IQ2XXS ? kTabBytes : wtype == BM_IQ3XXS ? kTabBytes3 : 0; }
+static inline int tab_bytes_rt(int wtype, bool wide = false) {
+    if (wtype == BM_IQ2XXS) return wide ? tab_bytes<BM_IQ2XXS, true>() : tab_bytes<BM_IQ2XXS>();
+    if (wtype == BM_IQ3XXS) return wide ? tab_bytes<BM_IQ3XXS, true>() : tab_bytes<BM_IQ3XXS>();
+    return 0;
+}
 
 } // namespace bmk
 

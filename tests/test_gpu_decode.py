@@ -655,6 +655,67 @@ def test_fused_step_with_larger_down_workgroups(gpu, types, hidden, ff, m, top_k
     L.free()
 
 
+# Gate . up of the IQ types with a table in LDS: up to 256 blocks of 32 row pairs the tables as they are, beyond in copies and 64 row pairs a
+# workgroup (here 256 and 264; one row block a slot more than the others that holds 8 or 40 rows; by dies with the last eight blocks not
+# whole), with slots that are served elsewhere and refused ones. The down half of 512 and 1024 threads takes the copies as well.
+@pytest.mark.parametrize("types,hidden,ff,m,top_k", (
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 512, 256, 32, 1),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 512, 256, 33, 1),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.Q6_K), 768, 768, 6, 2),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ3_XXS), 256, 512, 16, 4),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 256, 3328, 10, 7),
+))
+def test_fused_step_with_tables_in_copies(gpu, types, hidden, ff, m, top_k):
+    n_experts = 8
+    L = Layer(gpu, types, hidden, ff, n_experts, 670 + hidden + ff, cheap=ff > 2048)
+    rng = np.random.default_rng(671)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    gpu.fault_clear()
+    y, h, _, _ = run_fused_step(gpu, L, x, ids, wts, top_k, resid)
+    want_y, want_h = L.oracle(x, ids, wts, top_k)
+    assert_f32(h, want_h, "h")
+    assert_f32(y, (want_y.reshape(m, hidden) + resid).astype(np.float32).reshape(-1), "y + resid")
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    L.free()
+
+
+@pytest.mark.parametrize("wtype,k,rpe,n_slots", ((bm.IQ2_XXS, 512, 72, 85), (bm.IQ2_XXS, 512, 72, 86), (bm.IQ3_XXS, 768, 104, 65),
+                                                 (bm.IQ3_XXS, 1280, 256, 33)))
+def test_gate_up_with_tables_in_copies(gpu, wtype, k, rpe, n_slots):
+    rng = np.random.default_rng(680)
+    n_experts, kinds = 5, 3
+    wg, wu = stack(wtype, n_experts * rpe, k, 681), stack(wtype, n_experts * rpe, k, 682)
+    cols = [normal_f32(rng, k) for _ in range(kinds)]
+    dots = [[ora.gemv(wtype, w, n_experts * rpe, k, ora.quantize_col(wtype, c), 1).reshape(n_experts, rpe) for c in cols] for w in (wg, wu)]
+    sel = rng.integers(0, n_experts, n_slots).astype(np.uint32)
+    sel[[1, n_slots - 2]] = bm.HOST_SLOT, n_experts # served elsewhere; refused
+    dg, du, act = gpu.weights(wtype, n_experts * rpe, k, wg), gpu.weights(wtype, n_experts * rpe, k, wu), gpu.act(wtype, k, n_slots)
+    xd, seld = gpu.upload(np.stack([cols[s % kinds] for s in range(n_slots)]), np.float32), gpu.upload(sel, np.uint32)
+    h = gpu.buffer(np.float32, n_slots * rpe)
+    h.upload(np.full(n_slots * rpe, 7.0, np.float32))
+    act_h = gpu.act(bm.Q6_K, rpe, n_slots) if rpe % 256 == 0 else None
+    gpu.fault_clear()
+    gpu.enqueue_quantize(xd, n_slots, act)
+    gpu.enqueue_gate_up(dg, du, act, seld, n_slots, rpe, 1, h, act_h)
+    got = h.download().reshape(n_slots, rpe)
+    assert gpu.fault()[1] == 1 << bm.SITE_EXPERT_ID
+    gpu.fault_clear()
+    for s in range(n_slots):
+        e, c = int(sel[s]), s % kinds
+        if e == bm.HOST_SLOT:
+            assert (got[s] == 7.0).all()
+        elif e >= n_experts:
+            assert np.isnan(got[s]).all()
+        else:
+            want = ora.swiglu(dots[0][c][e], dots[1][c][e])
+            assert_f32(got[s], want, f"slot {s}")
+            if act_h is not None:
+                assert np.array_equal(act_h.download(s), ora.quantize_col(bm.Q6_K, want)), f"act_h slot {s}"
+    for b in (dg, du, act, xd, seld, h) + (() if act_h is None else (act_h,)):
+        b.free()
+
+
 def test_fused_step_at_the_token_limit(gpu):
     """bm_moe_decode takes 1..=1024 tokens a launch: the limit itself against the oracle, one more refused by name."""
     L = Layer(gpu, (bm.Q4_K, bm.Q4_K, bm.Q6_K), 256, 256, 9, 650)
