@@ -940,11 +940,10 @@ int bm_scratch_create(bm_ctx *ctx, int gate_type, int down_type, int hidden, int
     // the per-slot step below 22 tokens (Q4_K gate/up, Q6_K down, top-8 of 128, hidden 2048, ff 768, us a step, per slot / grouped:
     // 16 tokens 63 / 81, 24: 85 / 84, 128: 328 / 177), then by path_choice
     s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 0;
-    // Where both stacks are on Q8_K columns and the experts are large, the grouped step - for few slots an
-    // expert the per-slot gate . up launch and the down tiles, see bm_moe_forward - is ahead of the per-slot step from the first
-    // token: every workgroup of the per-slot down launch encodes all of a token's h rows itself, work that grows with hidden x ff
-    // (DeepSeek-V3 shape, hidden 7168, ff 2048, IQ2_XXS, us a step per slot / grouped: 1 token 61.5 / 57.9, 4 tokens 171 / 147,
-    // 16 tokens 589 / 481; at hidden 2048, ff 768 the per-slot step leads up to 12 tokens: 1 token 16.0 / 23.7)
+    // Where both stacks are on Q8_K columns and the experts are large, the grouped step (slot by slot at few slots, see slot_by_slot) is ahead of the
+    // per-slot step from the first token: every workgroup of the per-slot down launch encodes all of a token's h rows itself, work that grows
+    // with hidden x ff (DeepSeek-V3 shape, hidden 7168, ff 2048, IQ2_XXS, us a step per slot / grouped: 1 token 61.5 / 57.9, 4 tokens 171 /
+    // 147, 16 tokens 589 / 481; at hidden 2048, ff 768 the per-slot step leads up to 12 tokens: 1 token 16.0 / 23.7)
     if (act_form(gate_type) != 0 && act_form(down_type) != 0 && (int64_t)hidden * ff >= ((int64_t)1 << 23)) s->grouped_from = 1;
     const size_t slots = (size_t)max_tokens * n_slots_per_token;
     int rc = bm_act_create(ctx, gate_type, hidden, max_tokens, &s->act_x);
@@ -1035,6 +1034,23 @@ static bool gemm_ahead(const bm_scratch *s, int m) {
     return tiles > line.launches + line.die * v * std::ceil(std::max(experts, n / 64 + experts / 2) / 8);
 }
 
+// Whether a step of both stacks on Q8_K columns goes slot by slot through launches of its own: the columns quantized once, gate . up and down a
+// workgroup a slot's rows.
+// In place of the grouped step's tiles: the one-column walks (activation operands read a super-block ahead, the IQ tables in copies) are that
+// much cheaper than the tile launches' that rows read again for another slot of their expert cost less than tiles of few slots, as long as the
+// caches serve most of them: up to 500 MB of rows asked for, repeats and all, or with no more slots than experts. (650 random layers of 0.7 to 8
+// slots an expert, cold weights, over the tile launches: 0.83 on average, 1.03 at worst, and 2.5 % behind the better of the two; by MB asked
+// for 0.7 up to 128, 0.8 to 500, 0.95 to 768, 1.2 beyond; the large IQ2_XXS layer, 4 tokens, 175 -> 155 us with the shared expert and the router.)
+// In place of the per-slot step's two launches, where they ask for 128 MB or more: there every workgroup quantizes the columns it reads itself, which
+// three launches more cost less than by then (over it, by MB: 1.1 at 32, 1.05 at 64, 0.98 at 128 to 256, 0.92 beyond; 280 random layers below 22 tokens).
+static bool slot_by_slot(const bm_scratch *s, int m, int path) {
+    if (act_form(s->gate_type) == 0 || act_form(s->down_type) == 0 || m > bmk::kMaxDecodeTokens || !per_slot_fits(s)) return false;
+    const int64_t slots = (int64_t)m * s->spt;
+    const int64_t asked = slots * (2 * s->ff * bm_row_bytes(s->gate_type, s->hidden) + s->hidden * bm_row_bytes(s->down_type, s->ff));
+    if (path == BM_PATH_PER_SLOT && asked < 128000000) return false;
+    return path != BM_PATH_GEMM && (slots <= s->n_experts || asked <= 500000000);
+}
+
 // The path a call with m tokens takes, and the f32 order of its GEMMs: the one place where it is chosen.
 struct PathChoice {
     int path, mode;
@@ -1075,31 +1091,26 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     if (m < 1 || m > s->max_tokens) return fail(ctx, BM_ESHAPE, "%s: m = %d tokens, the scratch holds 1..=%d", what, m, s->max_tokens);
     const int spt = s->spt, n_slots = m * spt, hidden = s->hidden, ff = s->ff, n_experts = s->n_experts;
     const bool down_q8k = act_form(s->down_type) != 0;
+    auto combine = [&] { // the slots' weighted sum; a slot that names no expert of the stack adds nothing, as in the per-slot path
+        return driver(ctx, what, bmk::combine_tokens(launch_of(ctx), s->down, w_dev, nullptr, resid_dev, hidden, spt, m, y_dev, sel_dev,
+                                                     (uint32_t)n_experts));
+    };
     const PathChoice choice = path_choice(s, m);
+    if (((uintptr_t)x_dev & 15) == 0 && slot_by_slot(s, m, choice.path)) { // (the other steps take such an x, or refuse it)
+        int rc = bm_quantize(ctx, x_dev, m, s->act_x);
+        if (!rc) rc = bm_gate_up(ctx, wg, wu, s->act_x, sel_dev, n_slots, ff, spt, rule, s->g, nullptr);
+        if (!rc) // (a slot without an expert of the stack: its rows of h hold nothing, its column is left alone)
+            rc = driver(ctx, what, bmk::quantize(launch_of(ctx), s->down_type, s->g, n_slots, ff, s->act_h->dev, nullptr, sel_dev,
+                                                 (uint32_t)n_experts));
+        if (!rc) rc = bm_gemv_sel(ctx, wd, s->act_h, sel_dev, n_slots, hidden, s->down);
+        if (!rc) rc = combine();
+        return rc;
+    }
     switch (choice.path) {
     case BM_PATH_PER_SLOT:
         return bm_moe_decode(ctx, wg, wu, wd, x_dev, sel_dev, w_dev, resid_dev, spt, m, rule, s->act_h, nullptr,
                              down_q8k ? s->g : nullptr, y_dev);
     case BM_PATH_GROUPED: {
-        // Few slots an expert (no more slots than experts: nearly every tile is one slot) and h on its way through f32 rows:
-        // the per-slot gate . up launch is the faster one there (its one-column walk reads the activation operands a
-        // super-block ahead: 83 against 102 us at the DeepSeek-V3 shape, 4 tokens) and the tile launch the faster down (54
-        // against 84 us), so the step takes one of each; the down tiles then read their columns in slot order. The tokens'
-        // columns are quantized once, beside the tables in their launch, not by every workgroup of the gate . up launch
-        // (whose vector ALU is what bounds it at these types: 180 -> 172 us a step).
-        if (down_q8k && act_form(s->gate_type) != 0 && n_slots <= n_experts && m <= bmk::kMaxDecodeTokens && per_slot_fits(s) &&
-            n_experts <= bmk::kBucketExperts && n_slots <= bmk::kTileMaxSlots) {
-            int rc = bm_tables_quantize(ctx, sel_dev, n_slots, n_experts, s->order, s->start, s->tiles, x_dev, m, s->act_x);
-            if (!rc) rc = bm_gate_up(ctx, wg, wu, s->act_x, sel_dev, n_slots, ff, spt, rule, s->g, nullptr);
-            if (!rc) // (a slot without an expert of the stack: its rows of h hold nothing, its column is left alone)
-                rc = driver(ctx, what, bmk::quantize(launch_of(ctx), s->down_type, s->g, n_slots, ff, s->act_h->dev, nullptr, sel_dev,
-                                                     (uint32_t)n_experts));
-            if (!rc)
-                rc = driver(ctx, what, bmk::gemv_tiles(launch_of(ctx), wd->wtype, wd->dev, n_experts, ff, s->act_h->dev, s->order, s->start,
-                                                       s->tiles, n_slots, hidden, s->down, true));
-            if (rc) return rc;
-            break;
-        }
         int rc = bm_tables_quantize(ctx, sel_dev, n_slots, n_experts, s->order, s->start, s->tiles, x_dev, m, s->act_x);
         if (!rc && !down_q8k)
             rc = bm_gate_up_tiles(ctx, wg, wu, s->act_x, s->order, s->start, s->tiles, n_slots, ff, spt, rule, nullptr, s->act_h);
@@ -1120,9 +1131,7 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
         break;
     }
     }
-    // the slots' weighted sum; a slot that names no expert of the stack adds nothing, as in the per-slot path
-    return driver(ctx, what, bmk::combine_tokens(launch_of(ctx), s->down, w_dev, nullptr, resid_dev, hidden, spt, m, y_dev, sel_dev,
-                                                 (uint32_t)n_experts));
+    return combine();
 }
 
 // crates/gpu/src/kquant/act.rs:71-125 Act::code: what the device rules can run, refused by name otherwise.

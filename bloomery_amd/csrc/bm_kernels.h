@@ -118,7 +118,7 @@ hipError_t gate_up_tiles(const Launch &L, int wtype, const uint8_t *wg, const ui
                          uint8_t *act_h);
 hipError_t gemv_tiles(const Launch &L, int wtype, const uint8_t *w, int n_experts, int k, const uint8_t *act,
                       const uint32_t *order, const uint32_t *start, const uint32_t *tiles, int n_slots,
-                      int rows_per_expert, float *y, bool by_slot = false);
+                      int rows_per_expert, float *y);
 
 // ------------------------------------------------------------------------------------- prefill (bm_prefill.hip)
 

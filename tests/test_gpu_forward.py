@@ -22,7 +22,7 @@ PATHS = ((bm.PATH_PER_SLOT, "per slot"), (bm.PATH_GROUPED, "grouped"), (bm.PATH_
     ((bm.IQ4_XS, bm.IQ4_XS, bm.Q3_K), 512, 512, 5, 3, 25),   # the added types through the GEMM path as well
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.Q6_K), 768, 256, 4, 2, 18),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 512, 512, 40, 4, 6),  # no more slots than experts, Q8_K columns on both sides: the
-    ((bm.IQ4_XS, bm.IQ4_XS, bm.Q3_K), 512, 256, 64, 3, 7),       # grouped path's per-slot gate . up launch and slot-ordered down tiles
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.Q3_K), 512, 256, 64, 3, 7),       # grouped path's launches go slot by slot
 ))
 def test_every_path_gives_the_oracles_bits(gpu, types, hidden, ff, n_experts, top_k, m):
     L = Layer(gpu, types, hidden, ff, n_experts, 5100 + hidden)
@@ -49,6 +49,37 @@ def test_every_path_gives_the_oracles_bits(gpu, types, hidden, ff, n_experts, to
             assert_f32(y.download()[:3 * hidden], want[:3 * hidden], f"{name}, three tokens")
         assert gpu.fault() == (bm.FAULT_NONE, 0)
     finally:
+        sc.free()
+        for b in (xd, sel, wd, rd, y):
+            b.free()
+        L.free()
+
+
+@pytest.mark.parametrize("m", (19, 20))
+def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
+    """Stacks on Q8_K columns whose rows are 6.7 MB an expert: 20 slots ask for 128 MB, from where the per-slot step quantizes its columns in
+    launches of their own. One slot is served elsewhere and one names no expert; neither adds anything."""
+    hidden, ff, n_experts, top_k = 2048, 2048, 8, 1
+    L = Layer(gpu, (bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), hidden, ff, n_experts, 5200, cheap=True)
+    rng = np.random.default_rng(5201)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    want_y, _ = L.oracle(x, ids, wts, top_k)
+    want = (want_y.reshape(m, hidden) + resid).astype(np.float32)
+    ids[2], ids[5] = bm.HOST_SLOT, n_experts
+    want[[2, 5]] = resid[[2, 5]]
+    xd, sel, wd, rd = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.upload(wts, np.float32), gpu.upload(resid, np.float32)
+    y = gpu.buffer(np.float32, m * hidden).fill_bytes(0xFF)
+    sc = gpu.scratch(bm.IQ4_XS, bm.IQ4_XS, hidden, ff, n_experts, top_k, 32)
+    gpu.fault_clear()
+    try:
+        assert sc.path_for(m) == bm.PATH_PER_SLOT
+        for _ in range(2):
+            gpu.enqueue_moe_forward(sc, L.dg, L.du, L.dd, xd, sel, wd, rd, m, y)
+            assert_f32(y.download(), want.reshape(-1), "y")
+        assert gpu.fault()[1] == 1 << bm.SITE_EXPERT_ID
+    finally:
+        gpu.fault_clear()
         sc.free()
         for b in (xd, sel, wd, rd, y):
             b.free()
