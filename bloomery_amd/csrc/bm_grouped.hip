@@ -93,9 +93,10 @@ __global__ __launch_bounds__(1024) void k_tables_quant(const u32 *sel, u32 n_slo
             if (b >= m * (k / 256)) return; // whole waves leave
             q8k_wave_block(*reinterpret_cast<const float4 *>(x + (size_t)b * 256 + 4 * lane), act + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
         } else {
-            const long at = ((long)(blockIdx.x - 1) * 1024 + threadIdx.x) * 8;
-            if (at >= (long)m * k) return; // whole quads leave: a block is 32 values, k a multiple of 256
-            const int col = (int)(at / k), o = (int)(at % k);
+            const u32 i = (blockIdx.x - 1u) * 1024u + threadIdx.x, line = (u32)k / 8u;
+            if (i >= (u32)m * line) return; // whole quads leave: a block is 32 values, k a multiple of 256
+            const int col = (int)(i / line), o = 8 * (int)(i % line);
+            const size_t at = (size_t)i * 8;
             const float4 a = *reinterpret_cast<const float4 *>(x + at), b = *reinterpret_cast<const float4 *>(x + at + 4);
             const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
             q82_quad8(v, act + (size_t)col * (k / 256) * BM_Q82_SB_EXT, k / 256, o >> 5, threadIdx.x & 3, fault, layer);

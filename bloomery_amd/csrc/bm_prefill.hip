@@ -50,9 +50,10 @@ __global__ __launch_bounds__(kRouteThreads) void k_route(const u32 *ids, u32 n_s
             if (b >= m * (k / 256)) return; // whole waves leave
             q8k_wave_block(*reinterpret_cast<const float4 *>(x + (size_t)b * 256 + 4 * lane), act + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
         } else {
-            const long at = ((long)qb * kRouteThreads + threadIdx.x) * 8;
-            if (at >= (long)m * k) return; // whole quads leave: a block is 32 values, k a multiple of 256
-            const int col = (int)(at / k), o = (int)(at % k);
+            const u32 i = qb * kRouteThreads + threadIdx.x, line = (u32)k / 8u;
+            if (i >= (u32)m * line) return; // whole quads leave: a block is 32 values, k a multiple of 256
+            const int col = (int)(i / line), o = 8 * (int)(i % line);
+            const size_t at = (size_t)i * 8;
             const float4 a = *reinterpret_cast<const float4 *>(x + at), b = *reinterpret_cast<const float4 *>(x + at + 4);
             const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
             q82_quad8(v, act + (size_t)col * (k / 256) * BM_Q82_SB_EXT, k / 256, o >> 5, threadIdx.x & 3, fault, layer);
@@ -121,12 +122,11 @@ __device__ __forceinline__ bool swiglu_column_skipped(const u32 *sel, u32 n_expe
 
 __global__ __launch_bounds__(256) void k_swiglu_quant(const float *g, const float *u, int m, int k, uint8_t *act,
                                                       GateRule rule, const u32 *sel, u32 n_experts, u32 *fault, u32 layer) {
-    const int bpc = k / 32;
-    const long gblk = (long)blockIdx.x * 8 + (threadIdx.x >> 5);
-    if (gblk >= (long)m * bpc) return;
+    const u32 bpc = (u32)k / 32u, gblk = blockIdx.x * 8u + (threadIdx.x >> 5);
+    if (gblk >= (u32)m * bpc) return;
     const int col = (int)(gblk / bpc), blk = (int)(gblk % bpc), lane32 = threadIdx.x & 31;
     if (swiglu_column_skipped(sel, n_experts, col, blk == 0 && lane32 == 0, fault, layer)) return; // uniform over the half wave
-    const size_t at = (size_t)col * k + 32 * blk + lane32;
+    const size_t at = (size_t)gblk * 32 + lane32;
     bool odd;
     const float v = bm_gate_rule(rule.act, rule.limit, g[at], u[at], odd);
     if (odd) bm_raise(fault, layer, kSiteF32Product);
@@ -163,9 +163,11 @@ __global__ __launch_bounds__(256) void k_swiglu_quant_q8k(const float *g, const 
 // The Q8_2_X4 form with eight values a thread, a block a quad of lanes: two 16-byte loads of each input a thread.
 __global__ __launch_bounds__(256) void k_swiglu_quant_wide(const float *g, const float *u, int m, int k, uint8_t *act,
                                                            GateRule rule, const u32 *sel, u32 n_experts, u32 *fault, u32 layer) {
-    const long at = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
-    if (at >= (long)m * k) return;
-    const int col = (int)(at / k), o = (int)(at % k);
+    // (thread numbers fit 32 bits, as a grid's threads do; a division of 64 bits takes some hundred and fifty instructions)
+    const u32 i = blockIdx.x * 256u + threadIdx.x, line = (u32)k / 8u;
+    if (i >= (u32)m * line) return;
+    const int col = (int)(i / line), o = 8 * (int)(i % line);
+    const size_t at = (size_t)i * 8;
     if (swiglu_column_skipped(sel, n_experts, col, o == 0, fault, layer)) return; // uniform over a block's quad of lanes
     const float4 g0 = *reinterpret_cast<const float4 *>(g + at), g1 = *reinterpret_cast<const float4 *>(g + at + 4);
     const float4 u0 = *reinterpret_cast<const float4 *>(u + at), u1 = *reinterpret_cast<const float4 *>(u + at + 4);
@@ -174,9 +176,9 @@ __global__ __launch_bounds__(256) void k_swiglu_quant_wide(const float *g, const
     float v[8];
     bool any_odd = false;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int j = 0; j < 8; j++) {
         bool odd;
-        v[i] = bm_gate_rule(rule.act, rule.limit, gv[i], uv[i], odd);
+        v[j] = bm_gate_rule(rule.act, rule.limit, gv[j], uv[j], odd);
         any_odd |= odd;
     }
     if (any_odd) bm_raise(fault, layer, kSiteF32Product);

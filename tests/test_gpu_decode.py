@@ -1063,6 +1063,23 @@ def test_combine_adds_the_residual(gpu):
         b.free()
 
 
+@pytest.mark.parametrize("n_slots", [1, 2, 3, 4, 5, 6, 7, 8, 9, 15, 16, 23])
+@pytest.mark.parametrize("rows, m", [(2048, 3), (37, 5), (1030, 255), (2048, 129), (260, 1031)])
+def test_combine_takes_slots_in_batches(gpu, rows, m, n_slots):
+    # batches of eight slots and what is left by halves; a value a thread, or four from 2^18 values on where rows allow it
+    rng = np.random.default_rng(rows + n_slots)
+    down, w = normal_f32(rng, m * n_slots * rows), normal_f32(rng, m * n_slots)
+    shexp, resid = normal_f32(rng, m * rows), normal_f32(rng, m * rows)
+    bufs = [gpu.upload(v) for v in (down, w, shexp, resid)]
+    y = gpu.buffer(np.float32, m * rows)
+    gpu.enqueue_combine_tokens(bufs[0], bufs[1], bufs[3], rows, n_slots, m, y)
+    assert_f32(y.download(), ora.combine_tokens(down, w, resid, rows, n_slots, m), "combine + resid")
+    gpu.enqueue_moe_combine(*bufs, rows, n_slots, m, y)
+    assert_f32(y.download(), ora.moe_combine(down, w, shexp, resid, rows, n_slots, m), "moe_combine")
+    for b in bufs + [y]:
+        b.free()
+
+
 def test_shape_refusals_are_named(gpu):
     # crates/gpu/src/q4k_sel.rs:990-1042: refused on the host, before any launch, with the entry point's name
     w4 = gpu.weights(bm.Q4_K, 64, 512, np.zeros(64 * bm.row_bytes(bm.Q4_K, 512), np.uint8))
