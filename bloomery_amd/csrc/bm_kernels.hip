@@ -809,29 +809,38 @@ __global__ __launch_bounds__(256) void k_gate_up_x(const float *x, const uint8_t
 // ------------------------------------------------------------- the fused step for the types that take Q8_K columns
 
 // `cols` columns of nb blocks each, f32 rows at x (column c at x + c * nb * 256), into LDS at `dst` by the workgroup's
-// waves, block by block. T: the workgroup's thread count.
-template <int T = 256>
-__device__ __forceinline__ void q8k_stage_cols(const float *x, uint8_t *dst, int cols, int nb, u32 *fault, u32 layer,
-                                               const u32 *ids = nullptr, u32 n_experts = 0) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int n_waves = T / 64;
-    const int total = cols * nb;
-    constexpr int kAhead = T == 256 ? 6 : T == 512 ? 3 : 2; // blocks whose loads a wave has in flight
-    for (int b0 = wave; b0 < total; b0 += kAhead * n_waves) {
-        float4 x4[kAhead];
-#pragma unroll
-        for (int u = 0; u < kAhead; u++) {
-            const int b = b0 + u * n_waves;
-            x4[u] = *reinterpret_cast<const float4 *>(x + (size_t)(b < total ? b : b0) * 256 + 4 * lane);
-        }
-#pragma unroll
-        for (int u = 0; u < kAhead; u++) {
-            const int b = b0 + u * n_waves;
-            // with ids: a column whose slot is not live is not encoded (its rows may hold anything)
-            if (b < total && (!ids || ids[b / nb] < n_experts)) q8k_wave_block(x4[u], dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
-        }
+// waves, block by block. In two steps, as Q82Cols below: a wave's first kAhead blocks are requested in front of the weight rows (memory
+// answers in order: asked for behind them, the quantizer began when the rows were there), and encoded while those are on their way. (us a
+// launch: 5 tokens x 8 slots of 768 values, IQ4_XS down rows 16.0 -> 13.8.)
+// T: the workgroup's thread count.
+template <int T>
+struct Q8kCols {
+    static constexpr int kWaves = T / 64, kAhead = T == 256 ? 6 : T == 512 ? 3 : 2;
+    float4 x4[kAhead];
+    __device__ __forceinline__ static int wave() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+    __device__ __forceinline__ static float4 block(const float *x, int b) {
+        return *reinterpret_cast<const float4 *>(x + (size_t)b * 256 + 4 * (threadIdx.x & 63));
     }
-}
+    __device__ __forceinline__ void load(const float *x, int cols, int nb) {
+#pragma unroll
+        for (int u = 0; u < kAhead; u++)
+            if (wave() + u * kWaves < cols * nb) x4[u] = block(x, wave() + u * kWaves);
+        __asm__ volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // `live` (a column's number): a column whose slot is not live is not encoded (its rows may hold anything)
+    template <class Live>
+    __device__ __forceinline__ void encode(const float *x, uint8_t *dst, int cols, int nb, u32 *fault, u32 layer, Live live) const {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const int b = wave() + u * kWaves;
+            if (b < cols * nb && live(b / nb)) q8k_wave_block(x4[u], dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
+        }
+        for (int b = wave() + kAhead * kWaves; b < cols * nb; b += kWaves)
+            if (live(b / nb)) q8k_wave_block(block(x, b), dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
+    }
+};
 
 // `cols` columns of nb super-blocks each, f32 rows at x (column c at x + c * nb * 256), into LDS at `dst` as Q8_2_X4
 // columns with their tables: a 32-value block is four consecutive lanes of eight values. In two steps, for a workgroup
@@ -899,6 +908,8 @@ __global__ __launch_bounds__(T) void k_gate_up_xq(const float *x, const uint8_t 
     const int hidden = na * 256, ff = nh * 256;
     const int r0 = rb * (T / 8), r = r0 + (tid >> 3);
     if (T > 256 && r0 >= ff) return; // (by dies, the last eight blocks need not be whole)
+    Q8kCols<T> xrow;
+    xrow.load(x + (size_t)t * hidden, 1, na);
     const u32 id = sel[slot];
     uint8_t *hcol = act_h ? act_h + (size_t)slot * nh * BM_Q82_SB_EXT : nullptr;
     if (id >= n_experts) { // uniform over the workgroup
@@ -915,7 +926,7 @@ __global__ __launch_bounds__(T) void k_gate_up_xq(const float *x, const uint8_t 
     const Iq2Tables tb = stage_tables_as<WA, WIDE, T>(lds);
     uint8_t *col = lds + tab_bytes<WA, WIDE>();
     const int col_bytes = bm_act_col_bytes<WA>(na);
-    q8k_stage_cols<T>(x + (size_t)t * hidden, col, 1, na, fault, layer);
+    xrow.encode(x + (size_t)t * hidden, col, 1, na, fault, layer, [](int) { return true; });
     __syncthreads();
     if (act_x && rb == 0 && slot % spt == 0) stage_bytes<T>(act_x + (size_t)t * col_bytes, col, col_bytes);
     float v[1];
@@ -948,10 +959,13 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
     const int col_bytes = bm_act_col_bytes<WT>(n);
     const uint8_t *wrow = w + (size_t)(active ? row : 0) * row_bytes;
     const float *xc = x + (size_t)c * k;
-    // the column's first 2048 values are asked for in front of the rows: vector loads come back in the order they were asked
+    // the column's first values (2048, or 6144) are asked for in front of the rows: vector loads come back in the order they were asked
     // for, and behind the rows' requests the quantizer would wait for those as well
     float4 x_lo = make_float4(0, 0, 0, 0), x_hi = x_lo;
-    if constexpr (!bm_takes_q8k(WT)) {
+    [[maybe_unused]] Q8kCols<256> xcol;
+    if constexpr (bm_takes_q8k(WT)) {
+        xcol.load(xc, 1, n);
+    } else {
         const int o = tid * 8 < k ? tid * 8 : k - 8;
         x_lo = *reinterpret_cast<const float4 *>(xc + o), x_hi = *reinterpret_cast<const float4 *>(xc + o + 4);
         __asm__ volatile("" ::: "memory");
@@ -962,7 +976,7 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *col = lds + tab_bytes<WT>();
     if constexpr (bm_takes_q8k(WT)) {
-        q8k_stage_cols(xc, col, 1, n, fault, layer);
+        xcol.encode(xc, col, 1, n, fault, layer, [](int) { return true; });
     } else { // a q8_2 block is four lanes of eight values; 2048 values a pass
         if (tid * 8 < k) {
             const float v8[8] = {x_lo.x, x_lo.y, x_lo.z, x_lo.w, x_hi.x, x_hi.y, x_hi.z, x_hi.w};
@@ -999,12 +1013,13 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     const int r = rb * D + dl;
     const int n = NB > 0 ? NB : nb;
     const u32 id = sel[t * spt + e];
-    // Q8_2_X4 columns: the token's f32 rows of h are asked for before anything that waits for the expert id, so they
-    // arrive with it and are encoded while the weight rows are on their way
-    Q82Cols<4, T> hrows;
-    if constexpr (!bm_takes_q8k(WT)) hrows.load(h + (size_t)t * spt * n * 256, spt * n * 32, n * 32, sel + t * spt);
-    const int si = tid < spt ? tid : 0;
+    const int si = (tid & 63) < spt ? tid & 63 : 0; // (every wave has the token's ids, slot l's in lane l: at most 64 slots)
     const u32 my_sel = sel[t * spt + si];
+    // the token's f32 rows of h are asked for before anything that waits for the expert id, so they arrive with it and are
+    // encoded while the weight rows are on their way
+    typename std::conditional<bm_takes_q8k(WT), Q8kCols<T>, Q82Cols<4, T>>::type hrows;
+    if constexpr (bm_takes_q8k(WT)) hrows.load(h + (size_t)t * spt * n * 256, spt, n);
+    else hrows.load(h + (size_t)t * spt * n * 256, spt * n * 32, n * 32, sel + t * spt);
     const float my_w = wts[t * spt + si];
     const bool live = id < n_experts;
     const bool active = dl < D && r < rpe && live;
@@ -1020,7 +1035,9 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
     float *s_w = part + D * spt;                                              // [spt]
     u32 *s_sel = reinterpret_cast<u32 *>(s_w + spt);                          // [spt]
-    if constexpr (bm_takes_q8k(WT)) q8k_stage_cols<T>(h + (size_t)t * spt * n * 256, cols, spt, n, fault, layer, sel + t * spt, n_experts);
+    if constexpr (bm_takes_q8k(WT))
+        hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, fault, layer,
+                     [&](int c) { return (u32)__builtin_amdgcn_readlane((int)my_sel, __builtin_amdgcn_readfirstlane(c)) < n_experts; });
     else hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, sel + t * spt, n_experts, fault, layer);
     if (tid < spt) {
         s_w[tid] = my_w;
