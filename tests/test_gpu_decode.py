@@ -920,6 +920,9 @@ def run_grouped(gpu, L, x, ids, wts, top_k, fused_quant):
     ((bm.Q3_K, bm.Q3_K, bm.Q3_K), 768, 512, 3, 9, 2),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 1024, 512, 5, 6, 3),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 768, 256, 4, 5, 4),
+    # columns a little over the 4096 bytes that are asked for at a time: 4160, and 4440 with half a piece at the end
+    ((bm.Q5_K, bm.Q5_K, bm.Q6_K), 2560, 512, 3, 11, 2),
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.Q4_K), 3840, 256, 4, 9, 3),
     # rows long enough that eight Q8_K columns pass the LDS mark where a tile launch goes as two, one for the tiles of
     # up to two slots and one for the wider ones: 18 slots over 6 experts give runs of both kinds
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ4_XS), 5120, 4608, 6, 9, 2),
