@@ -175,7 +175,7 @@ __global__ __launch_bounds__(T) void k_gemv(const uint8_t *w, long rows, int nb,
     const uint8_t *wrow = w + (size_t)(active ? row : 0) * row_bytes;
     // the columns' first bytes are asked for in front of the rows (vector loads come back in the order they were asked for:
     // behind the rows' requests the columns would wait for those as well); what a thread's few loads do not cover comes after
-    Stage<(T == 64 ? 5 : 2), T> st;
+    Stage<(T == 64 ? 3 : 2), T, !bm_takes_q8k(WT)> st;
     st.load(act + (size_t)col0 * col_bytes, m * col_bytes);
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
@@ -211,24 +211,13 @@ __global__ __launch_bounds__(C == 1 ? 512 : 1024) void k_gemv_cols(const uint8_t
     const int col_bytes = bm_act_col_bytes<WT>(n), bytes = m * col_bytes;
     const uint8_t *wrow = w + (size_t)(active ? row : 0) * row_bytes;
     const uint8_t *src = act + (size_t)col0 * col_bytes;
-    uint2 v[4]; // the columns' first bytes in front of the rows, as k_gemv
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int o = (r * T + tid) * 8;
-        v[r] = *reinterpret_cast<const uint2 *>(src + (o < bytes ? o : bytes - 8));
-    }
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
+    Stage<2, 256, !bm_takes_q8k(WT)> st; // the columns' first bytes in front of the rows, as k_gemv
+    st.load(src, bytes, T);
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables<WT>(lds, T);
     uint8_t *cols = lds + tab_bytes<WT>();
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int o = (r * T + tid) * 8;
-        if (o < bytes) *reinterpret_cast<uint2 *>(cols + o) = v[r];
-    }
-    for (int o = (4 * T + tid) * 8; o < bytes; o += T * 8) *reinterpret_cast<uint2 *>(cols + o) = *reinterpret_cast<const uint2 *>(src + o);
+    st.store(cols, src, bytes, T);
     __syncthreads();
     const int c0 = cg * C, mc = m - c0 < C ? m - c0 : C;
     float out[C];
@@ -306,7 +295,7 @@ __global__ __launch_bounds__(T) void k_gate_up(const uint8_t *wg, const uint8_t 
     const int spc_shift = (spc_word >> 24) - 1;
     const int token = spc_shift >= 0 ? slot >> spc_shift : slot / (spc_word & 0xffffff);
     const uint8_t *act_col = act + (size_t)token * col_bytes;
-    Stage<512 / T, T> st;
+    Stage<2, T, !bm_takes_q8k(WT)> st;
     st.load(act_col, col_bytes);
     if (id >= n_experts) { // uniform over the workgroup: no weight is read (crates/gpu/src/kquant/sel.rs:22-28)
         if (id == 0xffffffffu) return; // a slot served elsewhere: nothing written, nothing raised (sel.rs:153-161)
@@ -361,7 +350,7 @@ __global__ __launch_bounds__(256) void k_gemv_sel(const uint8_t *w, u32 n_expert
     const int n = NB > 0 ? NB : nb;
     const int col_bytes = bm_act_col_bytes<WT>(n);
     const uint8_t *act_col = act + (size_t)slot * col_bytes;
-    Stage<2> st;
+    Stage<1, 256, !bm_takes_q8k(WT)> st;
     st.load(act_col, col_bytes);
     if (id >= n_experts) { // the slot's rows stay untouched; a host slot is skipped silently
         if (tid == 0 && rb == 0 && id != 0xffffffffu) bm_raise(fault, layer, kSiteExpertId);
@@ -559,7 +548,7 @@ __device__ __forceinline__ void down_combine_body(uint8_t *lds, const uint8_t *w
     const int col_bytes = bm_act_col_bytes<WT>(n);
     const uint8_t *act_cols = act + (size_t)t * spt * col_bytes;
     // the token's columns are asked for before anything waits for the expert id: they arrive with it
-    Stage<5> st;
+    StageWords<5> st;
     st.load(act_cols, spt * col_bytes);
     if constexpr (eight) {
         __builtin_amdgcn_sched_barrier(0);
@@ -655,7 +644,7 @@ __global__ __launch_bounds__(256 * NB) void k_down_combine_q6k_split(const uint8
     constexpr size_t row_bytes = (size_t)NB * BM_Q6K_BLOCK;
     constexpr int col_bytes = bm_act_col_bytes<WT>(NB);
     const uint8_t *act_cols = act + (size_t)t * spt * col_bytes;
-    Stage<2, 256 * NB> st; // 16 bytes a thread of 768: the eight columns of 1248 bytes
+    StageWords<2, 256 * NB> st; // 16 bytes a thread of 768: the eight columns of 1248 bytes
     st.load(act_cols, spt * col_bytes);
     if (!live && id != 0xffffffffu && rb == 0 && dl == 0 && q == 0 && i == 0) bm_raise(fault, layer, kSiteExpertId);
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
