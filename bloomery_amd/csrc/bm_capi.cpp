@@ -1039,7 +1039,7 @@ static bool gemm_ahead(const bm_scratch *s, int m) {
 // In place of the grouped step's tiles: the one-column walks (activation operands read a super-block ahead, the IQ tables in copies) are that
 // much cheaper than the tile launches' that rows read again for another slot of their expert cost less than tiles of few slots, as long as the
 // caches serve most of them: up to 500 MB of rows asked for, repeats and all, or with no more slots than experts. (650 random layers of 0.7 to 8
-// slots an expert, cold weights, over the tile launches: 0.83 on average, 1.03 at worst, and 2.5 % behind the better of the two; by MB asked
+// slots an expert, cold weights, over the tile launches, then some 1 to 4 % slower than now: 0.83 on average, 1.03 at worst, and 2.5 % behind the better of the two; by MB asked
 // for 0.7 up to 128, 0.8 to 500, 0.95 to 768, 1.2 beyond; the large IQ2_XXS layer, 4 tokens, 175 -> 155 us with the shared expert and the router.)
 // In place of the per-slot step's two launches, where they ask for 128 MB or more: there every workgroup quantizes the columns it reads itself, which
 // three launches more cost less than by then (over it, by MB: 1.1 at 32, 1.05 at 64, 0.98 at 128 to 256, 0.92 beyond; 280 random layers below 22 tokens).
