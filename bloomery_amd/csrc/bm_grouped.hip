@@ -320,7 +320,8 @@ __global__ __launch_bounds__(256) void k_gemv_tiles(const uint8_t *w, u32 n_expe
             if (t.entry >= n_slots && t.row_block == 0) bm_raise(fault, layer, kSiteExpertId);
             slot_of[c_of] = t.entry;
         }
-        stage_tile_cols<MC>(cols, col_bytes, mc, [&](int c) { return act + (size_t)(t.j + c0 + c) * col_bytes; }); // (they lie side by side)
+        // the tile's columns lie side by side: as one run, so that short ones leave no thread idle
+        Stage<1, 256, !bm_takes_q8k(WT)>::rest(cols, act + (size_t)(t.j + c0) * col_bytes, mc * col_bytes, 256, 0);
         __syncthreads();
         float v[MC];
         row_dot<WT, U, NB, MC>(b, wrow, cols, col_bytes, mc, n, q, tb, v, NoTap{});

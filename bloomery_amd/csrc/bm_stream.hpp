@@ -165,8 +165,12 @@ struct Stage {
     __device__ __forceinline__ void store(uint8_t *dst, const uint8_t *src, int bytes, int threads = T) const {
 #pragma unroll
         for (int r = 0; r < R; r++) put(dst, (r * threads + (int)threadIdx.x) * 16, bytes, v[r]);
+        rest(dst, src, bytes, threads, R * threads * 16);
+    }
+    // What lies from `first` on, four pieces a thread at a time.
+    __device__ __forceinline__ static void rest(uint8_t *dst, const uint8_t *src, int bytes, int threads, int first) {
         constexpr int kMore = 4;
-        for (int base = R * threads * 16; base < bytes; base += kMore * threads * 16) {
+        for (int base = first; base < bytes; base += kMore * threads * 16) {
             uint4 x[kMore];
 #pragma unroll
             for (int r = 0; r < kMore; r++) x[r] = piece(src, base + (r * threads + (int)threadIdx.x) * 16, bytes);
