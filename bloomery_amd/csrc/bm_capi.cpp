@@ -1097,7 +1097,11 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
     };
     const PathChoice choice = path_choice(s, m);
     if (((uintptr_t)x_dev & 15) == 0 && slot_by_slot(s, m, choice.path)) { // (the other steps take such an x, or refuse it)
-        int rc = bm_quantize(ctx, x_dev, m, s->act_x);
+        // (In the per-slot step's place only the rows of tokens that some expert takes, as that step does: a batch may be filled up with rows that
+        // hold anything and have their slots served elsewhere. The grouped step quantizes, and answers for, every row.)
+        const bool taken_only = choice.path == BM_PATH_PER_SLOT;
+        int rc = driver(ctx, what, bmk::quantize(launch_of(ctx), s->gate_type, x_dev, m, hidden, s->act_x->dev, nullptr,
+                                                 taken_only ? sel_dev : nullptr, (uint32_t)n_experts, spt));
         if (!rc) rc = bm_gate_up(ctx, wg, wu, s->act_x, sel_dev, n_slots, ff, spt, rule, s->g, nullptr);
         if (!rc) // (a slot without an expert of the stack: its rows of h hold nothing, its column is left alone)
             rc = driver(ctx, what, bmk::quantize(launch_of(ctx), s->down_type, s->g, n_slots, ff, s->act_h->dev, nullptr, sel_dev,

@@ -82,16 +82,17 @@ __global__ __launch_bounds__(256) void k_quantize_q82x4(const float *x, int m, i
 }
 
 // x: m columns of k values -> Q8_K columns (crates/qdot/src/lib.rs:1787-1809). A wave a 256-value block.
-// sel (optional): column c belongs to slot c; a slot whose id names no expert of the stack (served elsewhere, or refused) keeps
-// its column as it stands and raises nothing here: its rows of x need not hold anything.
+// sel (optional): column c is read by slots c * spc .. c * spc + spc (at most 64); a column none of whose slots names an expert of the stack
+// (served elsewhere, or refused) stays as it stands and raises nothing here: its row of x need not hold anything.
 __global__ __launch_bounds__(256) void k_quantize_q8k(const float *x, int m, int k, uint8_t *act, const u32 *live,
-                                                      const u32 *sel, u32 n_experts, u32 *fault, u32 layer) {
+                                                      const u32 *sel, u32 spc, u32 n_experts, u32 *fault, u32 layer) {
     const u32 bpc = (u32)k / 256u, gblk = blockIdx.x * 4u + (u32)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (gblk >= (u32)m * bpc) return;
     const u32 col = gblk / bpc, lane = threadIdx.x & 63;
     if (live && col >= *live) return;
-    if (sel && sel[col] >= n_experts) return;
-    q8k_wave_block(bm_ld4f(x + (size_t)gblk * 256 + 4 * lane), act + (size_t)gblk * BM_Q8K_STRIDE, (int)lane, fault, layer);
+    const float4 v = bm_ld4f(x + (size_t)gblk * 256 + 4 * lane); // (asked for beside the ids)
+    if (sel && __ballot(lane < spc && sel[(size_t)col * spc + (lane < spc ? lane : 0)] < n_experts) == 0) return;
+    q8k_wave_block(v, act + (size_t)gblk * BM_Q8K_STRIDE, (int)lane, fault, layer);
 }
 
 // The same columns with eight values a thread, a block a quad of lanes (two 16-byte loads a thread, fewer and fatter
@@ -112,8 +113,8 @@ __global__ __launch_bounds__(256) void k_quantize_q82x4_wide(const float *x, int
 constexpr long kWideQuantValues = 1 << 18;
 
 hipError_t quantize(const Launch &L, int wtype, const float *x, int m, int k, uint8_t *act, const uint32_t *live,
-                    const uint32_t *sel, uint32_t n_experts) {
-    if (sel && !bm_takes_q8k(wtype)) return hipErrorInvalidValue; // the slot-aware form is the Q8_K quantizer's
+                    const uint32_t *sel, uint32_t n_experts, int slots_per_col) {
+    if (sel && (!bm_takes_q8k(wtype) || slots_per_col < 1 || slots_per_col > 64)) return hipErrorInvalidValue; // the slot-aware form is the Q8_K quantizer's
     if (!bm_takes_q8k(wtype) && (long)m * k >= kWideQuantValues && ((uintptr_t)x & 15) == 0) {
         const long threads = (long)m * k / 8;
         hipLaunchKernelGGL(k_quantize_q82x4_wide, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, L.stream, x, m, k, act,
@@ -122,7 +123,7 @@ hipError_t quantize(const Launch &L, int wtype, const float *x, int m, int k, ui
     }
     if (bm_takes_q8k(wtype)) {
         hipLaunchKernelGGL(k_quantize_q8k, dim3(((unsigned)m * (unsigned)(k / 256) + 3) / 4), dim3(256), 0, L.stream, x, m, k, act,
-                           live, sel, n_experts, L.fault, L.layer);
+                           live, sel, (u32)slots_per_col, n_experts, L.fault, L.layer);
     } else {
         const long blocks = (long)m * (k / 32);
         hipLaunchKernelGGL(k_quantize_q82x4, dim3((unsigned)((blocks + 7) / 8)), dim3(256), 0, L.stream, x, m, k, act,

@@ -86,6 +86,48 @@ def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
         L.free()
 
 
+@pytest.mark.parametrize("m,top_k", ((20, 1), (8, 3), (19, 1)))
+def test_rows_of_tokens_that_no_expert_takes_may_hold_anything(gpu, m, top_k):
+    """A per-slot step, in two launches (the last case) and in launches of its own (from 128 MB asked for on): a row whose slots are all
+    served elsewhere, or refused, is not read as numbers. It may hold NaN and infinities and raises nothing but the refused id; the
+    other tokens' rows, one of them with some slots served elsewhere, are the oracle's."""
+    hidden, ff, n_experts = 2048, 2048, 8
+    L = Layer(gpu, (bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), hidden, ff, n_experts, 5200, cheap=True)
+    rng = np.random.default_rng(5202)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    ids, wts = ids.reshape(m, top_k), wts.reshape(m, top_k)
+    if top_k > 1:
+        wts[4, :-1] = 0.0  # (the slots that are served elsewhere below)
+    want_y, _ = L.oracle(x, ids, wts, top_k)
+    want = (want_y.reshape(m, hidden) + resid).astype(np.float32)
+    ids[4, :-1] = bm.HOST_SLOT
+    ids[2], ids[m - 1] = bm.HOST_SLOT, bm.HOST_SLOT
+    x[2], x[m - 1, 5] = np.nan, np.inf
+    want[[2, m - 1]] = resid[[2, m - 1]]
+    xd, wd, rd = gpu.upload(x, np.float32), gpu.upload(wts, np.float32), gpu.upload(resid, np.float32)
+    y = gpu.buffer(np.float32, m * hidden)
+    sc = gpu.scratch(bm.IQ4_XS, bm.IQ4_XS, hidden, ff, n_experts, top_k, 32)
+    try:
+        assert sc.path_for(m) == bm.PATH_PER_SLOT
+        for refused in (False, True):
+            if refused:
+                ids[2] = n_experts
+            sel = gpu.upload(ids, np.uint32)
+            gpu.fault_clear()
+            y.fill_bytes(0xFF)
+            gpu.enqueue_moe_forward(sc, L.dg, L.du, L.dd, xd, sel, wd, rd, m, y)
+            assert_f32(y.download(), want.reshape(-1), f"refused {refused}")
+            assert gpu.fault()[1] == (1 << bm.SITE_EXPERT_ID if refused else 0)
+            sel.free()
+    finally:
+        gpu.fault_clear()
+        sc.free()
+        for b in (xd, wd, rd, y):
+            b.free()
+        L.free()
+
+
 @pytest.mark.parametrize("gate,down,hidden,ff,n_experts,top_k,gemm", (
     (bm.Q4_K, bm.Q6_K, 2048, 768, 128, 8, 196),      # many experts of few slots
     (bm.Q6_K, bm.Q6_K, 2048, 768, 128, 8, 179),
