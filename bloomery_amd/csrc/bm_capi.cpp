@@ -1047,8 +1047,11 @@ static bool slot_by_slot(const bm_scratch *s, int m, int path) {
     if (act_form(s->gate_type) == 0 || act_form(s->down_type) == 0 || m > bmk::kMaxDecodeTokens || !per_slot_fits(s)) return false;
     const int64_t slots = (int64_t)m * s->spt;
     const int64_t asked = slots * (2 * s->ff * bm_row_bytes(s->gate_type, s->hidden) + s->hidden * bm_row_bytes(s->down_type, s->ff));
+    if (path == BM_PATH_GEMM) return false;
+    // A path that the caller forces takes its own launches. The grouped step of no more slots than experts is this one: its tiles hold a slot each.
+    if (s->path != BM_PATH_AUTO) return path == BM_PATH_GROUPED && slots <= s->n_experts;
     if (path == BM_PATH_PER_SLOT && asked < 128000000) return false;
-    return path != BM_PATH_GEMM && (slots <= s->n_experts || asked <= 500000000);
+    return slots <= s->n_experts || asked <= 500000000;
 }
 
 // The path a call with m tokens takes, and the f32 order of its GEMMs: the one place where it is chosen.

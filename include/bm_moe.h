@@ -374,7 +374,7 @@ int bm_swiglu_quant_sel(bm_ctx *ctx, const float *g_dev, const float *u_dev, con
  * GEMV_COLS, prefill.rs:602-604 WIDE_FROM, :147 wide_steps), here with a grouped arm between the two:
  *   BM_PATH_PER_SLOT  bm_moe_decode: two launches, every slot streams its expert's rows (repeats come from the caches);
  *   BM_PATH_GROUPED   bm_tables_quantize, bm_gate_up_tiles (bm_quantize_ord for a down stack on Q8_K columns),
- *                     bm_gemv_tiles, the slots' sum: an expert's rows are read once for all of its slots;
+ *                     bm_gemv_tiles, the slots' sum: a tile of eight of an expert's slots reads its rows once;
  *   BM_PATH_GEMM      bm_route_fill_quantize, bm_gemm over the gate and the up, bm_swiglu_quant_sel, bm_gemm, the slots' sum: the
  *                     matrix cores (in the f32 order bm_set_gemm_mode sets; every stack type bm_gemm takes).
  * In the exact mode all three give the same bits in y_dev. bm_scratch holds what the paths need between their launches for
@@ -385,11 +385,13 @@ int bm_swiglu_quant_sel(bm_ctx *ctx, const float *g_dev, const float *u_dev, con
  * rule fitted to measurements of both expects to be ahead for the types, the shape, the number of experts and of slots (the
  * GEMM from 196 tokens at that layer shape, from 76 for one large expert with a slot a token). In the tolerance mode of bm_gemm the
  * GEMM is taken from 96 tokens on where the gate/up type has kernels of that mode; below 96 tokens a GEMM path runs in the exact order.
- * On the grouped path a batch with no more slots than experts whose h crosses in f32 rows takes the per-slot gate . up launch (over
- * columns made in the tables' launch) and the tile launch for down.
+ * Where gate/up and down stacks all dot against Q8_K columns a step can also go slot by slot through launches of its own, same bits: the tokens'
+ * columns quantized once, bm_gate_up, the quantizer of h, bm_gemv_sel, the slots' sum (x_dev 16-byte aligned). It is the grouped path's form for a batch
+ * with no more slots than experts, and under BM_PATH_AUTO it stands in for the per-slot and the grouped path wherever measurements put it
+ * ahead of their launches (by the bytes of expert rows that the slots ask for, the types and the slots an expert).
  * bm_scratch_set_path sets crossovers of the caller's own (0 keeps what is; gemm_from then holds for both modes, in the mode's own
- * f32 order) or forces one path.
- * bm_scratch_path_for: the path a call with m tokens takes. A slot whose id names no expert of the stack adds nothing to
+ * f32 order) or forces one path, which then runs the launches listed for it (the grouped one's form for few slots among them).
+ * bm_scratch_path_for: the path a call with m tokens takes, also where the slot-by-slot launches stand in for it. A slot whose id names no expert of the stack adds nothing to
  * the sum and raises BM_SITE_EXPERT_ID unless it is BM_HOST_SLOT, which every path skips silently (the GEMM path's route
  * table does not list it, and its SwiGLU quantizer is bm_swiglu_quant_sel). Calls that share a scratch must not overlap. */
 typedef struct bm_scratch bm_scratch;

@@ -1,6 +1,9 @@
 """GPU parity tests of bm_moe_forward, the one entry for any number of tokens: each of its three paths (per slot, grouped
 by expert, the grouped GEMM) gives the oracle's layer output bit for bit on the same seeded inputs, so the choice among
-them by batch size changes no bit; the automatic choice follows the crossovers; ids that name no expert add nothing."""
+them by batch size changes no bit; a forced path takes its own launches and the automatic choice follows the crossovers; ids that name no
+expert add nothing."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -12,6 +15,39 @@ from test_gpu_decode import Layer, assert_f32, gpu, route  # noqa: F401  (gpu: m
 pytestmark = pytest.mark.gpu
 
 PATHS = ((bm.PATH_PER_SLOT, "per slot"), (bm.PATH_GROUPED, "grouped"), (bm.PATH_GEMM, "gemm"))
+
+
+class _KernelNode(C.Structure):  # hipKernelNodeParams
+    _fields_ = [("threads", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("blocks", C.c_uint32 * 3), ("params", C.c_void_p),
+                ("lds", C.c_uint32)]
+
+
+def launches(gpu, enqueue):
+    """The workgroups' thread counts of the launches that `enqueue` makes, in order: captured on the context's stream, not run."""
+    with open("/proc/self/maps") as f:
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))  # the runtime that the library has loaded
+    graph, count = C.c_void_p(), C.c_size_t(0)
+    assert hip.hipStreamBeginCapture(C.c_void_p(gpu.stream()), 1) == 0  # (thread-local)
+    try:
+        enqueue()
+    finally:
+        assert hip.hipStreamEndCapture(C.c_void_p(gpu.stream()), C.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(count)) == 0
+    nodes, threads = (C.c_void_p * count.value)(), []
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(count)) == 0
+    for n in nodes:
+        p = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(C.c_void_p(n), C.byref(p)) == 0
+        threads.append(p.threads[0])
+    assert hip.hipGraphDestroy(graph) == 0
+    return threads
+
+
+def route_taken(gpu, enqueue):
+    """Which launches a step of two Q8_K stacks makes: the per-slot step's two, the grouped step's, which begin with the tables (a workgroup of
+    1024 threads), or slot by slot through launches of their own, which begin with the quantizer."""
+    t = launches(gpu, enqueue)
+    return "per slot" if len(t) == 2 else "tiles" if t[0] == 1024 else "slot by slot" if len(t) == 5 else t
 
 
 @pytest.mark.parametrize("types,hidden,ff,n_experts,top_k,m", (
@@ -86,9 +122,50 @@ def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
         L.free()
 
 
+@pytest.mark.parametrize("types,hidden,ff,n_experts,top_k,m,auto,grouped", (
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 2048, 8, 1, 19, "per slot", "tiles"),      # 127 MB asked for
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 2048, 8, 1, 20, "slot by slot", "tiles"),  # 134 MB
+    ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 2048, 2048, 8, 2, 13, "slot by slot", "tiles"),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 1024, 512, 6, 4, 9, "per slot", "tiles"),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 27, 3, 9, "per slot", "slot by slot"),  # a slot an expert
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 26, 3, 9, "per slot", "tiles"),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 512, 512, 64, 3, 24, "slot by slot", "tiles"),  # past the per-slot step's tokens
+))
+def test_a_forced_path_takes_its_own_launches(gpu, types, hidden, ff, n_experts, top_k, m, auto, grouped):
+    """Stacks on Q8_K columns on both sides: the per-slot and the grouped path forced, and what the automatic choice puts in their place, as
+    launches and in their outputs, with slots that are served elsewhere and refused ones."""
+    L = Layer(gpu, types, hidden, ff, n_experts, 5210 + m, cheap=True)
+    rng = np.random.default_rng(5211)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    wts[2, 0] = wts[m - 1, top_k - 1] = 0.0  # (the two slots that no expert takes below)
+    want = (L.oracle(x, ids, wts, top_k)[0].reshape(m, hidden) + resid).astype(np.float32).reshape(-1)
+    ids[2, 0], ids[m - 1, top_k - 1] = bm.HOST_SLOT, n_experts
+    xd, sel, wd, rd = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.upload(wts, np.float32), gpu.upload(resid, np.float32)
+    y = gpu.buffer(np.float32, m * hidden)
+    sc = gpu.scratch(types[0], types[2], hidden, ff, n_experts, top_k, m)
+    step = lambda: gpu.enqueue_moe_forward(sc, L.dg, L.du, L.dd, xd, sel, wd, rd, m, y)  # noqa: E731
+    try:
+        for path, takes in ((bm.PATH_AUTO, auto), (bm.PATH_PER_SLOT, "per slot"), (bm.PATH_GROUPED, grouped)):
+            sc.set_path(path)
+            assert route_taken(gpu, step) == takes, path
+            gpu.fault_clear()
+            for _ in range(2):
+                y.fill_bytes(0xFF)
+                step()
+                assert_f32(y.download(), want, f"path {path}")
+            assert gpu.fault()[1] == 1 << bm.SITE_EXPERT_ID
+    finally:
+        gpu.fault_clear()
+        sc.free()
+        for b in (xd, sel, wd, rd, y):
+            b.free()
+        L.free()
+
+
 @pytest.mark.parametrize("m,top_k", ((20, 1), (8, 3), (19, 1)))
 def test_rows_of_tokens_that_no_expert_takes_may_hold_anything(gpu, m, top_k):
-    """A per-slot step, in two launches (the last case) and in launches of its own (from 128 MB asked for on): a row whose slots are all
+    """A per-slot step of the automatic choice, in two launches (the last case) and in launches of its own (from 128 MB asked for on): a row whose slots are all
     served elsewhere, or refused, is not read as numbers. It may hold NaN and infinities and raises nothing but the refused id; the
     other tokens' rows, one of them with some slots served elsewhere, are the oracle's."""
     hidden, ff, n_experts = 2048, 2048, 8
@@ -240,8 +317,8 @@ def test_the_automatic_choice_follows_the_crossovers(gpu):
 
 
 def test_a_slot_without_an_expert_on_the_grouped_path_of_few_slots(gpu):
-    """The grouped path with no more slots than experts and Q8_K columns on both sides (the per-slot gate . up launch, the
-    slot-aware quantizer of h, the down tiles reading their columns in slot order): a host-served slot and an id past the stack
+    """The grouped path with no more slots than experts and Q8_K columns on both sides (gate . up and down slot by slot, the
+    slot-aware quantizer of h between them): a host-served slot and an id past the stack
     add nothing, the sums over the live slots are the oracle's, only the id past the stack raises; the scratch is poisoned first so
     that a stale row of h would show."""
     hidden, ff, n_experts, top_k, m = 512, 256, 16, 3, 3
