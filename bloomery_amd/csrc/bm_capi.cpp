@@ -1050,7 +1050,7 @@ static bool slot_by_slot(const bm_scratch *s, int m, int path) {
     if (path == BM_PATH_GEMM) return false;
     // A path that the caller forces takes its own launches. The grouped step of no more slots than experts is this one: its tiles hold a slot each.
     if (s->path != BM_PATH_AUTO) return path == BM_PATH_GROUPED && slots <= s->n_experts;
-    if (path == BM_PATH_PER_SLOT && asked < 128000000) return false;
+    if (path == BM_PATH_PER_SLOT) return asked >= 128000000;
     return slots <= s->n_experts || asked <= 500000000;
 }
 

@@ -126,6 +126,7 @@ def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
     ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 2048, 8, 1, 19, "per slot", "tiles"),      # 127 MB asked for
     ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 2048, 8, 1, 20, "slot by slot", "tiles"),  # 134 MB
     ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 2048, 2048, 8, 2, 13, "slot by slot", "tiles"),
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 3840, 4, 2, 21, "slot by slot", "tiles"),  # 526 MB, more slots than experts
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 1024, 512, 6, 4, 9, "per slot", "tiles"),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 27, 3, 9, "per slot", "slot by slot"),  # a slot an expert
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 26, 3, 9, "per slot", "tiles"),
