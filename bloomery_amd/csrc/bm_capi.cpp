@@ -1041,8 +1041,10 @@ static bool gemm_ahead(const bm_scratch *s, int m) {
 // caches serve most of them: up to 500 MB of rows asked for, repeats and all, or with no more slots than experts. (650 random layers of 0.7 to 8
 // slots an expert, cold weights, over the tile launches, then some 1 to 4 % slower than now: 0.83 on average, 1.03 at worst, and 2.5 % behind the better of the two; by MB asked
 // for 0.7 up to 128, 0.8 to 500, 0.95 to 768, 1.2 beyond; the large IQ2_XXS layer, 4 tokens, 175 -> 155 us with the shared expert and the router.)
-// In place of the per-slot step's two launches, where they ask for 128 MB or more: there every workgroup quantizes the columns it reads itself, which
-// three launches more cost less than by then (over it, by MB: 1.1 at 32, 1.05 at 64, 0.98 at 128 to 256, 0.92 beyond; 280 random layers below 22 tokens).
+// In place of the per-slot step's two launches, where they ask for 128 MB or more, 200 with one or two slots a token, whose columns are the
+// fewer to quantize: there every workgroup quantizes the columns it reads itself, which three launches more cost less than by then (over it, 900 random
+// layers below 22 tokens, by MB: 1.16 at 30 to 64, 1.08 to 96, 1.02 to 128, 0.98 to 160, 0.94 to 200, 0.91 to 256, 0.88 to 400, 0.84 beyond without
+// an end; one or two slots a token 1.04 from 128 to 160, 1.03 to 200, 0.98 to 400).
 static bool slot_by_slot(const bm_scratch *s, int m, int path) {
     if (act_form(s->gate_type) == 0 || act_form(s->down_type) == 0 || m > bmk::kMaxDecodeTokens || !per_slot_fits(s)) return false;
     const int64_t slots = (int64_t)m * s->spt;
@@ -1050,7 +1052,7 @@ static bool slot_by_slot(const bm_scratch *s, int m, int path) {
     if (path == BM_PATH_GEMM) return false;
     // A path that the caller forces takes its own launches. The grouped step of no more slots than experts is this one: its tiles hold a slot each.
     if (s->path != BM_PATH_AUTO) return path == BM_PATH_GROUPED && slots <= s->n_experts;
-    if (path == BM_PATH_PER_SLOT) return asked >= 128000000;
+    if (path == BM_PATH_PER_SLOT) return asked >= (s->spt > 2 ? 128000000 : 200000000);
     return slots <= s->n_experts || asked <= 500000000;
 }
 

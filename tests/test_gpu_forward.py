@@ -93,9 +93,9 @@ def test_every_path_gives_the_oracles_bits(gpu, types, hidden, ff, n_experts, to
 
 @pytest.mark.parametrize("m", (19, 20))
 def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
-    """Stacks on Q8_K columns whose rows are 6.7 MB an expert: 20 slots ask for 128 MB, from where the per-slot step quantizes its columns in
-    launches of their own. One slot is served elsewhere and one names no expert; neither adds anything."""
-    hidden, ff, n_experts, top_k = 2048, 2048, 8, 1
+    """Stacks on Q8_K columns whose rows are 10 MB an expert: 20 slots ask for 200 MB, from where the per-slot step of a slot a token quantizes its
+    columns in launches of their own. One slot is served elsewhere and one names no expert; neither adds anything."""
+    hidden, ff, n_experts, top_k = 2048, 3072, 8, 1
     L = Layer(gpu, (bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), hidden, ff, n_experts, 5200, cheap=True)
     rng = np.random.default_rng(5201)
     x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
@@ -123,9 +123,10 @@ def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
 
 
 @pytest.mark.parametrize("types,hidden,ff,n_experts,top_k,m,auto,grouped", (
-    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 2048, 8, 1, 19, "per slot", "tiles"),      # 127 MB asked for
-    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 2048, 8, 1, 20, "slot by slot", "tiles"),  # 134 MB
-    ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 2048, 2048, 8, 2, 13, "slot by slot", "tiles"),
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 3072, 8, 1, 19, "per slot", "tiles"),      # 191 MB asked for
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 3072, 8, 1, 20, "slot by slot", "tiles"),  # 201 MB
+    ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 2048, 2048, 8, 3, 8, "per slot", "tiles"),          # 125 MB, three slots a token
+    ((bm.Q3_K, bm.Q3_K, bm.IQ3_XXS), 2048, 2048, 8, 3, 9, "slot by slot", "tiles"),      # 141 MB
     ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 2048, 3840, 4, 2, 21, "slot by slot", "tiles"),  # 526 MB, more slots than experts
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 1024, 512, 6, 4, 9, "per slot", "tiles"),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 27, 3, 9, "per slot", "slot by slot"),  # a slot an expert
@@ -164,9 +165,9 @@ def test_a_forced_path_takes_its_own_launches(gpu, types, hidden, ff, n_experts,
         L.free()
 
 
-@pytest.mark.parametrize("m,top_k", ((20, 1), (8, 3), (19, 1)))
+@pytest.mark.parametrize("m,top_k", ((8, 3), (7, 3), (6, 3), (20, 1)))
 def test_rows_of_tokens_that_no_expert_takes_may_hold_anything(gpu, m, top_k):
-    """A per-slot step of the automatic choice, in two launches (the last case) and in launches of its own (from 128 MB asked for on): a row whose slots are all
+    """A per-slot step of the automatic choice, in launches of its own (24 and 21 slots, 160 and 140 MB asked for) and in two: a row whose slots are all
     served elsewhere, or refused, is not read as numbers. It may hold NaN and infinities and raises nothing but the refused id; the
     other tokens' rows, one of them with some slots served elsewhere, are the oracle's."""
     hidden, ff, n_experts = 2048, 2048, 8
