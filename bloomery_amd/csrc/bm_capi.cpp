@@ -1016,6 +1016,7 @@ static bool per_slot_fits(const bm_scratch *s) {
 //   hidden 7168, ff 1536, top-4 of 8:   Q4_K 22 tokens 213 / 92, 64: 391 / 142
 //   hidden 7168, ff 2048, top-8 of 256: IQ2_XXS 64 tokens 1363 / 3190, 192: 3013 / 3603
 //   hidden 2048, ff 768, top-2 of 256:  Q4_K 500 tokens 222 / 312, 1500: 430 / 342; IQ2_XXS 230: 151 / 391
+static double tiles_worth(double slots, double experts) { return std::max(experts / 2 + slots / 16, slots / 8 + experts / 4); }
 static bool gemm_ahead(const bm_scratch *s, int m) {
     struct Line {
         double launches, die, fits; // the GEMM's constant, what a 64-slot tile on the die costs, the factor of short columns
@@ -1030,17 +1031,21 @@ static bool gemm_ahead(const bm_scratch *s, int m) {
     const double v = (double)s->hidden * s->ff / (1 << 20), n = (double)m * s->spt, experts = s->n_experts;
     if (n < 1.5 * experts) return false;
     const double past = std::min(1.0, std::max(0.0, 2.0 * (s->hidden / line.short_hidden - 1.0)));
-    const double tiles = v * std::max(experts / 2 + n / 16, n / 8 + experts / 4) * (line.fits + (1.0 - line.fits) * past);
+    const double tiles = v * tiles_worth(n, experts) * (line.fits + (1.0 - line.fits) * past);
     return tiles > line.launches + line.die * v * std::ceil(std::max(experts, n / 64 + experts / 2) / 8);
 }
 
 // Whether a step of both stacks on Q8_K columns goes slot by slot through launches of its own: the columns quantized once, gate . up and down a
 // workgroup a slot's rows.
 // In place of the grouped step's tiles: the one-column walks (activation operands read a super-block ahead, the IQ tables in copies) are that
-// much cheaper than the tile launches' that rows read again for another slot of their expert cost less than tiles of few slots, as long as the
-// caches serve most of them: up to 500 MB of rows asked for, repeats and all, or with no more slots than experts. (650 random layers of 0.7 to 8
-// slots an expert, cold weights, over the tile launches, then some 1 to 4 % slower than now: 0.83 on average, 1.03 at worst, and 2.5 % behind the better of the two; by MB asked
-// for 0.7 up to 128, 0.8 to 500, 0.95 to 768, 1.2 beyond; the large IQ2_XXS layer, 4 tokens, 175 -> 155 us with the shared expert and the router.)
+// much cheaper than the tile launches' that rows read again for another slot of their expert cost less than tiles of few slots, with no more slots
+// than experts, or as long as the caches serve most of the rows (up to 500 MB asked for, repeats and all; by MB 0.95 times the tiles' time to 768, 1.2
+// beyond) and the tiles do not save too much decoding: a walk decodes its rows for every slot, a tile once for up to eight. What a slot's decoding costs
+// goes by the types' work a weight (IQ2_XXS 1, IQ3_XXS 0.7, IQ4_XS 0.4, Q3_K 0.3) and by the rows, whose ends cost as much as 1024 values; the line, 500
+// millions of such weights more than two tiles' worth each, is a fit. Rows of 4096 values and more stay slot by slot: eight of their columns leave a
+// compute unit few tile workgroups. (2628 random layers that the choice below gives to the grouped step, 0.7 to 1000 slots an expert, cold
+// weights: 0.77 of the tiles' time on average, more than 1.05 times in 13 of them and 1.13 at worst, 0.6 % behind the better of the two, in 900 others 13 and
+// 1.17; by the 500 MB alone 306 and 1.53, IQ2_XXS at 4 to 16 slots an expert and short rows most. The large IQ2_XXS layer, 4 tokens, 175 -> 155 us with the shared expert and the router.)
 // In place of the per-slot step's two launches, where they ask for 128 MB or more, 200 with one or two slots a token, whose columns are the
 // fewer to quantize: there every workgroup quantizes the columns it reads itself, which three launches more cost less than by then (over it, 900 random
 // layers below 22 tokens, by MB: 1.16 at 30 to 64, 1.08 to 96, 1.02 to 128, 0.98 to 160, 0.94 to 200, 0.91 to 256, 0.88 to 400, 0.84 beyond without
@@ -1053,7 +1058,12 @@ static bool slot_by_slot(const bm_scratch *s, int m, int path) {
     // A path that the caller forces takes its own launches. The grouped step of no more slots than experts is this one: its tiles hold a slot each.
     if (s->path != BM_PATH_AUTO) return path == BM_PATH_GROUPED && slots <= s->n_experts;
     if (path == BM_PATH_PER_SLOT) return asked >= (s->spt > 2 ? 128000000 : 200000000);
-    return slots <= s->n_experts || asked <= 500000000;
+    if (slots <= s->n_experts) return true;
+    if (asked > 500000000 || s->hidden >= 4096) return asked <= 500000000;
+    auto work = [](int type) { return type == BM_TYPE_IQ2_XXS ? 1.0 : type == BM_TYPE_IQ3_XXS ? 0.7 : type == BM_TYPE_IQ4_XS ? 0.4 : 0.3; };
+    const double hidden = s->hidden, ff = s->ff;
+    const double of_slot = (2 * work(s->gate_type) * ff * (hidden + 1024) + work(s->down_type) * hidden * (ff + 1024)) / (1 << 20);
+    return of_slot * ((double)slots - 2 * tiles_worth((double)slots, s->n_experts)) <= 500;
 }
 
 // The path a call with m tokens takes, and the f32 order of its GEMMs: the one place where it is chosen.

@@ -132,6 +132,10 @@ def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 27, 3, 9, "per slot", "slot by slot"),  # a slot an expert
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q3_K), 512, 256, 26, 3, 9, "per slot", "tiles"),
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ4_XS), 512, 512, 64, 3, 24, "slot by slot", "tiles"),  # past the per-slot step's tokens
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 512, 512, 16, 4, 76, "slot by slot", "tiles"),  # nineteen slots an expert: what its tiles save
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 512, 512, 16, 4, 77, "tiles", "tiles"),
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 4096, 1024, 4, 1, 74, "slot by slot", "tiles"),    # 495 MB
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 4096, 1024, 4, 1, 75, "tiles", "tiles"),           # 501 MB
 ))
 def test_a_forced_path_takes_its_own_launches(gpu, types, hidden, ff, n_experts, top_k, m, auto, grouped):
     """Stacks on Q8_K columns on both sides: the per-slot and the grouped path forced, and what the automatic choice puts in their place, as
@@ -149,7 +153,7 @@ def test_a_forced_path_takes_its_own_launches(gpu, types, hidden, ff, n_experts,
     step = lambda: gpu.enqueue_moe_forward(sc, L.dg, L.du, L.dd, xd, sel, wd, rd, m, y)  # noqa: E731
     try:
         for path, takes in ((bm.PATH_AUTO, auto), (bm.PATH_PER_SLOT, "per slot"), (bm.PATH_GROUPED, grouped)):
-            sc.set_path(path)
+            sc.set_path(path, 0, 4096)  # (the automatic choice among the two of them alone)
             assert route_taken(gpu, step) == takes, path
             gpu.fault_clear()
             for _ in range(2):
