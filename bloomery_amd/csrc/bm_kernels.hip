@@ -827,8 +827,17 @@ struct Q8kCols {
             const int b = wave() + u * kWaves;
             if (b < cols * nb && live(b / nb)) q8k_wave_block(x4[u], dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
         }
-        for (int b = wave() + kAhead * kWaves; b < cols * nb; b += kWaves)
-            if (live(b / nb)) q8k_wave_block(block(x, b), dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
+        for (int b0 = wave() + kAhead * kWaves; b0 < cols * nb; b0 += kAhead * kWaves) { // the rest, as many on their way at a time
+            float4 more[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; u++)
+                if (b0 + u * kWaves < cols * nb) more[u] = block(x, b0 + u * kWaves);
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int b = b0 + u * kWaves;
+                if (b < cols * nb && live(b / nb)) q8k_wave_block(more[u], dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
+            }
+        }
     }
 };
 
