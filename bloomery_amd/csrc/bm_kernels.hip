@@ -511,6 +511,13 @@ __device__ __forceinline__ float slot_sum(const float *v, const float *w, const 
     return with_resid ? __fadd_rn(acc, resid_v) : acc;
 }
 
+// Bytes between two slots' Q8_K columns in LDS beside the columns themselves. The IQ types with tables read a column 64 bytes a lane of the quad (four
+// lanes' eight bytes in every step), the quads of a wave as many columns as there are slots: columns an odd multiple of eight bytes apart fall on
+// banks of their own, columns of eight super-blocks, a multiple of 64 bytes, all on the same ones. (k_down_combine of IQ2_XXS without / with it, us: 2816
+// rows of 2048, 8 slots, 5 tokens 31.1 / 20.7; 7168 rows of 2048, 12 slots, 5 tokens 114 / 87; k_down_combine_hq of such rows 0.98 times its time, without it up to
+// 1.18 times what it took before a lane held whole sub-blocks.) Up to 32 slots: the entries answer for 4096 bytes of LDS beside the columns.
+__host__ __device__ constexpr int slot_col_pad(int wt, int nb, int spt) { return (wt == BM_IQ2XXS || wt == BM_IQ3XXS) && nb % 2 == 0 && spt <= 32 ? 8 : 0; }
+
 // The shared body of the down + combine workgroup: token t, output rows rb * D .. + D with D = 64 / spt, a quad for
 // every (row, slot).
 template <int WT, int U, int NB, bool EIGHT = false>
@@ -546,7 +553,7 @@ __device__ __forceinline__ void down_combine_body(uint8_t *lds, const uint8_t *w
     const float resid_v = resid && tid < D && rb * D + tid < rpe ? resid[(size_t)t * rpe + rb * D + tid] : 0.0f;
     const int n = NB > 0 ? NB : nb;
     const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
-    const int col_bytes = bm_act_col_bytes<WT>(n);
+    const int col_bytes = bm_act_col_bytes<WT>(n), pad = slot_col_pad(WT, n, spt), col_stride = col_bytes + pad;
     const uint8_t *act_cols = act + (size_t)t * spt * col_bytes;
     // the token's columns are asked for before anything waits for the expert id: they arrive with it
     StageWords<5> st;
@@ -562,7 +569,7 @@ __device__ __forceinline__ void down_combine_body(uint8_t *lds, const uint8_t *w
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *cols = lds + tab_bytes<WT>();
-    float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
+    float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_stride); // [D][spt]
     float *s_w = part + D * spt;                                              // [spt]
     u32 *s_sel = reinterpret_cast<u32 *>(s_w + spt);                          // [spt]
     Blk<WT> b[U];
@@ -573,7 +580,8 @@ __device__ __forceinline__ void down_combine_body(uint8_t *lds, const uint8_t *w
     preload<WT, U>(b, wrow, n, q);
     BM_TICK(t_asked, tid);
     BM_TICK(t_cols, st.v[4].x);
-    st.store(cols, act_cols, spt * col_bytes);
+    if constexpr (slot_col_pad(WT, 2, 1) != 0) st.store_apart(cols, act_cols, spt * col_bytes, col_bytes, pad);
+    else st.store(cols, act_cols, spt * col_bytes);
     if (tid < spt) {
         s_w[tid] = my_w;
         s_sel[tid] = my_sel;
@@ -586,7 +594,7 @@ __device__ __forceinline__ void down_combine_body(uint8_t *lds, const uint8_t *w
     BM_TOCK(2048, 5, t_asked);
     BM_TOCK(2048, 6, t_cols);
     float v[1];
-    row_dot<WT, U, NB, 1>(b, wrow, cols + (size_t)e * col_bytes, col_bytes, 1, n, q, tb, v, NoTap{});
+    row_dot<WT, U, NB, 1>(b, wrow, cols + (size_t)e * col_stride, col_stride, 1, n, q, tb, v, NoTap{});
     BM_MARK(2048, 2);
     if (q == 0 && dl < D) part[dl * spt + e] = v[0];
     __syncthreads();
@@ -820,12 +828,16 @@ struct Q8kCols {
     }
     // `live` (a column's number): a column whose slot is not live is not encoded (its rows may hold anything)
     template <class Live>
-    __device__ __forceinline__ void encode(const float *x, uint8_t *dst, int cols, int nb, u32 *fault, u32 layer, Live live) const {
+    __device__ __forceinline__ void encode(const float *x, uint8_t *dst, int cols, int nb, int col_stride, u32 *fault, u32 layer, Live live) const {
         const int lane = threadIdx.x & 63;
+        auto store = [&](int b, float4 v) __attribute__((always_inline)) {
+            const int c = b / nb;
+            if (live(c)) q8k_wave_block(v, dst + (size_t)c * col_stride + (size_t)(b - c * nb) * BM_Q8K_STRIDE, lane, fault, layer);
+        };
 #pragma unroll
         for (int u = 0; u < kAhead; u++) {
             const int b = wave() + u * kWaves;
-            if (b < cols * nb && live(b / nb)) q8k_wave_block(x4[u], dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
+            if (b < cols * nb) store(b, x4[u]);
         }
         for (int b0 = wave() + kAhead * kWaves; b0 < cols * nb; b0 += kAhead * kWaves) { // the rest, as many on their way at a time
             float4 more[kAhead];
@@ -834,8 +846,7 @@ struct Q8kCols {
                 if (b0 + u * kWaves < cols * nb) more[u] = block(x, b0 + u * kWaves);
 #pragma unroll
             for (int u = 0; u < kAhead; u++) {
-                const int b = b0 + u * kWaves;
-                if (b < cols * nb && live(b / nb)) q8k_wave_block(more[u], dst + (size_t)b * BM_Q8K_STRIDE, lane, fault, layer);
+                if (b0 + u * kWaves < cols * nb) store(b0 + u * kWaves, more[u]);
             }
         }
     }
@@ -925,7 +936,7 @@ __global__ __launch_bounds__(T) void k_gate_up_xq(const float *x, const uint8_t 
     const Iq2Tables tb = stage_tables_as<WA, WIDE, T>(lds);
     uint8_t *col = lds + tab_bytes<WA, WIDE>();
     const int col_bytes = bm_act_col_bytes<WA>(na);
-    xrow.encode(x + (size_t)t * hidden, col, 1, na, fault, layer, [](int) { return true; });
+    xrow.encode(x + (size_t)t * hidden, col, 1, na, 0, fault, layer, [](int) { return true; });
     __syncthreads();
     if (act_x && rb == 0 && slot % spt == 0) stage_bytes<T>(act_x + (size_t)t * col_bytes, col, col_bytes);
     float v[1];
@@ -975,7 +986,7 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *col = lds + tab_bytes<WT>();
     if constexpr (bm_takes_q8k(WT)) {
-        xcol.encode(xc, col, 1, n, fault, layer, [](int) { return true; });
+        xcol.encode(xc, col, 1, n, 0, fault, layer, [](int) { return true; });
     } else { // a q8_2 block is four lanes of eight values; 2048 values a pass
         if (tid * 8 < k) {
             const float v8[8] = {x_lo.x, x_lo.y, x_lo.z, x_lo.w, x_hi.x, x_hi.y, x_hi.z, x_hi.w};
@@ -1025,17 +1036,17 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     const float resid_v = resid && tid < D && rb * D + tid < rpe ? resid[(size_t)t * rpe + rb * D + tid] : 0.0f;
     if (!live && id != 0xffffffffu && rb == 0 && dl == 0 && q == 0) bm_raise(fault, layer, kSiteExpertId);
     const size_t row_bytes = (size_t)n * bm_block_bytes<WT>();
-    const int col_bytes = bm_act_col_bytes<WT>(n);
+    const int col_bytes = bm_act_col_bytes<WT>(n), col_stride = col_bytes + slot_col_pad(WT, n, spt);
     const uint8_t *wrow = w + ((size_t)(live ? id : 0) * rpe + (active ? r : 0)) * row_bytes;
     Blk<WT> b[U];
     preload<WT, U>(b, wrow, n, q);
     const Iq2Tables tb = stage_tables_as<WT, WIDE, T>(lds);
     uint8_t *cols = lds + tab_bytes<WT, WIDE>();
-    float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_bytes); // [D][spt]
+    float *part = reinterpret_cast<float *>(cols + (size_t)spt * col_stride); // [D][spt]
     float *s_w = part + D * spt;                                              // [spt]
     u32 *s_sel = reinterpret_cast<u32 *>(s_w + spt);                          // [spt]
     if constexpr (bm_takes_q8k(WT))
-        hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, fault, layer,
+        hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, col_stride, fault, layer,
                      [&](int c) { return (u32)__builtin_amdgcn_readlane((int)my_sel, __builtin_amdgcn_readfirstlane(c)) < n_experts; });
     else hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, sel + t * spt, n_experts, fault, layer);
     if (tid < spt) {
@@ -1045,9 +1056,9 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     __syncthreads();
     if (act_h && rb == 0) // the live slots' columns; the others keep what they held
         for (int c = 0; c < spt; c++)
-            if (s_sel[c] < n_experts) stage_bytes<T>(act_h + ((size_t)t * spt + c) * col_bytes, cols + (size_t)c * col_bytes, col_bytes);
+            if (s_sel[c] < n_experts) stage_bytes<T>(act_h + ((size_t)t * spt + c) * col_bytes, cols + (size_t)c * col_stride, col_bytes);
     float v[1];
-    row_dot<WT, U, NB, 1, WIDE>(b, wrow, cols + (size_t)e * col_bytes, col_bytes, 1, n, q, tb, v, NoTap{});
+    row_dot<WT, U, NB, 1, WIDE>(b, wrow, cols + (size_t)e * col_stride, col_stride, 1, n, q, tb, v, NoTap{});
     if (q == 0 && dl < D) part[dl * spt + e] = v[0];
     __syncthreads();
     if (tid < D && rb * D + tid < rpe) y[(size_t)t * rpe + rb * D + tid] = slot_sum(part + tid * spt, s_w, s_sel, spt, n_experts, resid_v, resid != nullptr);
@@ -1284,7 +1295,7 @@ hipError_t gemv_sel(const Launch &L, int wtype, const uint8_t *w, int n_experts,
 
 size_t down_combine_lds(int wtype, int k, int spt) {
     const int D = 64 / spt;
-    return tab_bytes_rt(wtype) + (size_t)spt * act_col_bytes(wtype, k) + ((size_t)D * spt + 2 * (size_t)spt) * sizeof(float);
+    return tab_bytes_rt(wtype) + (size_t)spt * (act_col_bytes(wtype, k) + slot_col_pad(wtype, k / 256, spt)) + ((size_t)D * spt + 2 * (size_t)spt) * sizeof(float);
 }
 
 hipError_t down_combine(const Launch &L, int wtype, const uint8_t *w, int n_experts, int k, const uint8_t *act,

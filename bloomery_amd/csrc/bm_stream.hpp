@@ -205,6 +205,17 @@ struct StageWords {
         for (int o = (R * T + (int)threadIdx.x) * 8; o < bytes; o += T * 8)
             *reinterpret_cast<uint2 *>(dst + o) = *reinterpret_cast<const uint2 *>(src + o);
     }
+    // Columns of col_bytes side by side in memory, `pad` bytes further apart in LDS.
+    __device__ __forceinline__ void store_apart(uint8_t *dst, const uint8_t *src, int bytes, int col_bytes, int pad) const {
+        const u32 inv = 0xffffffffu / (u32)(col_bytes / 8) + 1; // a word's column: exact, as words times words a column stay below 2^32
+        auto at = [&](int o) { return reinterpret_cast<uint2 *>(dst + o + pad * (int)__umulhi((u32)o / 8, inv)); };
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int o = (r * T + (int)threadIdx.x) * 8;
+            if (o < bytes) *at(o) = v[r];
+        }
+        for (int o = (R * T + (int)threadIdx.x) * 8; o < bytes; o += T * 8) *at(o) = *reinterpret_cast<const uint2 *>(src + o);
+    }
 };
 
 // The weight stream of a row is a ring of U super-blocks in registers: the first U - 1 are requested up front

@@ -716,6 +716,39 @@ def test_gate_up_with_tables_in_copies(gpu, wtype, k, rpe, n_slots):
         b.free()
 
 
+# The slots' columns lie eight bytes apart in LDS where a column of the IQ types with tables has an even number of super-blocks, up to 32 slots: even
+# and odd counts, eight (a multiple of the banks), slots that divide a workgroup's quads and ones that do not, 32 and 33 of them, more than the first
+# loads' bytes, and the larger workgroups of the launch that quantizes the rows itself.
+@pytest.mark.parametrize("wtype,k,top_k,m", ((bm.IQ2_XXS, 2048, 8, 3), (bm.IQ3_XXS, 2048, 5, 2), (bm.IQ2_XXS, 512, 7, 2), (bm.IQ3_XXS, 1536, 3, 33),
+                                             (bm.IQ3_XXS, 768, 8, 2), (bm.IQ2_XXS, 1024, 32, 1), (bm.IQ2_XXS, 1024, 33, 1), (bm.IQ3_XXS, 256, 64, 1)))
+def test_down_half_with_columns_apart(gpu, wtype, k, top_k, m):
+    rng = np.random.default_rng(690 + k + top_k)
+    n_experts, rows = 3, 70
+    w = stack(wtype, n_experts * rows, k, 691)
+    h, wts, resid = normal_f32(rng, (m * top_k, k)), normal_f32(rng, (m, top_k)), normal_f32(rng, (m, rows))
+    sel = rng.integers(0, n_experts, (m, top_k)).astype(np.uint32)
+    want_cols = [ora.quantize_col(wtype, c) for c in h]
+    down = np.stack([ora.gemv(wtype, w, n_experts * rows, k, c, 1).reshape(n_experts, rows)[e] for c, e in zip(want_cols, sel.reshape(-1))])
+    sel[0, top_k - 2], down[top_k - 2] = bm.HOST_SLOT, 0.0  # (a slot served elsewhere adds nothing)
+    want = ora.combine_tokens(down.reshape(-1), wts.reshape(-1), resid.reshape(-1), rows, top_k, m)
+    dw, act, act_h = gpu.weights(wtype, n_experts * rows, k, w), gpu.act(wtype, k, m * top_k), gpu.act(wtype, k, m * top_k)
+    hd, seld, wd, rd = gpu.upload(h, np.float32), gpu.upload(sel, np.uint32), gpu.upload(wts, np.float32), gpu.upload(resid, np.float32)
+    y = gpu.buffer(np.float32, m * rows)
+    gpu.fault_clear()
+    gpu.enqueue_quantize(hd, m * top_k, act)
+    gpu.enqueue_down_combine(dw, act, seld, wd, rd, top_k, m, rows, y)
+    assert_f32(y.download(), want, "from columns")
+    y.fill_bytes(0xFF)
+    gpu.enqueue_down_combine_h(dw, hd, act_h, seld, wd, rd, top_k, m, rows, y)
+    assert_f32(y.download(), want, "from rows")
+    for c in range(m * top_k):
+        if c != top_k - 2:
+            assert np.array_equal(act_h.download(c), want_cols[c]), f"column {c}"
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    for b in (dw, act, act_h, hd, seld, wd, rd, y):
+        b.free()
+
+
 def test_fused_step_at_the_token_limit(gpu):
     """bm_moe_decode takes 1..=1024 tokens a launch: the limit itself against the oracle, one more refused by name."""
     L = Layer(gpu, (bm.Q4_K, bm.Q4_K, bm.Q6_K), 256, 256, 9, 650)
