@@ -1232,9 +1232,10 @@ hipError_t gemv_x(const Launch &L, int wtype, const uint8_t *w, int64_t rows, in
 }
 
 // Whether a launch of one-column row dots takes the IQ tables in copies: `lds` bytes with them, `threads` a workgroup. Not where they leave a
-// compute unit fewer than sixteen waves.
-static bool copies_fit(int wtype, size_t lds, int threads) {
-    return (wtype == BM_IQ2XXS || wtype == BM_IQ3XXS) && (size_t)kMaxLds / lds * (size_t)threads >= 16 * 64;
+// compute unit fewer than sixteen waves, and not for rows of one super-block, which end before the larger tables are laid out (gate . up 1.2 times
+// the plain tables' launch, down 1.01 on average and up to 1.3).
+static bool copies_fit(int wtype, int nb, size_t lds, int threads) {
+    return (wtype == BM_IQ2XXS || wtype == BM_IQ3XXS) && nb >= 2 && (size_t)kMaxLds / lds * (size_t)threads >= 16 * 64;
 }
 #define BM_WITH_TABLES(PLAIN, WIDE)                                                                                    \
     {                                                                                                                  \
@@ -1242,11 +1243,17 @@ static bool copies_fit(int wtype, size_t lds, int threads) {
             if (wide) return launch(WIDE);                                                                             \
         return launch(PLAIN);                                                                                          \
     }
-// A gate . up launch of `blocks` workgroups of 32 row pairs as one of workgroups of 64 that hold the tables in copies: from more blocks than
-// compute units on, where two of the smaller ones would share a unit (below, a unit's only workgroup then takes twice as long: 700 random
-// layers of IQ2_XXS and IQ3_XXS, 1 to 24 tokens: up to 256 blocks 1.03, from there to 1024 0.97, past that 0.975 and 0.96; at worst 1.07).
+// A gate . up launch of `blocks` workgroups of 32 row pairs as one of workgroups of 64 that hold the tables in copies: where the blocks make an even
+// number of rounds over the compute units, so that two of the smaller workgroups would share a unit to the end (an odd round makes a larger
+// workgroup's unit work twice as long as the others': 1.02 to 1.06 times the plain tables' launch at three, five and seven rounds, 0.85 to 0.98 at two,
+// four, six and eight). Beyond eight rounds, where rounds no longer stand out, by the rows: from 13 super-blocks of IQ2_XXS (0.98 to 1.02, shorter ones 1.05
+// to 1.13), from 7 of IQ3_XXS (0.86 to 1.02). 1200 random launches of 1 to 28
+// super-blocks: the rule is 0.3 % behind the better side, 0.92 of the plain time where it takes the copies.
 static bool gate_up_in_copies(int wtype, int k, int64_t blocks) {
-    return blocks > kCardUnits && copies_fit(wtype, tab_bytes_rt(wtype, true) + (size_t)act_col_bytes(wtype, k) + 64 * sizeof(float), 512);
+    const int64_t rounds = (blocks + kCardUnits - 1) / kCardUnits;
+    const int nb = k / 256;
+    if (rounds <= 8 ? rounds % 2 != 0 : nb < (wtype == BM_IQ2XXS ? 13 : 7)) return false;
+    return copies_fit(wtype, nb, tab_bytes_rt(wtype, true) + (size_t)act_col_bytes(wtype, k) + 64 * sizeof(float), 512);
 }
 
 hipError_t gate_up(const Launch &L, int wtype, const uint8_t *wg, const uint8_t *wu, int n_experts, int k,
@@ -1436,8 +1443,9 @@ hipError_t down_combine_hq(const Launch &L, int wtype, const uint8_t *w, int n_e
     const size_t lds = down_combine_lds(wtype, k, spt) + (size_t)(D - 64 / spt) * spt * sizeof(float);
     const unsigned blocks = (unsigned)((rpe + D - 1) / D);
     const bool row_major = plain_order((int64_t)m * spt, m, blocks, T);
-    // (from 512 threads on: of 256 a compute unit holds too few beside the copies; 450 random launches 0.95 to 0.99, at worst 1.03)
-    const bool wide = copies_fit(wtype, lds + (size_t)(tab_bytes_rt(wtype, true) - tab_bytes_rt(wtype)), T);
+    // (from 512 threads on: of 256 a compute unit holds too few beside the copies; 980 random launches of two super-blocks and more 0.98, by rows 0.96 to
+    // 1.0, at worst 1.12, two super-blocks of IQ2_XXS)
+    const bool wide = copies_fit(wtype, nb, lds + (size_t)(tab_bytes_rt(wtype, true) - tab_bytes_rt(wtype)), T);
     const size_t bytes = lds + (size_t)(tab_bytes_rt(wtype, wide) - tab_bytes_rt(wtype));
     auto launch = [&](auto kern) {
         hipError_t e = allow_lds(kern, bytes);

@@ -655,15 +655,20 @@ def test_fused_step_with_larger_down_workgroups(gpu, types, hidden, ff, m, top_k
     L.free()
 
 
-# Gate . up of the IQ types with a table in LDS: up to 256 blocks of 32 row pairs the tables as they are, beyond in copies and 64 row pairs a
-# workgroup (here 256 and 264; one row block a slot more than the others that holds 8 or 40 rows; by dies with the last eight blocks not
-# whole), with slots that are served elsewhere and refused ones. The down half of 512 and 1024 threads takes the copies as well.
+# Gate . up of the IQ types with a table in LDS: up to 256 blocks of 32 row pairs and at odd numbers of rounds of as many the tables as they are,
+# at even ones in copies and 64 row pairs a workgroup, beyond eight rounds by the rows (here 256 blocks and 264; one row block a slot more than the
+# others that holds 8 or 40 rows; three, six, nine and ten rounds; by dies with the last eight blocks not whole), with slots that are served
+# elsewhere and refused ones; a super-block a row never. The down half of 512 and 1024 threads takes the copies as well.
 @pytest.mark.parametrize("types,hidden,ff,m,top_k", (
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 512, 256, 32, 1),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 512, 256, 33, 1),
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.Q6_K), 768, 768, 6, 2),
     ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ3_XXS), 256, 512, 16, 4),
     ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 256, 3328, 10, 7),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.IQ2_XXS), 512, 3328, 7, 2),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ3_XXS), 768, 3328, 7, 1),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ3_XXS), 1792, 256, 36, 8),
+    ((bm.IQ2_XXS, bm.IQ2_XXS, bm.Q6_K), 3328, 256, 40, 8),
 ))
 def test_fused_step_with_tables_in_copies(gpu, types, hidden, ff, m, top_k):
     n_experts = 8
