@@ -827,11 +827,12 @@ struct Q8kCols {
         __builtin_amdgcn_sched_barrier(0);
     }
     // `live` (a column's number): a column whose slot is not live is not encoded (its rows may hold anything)
-    template <class Live>
+    // (ONE column: no division by a run-time length)
+    template <bool ONE, class Live>
     __device__ __forceinline__ void encode(const float *x, uint8_t *dst, int cols, int nb, int col_stride, u32 *fault, u32 layer, Live live) const {
         const int lane = threadIdx.x & 63;
         auto store = [&](int b, float4 v) __attribute__((always_inline)) {
-            const int c = b / nb;
+            const int c = ONE ? 0 : b / nb;
             if (live(c)) q8k_wave_block(v, dst + (size_t)c * col_stride + (size_t)(b - c * nb) * BM_Q8K_STRIDE, lane, fault, layer);
         };
 #pragma unroll
@@ -936,7 +937,7 @@ __global__ __launch_bounds__(T) void k_gate_up_xq(const float *x, const uint8_t 
     const Iq2Tables tb = stage_tables_as<WA, WIDE, T>(lds);
     uint8_t *col = lds + tab_bytes<WA, WIDE>();
     const int col_bytes = bm_act_col_bytes<WA>(na);
-    xrow.encode(x + (size_t)t * hidden, col, 1, na, 0, fault, layer, [](int) { return true; });
+    xrow.template encode<true>(x + (size_t)t * hidden, col, 1, na, 0, fault, layer, [](int) { return true; });
     __syncthreads();
     if (act_x && rb == 0 && slot % spt == 0) stage_bytes<T>(act_x + (size_t)t * col_bytes, col, col_bytes);
     float v[1];
@@ -986,7 +987,7 @@ __global__ __launch_bounds__(256) void k_gemv_x(const float *x, const uint8_t *w
     const Iq2Tables tb = stage_tables<WT>(lds);
     uint8_t *col = lds + tab_bytes<WT>();
     if constexpr (bm_takes_q8k(WT)) {
-        xcol.encode(xc, col, 1, n, 0, fault, layer, [](int) { return true; });
+        xcol.template encode<true>(xc, col, 1, n, 0, fault, layer, [](int) { return true; });
     } else { // a q8_2 block is four lanes of eight values; 2048 values a pass
         if (tid * 8 < k) {
             const float v8[8] = {x_lo.x, x_lo.y, x_lo.z, x_lo.w, x_hi.x, x_hi.y, x_hi.z, x_hi.w};
@@ -1046,7 +1047,7 @@ __global__ __launch_bounds__(T) void k_down_combine_hq(const uint8_t *w, u32 n_e
     float *s_w = part + D * spt;                                              // [spt]
     u32 *s_sel = reinterpret_cast<u32 *>(s_w + spt);                          // [spt]
     if constexpr (bm_takes_q8k(WT))
-        hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, col_stride, fault, layer,
+        hrows.template encode<false>(h + (size_t)t * spt * n * 256, cols, spt, n, col_stride, fault, layer,
                      [&](int c) { return (u32)__builtin_amdgcn_readlane((int)my_sel, __builtin_amdgcn_readfirstlane(c)) < n_experts; });
     else hrows.encode(h + (size_t)t * spt * n * 256, cols, spt, n, sel + t * spt, n_experts, fault, layer);
     if (tid < spt) {
