@@ -290,7 +290,8 @@ __device__ __forceinline__ bool picks_from_places(const PickLds<PER> &L, u32 t, 
 // still on their way, and a barrier that waited for those to be acknowledged cost the routing 1 us.
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// One wave a token.
+// One wave a token. One or two picks (one, past 256 experts) go by the rounds: counting takes as long whatever their number (us a launch by rounds / by
+// counting, 64 tokens and fewer: one pick of 128 experts 2.8 / 3.3, of 256 3.2 / 3.7; two 2.9 / 3.2, 3.6 / 3.7; two of 590 7.1 / 6.6).
 template <int PER>
 __global__ __launch_bounds__(256) void k_route_softmax(const float *logits, u32 n_tok, u32 n_exp, u32 used, u32 renorm,
                                                        float *probs, u32 *ids, float *weights, u32 *fault, u32 layer) {
@@ -305,6 +306,11 @@ __global__ __launch_bounds__(256) void k_route_softmax(const float *logits, u32 
         v[j] = e < n_exp ? logits[(size_t)t * n_exp + e] : -INFINITY;
     }
     if (!logits_finite<PER>(v, n_exp)) return route_refuse(t, n_exp, used, probs, weights, fault, layer);
+    if (used <= (PER <= 4 ? 2u : 1u)) {
+        route_probs_wave<PER>(v, n_exp, p);
+        store_probs<PER>(p, t, n_exp, probs);
+        return route_pick_rounds<PER>(p, t, n_exp, used, renorm, ids, weights);
+    }
     places_clear(L);
     route_probs_wave<PER>(v, n_exp, p);
     store_probs<PER>(p, t, n_exp, probs);

@@ -69,6 +69,38 @@ def test_router_is_the_cpu_paths(gpu, n_experts, top_k, m, seed, renorm):
     assert gpu.fault() == (bm.FAULT_NONE, 0)
 
 
+@pytest.mark.parametrize("n_experts,top_k", ((128, 1), (128, 2), (129, 3), (600, 1), (257, 2), (256, 8), (128, 15), (256, 16), (64, 31), (62, 32), (63, 32),
+                                             (64, 32), (33, 32), (32, 32), (40, 17), (128, 32), (1024, 8), (1000, 32)))
+def test_picks_at_the_edges_of_the_counting(gpu, n_experts, top_k):
+    """The picks by rounds (one or two of them) and by counting what passes a bound from group maxima (of sixteen groups of lanes up to fifteen
+    picks, of 32 beyond): ordinary logits, sorted ones either way, large ones crowded into half of the groups (more entries pass than the
+    list holds), equal ones across the last place, and all equal. bm_route_softmax on them, and bm_norm_route over rows that are them."""
+    rng = np.random.default_rng(7400 + n_experts + top_k)
+    lane = np.arange(n_experts) % 64
+    rows = [normal_f32(rng, n_experts) * np.float32(s) for s in (0.3, 1, 4)]
+    rows += [np.sort(rows[1]), np.sort(rows[1])[::-1], np.where(lane < 32, 3, 0) + rows[0], np.where(lane % 4 == 0, 3, 0) + rows[0]]
+    tied = np.sort(rows[1])[::-1].copy()
+    tied[top_k - 1:top_k + 1] = tied[top_k - 1]
+    rows += [rng.permutation(tied), np.zeros(n_experts, np.float32)]
+    logits = np.ascontiguousarray(np.stack(rows), np.float32)
+    m, hidden = len(rows), (n_experts + 7) // 8 * 8
+    want = [ora.route_softmax_topk(row, top_k) for row in logits]
+    gpu.fault_clear()
+    ids, wts, _ = run_router(gpu, logits, top_k)
+    for t in range(m):
+        assert np.array_equal(ids[t], want[t][0]), f"row {t}"
+        assert_ulp(wts[t], want[t][1], f"weights of row {t}", odd_share=1.0)
+    # a row of the router picks one value of the token's row, so the logits are the row
+    rd, xd = gpu.upload(np.eye(n_experts, hidden), np.float32), gpu.upload(np.pad(logits, ((0, 0), (0, hidden - n_experts))), np.float32)
+    ld, idd, wd = gpu.buffer(np.float32, m * n_experts), gpu.buffer(np.uint32, m * top_k).fill_bytes(0xEE), gpu.buffer(np.float32, m * top_k)
+    gpu.enqueue_norm_route(rd, xd, None, 0.0, m, n_experts, hidden, top_k, True, None, ld, None, idd, wd)
+    assert np.array_equal(ld.download().reshape(m, n_experts), logits)
+    assert np.array_equal(idd.download().reshape(m, top_k), ids) and np.array_equal(wd.download().reshape(m, top_k), wts)
+    assert gpu.fault() == (bm.FAULT_NONE, 0)
+    for b in (rd, xd, ld, idd, wd):
+        b.free()
+
+
 def test_router_ties_go_to_the_smaller_id(gpu):
     logits = np.zeros((3, 128), np.float32)
     logits[1, [5, 77, 100]] = 2.0          # three equal winners, then equal losers
