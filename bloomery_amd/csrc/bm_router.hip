@@ -209,11 +209,13 @@ __device__ __forceinline__ void places_clear(PickLds<PER> &L) {
 
 // The places of the first `used` + 1 entries in descending order of v, by one wave: at[r] = e for the entry e that r others are
 // larger than. Entries of equal value have the same count: they take the same place and leave the next one as it was, so a
-// caller finds out, and picks by rounds; so it does where more than 64 entries pass the bound, which takes equal ones.
+// caller finds out, and picks by rounds; so it does where more than 64 entries pass the bound (equal ones, or large ones crowded into few groups).
 // Not every entry is compared with every other (128 of them: a quarter of it a wave, over LDS, took 0.9 us, and the rounds are a
 // chain of eighty dependent instructions each): an entry below `used` + 1 others' maxima cannot be among the first, so the maxima of
-// sixteen groups of lanes (of the 64 lanes, for more than fifteen picks) give a bound that about as many entries pass as are
-// wanted; those go to LDS, a lane each, and are compared with one another.
+// sixteen groups of lanes (of 32 for sixteen picks and more, of the 64 lanes for more still) give a bound that about as many entries pass as are
+// wanted; those go to LDS, a lane each, and are compared with one another. A group costs a step of the count: of sixteen picks of 128 experts 4.1 us
+// a k_route_softmax with 64 groups, 3.4 with 32. With no more than half again as many groups as picks too many entries pass (31 of 32 groups: the
+// list overflows, 256 experts 5.3 -> 13.7 us; 24 of 32 past 256 experts 8.3 -> 17.6).
 template <int PER>
 __device__ __forceinline__ void places_by_counting(const float (&v)[PER], u32 n_exp, u32 used, PickLds<PER> &L) {
     const u32 lane = threadIdx.x & 63;
@@ -227,6 +229,10 @@ __device__ __forceinline__ void places_by_counting(const float (&v)[PER], u32 n_
         top = fmaxf(top, bm_dppf<kDppXor2>(top));
 #pragma unroll
         for (u32 g = 0; g < 64; g += 4) count_group(g);
+    } else if (used < (PER <= 4 ? 24u : 20u)) {
+        top = fmaxf(top, bm_dppf<kDppXor1>(top));
+#pragma unroll
+        for (u32 g = 0; g < 64; g += 2) count_group(g);
     } else {
 #pragma unroll 16
         for (u32 g = 0; g < 64; g++) count_group(g);

@@ -69,11 +69,11 @@ def test_router_is_the_cpu_paths(gpu, n_experts, top_k, m, seed, renorm):
     assert gpu.fault() == (bm.FAULT_NONE, 0)
 
 
-@pytest.mark.parametrize("n_experts,top_k", ((128, 1), (128, 2), (129, 3), (600, 1), (257, 2), (256, 8), (128, 15), (256, 16), (64, 31), (62, 32), (63, 32),
+@pytest.mark.parametrize("n_experts,top_k", ((128, 1), (128, 2), (129, 3), (600, 1), (257, 2), (256, 8), (128, 15), (256, 16), (256, 23), (256, 24), (300, 19), (300, 20), (64, 31), (62, 32), (63, 32),
                                              (64, 32), (33, 32), (32, 32), (40, 17), (128, 32), (1024, 8), (1000, 32)))
 def test_picks_at_the_edges_of_the_counting(gpu, n_experts, top_k):
     """The picks by rounds (one or two of them) and by counting what passes a bound from group maxima (of sixteen groups of lanes up to fifteen
-    picks, of 32 beyond): ordinary logits, sorted ones either way, large ones crowded into half of the groups (more entries pass than the
+    picks, then of 32, of 64 from 24 or 20 on): ordinary logits, sorted ones either way, large ones crowded into half of the groups (more entries pass than the
     list holds), equal ones across the last place, and all equal. bm_route_softmax on them, and bm_norm_route over rows that are them."""
     rng = np.random.default_rng(7400 + n_experts + top_k)
     lane = np.arange(n_experts) % 64
