@@ -364,6 +364,12 @@ hipError_t route_softmax(const Launch &L, const float *logits, int n_tok, int n_
 // with a meaning, and a move to the next lane hands the accumulators on.
 constexpr int kRouterSb = 256 + 8; // floats from one super-block of a token's row in LDS to the next
 __host__ __device__ inline int router_line(int hidden) { return (hidden + 255) / 256 * kRouterSb; }
+// Super-blocks of a router row that a wave has in LDS at a time (n4: see norm_rows): of short rows no more than they have, which lets the more
+// workgroups stand on a compute unit (eight of them throughout: rows of 304 to 760 values took up to 1.39 times as long as with eight lanes a row).
+__host__ __device__ constexpr int router_lines(int n4, int hidden) {
+    const int sbs = (hidden + 255) / 256;
+    return n4 == 1 ? 4 : n4 == -2 && sbs < 8 ? sbs : 8;
+}
 
 // (k_norm_route's arguments: what the head of a logits workgroup needs stands in the first fourteen words, which are in registers when a
 // wave starts - m_word is the token count, bit 31 set where the quantized column is asked for - and the rest travels as one
@@ -392,7 +398,8 @@ static_assert(offsetof(NormRouteArgs, late) == 56, "fourteen words in front of t
 
 // The norm of T rows (of tokens t0 .., the last token's where there are fewer: its numbers again) into LDS, row after row of
 // router_line(hidden) floats, without a barrier behind it; and to normed_out where that is wanted. Without a gain the rows as they are. N4: 16-byte
-// pieces of a row a thread holds in registers (rows of up to 1024 N4 values); 0: rows of any length, through LDS. `behind_requests` is
+// pieces of a row a thread holds in registers (rows of whole super-blocks and up to 1024 N4 values; -2, -4: as many, and any rows of so many values);
+// 0: rows of any length, through LDS. `behind_requests` is
 // called when the rows have been asked for, `behind_sums` when their squares are summed.
 template <int T, int N4, class F, class G>
 __device__ __forceinline__ void norm_rows(float *xs, double (*s_part)[4], const float *x, const float *gain, float eps, int hidden, float *normed_out,
@@ -414,28 +421,29 @@ __device__ __forceinline__ void norm_rows(float *xs, double (*s_part)[4], const 
         *in_lds(tt, i) = v;
         if (normed_out && t0 + tt < m) reinterpret_cast<float4 *>(normed_out + row(tt))[i] = v;
     };
-    constexpr int kRegs = N4 ? N4 : 1;
+    constexpr bool kInRegs = N4 != 0, kRagged = N4 <= 0;
+    constexpr int kRegs = N4 > 0 ? N4 : N4 < 0 ? -N4 : 1;
     [[maybe_unused]] float4 xv[T][kRegs], gv[kRegs];
     [[maybe_unused]] unsigned long long tl_row = 0, tl_norm = 0;
     double sum[T];
 #pragma unroll
     for (int tt = 0; tt < T; tt++) sum[tt] = 0.0;
-    if constexpr (N4 != 0) {
+    if constexpr (kInRegs) {
 #pragma unroll
         for (int tt = 0; tt < T; tt++)
 #pragma unroll
-            for (int j = 0; j < N4; j++)
+            for (int j = 0; j < kRegs; j++)
                 if (tid + 256 * j < n4) xv[tt][j] = reinterpret_cast<const float4 *>(x + row(tt))[tid + 256 * j];
         if (gain)
 #pragma unroll
-            for (int j = 0; j < N4; j++)
+            for (int j = 0; j < kRegs; j++)
                 if (tid + 256 * j < n4) gv[j] = reinterpret_cast<const float4 *>(gain)[tid + 256 * j];
         behind_requests();
         if (gain)
 #pragma unroll
             for (int tt = 0; tt < T; tt++)
 #pragma unroll
-                for (int j = 0; j < N4; j++)
+                for (int j = 0; j < kRegs; j++)
                     if (tid + 256 * j < n4) squares(sum[tt], xv[tt][j]);
     } else {
         behind_requests();
@@ -449,19 +457,19 @@ __device__ __forceinline__ void norm_rows(float *xs, double (*s_part)[4], const 
                     put(tt, i, v);
                 }
             }
-        // the steps past a row's end, to a whole super-block: -0, which times +0 leaves a chain as it is
+    }
+    if constexpr (kRagged) // the steps past a row's end, to a whole super-block: -0, which times +0 leaves a chain as it is
         for (int tt = 0; tt < T; tt++)
             for (int k = hidden + tid; k < (hidden + 255) / 256 * 256; k += 256) xs[tt * line + k + 8 * (k >> 8)] = -0.0f;
-    }
     BM_RTICK(tl_row, sum[0]);
     BM_RTOCK(1, tl_row);
     if (!gain) {
         behind_sums();
-        if constexpr (N4 != 0)
+        if constexpr (kInRegs)
 #pragma unroll
             for (int tt = 0; tt < T; tt++)
 #pragma unroll
-                for (int j = 0; j < N4; j++)
+                for (int j = 0; j < kRegs; j++)
                     if (tid + 256 * j < n4) put(tt, tid + 256 * j, xv[tt][j]);
         return;
     }
@@ -486,11 +494,11 @@ __device__ __forceinline__ void norm_rows(float *xs, double (*s_part)[4], const 
     }
     BM_RTICK(tl_norm, scale[0]);
     BM_RTOCK(2, tl_norm);
-    if constexpr (N4 != 0) {
+    if constexpr (kInRegs) {
 #pragma unroll
         for (int tt = 0; tt < T; tt++)
 #pragma unroll
-            for (int j = 0; j < N4; j++)
+            for (int j = 0; j < kRegs; j++)
                 if (tid + 256 * j < n4) put(tt, tid + 256 * j, normed(scale[tt], gv[j], xv[tt][j]));
     } else {
         for (int tt = 0; tt < T; tt++)
@@ -500,7 +508,8 @@ __device__ __forceinline__ void norm_rows(float *xs, double (*s_part)[4], const 
 }
 
 // The logits of tokens t0 .. t0 + T - 1 against router rows e0 .. e0 + R - 1. A wave takes one row and all the
-// tokens, whose chains run side by side. N4: see norm_rows; 0 takes a hidden that is not whole super-blocks too.
+// tokens, whose chains run side by side. N4: see norm_rows. Rows of one pass (up to eight super-blocks) hold one set of operands: registers a
+// lane 74 (up to 1024 values), 100 (2048), 168 (4096, two sets), 186, of two tokens 99, 116, 234; ragged ones up to six more.
 template <int R, int T, int N4, bool COH>
 __device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *router, const float *x, const float *gain, float eps, int n_exp,
                                                    int hidden, int m, float *normed_out, float *logits, int t0, int e0) {
@@ -513,20 +522,26 @@ __device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *ro
     BM_RTOCK(0, tl_start);
     const int r = wave; // the wave's row
     const bool has_dot = wave < R;
-    const int acc_l = lane >> 3, sb_l = lane & 7, line = router_line(hidden), sbs = (hidden + 255) / 256, passes = (sbs + 7) / 8;
+    const int acc_l = lane >> 3, sb_l = lane & 7, line = router_line(hidden), sbs = (hidden + 255) / 256;
+    constexpr bool kRagged = N4 <= 0, kOnePass = N4 == 1 || N4 == 2 || N4 == -2; // (rows of up to 1024, 2048 values)
+    const int passes = kOnePass ? 1 : (sbs + 7) / 8;
+    constexpr int kLines = N4 == 1 ? 4 : 8;
+    constexpr bool kFewer = N4 == -2;
+    const int lines = router_lines(N4, hidden);
     const float *const wrow = router + (size_t)(e0 + r < n_exp ? e0 + r : n_exp - 1) * hidden;
     struct Row { // a lane's operands of a pass
         float w[32], x[T][32];
     };
     // The router's row comes in whole lines, a super-block an instruction, and goes through the wave's own eight super-blocks of LDS:
     // asked for straight into the lanes that use it, 32 bytes here and there, it kept the address unit busy for 33 cycles an instruction.
-    float4 *const ws = reinterpret_cast<float4 *>(xs + T * line + wave * (8 * kRouterSb));
-    v4f raw[8];
+    float4 *const ws = reinterpret_cast<float4 *>(xs + T * line + wave * (lines * kRouterSb));
+    v4f raw[kLines];
     auto ask = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < kLines; i++) {
+            if (kFewer && i >= lines) break;
             const int sb = 8 * q + i < sbs ? 8 * q + i : sbs - 1, at = 256 * sb + 4 * lane; // (past the row's end: its last, for no reader)
-            if constexpr (N4 != 0) {
+            if constexpr (!kRagged) {
                 raw[i] = *reinterpret_cast<const v4f *>(wrow + at);
             } else {
                 const bool in = at < hidden;
@@ -537,11 +552,12 @@ __device__ __forceinline__ void router_logits_body(uint8_t *lds, const float *ro
     };
     auto park = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) *reinterpret_cast<v4f *>(ws + (kRouterSb / 4) * i + lane) = raw[i];
+        for (int i = 0; i < kLines; i++)
+            if (!kFewer || i < lines) *reinterpret_cast<v4f *>(ws + (kRouterSb / 4) * i + lane) = raw[i];
         lds_of_wave();
     };
     auto read_row = [&](Row &o) __attribute__((always_inline)) {
-        const float *const from = reinterpret_cast<const float *>(ws) + kRouterSb * sb_l + acc_l;
+        const float *const from = reinterpret_cast<const float *>(ws) + kRouterSb * (sb_l < lines ? sb_l : lines - 1) + acc_l;
 #pragma unroll
         for (int j = 0; j < 32; j++) o.w[j] = from[8 * j];
         lds_of_wave();
@@ -818,9 +834,9 @@ __global__ __launch_bounds__(256) void k_norm_rows(const float *x, const float *
 // No unit is full (2048 tokens: one wave a SIMD, matrix cores busy 40 % of the cycles, LDS 23 %, vector ALU 12 %, waiting 23 %; 4096:
 // 52, 31, 15, 19 %): a wave's chain of matrix instructions, 256 cycles a step of 32 values, is stretched by the LDS accesses that stand
 // between them (26 KB a step and workgroup). Two tiles of experts a wave, which halve the reads of a matrix instruction, were no faster
-// (39.1 against 39.8 us at 4096 tokens: half the workgroups). Measured, with the norm's launch: 4096 tokens x 128 experts x 2048 values
+// (39.1 against 39.8 us at 4096 tokens: half the workgroups). Measured, with the norm's launch, against workgroups of a token each: 4096 tokens x 128 experts x 2048 values
 // 827 -> 40 us, 2048 tokens 416 -> 25, 333 tokens 71 -> 13.7, 64 tokens 16.7 -> 11.1; 1024 tokens x 256 experts x 7168 values
-// 2867 -> 64 us. The one-token workgroups of k_router_logits read and lay out the router's rows once a token.
+// 2867 -> 64 us. Workgroups of a token or two read the router's rows once a token or two.
 template <int SPLIT, int KC, bool RAGGED>
 __global__ __launch_bounds__(256) void k_router_tiles(const float *router, const float *x, int m, int n_exp, int hidden, float *logits) {
     constexpr int kTok = 16, kExp = SPLIT == 1 ? 64 : 16, kAcc = 8 / SPLIT, kRows = kTok + kExp;
@@ -956,22 +972,31 @@ __global__ __launch_bounds__(256) void k_router_tiles(const float *router, const
 }
 
 // LDS of a workgroup of so many tokens, whose dots take so many waves.
-static size_t router_lds_bytes(int tokens, int waves, int hidden) { return ((size_t)tokens * router_line(hidden) + (size_t)waves * 8 * kRouterSb) * sizeof(float); }
+static size_t router_lds_bytes(int tokens, int waves, int hidden, int n4) {
+    return ((size_t)tokens * router_line(hidden) + (size_t)waves * router_lines(n4, hidden) * kRouterSb) * sizeof(float);
+}
 
 bool router_logits_fits(int hidden) { return 16 * (size_t)(((hidden / 8 + 3) & ~3) + 8) * sizeof(float) + 16 <= (size_t)kMaxLds - 1024; }
 
-// Router rows and tokens a workgroup takes. A row and a token each while that leaves no more workgroups than stand on the card at once at three
-// waves a SIMD (two, where a row takes several passes): a launch of few workgroups is a wave's chain behind the norm of its token's
-// row, and nothing is shorter than one of each. Then four rows a token, a wave each, and from three workgroups a compute unit on two tokens
-// a workgroup, which ask for a row's bytes once - not where two rows of tokens leave a compute unit one workgroup.
-// (us a launch, 1 x 1 / 4 x 1 / 4 x 2, 128 experts: 2048 values 1 token 5.6 / 6.3 / 7.5, 4 tokens 6.0 / 6.4 / 7.6, 8 tokens 7.9 / 6.6 / 7.9, 24 tokens
-// 13.0 / 8.4 / 9.1, 32 tokens 15.9 / 10.5 / 9.6; 4096 values 4 tokens 7.7 / 8.5 / 10.4, 8 tokens 11.9 / 8.8 / 10.7, 24 tokens - / 14.7 / 12.6; 7168 values
-// 4 tokens 9.9 / 10.3 / 13.5, 24 tokens - / 19.6 / 24.3.)
+// Router rows and tokens a workgroup takes. A row and a token each while that leaves no more workgroups than stand on the card at once: a
+// launch of few workgroups is a wave's chain behind the norm of its token's row, and nothing is shorter than one of each (rows of up to 1024
+// values are so short that sharing the norm soon pays). Then four rows a token, a wave each, and from three workgroups a compute unit on two tokens
+// a workgroup, which ask for a row's bytes once: where that needs fewer rounds over the card. A compute unit holds two workgroups of 4 x 2 and three of
+// 4 x 1 of rows of 2304 to 4096 values (so 4 x 2 between one round of the one and of the other), two of either where such rows are ragged,
+// as many as have work of the short whole rows (always 4 x 1).
+// (us a launch, 1 x 1 / 4 x 1 / 4 x 2, 128 experts: 2048 values 1 token 5.5 / 6.2 / 7.4, 8 tokens 7.0 / 6.4 / 7.8; 4096 values 4 tokens 7.7 / 8.5 / 10.4, 8 tokens
+// 11.9 / 8.8 / 10.7; 7168 values 4 tokens 9.9 / 10.3 / 13.5. 3300 random launches of 8 to 8192 values, by such fours: 1300 to 2048 values 900 fours
+// 1.15 / 1.0 and 1.04 / 1.0 times the better of 4 x 1 and 4 x 2, 768 1.0 / 1.07; 4096 values 640 1.0 / 1.04, 900 1.12 / 1.0, 1300 1.0 / 1.04; up to 1024 values
+// 1.0 / 1.05 at 1300, ragged 1.07 / 1.0.)
 enum RouterForm { kForm1x1, kForm4x1, kForm4x2 };
 static long router_fours(int m, int n_exp) { return (long)m * ((n_exp + 3) / 4); }
 static RouterForm router_form(int m, int n_exp, int hidden) {
-    if ((long)m * n_exp <= (hidden <= 2048 ? 640 : 512)) return kForm1x1;
-    if (hidden <= 4096 && router_fours(m, n_exp) > (hidden <= 2048 ? 768 : 640)) return kForm4x2;
+    const bool ragged = hidden % 256 != 0;
+    const long fours = router_fours(m, n_exp);
+    if ((long)m * n_exp <= (hidden <= 1024 ? 256 : hidden <= 4096 && !ragged ? 640 : 512)) return kForm1x1;
+    if (hidden <= 1024) return ragged && fours > 1024 ? kForm4x2 : kForm4x1;
+    if (hidden <= 2048) return fours > 768 ? kForm4x2 : kForm4x1;
+    if (hidden <= 4096) return (ragged ? fours > 512 : fours > 768 && fours <= 1024) ? kForm4x2 : kForm4x1;
     return kForm4x1;
 }
 
@@ -983,24 +1008,29 @@ static hipError_t with_form(RouterForm form, int hidden, F f) {
     constexpr integral_constant<int, 2> two{};
     constexpr integral_constant<int, 4> four{};
     auto tokens = [&](auto n4) { return form == kForm1x1 ? f(one, one, n4) : form == kForm4x1 ? f(four, one, n4) : f(four, two, n4); };
+    if (hidden % 256 != 0 && hidden <= 2048) return tokens(integral_constant<int, -2>{});
+    if (hidden % 256 != 0 && hidden <= 4096) return tokens(integral_constant<int, -4>{});
     if (hidden % 256 != 0 || hidden > 8192) return tokens(integral_constant<int, 0>{});
-    if (hidden > 2048) return tokens(integral_constant<int, 8>{});
-    return tokens(two);
+    if (hidden > 4096) return tokens(integral_constant<int, 8>{});
+    if (hidden > 2048) return tokens(four);
+    return hidden > 1024 ? tokens(two) : tokens(one);
 }
 
-// Whether the norm and the logits go as two launches, rows and then tiles: from six workgroups of four rows a compute unit on, from five
-// for rows of up to 1024 values, whose tiles are short, and of more than 4096, of which fewer workgroups stand on a compute unit. (us, one launch /
-// the tiles' three, routing included, by such workgroups: 1024 values 1024 of them 7.9 / 10.0, 1536 10.8 / 10.0; 2048 values 1536 12.5 / 13.3, 2048 15.0 /
-// 13.5; 4096 values 1536 18.7 / 20.0, 2048 22.4 / 20.3; 7168 values 1024 23.2 / 28.8, 1536 31.4 / 29.4.) The tiles read
-// normed rows from memory: a caller that wants none of them stays with the workgroups that norm their own.
+// Whether the norm and the logits go as two launches, rows and then tiles: by workgroups of four rows, from the later the shorter the rows, whose
+// workgroups are the cheaper (and the more of them stand on a compute unit), and whose tiles are mostly their launch. (one launch / the tiles' two,
+// with the routing's as well where it is asked for, as times the better: up to 1024 values 2500 of them 1.0 / 1.13 to 1.18, 3500 1.08 / 1.03; 1280 to 2048
+// values 1800 1.01 / 1.14, 2200 1.09 / 1.04, ragged 2500 1.0 / 1.1, 3500 1.09 / 1.0; 2304 to 4096 values 1400 1.0 / 1.2, 1800 1.09 / 1.07, ragged 1800 1.0 / 1.09,
+// 2500 1.13 / 1.0; longer 1200 1.0 / 1.2, 1400 1.07 / 1.06.) The tiles read normed rows from memory: a caller that wants none of them stays with the workgroups that norm their own.
 static bool router_tiled(int m, int n_exp, int hidden, const float *gain, const float *normed_out) {
-    return router_fours(m, n_exp) > (hidden > 1024 && hidden <= 4096 ? 1536 : 1280) && (!gain || normed_out);
+    const bool ragged = hidden % 256 != 0;
+    const int from = hidden <= 1024 ? 3072 : hidden <= 2048 ? (ragged ? 3072 : 2048) : hidden <= 4096 ? (ragged ? 2048 : 1536) : 1280;
+    return router_fours(m, n_exp) > from && (!gain || normed_out);
 }
 
 static hipError_t router_tiles(const Launch &L, const float *router, const float *x, const float *gain, float eps, int m, int n_exp,
                                int hidden, float *normed_out, float *logits, uint8_t *act_x = nullptr, bool q8k = false) {
     if (normed_out || act_x) {
-        const size_t lds = router_lds_bytes(1, 0, hidden);
+        const size_t lds = router_lds_bytes(1, 0, hidden, 0);
         auto kern = hidden % 256 != 0 || hidden > 8192 ? k_norm_rows<0> : hidden > 2048 ? k_norm_rows<8> : k_norm_rows<2>;
         hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;
@@ -1027,7 +1057,7 @@ hipError_t router_logits(const Launch &L, const float *router, const float *x, c
     if (!router_logits_fits(hidden)) return hipErrorInvalidValue;
     return with_form(router_form(m, n_exp, hidden), hidden, [&](auto r, auto t, auto n4) {
         auto kern = k_router_logits<decltype(r)::value, decltype(t)::value, decltype(n4)::value>;
-        const size_t lds = router_lds_bytes(t, r, hidden);
+        const size_t lds = router_lds_bytes(t, r, hidden, n4);
         hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;
         const unsigned grid = (unsigned)((m + t - 1) / t) * (unsigned)((n_exp + r - 1) / r);
@@ -1048,7 +1078,7 @@ hipError_t norm_route(const Launch &L, const float *router, const float *x, cons
     return with_form(router_form(m, n_exp, hidden), hidden, [&](auto r, auto t, auto n4) {
         constexpr int R = decltype(r)::value, T = decltype(t)::value, N4 = decltype(n4)::value;
         auto kern = n_exp <= 128 ? k_norm_route<R, T, N4, 2> : n_exp <= 256 ? k_norm_route<R, T, N4, 4> : k_norm_route<R, T, N4, 16>;
-        const size_t lds = router_lds_bytes(T, R, hidden);
+        const size_t lds = router_lds_bytes(T, R, hidden, N4);
         hipError_t e = allow_lds(kern, lds);
         if (e != hipSuccess) return e;
         const unsigned grid = (unsigned)((m + T - 1) / T) * (unsigned)((n_exp + R - 1) / R) + (act_x ? (unsigned)m : 0u) + (unsigned)m;

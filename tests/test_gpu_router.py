@@ -325,10 +325,13 @@ def test_norm_route_is_the_two_launches_in_one(gpu, n_experts, hidden, m, top_k,
 @pytest.mark.parametrize("n_experts,hidden,m,top_k,with_gain", ((128, 256, 1, 15, True), (5, 2304, 3, 5, True), (127, 2048, 5, 8, True), (641, 2048, 1, 16, True),
                                                                 (130, 1792, 25, 32, False), (98, 2048, 33, 1, True), (257, 4352, 3, 9, True),
                                                                 (66, 4096, 41, 6, True), (131, 7168, 5, 8, True), (64, 8448, 9, 8, True), (70, 264, 3, 16, True),
-                                                                (129, 2312, 7, 17, False), (17, 20256, 33, 3, True)))
+                                                                (129, 2312, 7, 17, False), (17, 20256, 33, 3, True), (128, 1024, 5, 8, True), (64, 760, 9, 6, True),
+                                                                (130, 328, 33, 4, True), (64, 2040, 9, 8, False), (127, 1096, 25, 8, True), (66, 2560, 47, 6, True),
+                                                                (66, 2304, 62, 6, False), (131, 7168, 3, 8, True), (9, 2312, 5, 2, True), (64, 2312, 33, 4, True),
+                                                                (33, 4360, 3, 4, True), (257, 4360, 3, 8, False)))
 def test_norm_route_forms(gpu, n_experts, hidden, m, top_k, with_gain):
     """Every form of the fused launch's workgroups (bm_router.hip, router_form: a row and a token, four rows, four rows and two
-    tokens, with a last token by itself and rows left over) over rows of one super-block, of one whole pass of eight and a super-block more, of
+    tokens, with a last token by itself and rows left over), at each number of registers a row takes, over rows of one super-block, of one whole pass of eight and a super-block more, of
     lengths that are not whole super-blocks and the longest taken: normed rows, logits, ids against the oracle, the weights
     within its units; picks up to the most there are."""
     rng = np.random.default_rng(7000 + hidden + m)
@@ -358,7 +361,7 @@ def test_norm_route_forms(gpu, n_experts, hidden, m, top_k, with_gain):
             b.free()
 
 
-@pytest.mark.parametrize("n_experts,hidden,m,with_gain", ((129, 2048, 49, True), (16, 2048, 330, False), (17, 2056, 400, True), (1000, 512, 33, True),
+@pytest.mark.parametrize("n_experts,hidden,m,with_gain", ((129, 2048, 49, True), (129, 2048, 75, True), (16, 2048, 330, False), (17, 2056, 400, True), (17, 2056, 420, True), (1000, 512, 33, True),
                                                            (33, 520, 650, False), (130, 2048, 1100, True), (70, 2072, 2100, True), (65, 264, 4096, True)))
 def test_many_tokens_take_the_tiles_with_the_same_bits(gpu, n_experts, hidden, m, with_gain):
     """Batches whose norm and logits go as rows and tiles (bm_router.hip, router_tiled): rows that are whole groups of chunks and
