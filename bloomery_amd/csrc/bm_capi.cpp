@@ -1275,7 +1275,7 @@ int bm_router_logits(bm_ctx *ctx, const float *router_dev, const float *x_dev, c
     if (hidden < 8 || hidden % 8 != 0)
         return fail(ctx, BM_ESHAPE, "%s: hidden = %d is not a positive multiple of 8 (the f32 row dot's eight lanes)", what, hidden);
     if ((int64_t)n_tokens * n_experts > (1 << 30)) return fail(ctx, BM_ESHAPE, "%s: %d tokens x %d experts is past what a launch takes", what, n_tokens, n_experts);
-    if (!bmk::router_logits_fits(hidden)) return fail(ctx, BM_ESHAPE, "%s: two rows of hidden = %d do not fit the workgroup's LDS", what, hidden);
+    if (!bmk::router_logits_fits(hidden)) return fail(ctx, BM_ESHAPE, "%s: hidden = %d, the router takes rows of up to %d values", what, hidden, bmk::kRouteMaxHidden);
     if ((((uintptr_t)router_dev | (uintptr_t)x_dev | (uintptr_t)gain_dev | (uintptr_t)normed_dev) & 15) != 0)
         return fail(ctx, BM_ESHAPE, "%s: router_dev %p, x_dev %p, gain_dev %p and normed_dev %p must be 16-byte aligned", what,
                     (const void *)router_dev, (const void *)x_dev, (const void *)gain_dev, (const void *)normed_dev);
@@ -1299,7 +1299,7 @@ int bm_norm_route(bm_ctx *ctx, const float *router_dev, const float *x_dev, cons
                     bmk::kRouteMaxPicks);
     if (hidden < 8 || hidden % 8 != 0)
         return fail(ctx, BM_ESHAPE, "%s: hidden = %d is not a positive multiple of 8 (the f32 row dot's eight lanes)", what, hidden);
-    if (!bmk::router_logits_fits(hidden)) return fail(ctx, BM_ESHAPE, "%s: two rows of hidden = %d do not fit the workgroup's LDS", what, hidden);
+    if (!bmk::router_logits_fits(hidden)) return fail(ctx, BM_ESHAPE, "%s: hidden = %d, the router takes rows of up to %d values", what, hidden, bmk::kRouteMaxHidden);
     if ((((uintptr_t)router_dev | (uintptr_t)x_dev | (uintptr_t)gain_dev | (uintptr_t)normed_dev) & 15) != 0)
         return fail(ctx, BM_ESHAPE, "%s: router_dev %p, x_dev %p, gain_dev %p and normed_dev %p must be 16-byte aligned", what,
                     (const void *)router_dev, (const void *)x_dev, (const void *)gain_dev, (const void *)normed_dev);

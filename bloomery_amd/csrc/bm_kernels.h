@@ -156,7 +156,7 @@ hipError_t gemm_half(const Launch &L, int wtype, const uint8_t *w, int n_experts
 
 // ---------------------------------------------------------------------------------------- router (bm_router.hip)
 
-constexpr int kRouteMaxExperts = 1024, kRouteMaxPicks = 32;
+constexpr int kRouteMaxExperts = 1024, kRouteMaxPicks = 32, kRouteMaxHidden = 20256;
 // probs may be NULL. logits[n_tok * n_exp], ids / weights[n_tok * used].
 hipError_t route_softmax(const Launch &L, const float *logits, int n_tok, int n_exp, int used, int renorm, float *probs,
                          uint32_t *ids, float *weights);

@@ -363,7 +363,7 @@ hipError_t route_softmax(const Launch &L, const float *logits, int n_tok, int n_
 // banks. Then the chains run super-block by super-block: every lane does its 32 steps, only the lanes of the chains' present place
 // with a meaning, and a move to the next lane hands the accumulators on.
 constexpr int kRouterSb = 256 + 8; // floats from one super-block of a token's row in LDS to the next
-__host__ __device__ inline int router_line(int hidden) { return (hidden + 255) / 256 * kRouterSb; }
+__host__ __device__ constexpr int router_line(int hidden) { return (hidden + 255) / 256 * kRouterSb; }
 // Super-blocks of a router row that a wave has in LDS at a time (n4: see norm_rows): of short rows no more than they have, which lets the more
 // workgroups stand on a compute unit (eight of them throughout: rows of 304 to 760 values took up to 1.39 times as long as with eight lanes a row).
 __host__ __device__ constexpr int router_lines(int n4, int hidden) {
@@ -972,11 +972,14 @@ __global__ __launch_bounds__(256) void k_router_tiles(const float *router, const
 }
 
 // LDS of a workgroup of so many tokens, whose dots take so many waves.
-static size_t router_lds_bytes(int tokens, int waves, int hidden, int n4) {
+static constexpr size_t router_lds_bytes(int tokens, int waves, int hidden, int n4) {
     return ((size_t)tokens * router_line(hidden) + (size_t)waves * router_lines(n4, hidden) * kRouterSb) * sizeof(float);
 }
 
-bool router_logits_fits(int hidden) { return 16 * (size_t)(((hidden / 8 + 3) & ~3) + 8) * sizeof(float) + 16 <= (size_t)kMaxLds - 1024; }
+// The longest rows the router takes are the entries' contract (kRouteMaxHidden); every form's LDS holds them beside its arrays of fixed size.
+static_assert(router_lds_bytes(1, 4, kRouteMaxHidden, 0) + sizeof(PickLds<16>) + 1024 <= (size_t)kMaxLds, "four rows a workgroup, rows of any length");
+static_assert(router_lds_bytes(2, 4, 4096, 4) + sizeof(PickLds<16>) + 1024 <= (size_t)kMaxLds, "four rows and two tokens, rows of up to 4096 values");
+bool router_logits_fits(int hidden) { return hidden <= kRouteMaxHidden; }
 
 // Router rows and tokens a workgroup takes. A row and a token each while that leaves no more workgroups than stand on the card at once: a
 // launch of few workgroups is a wave's chain behind the norm of its token's row, and nothing is shorter than one of each (rows of up to 1024

@@ -532,3 +532,16 @@ def test_norm_route_raises_and_refuses_like_its_parts(gpu):
         assert e.value.code == bm.ESHAPE and word in str(e.value) and "bm_norm_route" in str(e.value)
     for b in (rd, xd, logits, ids, wts):
         b.free()
+
+
+def test_rows_past_the_longest_are_refused(gpu):
+    """20256 values are taken (test_norm_route_forms), the next length is refused by both entries before any launch."""
+    rd, xd, out = gpu.buffer(np.float32, 4 * 20264), gpu.buffer(np.float32, 20264), gpu.buffer(np.float32, 16)
+    ids = gpu.buffer(np.uint32, 4)
+    for call, name in ((lambda: gpu.enqueue_norm_route(rd, xd, None, 0.0, 1, 4, 20264, 2, True, None, out, None, ids, out), "bm_norm_route"),
+                       (lambda: gpu.enqueue_router_logits(rd, xd, None, 0.0, 1, 4, 20264, None, out), "bm_router_logits")):
+        with pytest.raises(bm.GpuError) as e:
+            call()
+        assert e.value.code == bm.ESHAPE and "20256" in str(e.value) and name in str(e.value)
+    for b in (rd, xd, out, ids):
+        b.free()
