@@ -1035,6 +1035,33 @@ static bool gemm_ahead(const bm_scratch *s, int m) {
     return tiles > line.launches + line.die * v * std::ceil(std::max(experts, n / 64 + experts / 2) / 8);
 }
 
+// The path a call with m tokens takes, and the f32 order of its GEMMs.
+struct PathChoice {
+    int path, mode;
+};
+
+// Whether slot by slot is ahead of the exact GEMM, by an estimate of either's time in us (stacks on Q8_K columns, where the grouped path would go slot by
+// slot). Slot by slot: five short launches, and the walks' time by slots and weights, each row's end as much as 128 values. The
+// GEMM: its launches, h through its f32 rows, and tiles of 64 rows by as many slots in rounds over the card, each a chain of super-blocks that is as long
+// for one slot as for 64. (gemm_ahead weighs the GEMM against tile launches, which take longer than this form where experts are few and have few slots.
+// 10000 random layers at one to five times the tokens from which it takes the GEMM, 1 to 128 experts, hidden 256 to 7168, ff 256 to 3072, cold weights: either estimate is
+// within 8 % on average; the half that go slot by slot take 0.752 of the GEMM's time, 59 of them more than 1.05 times and 1.19 at worst; all of
+// them 0.6 % behind the better side, by the GEMM alone 16 %; of 4000 others six above 1.05. IQ4_XS, hidden 1792, ff 256, 2 experts, 31 tokens 27.8 -> 15.5 us.)
+static bool slots_ahead_of_gemm(const bm_scratch *s, double slots) {
+    struct Cost {
+        double walk, chain; // us a slot and 2^20 weights; us a super-block of a round
+    };
+    auto cost = [](int type) {
+        return type == BM_TYPE_IQ2_XXS ? Cost{0.073, 3.1} : type == BM_TYPE_IQ3_XXS ? Cost{0.085, 3.2} : type == BM_TYPE_IQ4_XS ? Cost{0.08, 2.2} : Cost{0.073, 1.85};
+    };
+    const Cost gate = cost(s->gate_type), down = cost(s->down_type);
+    const double hidden = s->hidden, ff = s->ff, tiles = std::max((double)s->n_experts, slots / 64 + s->n_experts / 2.0);
+    const double walks = 12 + slots * (2 * gate.walk * ff * (hidden + 128) + down.walk * hidden * (ff + 128)) / (1 << 20);
+    const double rounds_a = std::max(1.0, 2 * tiles * std::ceil(ff / 64) / 350), rounds_b = std::max(1.0, tiles * std::ceil(hidden / 64) / 350);
+    const double gemm = 14 + 1e-5 * slots * ff + gate.chain * hidden / 256 * rounds_a + down.chain * ff / 256 * rounds_b;
+    return walks < 0.95 * gemm;
+}
+
 // Whether a step of both stacks on Q8_K columns goes slot by slot through launches of its own: the columns quantized once, gate . up and down a
 // workgroup a slot's rows.
 // In place of the grouped step's tiles: the one-column walks (activation operands read a super-block ahead, the IQ tables in copies) are that
@@ -1050,14 +1077,16 @@ static bool gemm_ahead(const bm_scratch *s, int m) {
 // fewer to quantize: there every workgroup quantizes the columns it reads itself, which three launches more cost less than by then (over it, 900 random
 // layers below 22 tokens, by MB: 1.16 at 30 to 64, 1.08 to 96, 1.02 to 128, 0.98 to 160, 0.94 to 200, 0.91 to 256, 0.88 to 400, 0.84 beyond without
 // an end; one or two slots a token 1.04 from 128 to 160, 1.03 to 200, 0.98 to 400).
-static bool slot_by_slot(const bm_scratch *s, int m, int path) {
+// In place of the GEMM in the exact order, where the grouped path would go so and slots_ahead_of_gemm; not where the caller has set the GEMM's line.
+static bool slot_by_slot(const bm_scratch *s, int m, PathChoice choice) {
+    const int path = choice.path;
     if (act_form(s->gate_type) == 0 || act_form(s->down_type) == 0 || m > bmk::kMaxDecodeTokens || !per_slot_fits(s)) return false;
     const int64_t slots = (int64_t)m * s->spt;
     const int64_t asked = slots * (2 * s->ff * bm_row_bytes(s->gate_type, s->hidden) + s->hidden * bm_row_bytes(s->down_type, s->ff));
-    if (path == BM_PATH_GEMM) return false;
     // A path that the caller forces takes its own launches. The grouped step of no more slots than experts is this one: its tiles hold a slot each.
     if (s->path != BM_PATH_AUTO) return path == BM_PATH_GROUPED && slots <= s->n_experts;
     if (path == BM_PATH_PER_SLOT) return asked >= (s->spt > 2 ? 128000000 : 200000000);
+    if (path == BM_PATH_GEMM && (choice.mode != BM_GEMM_EXACT || s->gemm_from || !slots_ahead_of_gemm(s, (double)slots))) return false;
     if (slots <= s->n_experts) return true;
     if (asked > 500000000 || s->hidden >= 4096) return asked <= 500000000;
     auto work = [](int type) { return type == BM_TYPE_IQ2_XXS ? 1.0 : type == BM_TYPE_IQ3_XXS ? 0.7 : type == BM_TYPE_IQ4_XS ? 0.4 : 0.3; };
@@ -1066,10 +1095,7 @@ static bool slot_by_slot(const bm_scratch *s, int m, int path) {
     return of_slot * ((double)slots - 2 * tiles_worth((double)slots, s->n_experts)) <= 500;
 }
 
-// The path a call with m tokens takes, and the f32 order of its GEMMs: the one place where it is chosen.
-struct PathChoice {
-    int path, mode;
-};
+// The one place where the path is chosen.
 static PathChoice path_choice(const bm_scratch *s, int m) {
     const bool gemm_ok = bmk::gemm_supported(s->gate_type) && bmk::gemm_supported(s->down_type);
     const bool per_slot_ok = m <= bmk::kMaxDecodeTokens && per_slot_fits(s);
@@ -1111,7 +1137,7 @@ int bm_moe_forward(bm_ctx *ctx, bm_scratch *s, const bm_weights *wg, const bm_we
                                                      (uint32_t)n_experts));
     };
     const PathChoice choice = path_choice(s, m);
-    if (((uintptr_t)x_dev & 15) == 0 && slot_by_slot(s, m, choice.path)) { // (the other steps take such an x, or refuse it)
+    if (((uintptr_t)x_dev & 15) == 0 && slot_by_slot(s, m, choice)) { // (the other steps take such an x, or refuse it)
         // (In the per-slot step's place only the rows of tokens that some expert takes, as that step does: a batch may be filled up with rows that
         // hold anything and have their slots served elsewhere. The grouped step quantizes, and answers for, every row.)
         const bool taken_only = choice.path == BM_PATH_PER_SLOT;

@@ -387,8 +387,9 @@ int bm_swiglu_quant_sel(bm_ctx *ctx, const float *g_dev, const float *u_dev, con
  * GEMM is taken from 96 tokens on where the gate/up type has kernels of that mode; below 96 tokens a GEMM path runs in the exact order.
  * Where gate/up and down stacks all dot against Q8_K columns a step can also go slot by slot through launches of its own, same bits: the tokens'
  * columns quantized once, bm_gate_up, the quantizer of h, bm_gemv_sel, the slots' sum (x_dev 16-byte aligned). It is the grouped path's form for a batch
- * with no more slots than experts, and under BM_PATH_AUTO it stands in for the per-slot and the grouped path wherever measurements put it
- * ahead of their launches (by the bytes of expert rows that the slots ask for, the types and the slots an expert).
+ * with no more slots than experts, and under BM_PATH_AUTO it stands in for the per-slot path, the grouped one and the GEMM in the exact order
+ * (where the GEMM's line is not the caller's) wherever measurements put it ahead of their launches (by the bytes of expert rows that the
+ * slots ask for, the types, the shape and the slots an expert).
  * bm_scratch_set_path sets crossovers of the caller's own (0 keeps what is; gemm_from then holds for both modes, in the mode's own
  * f32 order) or forces one path, which then runs the launches listed for it (the grouped one's form for few slots among them).
  * bm_scratch_path_for: the path a call with m tokens takes, also where the slot-by-slot launches stand in for it. A slot whose id names no expert of the stack adds nothing to

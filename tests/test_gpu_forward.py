@@ -169,6 +169,50 @@ def test_a_forced_path_takes_its_own_launches(gpu, types, hidden, ff, n_experts,
         L.free()
 
 
+@pytest.mark.parametrize("types,hidden,ff,n_experts,top_k,m,mode,slots", (
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 1792, 256, 2, 1, 31, bm.GEMM_EXACT, True),   # fifteen slots an expert: half the GEMM's time
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), 1792, 256, 2, 1, 31, bm.GEMM_FAST, True),    # below 96 tokens the exact order in this mode too
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.Q3_K), 512, 256, 4, 2, 99, bm.GEMM_EXACT, True),
+    ((bm.IQ4_XS, bm.IQ4_XS, bm.Q3_K), 512, 256, 4, 2, 100, bm.GEMM_EXACT, False),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ2_XXS), 256, 512, 1, 1, 266, bm.GEMM_EXACT, True),
+    ((bm.IQ3_XXS, bm.IQ3_XXS, bm.IQ2_XXS), 256, 512, 1, 1, 267, bm.GEMM_EXACT, False),
+))
+def test_few_slots_of_few_experts_go_slot_by_slot_in_the_gemms_place(gpu, types, hidden, ff, n_experts, top_k, m, mode, slots):
+    """Stacks on Q8_K columns where the path is the GEMM's: on both sides of the line from which its launches run, in its exact order; a
+    caller's own line or a forced path takes them at once. Outputs are the oracle's either way."""
+    L = Layer(gpu, types, hidden, ff, n_experts, 5230 + m, cheap=True)
+    rng = np.random.default_rng(5231)
+    x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
+    ids, wts = route(rng, m, n_experts, top_k)
+    wts[2, 0] = wts[m - 1, top_k - 1] = 0.0  # (the two slots that no expert takes below)
+    want = (L.oracle(x, ids, wts, top_k)[0].reshape(m, hidden) + resid).astype(np.float32).reshape(-1)
+    ids[2, 0], ids[m - 1, top_k - 1] = bm.HOST_SLOT, n_experts
+    xd, sel, wd, rd = gpu.upload(x, np.float32), gpu.upload(ids, np.uint32), gpu.upload(wts, np.float32), gpu.upload(resid, np.float32)
+    y = gpu.buffer(np.float32, m * hidden)
+    sc = gpu.scratch(types[0], types[2], hidden, ff, n_experts, top_k, m)
+    step = lambda: gpu.enqueue_moe_forward(sc, L.dg, L.du, L.dd, xd, sel, wd, rd, m, y)  # noqa: E731
+    gpu.set_gemm_mode(mode)
+    try:
+        ways = ((bm.PATH_AUTO, 0, slots), (bm.PATH_GEMM, 0, False), (bm.PATH_AUTO, 1, False))
+        for path, line, takes in ways if mode == bm.GEMM_EXACT else ways[:1]:
+            sc.set_path(path, 0, line)
+            assert sc.path_for(m) == bm.PATH_GEMM
+            assert (route_taken(gpu, step) == "slot by slot") == takes, (path, line)
+            gpu.fault_clear()
+            for _ in range(2):
+                y.fill_bytes(0xFF)
+                step()
+                assert_f32(y.download(), want, f"path {path}, line {line}")
+            assert gpu.fault()[1] == 1 << bm.SITE_EXPERT_ID
+    finally:
+        gpu.set_gemm_mode(bm.GEMM_EXACT)
+        gpu.fault_clear()
+        sc.free()
+        for b in (xd, sel, wd, rd, y):
+            b.free()
+        L.free()
+
+
 @pytest.mark.parametrize("m,top_k", ((8, 3), (7, 3), (6, 3), (20, 1)))
 def test_rows_of_tokens_that_no_expert_takes_may_hold_anything(gpu, m, top_k):
     """A per-slot step of the automatic choice, in launches of its own (24 and 21 slots, 160 and 140 MB asked for) and in two: a row whose slots are all
