@@ -442,7 +442,7 @@ def bench_dsv3(args, bm, ora, threads):
     def step(i, which=("shared", "routed")):
         """The shared expert, then bm_moe_forward over the routed ones with the shared expert's rows as the added term
         ((routed sum + shared), the reference's grouping): at this shape its grouped path, which for so few slots an expert is
-        the table, the per-slot gate . up launch from the token rows, the quantizer of h, the down tiles and the slot sum."""
+        the columns quantized once, gate . up slot by slot, the quantizer of h, down slot by slot and the slot sum."""
         st = i % sets
         s_ptr, x_ptr = sel.ptr + 4 * st * n_slots, xd.ptr + 4 * st * m * hidden
         if "shared" in which:

@@ -940,10 +940,12 @@ int bm_scratch_create(bm_ctx *ctx, int gate_type, int down_type, int hidden, int
     // the per-slot step below 22 tokens (Q4_K gate/up, Q6_K down, top-8 of 128, hidden 2048, ff 768, us a step, per slot / grouped:
     // 16 tokens 63 / 81, 24: 85 / 84, 128: 328 / 177), then by path_choice
     s->path = BM_PATH_AUTO, s->grouped_from = 22, s->gemm_from = 0;
-    // Where both stacks are on Q8_K columns and the experts are large, the grouped step (slot by slot at few slots, see slot_by_slot) is ahead of the
-    // per-slot step from the first token: every workgroup of the per-slot down launch encodes all of a token's h rows itself, work that grows
-    // with hidden x ff (DeepSeek-V3 shape, hidden 7168, ff 2048, IQ2_XXS, us a step per slot / grouped: 1 token 61.5 / 57.9, 4 tokens 171 /
-    // 147, 16 tokens 589 / 481; at hidden 2048, ff 768 the per-slot step leads up to 12 tokens: 1 token 16.0 / 23.7)
+    // Where both stacks are on Q8_K columns and the experts are large, the grouped path (slot by slot at few slots, see slot_by_slot; the tiles and
+    // the GEMM where an expert has many) stands from the first token: every workgroup of the per-slot down launch encodes all of a token's h rows
+    // itself, work that grows with hidden x ff (DeepSeek-V3 shape, hidden 7168, ff 2048, IQ2_XXS, us a step per slot / as chosen: 1 token 36.8 / 39.9,
+    // 2 tokens 66.7 / 63.6, 4 tokens 128 / 112, 16 tokens 454 / 394; 1500 random layers of 2^23 weights and more, 1 to 4 tokens, per slot over
+    // as chosen by the MB of rows asked for: 0.93 to 64, 0.97 to 128, 0.99 to 256, 1.02 beyond and up to 1.47. At hidden 2048, ff 768 the per-slot step leads up to 12
+    // tokens: 1 token 14.2 / 18.2 grouped, 8 tokens 34.2 / 37.4, 12 tokens 48.0 / 47.1.)
     if (act_form(gate_type) != 0 && act_form(down_type) != 0 && (int64_t)hidden * ff >= ((int64_t)1 << 23)) s->grouped_from = 1;
     const size_t slots = (size_t)max_tokens * n_slots_per_token;
     int rc = bm_act_create(ctx, gate_type, hidden, max_tokens, &s->act_x);

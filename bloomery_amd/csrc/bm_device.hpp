@@ -702,9 +702,8 @@ struct Iq2Tables {
 // lookups of a table that lies there once come about three deep: two thirds of the tables' LDS time. Larger workgroups hold the grid in copies,
 // an entry's 256 bytes apart from the next one's and each lane's on banks of its own. That leaves LDS time for entries of sixteen bytes
 // where a code is then one instruction less, and makes an entry's address one byte permute of the index and the lane's copy.
-// (Gate . up of IQ2_XXS, 2048 rows of 7168, 32 slots: LDS 87 % busy with the tables as they are, 46 % in copies, the launch 71 us against 69: what is left
-// is memory, whose rate for rows read 66 bytes at a time from sixteen places is 4.2 TB/s where the same bytes in order come at 5.6. IQ3_XXS, 768
-// rows of 2048, 40 slots: 17.4 against 15.5.)
+// (Gate . up of IQ2_XXS, 2048 rows of 7168: bank conflicts 38 % of the cycles with the tables as they are, 25 % in copies, 2.14 and 2.05 us a slot; LDS 70
+// and 72 % busy, since a copy's entry is twice the bytes, the vector ALU 84 and 81 %. IQ3_XXS, 768 rows of 2048, 40 slots: 17.4 against 15.5 us.)
 template <int WT, bool WIDE>
 struct IqGeom {
     static constexpr int kEntry = WIDE && WT == BM_IQ2XXS ? 16 : 8;

@@ -188,10 +188,10 @@ __device__ __forceinline__ bool tile_checked(Tile *t, u32 n_slots, u32 *fault, u
     return true;
 }
 
-// A tile's activation columns into LDS, column c from `from(c)`. All of them are asked for at once, 4096 bytes of each at a time: column after
-// column, eight bytes a thread, is sixteen round trips for eight columns of 2048 values. (Median and least us a launch, 64 tokens, top-8 of 128
-// experts of 768 x 2048: gate . up Q5_K 85.9, 77.0 -> 82.8, 73.3; down Q6_K 50.9, 47.0 -> 51.4, 45.8; forty random layers of 20 to 160 tokens
-// 0.963 to 1.011 of their time, those on tiles 0.98 on average.)
+// A gate . up tile's activation columns into LDS, column c from `from(c)`. All of them are asked for at once, 4096 bytes of each at a time: column
+// after column, eight bytes a thread, is sixteen round trips for eight columns of 2048 values. (Median and least us a launch, 64 tokens, top-8 of 128
+// experts of 768 x 2048, Q5_K: 85.9, 77.0 -> 82.8, 73.3. With the down tiles, whose columns are one run: forty random layers of 20 to 160 tokens 0.963 to
+// 1.011 of their time, those on tiles 0.98 on average.)
 template <int MC, class From>
 __device__ __forceinline__ void stage_tile_cols(uint8_t *cols, int col_bytes, int mc, const From &from) {
     for (int base = 0; base < col_bytes; base += 16 * 256) {
