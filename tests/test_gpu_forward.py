@@ -93,9 +93,10 @@ def test_every_path_gives_the_oracles_bits(gpu, types, hidden, ff, n_experts, to
 
 @pytest.mark.parametrize("m", (19, 20))
 def test_per_slot_step_on_either_side_of_its_own_launches(gpu, m):
-    """Stacks on Q8_K columns whose rows are 10 MB an expert: 20 slots ask for 200 MB, from where the per-slot step of a slot a token quantizes its
-    columns in launches of their own. One slot is served elsewhere and one names no expert; neither adds anything."""
-    hidden, ff, n_experts, top_k = 2048, 3072, 8, 1
+    """Stacks on Q8_K columns whose rows are 6.7 MB an expert: 20 slots ask for 128 MB, from where the per-slot step quantizes its columns in
+    launches of their own with three slots a token and more (with one, as here, from 200 MB: test_a_forced_path_takes_its_own_launches). One
+    slot is served elsewhere and one names no expert; neither adds anything."""
+    hidden, ff, n_experts, top_k = 2048, 2048, 8, 1
     L = Layer(gpu, (bm.IQ4_XS, bm.IQ4_XS, bm.IQ4_XS), hidden, ff, n_experts, 5200, cheap=True)
     rng = np.random.default_rng(5201)
     x, resid = normal_f32(rng, (m, hidden)), normal_f32(rng, (m, hidden))
