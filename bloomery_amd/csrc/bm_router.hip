@@ -213,8 +213,10 @@ __device__ __forceinline__ void places_clear(PickLds<PER> &L) {
 // Not every entry is compared with every other (128 of them: a quarter of it a wave, over LDS, took 0.9 us, and the rounds are a
 // chain of eighty dependent instructions each): an entry below `used` + 1 others' maxima cannot be among the first, so the maxima of
 // sixteen groups of lanes (of 32 for sixteen picks and more, of the 64 lanes for more still) give a bound that about as many entries pass as are
-// wanted; those go to LDS, a lane each, and are compared with one another. A group costs a step of the count: of sixteen picks of 128 experts 4.1 us
-// a k_route_softmax with 64 groups, 3.4 with 32. With no more than half again as many groups as picks too many entries pass (31 of 32 groups: the
+// wanted; those go to LDS, a lane each, and are compared with one another. A group costs a step of the count: of sixteen picks of 128 experts 4.2 us
+// a k_route_softmax with 64 groups, 3.8 with 32. (Counts of 32 and 64 are one loop: as code of its own, which fewer picks jump over, the count of 32 made
+// eight picks' k_route_softmax 5.0 -> 5.1 us and k_norm_route of 4 tokens x 256 experts x 7168 values 11.6 -> 12.4 where other launches stand between:
+// instructions come from memory in order.) With no more than half again as many groups as picks too many entries pass (31 of 32 groups: the
 // list overflows, 256 experts 5.3 -> 13.7 us; 24 of 32 past 256 experts 8.3 -> 17.6).
 template <int PER>
 __device__ __forceinline__ void places_by_counting(const float (&v)[PER], u32 n_exp, u32 used, PickLds<PER> &L) {
@@ -229,13 +231,13 @@ __device__ __forceinline__ void places_by_counting(const float (&v)[PER], u32 n_
         top = fmaxf(top, bm_dppf<kDppXor2>(top));
 #pragma unroll
         for (u32 g = 0; g < 64; g += 4) count_group(g);
-    } else if (used < (PER <= 4 ? 24u : 20u)) {
-        top = fmaxf(top, bm_dppf<kDppXor1>(top));
-#pragma unroll
-        for (u32 g = 0; g < 64; g += 2) count_group(g);
     } else {
-#pragma unroll 16
-        for (u32 g = 0; g < 64; g++) count_group(g);
+        const u32 lanes = used < (PER <= 4 ? 24u : 20u) ? 2 : 1;
+        const float pair = fmaxf(top, bm_dppf<kDppXor1>(top));
+        if (lanes == 2) top = pair;
+        for (u32 g0 = 0; g0 < 64; g0 += 16 * lanes)
+#pragma unroll
+            for (u32 g = 0; g < 16; g++) count_group(g0 + g * lanes);
     }
     // the maximum with `used` above it: no entry below it is wanted (none, where maxima are equal or fewer: then every entry may be)
     const unsigned long long bound_at = __ballot(above == used);
@@ -297,7 +299,8 @@ __device__ __forceinline__ bool picks_from_places(const PickLds<PER> &L, u32 t, 
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // One wave a token. One or two picks (one, past 256 experts) go by the rounds: counting takes as long whatever their number (us a launch by rounds / by
-// counting, 64 tokens and fewer: one pick of 128 experts 2.8 / 3.3, of 256 3.2 / 3.7; two 2.9 / 3.2, 3.6 / 3.7; two of 590 7.1 / 6.6).
+// counting, 64 tokens and fewer: one pick of 128 experts 2.8 / 3.3, of 256 3.2 / 3.7; two 2.9 / 3.2, 3.6 / 3.7; two of 590 7.1 / 6.6). One copy of the
+// rounds serves them and the ties.
 template <int PER>
 __global__ __launch_bounds__(256) void k_route_softmax(const float *logits, u32 n_tok, u32 n_exp, u32 used, u32 renorm,
                                                        float *probs, u32 *ids, float *weights, u32 *fault, u32 layer) {
@@ -312,18 +315,16 @@ __global__ __launch_bounds__(256) void k_route_softmax(const float *logits, u32 
         v[j] = e < n_exp ? logits[(size_t)t * n_exp + e] : -INFINITY;
     }
     if (!logits_finite<PER>(v, n_exp)) return route_refuse(t, n_exp, used, probs, weights, fault, layer);
-    if (used <= (PER <= 4 ? 2u : 1u)) {
-        route_probs_wave<PER>(v, n_exp, p);
-        store_probs<PER>(p, t, n_exp, probs);
-        return route_pick_rounds<PER>(p, t, n_exp, used, renorm, ids, weights);
-    }
     places_clear(L);
     route_probs_wave<PER>(v, n_exp, p);
     store_probs<PER>(p, t, n_exp, probs);
+    if (used > (PER <= 4 ? 2u : 1u)) {
 #pragma unroll
-    for (int j = 0; j < PER; j++) L.p[(threadIdx.x & 63) + 64 * j] = p[j];
-    places_by_counting<PER>(p, n_exp, used, L);
-    if (!picks_from_places(L, t, n_exp, used, renorm, ids, weights)) route_pick_rounds<PER>(p, t, n_exp, used, renorm, ids, weights);
+        for (int j = 0; j < PER; j++) L.p[(threadIdx.x & 63) + 64 * j] = p[j];
+        places_by_counting<PER>(p, n_exp, used, L);
+        if (picks_from_places(L, t, n_exp, used, renorm, ids, weights)) return;
+    }
+    route_pick_rounds<PER>(p, t, n_exp, used, renorm, ids, weights);
 }
 
 hipError_t route_softmax(const Launch &L, const float *logits, int n_tok, int n_exp, int used, int renorm, float *probs,
@@ -1004,6 +1005,8 @@ static RouterForm router_form(int m, int n_exp, int hidden) {
 }
 
 // Calls f with the form's rows and tokens and the pieces of a row a thread holds as constants.
+// (The order is the kernels' order in the library: the forms of whole rows together, in front. k_norm_route of 4 tokens x 256 experts x 7168 values among
+// a layer's other launches, us: 12.2 behind the ragged forms' kernels, 11.4 in front of them.)
 template <class F>
 static hipError_t with_form(RouterForm form, int hidden, F f) {
     using std::integral_constant;
@@ -1011,12 +1014,15 @@ static hipError_t with_form(RouterForm form, int hidden, F f) {
     constexpr integral_constant<int, 2> two{};
     constexpr integral_constant<int, 4> four{};
     auto tokens = [&](auto n4) { return form == kForm1x1 ? f(one, one, n4) : form == kForm4x1 ? f(four, one, n4) : f(four, two, n4); };
-    if (hidden % 256 != 0 && hidden <= 2048) return tokens(integral_constant<int, -2>{});
-    if (hidden % 256 != 0 && hidden <= 4096) return tokens(integral_constant<int, -4>{});
-    if (hidden % 256 != 0 || hidden > 8192) return tokens(integral_constant<int, 0>{});
-    if (hidden > 4096) return tokens(integral_constant<int, 8>{});
-    if (hidden > 2048) return tokens(four);
-    return hidden > 1024 ? tokens(two) : tokens(one);
+    if (hidden % 256 == 0) {
+        if (hidden <= 1024) return tokens(one);
+        if (hidden <= 2048) return tokens(two);
+        if (hidden <= 4096) return tokens(four);
+        if (hidden <= 8192) return tokens(integral_constant<int, 8>{});
+    }
+    if (hidden <= 2048) return tokens(integral_constant<int, -2>{});
+    if (hidden <= 4096) return tokens(integral_constant<int, -4>{});
+    return tokens(integral_constant<int, 0>{});
 }
 
 // Whether the norm and the logits go as two launches, rows and then tiles: by workgroups of four rows, from the later the shorter the rows, whose
